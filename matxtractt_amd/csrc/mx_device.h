@@ -177,6 +177,33 @@ constexpr int kSliceChunkCost = 2;     // what ending a chunk costs a wave, in s
 inline int slice_step_entries(mx_dtype) { return 1; }  // entries a lane takes per step; chunks end between steps
 constexpr int kSliceLightSegs = 8;     // rows with at most this many virtual rows are summed by one lane
 
+// The CSR part of a matrix whose rows repeat a pattern of column offsets (a stencil, a few diagonals):
+// chunks of 64 * R consecutive rows (R = 2 binary64, 4 binary16), one per wave, each with the ascending
+// list of the offsets (column - row) that its rows have.  Per chunk and unit -- unitBytes per lane, one
+// contiguous stretch per wave -- the values of U offsets for the R rows of every lane; a place that no
+// entry owns holds -0.0 (any binary64 whose upper half is 0x80000000) or code 255.
+struct DeviceOffsets {
+    int rows = 0, cols = 0, nnz = 0, nChunks = 0;
+    int units = 0, unitBytes = 0;  // units of all chunks; bytes per lane and unit (16 of values, 8 of codes)
+    long long nOffs = 0;
+    int *chunk = nullptr;    // [nChunks][4] {first unit, first offset, units, flags: 1 = reaches outside x, 2 = reaches past the last row}
+    int *offs = nullptr;     // [nOffs] U per unit, the last of a chunk repeated up to whole units
+    void *stream = nullptr;  // [units][64] unitBytes each
+    void *dict = nullptr;    // [256] values, when the units hold codes
+    int nDict = 0;
+    bool keep = false;       // the units are read with plain loads (they may stay in the caches), not streamed
+};
+constexpr int kOffsetsMost = 64;           // most offsets of a chunk
+constexpr int kOffsetsRowsLeast = 1024;    // fewest rows of a matrix that takes the form
+constexpr double kOffsetsFill = 1.2;       // most places per entry: 9.6 bytes per binary64 entry, as much as with a column offset of two bytes
+constexpr int offsets_unit_bytes(bool dict) { return dict ? 8 : 16; }
+void free_offsets(DeviceOffsets &D);
+// Lays the matrix out in this form if it suits it (D.nChunks > 0 then); otherwise D stays empty and MX_OK is returned.
+// (weak: a host-only link of the library's C++ files has no device code to call)
+__attribute__((weak)) int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev,
+                                               const void *val_dev, DeviceOffsets &D, hipStream_t s);
+__attribute__((weak)) hipError_t launch_offsets(mx_dtype dtype, const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s);
+
 // The sums of the virtual rows (DeviceSlices::partial) of mx_spmv_static live in a fixed array
 // in device memory instead of the plan's own buffer: static_scratch gives the address of the
 // current device's copy (looked up once per device, no allocation).
@@ -227,6 +254,12 @@ constexpr int kSlicePadSteps = 16;  // spare zero steps after the last of the st
 int build_slices_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev, const void *val_dev,
                         int nCU, int S, const char *elsewhere_dev, DeviceSlices &D, hipStream_t s, std::vector<int> *segPtrOut = nullptr,
                         std::vector<int> *segIdxOut = nullptr, int fused = 0);
+
+// The value dictionary of a matrix in device memory, as make_value_dict gives it on the host: at most `most`
+// distinct bit patterns, numbered in the order of their first entry.  *codes = nnz bytes in device memory (the
+// caller releases them; null when the matrix has more values), dict = 256 values in host memory, zero-padded.
+int value_dict_device(mx_dtype dtype, const void *val_dev, int nnz, int most, void **codes, std::vector<unsigned char> &dict, int *nDict,
+                      hipStream_t s);
 
 // For plans made from a matrix that lives in device memory: the caller's arrays looked at before
 // they are used as addresses; the mean number of distinct lines of x per wave-wide gather (sampled
