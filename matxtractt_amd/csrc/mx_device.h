@@ -194,8 +194,13 @@ struct DeviceOffsets {
     bool keep = false;       // the units are read with plain loads (they may stay in the caches), not streamed
 };
 constexpr int kOffsetsMost = 64;           // most offsets of a chunk
-constexpr int kOffsetsRowsLeast = 1024;    // fewest rows of a matrix that takes the form
+constexpr int kOffsetsRowsLeast = 1024;    // fewest rows of a matrix that takes the form (2431 rows: 3.3 us, row tiles 3.3)
 constexpr double kOffsetsFill = 1.2;       // most places per entry: 9.6 bytes per binary64 entry, as much as with a column offset of two bytes
+// What a product may touch for its units to be read with plain loads.  Plain / streaming loads, us, back to back | three
+// plans in turn: 67 MB 11.9 / 12.2 | 11.8 / 13.1; 98 MB 15.6 / 16.7 | 17.4 / 17.6; 142 MB 21.3 / 23.0 | 28.8 / 25.1;
+// 166 MB 24.2 / 26.8 | 32.3 / 28.7: from half of the memory-side cache on, anything else a program touches costs more
+// than staying there gives.
+constexpr long long kOffsetsKeepBytes = 128LL << 20;
 constexpr int offsets_unit_bytes(bool dict) { return dict ? 8 : 16; }
 void free_offsets(DeviceOffsets &D);
 // Lays the matrix out in this form if it suits it (D.nChunks > 0 then); otherwise D stays empty and MX_OK is returned.

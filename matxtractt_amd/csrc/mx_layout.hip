@@ -539,6 +539,17 @@ static int device_value_dict(const V *val, int nnz, mxl::Buf &codes, std::vector
     return MX_OK;
 }
 
+int value_dict_device(mx_dtype dtype, const void *val_dev, int nnz, int most, void **codes, std::vector<unsigned char> &dict, int *nDict,
+                      hipStream_t s)
+{
+    mxl::Buf c;
+    *codes = nullptr;
+    const int rc = dtype == MX_F64 ? device_value_dict<double>((const double *)val_dev, nnz, c, dict, nDict, s, most)
+                                   : device_value_dict<_Float16>((const _Float16 *)val_dev, nnz, c, dict, nDict, s, most);
+    if (rc == MX_OK) *codes = c.take();
+    return rc;
+}
+
 template <typename V>
 static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr, const int *col, const V *val, int nCU,
                                  int S, const char *elsewhere, DeviceSlices &D, hipStream_t s, std::vector<int> *segPtrOut,

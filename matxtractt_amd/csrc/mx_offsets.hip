@@ -79,15 +79,20 @@ __device__ __forceinline__ void unit_add(const typename Form<VT, DICT>::Unit &u,
         }
 }
 
-// One wave per chunk of 64 * R consecutive rows, R of them per lane.  Per unit (16 bytes of values per
-// lane, 8 bytes of codes) a lane reads its values -- the wave one contiguous stretch -- and for each of
-// the unit's offsets R consecutive x, again contiguous across the wave; the offsets are the same for
-// all lanes (scalar loads).  No column ids, no LDS, no cross-lane traffic; y is written once, in order.
-// What bounds it is the stream of values.  Units are taken eight offsets' worth at a time, all loads
-// of a round ahead of its sums; the remainder in halves, so that nothing is loaded twice.
+// A chunk is 64 * R consecutive rows, R of them per lane, and W waves share one: each takes a contiguous
+// part of its units, and with W > 1 the parts are added up through LDS in the order of the waves.  Per unit
+// (16 bytes of values per lane, 8 bytes of codes) a lane reads its values -- the wave one contiguous
+// stretch -- and for each of the unit's offsets R consecutive x, again contiguous across the wave; the
+// offsets are the same for all lanes (scalar loads).  No column ids, no cross-lane traffic; y is written
+// once, in order.  What bounds it is the stream of values (275.9 MB a product in 48.3 us, 5.7 TB/s; 17.4 MB that stay
+// in the caches in 6.0), or on small matrices the trips to memory of a wave: a round takes eight offsets' worth (four at the end if that is enough), all of its loads ahead of its
+// sums; a place beyond the wave's last unit reads that unit again and counts as "no entry".
 // A chunk whose offsets reach outside x for some row (flag 1) or past the last row (flag 2) takes the
 // form with every column clamped.
-template <typename VT, bool DICT, bool KEEP>
+// Measured against the forms these matrices had before, three plans in turn (us): 27 points, 18.9 million binary64
+// entries of their own value 28.6, row tiles 47.0; 26.5 million with two values 13.7, slices with one byte per value
+// 35.7; 31.6 million binary16 12.7, slices 38.3; 56 thousand binary64 3.3, row tiles 3.3.
+template <typename VT, bool DICT, bool KEEP, int W>
 __global__ __launch_bounds__(kBlock) void csr_offsets_kernel(const int4 *__restrict__ chunk, const int *__restrict__ offs,
                                                              const void *__restrict__ stream, const VT *__restrict__ dictG,
                                                              const VT *__restrict__ x, VT *__restrict__ y, int rows, int cols,
@@ -96,64 +101,71 @@ __global__ __launch_bounds__(kBlock) void csr_offsets_kernel(const int4 *__restr
     typedef Form<VT, DICT> F;
     typedef typename F::AT AT;
     typedef typename F::Unit Unit;
-    constexpr int R = F::R, U = F::U;
+    constexpr int R = F::R, U = F::U, WAVES = kBlock / 64;
     __shared__ AT dictL[DICT ? 256 : 1];
-    const int waves = blockDim.x >> 6;
+    __shared__ AT part[W > 1 ? WAVES : 1][W > 1 ? 64 * R : 1];
     if constexpr (DICT) {
-        for (int i = threadIdx.x; i < 256; i += blockDim.x) dictL[i] = (AT)dictG[i];
+        dictL[threadIdx.x] = (AT)dictG[threadIdx.x];
         __syncthreads();
     }
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), w = wave % W;
     // every XCD walks one contiguous range of chunks: the x of neighbouring chunks lives in one L2
     const int q = gridDim.x >> 3, rem = gridDim.x & 7, xcd = blockIdx.x & 7;
     const int block = xcd * q + min(xcd, rem) + (int)(blockIdx.x >> 3);
-    const int c = __builtin_amdgcn_readfirstlane(block * waves + (int)(threadIdx.x >> 6));
-    if (c >= nChunks) return;
-    const int4 d = chunk[c];
-    const int nUnits = __builtin_amdgcn_readfirstlane(d.z), flags = __builtin_amdgcn_readfirstlane(d.w);
-    const Unit *su = (const Unit *)stream + (size_t)__builtin_amdgcn_readfirstlane(d.x) * 64 + lane;
-    const int *of = offs + __builtin_amdgcn_readfirstlane(d.y);
+    const int c = block * (WAVES / W) + wave / W;
+    const bool live = c < nChunks;
+    const int4 d = chunk[live ? c : nChunks - 1];
+    const int all = __builtin_amdgcn_readfirstlane(d.z), flags = __builtin_amdgcn_readfirstlane(d.w), share = (all + W - 1) / W;
+    const int u0 = min(w * share, all), nUnits = live ? min(share, all - u0) : 0;  // this wave's part
+    // (a scalar base and a 32-bit offset per lane: the address of a load costs no vector registers)
+    const unsigned char *su = (const unsigned char *)stream + ((size_t)__builtin_amdgcn_readfirstlane(d.x) + u0) * (64 * F::kUnitBytes);
+    const int *of = offs + __builtin_amdgcn_readfirstlane(d.y) + u0 * U;
+    const unsigned suLane = (unsigned)lane * F::kUnitBytes, xLane = (unsigned)lane * (R * (unsigned)sizeof(VT));
     const int r0 = c * F::kRows + R * lane;
     AT acc[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) acc[i] = 0;
     if (flags == 0) {
-        const VT *xr = x + r0;
-        auto round = [&](int u0, auto n) {  // `n` units from u0 on
+        const VT *xc = x + (size_t)c * F::kRows;
+        auto round = [&](int u, auto n, auto masked) {  // `n` units from u on
             constexpr int N = decltype(n)::value;
+            constexpr bool MASK = decltype(masked)::value;
             Unit v[N];
             VT xv[N][U][R];
 #pragma unroll
-            for (int k = 0; k < N; ++k) v[k] = unit_load<KEEP>(su + (size_t)(u0 + k) * 64);
+            for (int k = 0; k < N; ++k) {
+                const int at = MASK ? min(u + k, nUnits - 1) : u + k;
+                v[k] = unit_load<KEEP>((const Unit *)(su + (size_t)at * (64 * F::kUnitBytes) + suLane));
+            }
 #pragma unroll
             for (int k = 0; k < N; ++k)
 #pragma unroll
                 for (int j = 0; j < U; ++j) {
-                    const typename F::XV t = *(const typename F::XV *)(xr + of[(u0 + k) * U + j]);
+                    const int at = MASK ? min(u + k, nUnits - 1) : u + k;
+                    const typename F::XV t = *(const typename F::XV *)((const unsigned char *)(xc + of[at * U + j]) + xLane);
 #pragma unroll
                     for (int i = 0; i < R; ++i) xv[k][j][i] = t[i];
                 }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int k = 0; k < N; ++k) unit_add<VT, DICT>(v[k], xv[k], acc, dictL);
+            for (int k = 0; k < N; ++k) {
+                if (MASK && u + k >= nUnits) {
+#pragma unroll
+                    for (int i = 0; i < F::kUnitBytes / 4; ++i) v[k][i] = DICT ? -1 : sizeof(VT) == 8 ? (int)0x80000000 : (int)0x80008000;
+                }
+                unit_add<VT, DICT>(v[k], xv[k], acc, dictL);
+            }
         };
         constexpr int N = 8 / U;
         int u = 0;
-        for (; u + N <= nUnits; u += N) round(u, std::integral_constant<int, N>());
-        if constexpr (N >= 8)
-            if ((nUnits - u) & 4) {
-                round(u, std::integral_constant<int, 4>());
-                u += 4;
-            }
-        if constexpr (N >= 4)
-            if ((nUnits - u) & 2) {
-                round(u, std::integral_constant<int, 2>());
-                u += 2;
-            }
-        if constexpr (N >= 2)
-            if ((nUnits - u) & 1) round(u, std::integral_constant<int, 1>());
+        for (; u + N <= nUnits; u += N) round(u, std::integral_constant<int, N>(), std::false_type());
+        if (u < nUnits) {
+            if (N > 1 && nUnits - u <= N / 2) round(u, std::integral_constant<int, (N > 1 ? N / 2 : 1)>(), std::true_type());
+            else round(u, std::integral_constant<int, N>(), std::true_type());
+        }
     } else {
         for (int u = 0; u < nUnits; ++u) {
-            const Unit v = unit_load<KEEP>(su + (size_t)u * 64);
+            const Unit v = unit_load<KEEP>((const Unit *)(su + (size_t)u * (64 * F::kUnitBytes) + suLane));
             VT xv[U][R];
 #pragma unroll
             for (int j = 0; j < U; ++j) {
@@ -164,6 +176,17 @@ __global__ __launch_bounds__(kBlock) void csr_offsets_kernel(const int4 *__restr
             unit_add<VT, DICT>(v, xv, acc, dictL);
         }
     }
+    if constexpr (W > 1) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) part[wave][i * 64 + lane] = acc[i];
+        __syncthreads();
+        if (w != 0) return;
+#pragma unroll
+        for (int k = 1; k < W; ++k)
+#pragma unroll
+            for (int i = 0; i < R; ++i) acc[i] += part[wave + k][i * 64 + lane];
+    }
+    if (!live) return;
     if (r0 + R <= rows && !accumulate) {
         typename F::XV t;
 #pragma unroll
@@ -450,13 +473,12 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     return MX_OK;
 }
 
-template <typename VT>
+template <typename VT, int W>
 static hipError_t launch_offsets_t(const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s)
 {
-    // (few chunks: a wave per workgroup, so that they spread over all CUs)
-    const int waves = D.nChunks < 2048 ? 1 : 4, wgs = (D.nChunks + waves - 1) / waves;
+    const int perWG = mxo::kBlock / 64 / W, wgs = (D.nChunks + perWG - 1) / perWG;
 #define MX_LAUNCH_OFFSETS(DICT, KEEP)                                                                                                    \
-    hipLaunchKernelGGL((mxo::csr_offsets_kernel<VT, DICT, KEEP>), dim3(wgs), dim3(64 * waves), 0, s, (const int4 *)D.chunk, D.offs,       \
+    hipLaunchKernelGGL((mxo::csr_offsets_kernel<VT, DICT, KEEP, W>), dim3(wgs), dim3(mxo::kBlock), 0, s, (const int4 *)D.chunk, D.offs,    \
                        (const void *)D.stream, (const VT *)D.dict, (const VT *)x, (VT *)y, D.rows, D.cols, D.nChunks, accumulate)
     if (D.nDict > 0 && D.keep) MX_LAUNCH_OFFSETS(true, true);
     else if (D.nDict > 0) MX_LAUNCH_OFFSETS(true, false);
@@ -468,7 +490,13 @@ static hipError_t launch_offsets_t(const DeviceOffsets &D, const void *x, void *
 hipError_t launch_offsets(mx_dtype dtype, const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s)
 {
     if (D.nChunks <= 0) return hipSuccess;
-    return dtype == MX_F64 ? launch_offsets_t<double>(D, x, y, accumulate, s) : launch_offsets_t<_Float16>(D, x, y, accumulate, s);
+    // Four waves a chunk: a wave's trips to memory are fewer and more of them are in flight on a matrix of few chunks
+    // (one / two / four waves, us, binary64: 22 thousand rows 6.3 / 4.2 / 3.2; 717 thousand 33.1 / 31.2 / 28.6; 1.2 million
+    // 52.9 / 51.3 / 48.3).  With one byte per binary64 value the kernel is bound by what a wave computes and the sum of
+    // the parts costs more than it gives from about two thousand chunks on (290 thousand rows 6.5 / 6.1 / 6.4, 717
+    // thousand 10.9 / 10.5 / 11.7, a million 13.1 / 13.7 / 14.8).
+    if (dtype == MX_F16) return launch_offsets_t<_Float16, 4>(D, x, y, accumulate, s);
+    return D.nDict > 0 && D.nChunks >= 2048 ? launch_offsets_t<double, 2>(D, x, y, accumulate, s) : launch_offsets_t<double, 4>(D, x, y, accumulate, s);
 }
 
 }  // namespace mx

@@ -28,11 +28,21 @@ extern "C" int mx_device_count(void)
     return n;
 }
 
+void mx::free_offsets(mx::DeviceOffsets &D)
+{
+    (void)hipFree(D.chunk);
+    (void)hipFree(D.offs);
+    (void)hipFree(D.stream);
+    (void)hipFree(D.dict);
+    D = mx::DeviceOffsets();
+}
+
 extern "C" void mx_plan_destroy(mx_plan *plan)
 {
     if (!plan) return;
     free_csr(plan->csr);
     free_slices(plan->slices);
+    mx::free_offsets(plan->offsets);
     free_tiles(plan->tiles);
     free_tiles(plan->strips);
     (void)hipFree(plan->ywide);
@@ -45,7 +55,7 @@ extern "C" void mx_plan_destroy(mx_plan *plan)
 // Bytes of the sums of a plan's virtual rows (what upload_slices allocates for them).
 size_t mxp::partial_bytes(const mx_plan *plan)
 {
-    if (plan->csr_variant == 0) return 0;
+    if (plan->csr_variant != 1 && plan->csr_variant != 2) return 0;
     return ((size_t)plan->slices.chunks * 64 + 64) * (plan->dtype == MX_F64 ? 8 : 4);
 }
 
@@ -207,8 +217,12 @@ double mxp::touched_bytes(const mx_plan *plan)
 {
     const double es = mx::elem_size(plan->dtype);
     double b = (double)plan->cols * es + (double)plan->rows * es;
-    if (plan->csr_variant != 1) b += (double)plan->csr.nnz * ((plan->csr.useDict ? 1.0 : es) + 4.0) + ((double)plan->rows + 1) * 4;
-    if (plan->csr_variant != 0) b += (double)slice_entry_bytes(plan) + (double)slice_handoff_bytes(plan) - (double)plan->rows * es;
+    if (plan->csr_variant == 3) {
+        const mx::DeviceOffsets &D = plan->offsets;
+        b += (double)D.units * 64 * D.unitBytes + (double)D.nOffs * 4 + (double)D.nChunks * 16;
+    }
+    if (plan->csr_variant == 0 || plan->csr_variant == 2) b += (double)plan->csr.nnz * ((plan->csr.useDict ? 1.0 : es) + 4.0) + ((double)plan->rows + 1) * 4;
+    if (plan->csr_variant == 1 || plan->csr_variant == 2) b += (double)slice_entry_bytes(plan) + (double)slice_handoff_bytes(plan) - (double)plan->rows * es;
     if (plan->tiles.steps)
         b += (double)plan->tiles.steps * (mx::kTileHdr * 4.0 + 64 * 4.0) + (double)plan->tiles.stored * es;
     if (plan->strips.steps) b += (double)plan->strips.steps * (mx::kTileHdr * 4.0) + (double)plan->strips.stored * es;
@@ -230,6 +244,13 @@ void mxp::decide_keep(mx_plan *plan, int flags)
 {
     mx::DeviceSlices &L = plan->slices;
     L.keep = false;
+    if (plan->csr_variant == 3) {
+        const int env = mx::opt().csr_keep;
+        if ((flags & MX_PLAN_STREAM) || env == 0) plan->offsets.keep = false;
+        else if ((flags & MX_PLAN_KEEP) || env == 1) plan->offsets.keep = true;
+        else plan->offsets.keep = touched_bytes(plan) <= (double)mx::kOffsetsKeepBytes;
+        return;
+    }
     if (plan->csr_variant == 0) return;
     const int env = mx::opt().csr_keep;
     if ((flags & MX_PLAN_STREAM) || env == 0) return;
@@ -268,6 +289,23 @@ CsrChoice mxp::choose_csr_form(mx_dtype dtype, int rows, int cols, const int *ro
     return c;
 }
 
+bool mxp::may_look_for_form(int flags)
+{
+    const mx::Options &o = mx::opt();
+    return !(flags & (MX_PLAN_CSR_ROWS | MX_PLAN_CSR_SLICES | MX_PLAN_FUSE)) && o.csr_kernel == 0 && o.csr_fused != 1 && !o.autotune;
+}
+int mxp::try_offsets(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took)
+{
+    *took = false;
+    const int rc = mx::build_offsets_device(plan->dtype, plan->rows, plan->cols, nnz, rowPtr_dev, colInd_dev, val_dev, plan->offsets, nullptr);
+    if (rc || plan->offsets.nChunks == 0) return rc;
+    plan->csr_variant = 3;
+    plan->csr_nnz = nnz;
+    decide_keep(plan, flags);
+    *took = true;
+    return MX_OK;
+}
+
 // Puts the CSR part on the device.  Three executable forms exist: row tiles with direct x
 // gathers; column slices with x resident in LDS; and a split in which the long rows (most of
 // the entries of a matrix with a heavy tail of row lengths) take the slices and the many short
@@ -281,13 +319,28 @@ CsrChoice mxp::choose_csr_form(mx_dtype dtype, int rows, int cols, const int *ro
 // `stripRows` (optional): rows that the strip form of the tile kernel writes (and the CSR part has
 // nothing for).
 // `segOut` (optional): receives the virtual rows of every matrix row when the slice form is taken.
+// `alone`: no tile form has a part in the product.
 int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const void *val, int flags, const char *stripRows,
-                        std::pair<std::vector<int>, std::vector<int>> *segOut)
+                        std::pair<std::vector<int>, std::vector<int>> *segOut, bool alone)
 {
     const int rows = plan->rows, cols = plan->cols;
     const int nnz = rowPtr[rows];
     const size_t es = (size_t)mx::elem_size(plan->dtype);
     plan->csr_nnz = nnz;
+    if (alone && may_look_for_form(flags)) {
+        // (the offset form is found and laid out on the device, whatever MX_LAYOUT says)
+        int *rp = nullptr, *ci = nullptr;
+        void *va = nullptr;
+        bool took = false;
+        int e = upload(&rp, rowPtr, (size_t)rows + 1);
+        if (!e) e = upload(&ci, col, (size_t)nnz);
+        if (!e) e = upload_bytes(&va, val, (size_t)nnz * es);
+        if (!e) e = try_offsets(plan, nnz, rp, ci, va, flags, &took);
+        (void)hipFree(rp);
+        (void)hipFree(ci);
+        (void)hipFree(va);
+        if (e || took) return e;
+    }
     hipDeviceProp_t prop;
     int dev = 0;
     MX_HIP(hipGetDevice(&dev));
@@ -908,7 +961,8 @@ static int create_plan(const mx_partition *P, int flags, mx_plan **out, bool noB
             const bool blocks64 = P->dtype == MX_F64 && !stripChunks.empty();
             std::pair<std::vector<int>, std::vector<int>> seg;  // virtual rows of every row (slice form)
             rc = setup_csr_part(plan, rowPtr.data(), col.data(), val.data(), flags, stripRows.empty() ? nullptr : stripRows.data(),
-                                blocks64 ? &seg : nullptr);
+                                blocks64 ? &seg : nullptr,
+                                stripChunks.empty() && std::find(sel.begin(), sel.end(), (char)1) == sel.end());
             if (rc) return fail(rc);
             phase("CSR part (layouts, trial)");
 

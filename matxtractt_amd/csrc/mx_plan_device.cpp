@@ -21,9 +21,10 @@ using namespace mxp;
 // The CSR part of a plan from arrays in device memory: the form is chosen as setup_csr_part chooses
 // it -- the same counts, taken on the device -- and only that form is built, there.  Nothing of the
 // matrix crosses to the host but its row pointers (for the row-tile form) or the lengths of its
-// chunks (for the slice form).  `elsewhere_dev` (optional): marks of rows that another kernel writes.
+// chunks (for the slice form).  `elsewhere_dev` (optional): marks of rows that another kernel writes; `alone`: no tile
+// form has a part in the product.
 static int setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags,
-                                 const char *elsewhere_dev, std::pair<std::vector<int>, std::vector<int>> *segOut = nullptr)
+                                 const char *elsewhere_dev, std::pair<std::vector<int>, std::vector<int>> *segOut = nullptr, bool alone = true)
 {
     const mx_dtype dtype = plan->dtype;
     const int rows = plan->rows, cols = plan->cols;
@@ -35,6 +36,11 @@ static int setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, 
     MX_HIP(hipGetDeviceProperties(&prop, dev));
     const int nCU = std::max(1, prop.multiProcessorCount);
     const int S = rows > 0 ? slice_count(dtype, rows, cols, nnz, nCU) : 0;
+    if (alone && may_look_for_form(flags)) {
+        bool took = false;
+        if ((rc = try_offsets(plan, nnz, rowPtr_dev, colInd_dev, val_dev, flags, &took))) return rc;
+        if (took) return MX_OK;
+    }
     bool want[2] = {true, S > 0};
     const int env = mx::opt().csr_kernel;
     if (env == 3 || plan_autotune()) {
@@ -443,7 +449,8 @@ int mxp::create_plan_device(mx_dtype dtype, int rows, int cols, int nnz, const i
         if ((rc = H.csr_part(keepStrips, keepGeneral, keepBlocks, &partPtr, &partCol, &partVal, &partNnz, &stripRows))) return fail(rc);
         phase("CSR part assembled (device)");
         std::pair<std::vector<int>, std::vector<int>> seg;  // virtual rows of every row (slice form), for the blocks
-        if ((rc = setup_csr_part_device(plan, partNnz, partPtr, partCol, partVal, flags, stripRows, keepBlocks ? &seg : nullptr)))
+        if ((rc = setup_csr_part_device(plan, partNnz, partPtr, partCol, partVal, flags, stripRows, keepBlocks ? &seg : nullptr,
+                                        !keepStrips && !keepGeneral && !keepBlocks)))
             return fail(rc);
         phase("CSR part layout (device)");
         if (keepBlocks && plan->csr_variant == 1) {

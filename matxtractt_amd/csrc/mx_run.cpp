@@ -50,6 +50,10 @@ extern "C" int mx_debug_fused_misplaced(int set)
 int mxp::launch_csr_part(mx_plan *plan, const void *x, void *y, int accumulate, hipStream_t s, const mx::DeviceTiles *strips, void *partial,
                          void *ywide)
 {
+    if (plan->csr_variant == 3) {
+        MX_HIP(mx::launch_offsets(plan->dtype, plan->offsets, x, y, accumulate, s));
+        return MX_OK;
+    }
     if (plan->csr_variant != 0 && ((uintptr_t)x & 15)) {
         set_error("mx_spmv: x must be 16-byte aligned for this plan");
         return MX_ERR_ARG;
@@ -100,7 +104,7 @@ int mxp::launch_csr_part(mx_plan *plan, const void *x, void *y, int accumulate, 
 static int check_x(const mx_plan *plan, const void *x, const char *who)
 {
     if (!((uintptr_t)x & 15)) return MX_OK;
-    if (plan->csr_variant != 0) {
+    if (plan->csr_variant == 1 || plan->csr_variant == 2) {
         set_error(std::string(who) + ": x must be 16-byte aligned for this plan (its CSR part keeps x in LDS)");
         return MX_ERR_ARG;
     }
@@ -210,7 +214,7 @@ extern "C" int mx_time_csr_main(mx_plan *plan, const void *x_dev, void *y_dev, i
     if (int bad = check_x(plan, x_dev, "mx_time_csr_main")) return bad;
     int rc = time_loop(plan, warm, iters, [&]() -> int {
         // the kernel that holds most of the entries
-        if (plan->csr_variant == 1 && plan->fused)
+        if (plan->csr_variant == 3 || (plan->csr_variant == 1 && plan->fused))
             return launch_csr_part(plan, x_dev, y_dev, 0, s);
         if (plan->csr_variant == 1 || (plan->csr_variant == 2 && plan->slices.nnz > plan->csr.nnz))
             MX_HIP(mx::launch_slices(plan->dtype, plan->slices, x_dev, y_dev, 0, s, 1));
@@ -349,7 +353,11 @@ extern "C" int mx_time_kernels(mx_plan *plan, const void *x_dev, void *y_dev, in
     };
     if ((rc = check_x(plan, x_dev, "mx_time_kernels"))) return rc;
     bool xCounted = false;
-    if (plan->csr_variant != 1 && plan->csr.nBlocks > 0) {
+    if (plan->csr_variant == 3)
+        add(std::string("csr_offsets_kernel<") + vt + (plan->offsets.nDict > 0 ? ",dict" : "") + (plan->offsets.keep ? ",keep>" : ">"),
+            (double)plan->csr_nnz * (es + 4) + xBytes + yBytes, plan->csr_nnz,
+            [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, 0, s); });
+    if (plan->csr_variant != 1 && plan->csr_variant != 3 && plan->csr.nBlocks > 0) {
         const bool last = plan->csr_variant == 0;  // writes y for good
         add(std::string("csr_rows_kernel<") + vt + (plan->csr.useDict ? ",dict>" : ">"),
             (double)plan->csr.nnz * (es + 4) + xBytes + (last ? yBytes : 0.0), plan->csr.nnz, [&]() -> int {
@@ -363,7 +371,7 @@ extern "C" int mx_time_kernels(mx_plan *plan, const void *x_dev, void *y_dev, in
         add(std::string("csr_slice_kernel<") + vt + (plan->slices.useDict ? ",dict" : "") + ",fused" + (plan->slices.keep ? ",keep>" : ">"),
             (double)plan->slices.nnz * (es + 4) + xBytes + yBytes, plan->slices.nnz,
             [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, 0, s, nullptr, nullptr, wide); });
-    } else if (plan->csr_variant != 0) {
+    } else if (plan->csr_variant == 1 || plan->csr_variant == 2) {
         add(std::string("csr_slice_kernel<") + vt + (plan->slices.useDict ? ",dict" : "") + (plan->slices.keep ? ",keep>" : ">"),
             (double)plan->slices.nnz * (es + 4) + (xCounted ? 0.0 : xBytes), plan->slices.nnz, [&]() -> int {
                 MX_HIP(mx::launch_slices(plan->dtype, plan->slices, x_dev, y_dev, 0, s, 1));

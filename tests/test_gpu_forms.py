@@ -1,26 +1,98 @@
 """GPU tests of the forms of the CSR part that a plan makes and picks on the device: value dictionaries,
 offset patterns, row windows.  Against the host's layouts where they exist, against the oracle otherwise."""
-import os
-import sys
-
 import numpy as np
 import pytest
 
-sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def mx():
-    import matxtractt_amd as m
-    assert m.device_count() > 0, "libmatxtract_hip.so sees no HIP device"
-    return m
+def _exact(ora, A, x):
+    """The oracle's y on integer data: the sums are exact in the accumulator (below 2^24), rounded once to the value type."""
+    y = ora.spmv_f64(A.val, A.rowPtr, A.colInd, x) if x.dtype == np.float64 else ora.spmv_f16_f32acc(A.val, A.rowPtr, A.colInd, x)[0]
+    return np.asarray(y).astype(x.dtype)
 
 
-@pytest.fixture(scope="module")
-def ora():
-    from oracle import mx_oracle
-    return mx_oracle
+def _diagonals(mx, rng, rows, cols, offs, dtype, few, holes=0.0):
+    """Rows with the column offsets `offs` where they lie inside the matrix, some of them missing; integer values."""
+    r = np.repeat(np.arange(rows), len(offs))
+    c = r + np.tile(offs, rows)
+    ok = (c >= 0) & (c < cols) & (rng.random(r.size) >= holes)
+    r, c = r[ok], c[ok]
+    ptr = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=rows))]).astype(np.int32)
+    val = rng.choice([-3, -1, 1, 2], r.size) if few else rng.integers(1, 400, r.size) * rng.choice([-1, 1], r.size)
+    return mx.Csr(rows, cols, ptr, c.astype(np.int32), val.astype(dtype))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float16])
+@pytest.mark.parametrize("few", [False, True])
+@pytest.mark.parametrize("rows,cols,offs", [
+    (1024, 1024, [0]),                                   # one offset, whole chunks
+    (1025, 1025, [-1, 0, 1]),                            # one row beyond them
+    (1151, 1300, [-130, -1, 0, 1, 130]),                 # more columns than rows
+    (5000, 3000, [-2500, -7, 3, 64]),                    # fewer: the last rows have few entries or none
+    (30011, 30011, list(range(-32, 32))),                # as many offsets as a chunk may have
+    (30011, 30011, list(range(-32, 33))),                # one more: another form takes the matrix
+    (40000, 40000, sorted({dx + 20 * (dy + 50 * dz) for dx in (-1, 0, 1) for dy in (-1, 0, 1) for dz in (-1, 0, 1)})),
+    (270000, 270000, [-700, -3, -2, 0, 2, 3, 700]),      # more than 2048 chunks of binary64 rows
+])
+def test_offset_form(mx, ora, dtype, few, rows, cols, offs):
+    """Matrices whose rows repeat a pattern of column offsets: the product from both routes equals the oracle's
+    (integers: every sum is exact), entries kept or streamed, over an old y and with every chunk's edges outside x; a
+    row's sum is not touched by an infinite x that the row does not name."""
+    import torch
+    rng = np.random.default_rng(rows + len(offs))
+    A = _diagonals(mx, rng, rows, cols, np.array(offs), dtype, few, holes=0.05 if len(offs) > 8 else 0.0)
+    small = few or dtype == np.float64
+    x = rng.integers(-2, 3, cols).astype(dtype) if small else rng.choice([-1, 0, 0, 0, 0, 0, 0, 0, 0, 1], cols).astype(dtype)
+    takes = len(offs) <= 64
+    xd = torch.from_numpy(x).cuda()
+    dev = [torch.from_numpy(a).cuda() for a in (A.rowPtr, A.colInd, A.val)]
+    ref = _exact(ora, A, x)
+    P = mx.Partition(A, 0.0, 0.0)
+    arrays = None
+    for plan in (mx.Plan(P), mx.Plan.from_device(*dev, cols, 0.0, 0.0), mx.Plan.from_device(*dev, cols, 0.0, 0.0, mx.MX_PLAN_STREAM)):
+        assert (plan.info["csr_variant"] == 3) == takes, plan.info
+        if takes:
+            assert (plan.info["csr_value_dict"] > 0) == (few and A.nnz >= 65536)
+            assert arrays is None or plan.arrays() == arrays
+            arrays = plan.arrays()
+        y = torch.full((rows,), 7.0, dtype=xd.dtype, device="cuda")
+        plan.spmv(xd, y)
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy(), ref)
+    bad = x.copy()
+    bad[[0, cols // 2, cols - 1]] = np.inf
+    touched = np.zeros(rows, bool)
+    touched[np.repeat(np.arange(rows), np.diff(A.rowPtr))[~np.isfinite(bad[A.colInd])]] = True
+    got = plan.spmv(torch.from_numpy(bad).cuda()).cpu().numpy()
+    assert np.array_equal(~np.isfinite(got), touched)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float16])
+@pytest.mark.parametrize("what", ["twice", "minus zero", "any order"])
+def test_matrices_the_offset_form_leaves_or_takes(mx, ora, dtype, what):
+    """A column named twice or a stored -0.0 sends the matrix to another form; rows in any order do not."""
+    import torch
+    rng = np.random.default_rng(8)
+    A = _diagonals(mx, rng, 4000, 4000, np.array([-50, -1, 0, 1, 50]), dtype, False)
+    ci, va = A.colInd.copy(), A.val.copy()
+    p = A.rowPtr[2000]
+    if what == "twice":
+        ci[p] = ci[p + 1]
+    elif what == "minus zero":
+        va[p] = -0.0
+    else:
+        for r in range(0, 4000, 3):
+            s = slice(A.rowPtr[r], A.rowPtr[r + 1])
+            o = rng.permutation(s.stop - s.start)
+            ci[s], va[s] = ci[s][o], va[s][o]
+    B = mx.Csr(4000, 4000, A.rowPtr, ci, va)
+    x = rng.integers(-1, 2, 4000).astype(dtype)
+    ref = _exact(ora, B, x)
+    plan = mx.Plan.from_device(*(torch.from_numpy(a).cuda() for a in (B.rowPtr, B.colInd, B.val)), 4000, 0.0, 0.0)
+    assert (plan.info["csr_variant"] == 3) == (what == "any order")
+    got = plan.spmv(torch.from_numpy(x).cuda()).cpu().numpy()
+    assert np.array_equal(got, ref)
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float16])
