@@ -175,6 +175,7 @@ SIGNATURES = {
     "mx_du_tcspmv_f64": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _pd]),
     "mx_du_tcspmv_f16": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _pd]),
     "mx_device_count": (_i, []),
+    "mx_release_memory": (None, []),
     "mx_probe_mfma_f64": (_i, [_vp, _vp, _vp]),
     "mx_probe_mfma_f16": (_i, [_vp, _vp, _vp]),
 }

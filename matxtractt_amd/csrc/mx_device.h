@@ -6,6 +6,33 @@
 
 namespace mx {
 
+// ---- device memory (mx_util.cpp).  Making a plan takes and gives back a hundred arrays, and hipMalloc and hipFree
+// of large ones cost more than the kernels that fill them (64 MB: 21 + 52 us in an idle process, several times that
+// beside other allocations).  dev_malloc and dev_free stand in for them and keep what was given back:
+//  * inside a MemScope -- one per entry point that works on a stream -- a freed block serves the thread's next
+//    request at once, in the order of that stream, and becomes anybody's when the scope ends, after the stream has
+//    been waited for;
+//  * inside IdleFrees, which waits for the device first, it is anybody's at once (plans that are destroyed: their
+//    streams are the callers');
+//  * elsewhere dev_free waits for the device, as hipFree does.
+// Idle blocks hold at most 1/128 of the device's memory, go back to the device after 64 calls in which nobody asked
+// for them, all of them when an allocation fails, and on mx_release_memory.
+hipError_t dev_malloc(void **out, size_t bytes);
+hipError_t dev_free(void *p);
+void release_idle_memory();
+struct MemScope {
+    explicit MemScope(hipStream_t s);
+    ~MemScope();
+    MemScope(const MemScope &) = delete;
+    MemScope &operator=(const MemScope &) = delete;
+};
+struct IdleFrees {
+    IdleFrees();
+    ~IdleFrees();
+    IdleFrees(const IdleFrees &) = delete;
+    IdleFrees &operator=(const IdleFrees &) = delete;
+};
+
 // CSR matrix resident on the device, plus the row ranges of the CSR kernel's workgroups.
 // col/val carry kCsrPad extra zero entries so that a wave's aligned 128-bit loads may overrun.
 struct DeviceCsr {

@@ -32,6 +32,21 @@ int need_device()
 }
 
 
+int compute_units(int *n)
+{
+    static std::atomic<int> known[64];
+    int dev = 0, cu = 0;
+    MX_HIP(hipGetDevice(&dev));
+    if (dev >= 0 && dev < 64 && (cu = known[dev].load()) > 0) {
+        *n = cu;
+        return MX_OK;
+    }
+    MX_HIP(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev));
+    *n = std::max(1, cu);
+    if (dev >= 0 && dev < 64) known[dev].store(*n);
+    return MX_OK;
+}
+
 int upload_bytes(void **dst, const void *src, size_t n, size_t pad)
 {
     return upload<unsigned char>((unsigned char **)dst, (const unsigned char *)src, n, pad);
@@ -60,48 +75,48 @@ void pack_rows(const int *rowPtr, int rows, int npt, std::vector<int> &desc)
 
 void free_csr(mx::DeviceCsr &A)
 {
-    (void)hipFree(A.rowPtr);
-    (void)hipFree(A.col);
-    (void)hipFree(A.col16);
-    (void)hipFree(A.colBase);
-    (void)hipFree(A.val);
-    (void)hipFree(A.codes);
-    (void)hipFree(A.dict);
-    (void)hipFree(A.blockDesc);
+    (void)mx::dev_free(A.rowPtr);
+    (void)mx::dev_free(A.col);
+    (void)mx::dev_free(A.col16);
+    (void)mx::dev_free(A.colBase);
+    (void)mx::dev_free(A.val);
+    (void)mx::dev_free(A.codes);
+    (void)mx::dev_free(A.dict);
+    (void)mx::dev_free(A.blockDesc);
     A = mx::DeviceCsr();
 }
 
 void free_tiles(mx::DeviceTiles &T)
 {
-    (void)hipFree(T.waveDesc);
-    (void)hipFree(T.hdr);
-    (void)hipFree(T.atox);
-    (void)hipFree(T.tcVal);
-    (void)hipFree(T.vidx);
+    (void)mx::dev_free(T.waveDesc);
+    (void)mx::dev_free(T.hdr);
+    (void)mx::dev_free(T.atox);
+    (void)mx::dev_free(T.tcVal);
+    (void)mx::dev_free(T.vidx);
     T = mx::DeviceTiles();
 }
 
 void free_slices(mx::DeviceSlices &P)
 {
-    (void)hipFree(P.waveDesc);
-    (void)hipFree(P.chunkEnd);
-    (void)hipFree(P.wgDesc);
-    (void)hipFree(P.ecol);
-    (void)hipFree(P.eval);
-    (void)hipFree(P.ecode);
-    (void)hipFree(P.dict);
-    (void)hipFree(P.partial);
-    (void)hipFree(P.rowInfo);
-    (void)hipFree(P.lightRow);
-    (void)hipFree(P.lightIdx);
-    (void)hipFree(P.heavyInfo);
-    (void)hipFree(P.segIdx);
-    (void)hipFree(P.wgGroups);
-    (void)hipFree(P.groupNeed);
-    (void)hipFree(P.groupCount);
-    (void)hipFree(P.fusedTarget);
-    (void)hipFree(P.fusedSums);
-    (void)hipFree(P.claim);
+    (void)mx::dev_free(P.waveDesc);
+    (void)mx::dev_free(P.chunkEnd);
+    (void)mx::dev_free(P.wgDesc);
+    (void)mx::dev_free(P.ecol);
+    (void)mx::dev_free(P.eval);
+    (void)mx::dev_free(P.ecode);
+    (void)mx::dev_free(P.dict);
+    (void)mx::dev_free(P.partial);
+    (void)mx::dev_free(P.rowInfo);
+    (void)mx::dev_free(P.lightRow);
+    (void)mx::dev_free(P.lightIdx);
+    (void)mx::dev_free(P.heavyInfo);
+    (void)mx::dev_free(P.segIdx);
+    (void)mx::dev_free(P.wgGroups);
+    (void)mx::dev_free(P.groupNeed);
+    (void)mx::dev_free(P.groupCount);
+    (void)mx::dev_free(P.fusedTarget);
+    (void)mx::dev_free(P.fusedSums);
+    (void)mx::dev_free(P.claim);
     P = mx::DeviceSlices();
 }
 
@@ -717,10 +732,10 @@ int upload_slices(mx_dtype dtype, int rows, int cols, const int *rowPtr, const i
         if (!rc)
             rc = mx::build_slices_device(dtype, rows, cols, nnz, dRowPtr, dCol, dVal, nCU, S, (const char *)dElse, D, nullptr,
                                          segOut ? &segOut->first : nullptr, segOut ? &segOut->second : nullptr, fused);
-        (void)hipFree(dRowPtr);
-        (void)hipFree(dCol);
-        (void)hipFree(dVal);
-        (void)hipFree(dElse);
+        (void)mx::dev_free(dRowPtr);
+        (void)mx::dev_free(dCol);
+        (void)mx::dev_free(dVal);
+        (void)mx::dev_free(dElse);
         return rc;
     }
     HostSlices H;
@@ -1359,9 +1374,9 @@ extern "C" int mx_slice_layout_device(const mx_csr *A, int nCU, mx_slice_layout_
     if (!rc) rc = upload(&dCol, A->colInd, (size_t)A->nnz);
     if (!rc) rc = upload_bytes(&dVal, A->val, (size_t)A->nnz * es);
     if (!rc) rc = mx::build_slices_device(A->dtype, A->rows, A->cols, A->nnz, dRowPtr, dCol, dVal, nCU, S, nullptr, D, nullptr, &segPtr, &segIdx);
-    (void)hipFree(dRowPtr);
-    (void)hipFree(dCol);
-    (void)hipFree(dVal);
+    (void)mx::dev_free(dRowPtr);
+    (void)mx::dev_free(dCol);
+    (void)mx::dev_free(dVal);
     if (rc) {
         free_slices(D);
         return rc;

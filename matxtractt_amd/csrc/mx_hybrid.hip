@@ -36,7 +36,7 @@ struct Buf {  // device memory released at scope exit unless taken
     ~Buf() { release(); }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p) (void)mx::dev_free(p);
         p = nullptr;
     }
     template <typename T>
@@ -851,7 +851,7 @@ int HybridDevice::analyse(mx_dtype dtype, int rows, int cols, int nnz, const int
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     {
         const size_t dcB = al((size_t)cols * 4 + 4), drB = al((size_t)rows * 4 + 4);
-        MXH_TRY(hipMalloc(&I.order.p, dcB + drB));
+        MXH_TRY(mx::dev_malloc(&I.order.p, dcB + drB));
         I.dc = (int *)I.order.p;
         I.dr = (int *)((unsigned char *)I.order.p + dcB);
     }
@@ -865,7 +865,7 @@ int HybridDevice::analyse(mx_dtype dtype, int rows, int cols, int nnz, const int
     {
         const size_t ddpB = al(((size_t)I.dRows + 1) * 4), ddcB = al((size_t)I.nDD * 4 + 4), ddvB = al((size_t)I.nDD * es + 8),
                      cdpB = al(((size_t)rows + 1) * 4), cdcB = al((size_t)I.nCD * 4 + 4), cdvB = al((size_t)I.nCD * es + 8);
-        MXH_TRY(hipMalloc(&I.split.p, ddpB + ddcB + ddvB + cdpB + cdcB + cdvB));
+        MXH_TRY(mx::dev_malloc(&I.split.p, ddpB + ddcB + ddvB + cdpB + cdcB + cdvB));
         unsigned char *b = (unsigned char *)I.split.p;
         I.ddp = (int *)b;
         I.ddc = (int *)(b + ddpB);
@@ -926,11 +926,11 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         Buf flag, notSel, pos, tmp;
         size_t scanBytes = 0;
         MXH_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, (size_t)cols, rocprim::plus<int>(), s));
-        MXH_TRY(hipMalloc(&flag.p, (size_t)cols + 4));
-        MXH_TRY(hipMalloc(&notSel.p, (size_t)cols * 4 + 4));
-        MXH_TRY(hipMalloc(&pos.p, (size_t)cols * 4 + 4));
-        MXH_TRY(hipMalloc(&tmp.p, scanBytes + 256));
-        MXH_TRY(hipMalloc(&I.colOrig.p, (size_t)cols * 4 + 4));
+        MXH_TRY(mx::dev_malloc(&flag.p, (size_t)cols + 4));
+        MXH_TRY(mx::dev_malloc(&notSel.p, (size_t)cols * 4 + 4));
+        MXH_TRY(mx::dev_malloc(&pos.p, (size_t)cols * 4 + 4));
+        MXH_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
+        MXH_TRY(mx::dev_malloc(&I.colOrig.p, (size_t)cols * 4 + 4));
         MXH_TRY(hipMemsetAsync(flag.p, 0, (size_t)cols + 4, s));
         if (I.dCols > 0) {
             hipLaunchKernelGGL(mark_kernel, grid(I.dCols), dim3(kBlock), 0, s, (const int *)I.dc, I.dCols, flag.as<unsigned char>());
@@ -942,7 +942,7 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         hipLaunchKernelGGL(col_orig_kernel, grid(cols), dim3(kBlock), 0, s, (const int *)I.dc, (const unsigned char *)flag.p,
                            (const int *)pos.p, cols, I.dCols, I.colOrig.as<int>());
         MXH_TRY(hipGetLastError());
-        MXH_TRY(hipMalloc(&I.ddRowOf.p, (size_t)rows * 4 + 4));
+        MXH_TRY(mx::dev_malloc(&I.ddRowOf.p, (size_t)rows * 4 + 4));
         MXH_TRY(hipMemsetAsync(I.ddRowOf.p, 0xff, (size_t)rows * 4 + 4, s));
         if (I.dRows > 0) {
             hipLaunchKernelGGL(dd_row_of_kernel, grid(I.dRows), dim3(kBlock), 0, s, (const int *)I.dr, I.dRows, I.ddRowOf.as<int>());
@@ -950,10 +950,10 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         }
         MXH_TRY(hipStreamSynchronize(s));
     }
-    MXH_TRY(hipMalloc(&I.taken.p, (size_t)I.dRows + 4));
+    MXH_TRY(mx::dev_malloc(&I.taken.p, (size_t)I.dRows + 4));
     MXH_TRY(hipMemsetAsync(I.taken.p, 0, (size_t)I.dRows + 4, s));
     Buf totals;
-    MXH_TRY(hipMalloc(&totals.p, 8 * 8));
+    MXH_TRY(mx::dev_malloc(&totals.p, 8 * 8));
     MXH_TRY(hipMemsetAsync(totals.p, 0, 8 * 8, s));
     unsigned long long *tot = totals.as<unsigned long long>();
 
@@ -964,9 +964,9 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         MXH_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, (size_t)I.dRows + 1, rocprim::plus<int>(), s));
         MXH_TRY(rocprim::inclusive_scan(nullptr, b2, (const int *)nullptr, (int *)nullptr, (size_t)I.dRows + 1, rocprim::plus<int>(), s));
         scanBytes = std::max(scanBytes, b2);
-        MXH_TRY(hipMalloc(&isCand.p, ((size_t)I.dRows + 1) * 4));
-        MXH_TRY(hipMalloc(&candPos.p, ((size_t)I.dRows + 1) * 4));
-        MXH_TRY(hipMalloc(&tmp.p, scanBytes + 256));
+        MXH_TRY(mx::dev_malloc(&isCand.p, ((size_t)I.dRows + 1) * 4));
+        MXH_TRY(mx::dev_malloc(&candPos.p, ((size_t)I.dRows + 1) * 4));
+        MXH_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
         MXH_TRY(hipMemsetAsync(isCand.p, 0, ((size_t)I.dRows + 1) * 4, s));
         hipLaunchKernelGGL(strip_candidates_kernel, grid(I.dRows), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const int *)I.dc,
                            (const int *)I.dr, (const int *)I.cdp, I.dRows, cols, isCand.as<int>());
@@ -978,9 +978,9 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         I.nCand = nCand;
         if (nCand > 0) {
             const size_t nc = (size_t)nCand;
-            MXH_TRY(hipMalloc(&I.candRow.p, nc * 4));
-            MXH_TRY(hipMalloc(&I.candKey.p, nc * 8 * 4));
-            MXH_TRY(hipMalloc(&I.candNb.p, nc * 4));
+            MXH_TRY(mx::dev_malloc(&I.candRow.p, nc * 4));
+            MXH_TRY(mx::dev_malloc(&I.candKey.p, nc * 8 * 4));
+            MXH_TRY(mx::dev_malloc(&I.candNb.p, nc * 4));
             hipLaunchKernelGGL(candidate_keys_kernel, grid(I.dRows), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc,
                                (const int *)I.dc, (const int *)I.dr, (const int *)I.cdp, (const int *)isCand.p, (const int *)candPos.p, I.dRows,
                                cols, I.candRow.as<int>(), I.candKey.as<int>(), I.candNb.as<int>());
@@ -992,11 +992,11 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
             size_t sortBytes = 0;
             MXH_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned *)nullptr, (unsigned *)nullptr, (const int *)nullptr,
                                               (int *)nullptr, nc, 0u, bits, s));
-            MXH_TRY(hipMalloc(&I.perm.p, nc * 4));
-            MXH_TRY(hipMalloc(&permB.p, nc * 4));
-            MXH_TRY(hipMalloc(&keyA.p, nc * 4));
-            MXH_TRY(hipMalloc(&keyB.p, nc * 4));
-            MXH_TRY(hipMalloc(&sortTmp.p, sortBytes + 256));
+            MXH_TRY(mx::dev_malloc(&I.perm.p, nc * 4));
+            MXH_TRY(mx::dev_malloc(&permB.p, nc * 4));
+            MXH_TRY(mx::dev_malloc(&keyA.p, nc * 4));
+            MXH_TRY(mx::dev_malloc(&keyB.p, nc * 4));
+            MXH_TRY(mx::dev_malloc(&sortTmp.p, sortBytes + 256));
             hipLaunchKernelGGL(iota_kernel, grid(nCand), dim3(kBlock), 0, s, I.perm.as<int>(), nCand);
             MXH_TRY(hipGetLastError());
             for (int k = 7; k >= 0; --k) {
@@ -1009,9 +1009,9 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
             }
             // runs of equal block sets and their chunks
             Buf head, runChunks, runChunk0;
-            MXH_TRY(hipMalloc(&head.p, (nc + 1) * 4));
-            MXH_TRY(hipMalloc(&I.runIdIncl.p, (nc + 1) * 4));
-            MXH_TRY(hipMalloc(&I.runStart.p, (nc + 2) * 4));
+            MXH_TRY(mx::dev_malloc(&head.p, (nc + 1) * 4));
+            MXH_TRY(mx::dev_malloc(&I.runIdIncl.p, (nc + 1) * 4));
+            MXH_TRY(mx::dev_malloc(&I.runStart.p, (nc + 2) * 4));
             hipLaunchKernelGGL(run_heads_kernel, grid(nCand), dim3(kBlock), 0, s, (const int *)I.candKey.p, (const int *)I.perm.p, nCand,
                                head.as<int>());
             MXH_TRY(hipGetLastError());
@@ -1022,8 +1022,8 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
             hipLaunchKernelGGL(run_starts_kernel, grid(nCand), dim3(kBlock), 0, s, (const int *)head.p, (const int *)I.runIdIncl.p, nCand,
                                I.runStart.as<int>());
             MXH_TRY(hipGetLastError());
-            MXH_TRY(hipMalloc(&runChunks.p, ((size_t)nRuns + 1) * 4));
-            MXH_TRY(hipMalloc(&runChunk0.p, ((size_t)nRuns + 1) * 4));
+            MXH_TRY(mx::dev_malloc(&runChunks.p, ((size_t)nRuns + 1) * 4));
+            MXH_TRY(mx::dev_malloc(&runChunk0.p, ((size_t)nRuns + 1) * 4));
             MXH_TRY(hipMemsetAsync(runChunks.p, 0, ((size_t)nRuns + 1) * 4, s));
             hipLaunchKernelGGL(run_chunks_kernel, grid(nRuns), dim3(kBlock), 0, s, (const int *)I.runStart.p, nRuns, runChunks.as<int>());
             MXH_TRY(hipGetLastError());
@@ -1036,11 +1036,11 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
             I.nChunks = nChunks;
             if (nChunks > 0) {
                 const size_t nk = (size_t)nChunks;
-                MXH_TRY(hipMalloc(&I.memberChunk.p, nc * 4));
-                MXH_TRY(hipMalloc(&I.chunkRows.p, nk * 8 * 4));
-                MXH_TRY(hipMalloc(&I.chunkKey.p, nk * 8 * 4));
-                MXH_TRY(hipMalloc(&I.chunkNb.p, nk * 4));
-                MXH_TRY(hipMalloc(&I.chunkNnz.p, nk * 4));
+                MXH_TRY(mx::dev_malloc(&I.memberChunk.p, nc * 4));
+                MXH_TRY(mx::dev_malloc(&I.chunkRows.p, nk * 8 * 4));
+                MXH_TRY(mx::dev_malloc(&I.chunkKey.p, nk * 8 * 4));
+                MXH_TRY(mx::dev_malloc(&I.chunkNb.p, nk * 4));
+                MXH_TRY(mx::dev_malloc(&I.chunkNnz.p, nk * 4));
                 MXH_TRY(hipMemsetAsync(I.chunkRows.p, 0xff, nk * 8 * 4, s));
                 hipLaunchKernelGGL(chunk_members_kernel, grid(nCand), dim3(kBlock), 0, s, (const int *)I.perm.p, (const int *)I.candRow.p,
                                    (const int *)I.candKey.p, (const int *)I.candNb.p, (const int *)I.runIdIncl.p, (const int *)I.runStart.p,
@@ -1070,11 +1070,11 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         size_t sortBytes = 0;
         MXH_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
                                           (const int *)nullptr, (int *)nullptr, n, 0u, 64u, s));
-        MXH_TRY(hipMalloc(&keyIn.p, n * 8));
-        MXH_TRY(hipMalloc(&payIn.p, n * 4));
-        MXH_TRY(hipMalloc(&I.blkKey.p, n * 8));
-        MXH_TRY(hipMalloc(&I.blkPay.p, n * 4));
-        MXH_TRY(hipMalloc(&sortTmp.p, sortBytes + 256));
+        MXH_TRY(mx::dev_malloc(&keyIn.p, n * 8));
+        MXH_TRY(mx::dev_malloc(&payIn.p, n * 4));
+        MXH_TRY(mx::dev_malloc(&I.blkKey.p, n * 8));
+        MXH_TRY(mx::dev_malloc(&I.blkPay.p, n * 4));
+        MXH_TRY(mx::dev_malloc(&sortTmp.p, sortBytes + 256));
         hipLaunchKernelGGL(block_keys_kernel, grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const int *)I.dc,
                            (const int *)I.dr, I.dRows, I.nDD, keyIn.as<unsigned long long>());
         MXH_TRY(hipGetLastError());
@@ -1135,15 +1135,15 @@ static int csr_part_t(HybridDevice::Impl &I, bool keepStrips, bool keepGeneral, 
     size_t scanBytes = 0;
     MXH_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, (size_t)std::max(rows, blocks ? I.nDD : 0) + 1,
                                     rocprim::plus<int>(), s));
-    MXH_TRY(hipMalloc(&len.p, ((size_t)rows + 1) * 4));
-    MXH_TRY(hipMalloc(&ptr.p, ((size_t)rows + 1) * 4));
-    MXH_TRY(hipMalloc(&tmp.p, scanBytes + 256));
-    if (taken) MXH_TRY(hipMalloc(&marks.p, (size_t)rows + 4));
+    MXH_TRY(mx::dev_malloc(&len.p, ((size_t)rows + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&ptr.p, ((size_t)rows + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
+    if (taken) MXH_TRY(mx::dev_malloc(&marks.p, (size_t)rows + 4));
     if (blocks) {
         Buf keep;
-        MXH_TRY(hipMalloc(&keep.p, ((size_t)I.nDD + 1) * 4));
-        MXH_TRY(hipMalloc(&keptBefore.p, ((size_t)I.nDD + 1) * 4));
-        MXH_TRY(hipMalloc(&marks.p, (size_t)rows + 4));
+        MXH_TRY(mx::dev_malloc(&keep.p, ((size_t)I.nDD + 1) * 4));
+        MXH_TRY(mx::dev_malloc(&keptBefore.p, ((size_t)I.nDD + 1) * 4));
+        MXH_TRY(mx::dev_malloc(&marks.p, (size_t)rows + 4));
         MXH_TRY(hipMemsetAsync(marks.p, 0, (size_t)rows + 4, s));
         hipLaunchKernelGGL(block_keep_kernel, grid((long long)I.nDD + 1), dim3(kBlock), 0, s, (const int *)I.entryBlock.p, I.nDD, keep.as<int>());
         MXH_TRY(hipGetLastError());
@@ -1155,7 +1155,7 @@ static int csr_part_t(HybridDevice::Impl &I, bool keepStrips, bool keepGeneral, 
                            marks.as<char>());
         MXH_TRY(hipStreamSynchronize(s));  // (`keep` leaves scope)
     } else if (general) {
-        MXH_TRY(hipMalloc(&kept.p, (size_t)I.dRows * 4 + 4));
+        MXH_TRY(mx::dev_malloc(&kept.p, (size_t)I.dRows * 4 + 4));
         hipLaunchKernelGGL((dd_rows_kernel<V, true>), grid(I.dRows), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc,
                            (const V *)I.ddv, (const int *)I.dc, (const int *)I.dr, taken, (const int *)I.T.chunkPtr,
                            (const int *)I.T.sparse_AToX_index, (const int *)I.usedCols.p, (const unsigned char *)I.selFrag.p, I.dRows, K,
@@ -1173,8 +1173,8 @@ static int csr_part_t(HybridDevice::Impl &I, bool keepStrips, bool keepGeneral, 
     int n = 0;
     MXH_TRY(hipMemcpyAsync(&n, ptr.as<int>() + rows, 4, hipMemcpyDeviceToHost, s));
     MXH_TRY(hipStreamSynchronize(s));
-    MXH_TRY(hipMalloc(&col.p, (size_t)n * 4 + 4));
-    MXH_TRY(hipMalloc(&val.p, (size_t)n * sizeof(V) + 8));
+    MXH_TRY(mx::dev_malloc(&col.p, (size_t)n * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&val.p, (size_t)n * sizeof(V) + 8));
     if (I.nCD > 0) {
         hipLaunchKernelGGL(part_residual_kernel<V>, grid(I.nCD), dim3(kBlock), 0, s, (const int *)I.cdp, (const int *)I.cdc, (const V *)I.cdv,
                            (const int *)I.colOrig.p, (const int *)ptr.p, rows, I.nCD, col.as<int>(), val.as<V>());
@@ -1234,10 +1234,10 @@ int HybridDevice::block_chunks(std::vector<int> &blocks, std::vector<int> &block
     MXH_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, n + 1, rocprim::plus<int>(), s));
     MXH_TRY(rocprim::inclusive_scan(nullptr, b2, (const int *)nullptr, (int *)nullptr, n + 1, rocprim::plus<int>(), s));
     scanBytes = std::max(scanBytes, b2);
-    MXH_TRY(hipMalloc(&selHead.p, (n + 1) * 4));
-    MXH_TRY(hipMalloc(&blockId.p, (n + 1) * 4));
-    MXH_TRY(hipMalloc(&tmp.p, scanBytes + 256));
-    MXH_TRY(hipMalloc(&I.entryBlock.p, n * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&selHead.p, (n + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&blockId.p, (n + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
+    MXH_TRY(mx::dev_malloc(&I.entryBlock.p, n * 4 + 4));
     MXH_TRY(hipMemsetAsync(I.entryBlock.p, 0xff, n * 4 + 4, s));
     hipLaunchKernelGGL(block_heads_kernel, grid((long long)n + 1), dim3(kBlock), 0, s, (const unsigned long long *)I.blkKey.p, I.nDD, 48, I.cols,
                        selHead.as<int>());
@@ -1248,10 +1248,10 @@ int HybridDevice::block_chunks(std::vector<int> &blocks, std::vector<int> &block
     MXH_TRY(hipStreamSynchronize(s));
     if (nBlk <= 0) return MX_OK;
     const size_t nbk = (size_t)nBlk;
-    MXH_TRY(hipMalloc(&I.blkBr.p, nbk * 4 + 4));
-    MXH_TRY(hipMalloc(&I.blkBc.p, nbk * 4 + 4));
-    MXH_TRY(hipMalloc(&head.p, nbk * 4 + 4));
-    MXH_TRY(hipMalloc(&I.blkChunkIdIncl.p, nbk * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&I.blkBr.p, nbk * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&I.blkBc.p, nbk * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&head.p, nbk * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&I.blkChunkIdIncl.p, nbk * 4 + 4));
     hipLaunchKernelGGL(block_records_kernel, grid(I.nDD), dim3(kBlock), 0, s, (const unsigned long long *)I.blkKey.p, (const int *)I.blkPay.p,
                        (const int *)selHead.p, (const int *)blockId.p, I.nDD, I.blkBr.as<int>(), I.blkBc.as<int>(), I.entryBlock.as<int>());
     MXH_TRY(hipGetLastError());
@@ -1262,9 +1262,9 @@ int HybridDevice::block_chunks(std::vector<int> &blocks, std::vector<int> &block
     int nChunks = 0;
     MXH_TRY(hipMemcpyAsync(&nChunks, I.blkChunkIdIncl.as<int>() + (nbk - 1), 4, hipMemcpyDeviceToHost, s));
     MXH_TRY(hipStreamSynchronize(s));
-    MXH_TRY(hipMalloc(&I.blkChunkStart.p, ((size_t)nChunks + 1) * 4));
-    MXH_TRY(hipMalloc(&I.blkChunkBr.p, ((size_t)nChunks + 1) * 4));
-    MXH_TRY(hipMalloc(&nb.p, ((size_t)nChunks + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&I.blkChunkStart.p, ((size_t)nChunks + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&I.blkChunkBr.p, ((size_t)nChunks + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&nb.p, ((size_t)nChunks + 1) * 4));
     hipLaunchKernelGGL(block_chunk_starts_kernel, grid(nBlk), dim3(kBlock), 0, s, (const int *)head.p, (const int *)I.blkChunkIdIncl.p,
                        (const int *)I.blkBr.p, nBlk, I.blkChunkStart.as<int>(), I.blkChunkBr.as<int>());
     MXH_TRY(hipGetLastError());
@@ -1289,20 +1289,20 @@ int HybridDevice::block_layout(const std::vector<int> &stepDesc, const std::vect
     hipStream_t s = I.s;
     const int steps = (int)(stepDesc.size() / 10);
     Buf dDesc, dBlock0;
-    MXH_TRY(hipMalloc(&dDesc.p, stepDesc.size() * 4 + 4));
-    MXH_TRY(hipMalloc(&dBlock0.p, chunkBlock0.size() * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&dDesc.p, stepDesc.size() * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&dBlock0.p, chunkBlock0.size() * 4 + 4));
     MXH_TRY(hipMemcpyAsync(dDesc.p, stepDesc.data(), stepDesc.size() * 4, hipMemcpyHostToDevice, s));
     MXH_TRY(hipMemcpyAsync(dBlock0.p, chunkBlock0.data(), chunkBlock0.size() * 4, hipMemcpyHostToDevice, s));
     const size_t nWave = waveDesc.size() + 64, nHdr = (size_t)steps * kTileHdr + 256, nAtox = (size_t)steps * 64 + 256,
                  valBytes = (size_t)totalBlocks * 64 * 8 + 8192;
-    MXH_TRY(hipMalloc((void **)&T.waveDesc, nWave * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.waveDesc, nWave * 4));
     MXH_TRY(hipMemsetAsync(T.waveDesc, 0, nWave * 4, s));
     MXH_TRY(hipMemcpyAsync(T.waveDesc, waveDesc.data(), waveDesc.size() * 4, hipMemcpyHostToDevice, s));
-    MXH_TRY(hipMalloc((void **)&T.hdr, nHdr * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.hdr, nHdr * 4));
     MXH_TRY(hipMemsetAsync(T.hdr, 0, nHdr * 4, s));
-    MXH_TRY(hipMalloc((void **)&T.atox, nAtox * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.atox, nAtox * 4));
     MXH_TRY(hipMemsetAsync(T.atox, 0, nAtox * 4, s));
-    MXH_TRY(hipMalloc(&T.tcVal, valBytes));
+    MXH_TRY(mx::dev_malloc(&T.tcVal, valBytes));
     MXH_TRY(hipMemsetAsync(T.tcVal, 0, valBytes, s));
     hipLaunchKernelGGL(block_steps_kernel, dim3(steps), dim3(64), 0, s, (const int *)dDesc.p, (const int *)I.blkChunkStart.p,
                        (const int *)I.blkChunkBr.p, (const int *)I.blkBc.p, I.rows, steps, T.hdr, T.atox);
@@ -1335,19 +1335,19 @@ int HybridDevice::tile_chunks(bool keepStrips, std::vector<int> &blocks)
     MXH_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
                                       (const int *)nullptr, (int *)nullptr, nKey, 0u, 64u, s));
     MXH_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, (size_t)chunkNum + 1, rocprim::plus<int>(), s));
-    MXH_TRY(hipMalloc(&I.selFrag.p, (size_t)nFrags + 4));
-    MXH_TRY(hipMalloc(&I.usedCols.p, (size_t)chunkNum * 4 + 4));
-    MXH_TRY(hipMalloc(&I.nrefs.p, ((size_t)chunkNum + 1) * 4));
-    MXH_TRY(hipMalloc(&I.refStart.p, ((size_t)chunkNum + 1) * 4));
-    MXH_TRY(hipMalloc(&I.selPos.p, ((size_t)chunkNum + 1) * 4));
-    MXH_TRY(hipMalloc(&I.where.p, nKey * 4 + 4));
-    MXH_TRY(hipMalloc(&keyIn.p, nKey * 8));
-    MXH_TRY(hipMalloc(&keyOut.p, nKey * 8));
-    MXH_TRY(hipMalloc(&payIn.p, nKey * 4));
-    MXH_TRY(hipMalloc(&payOut.p, nKey * 4));
-    MXH_TRY(hipMalloc(&sortTmp.p, sortBytes + 256));
-    MXH_TRY(hipMalloc(&scanTmp.p, scanBytes + 256));
-    MXH_TRY(hipMalloc(&isSel.p, ((size_t)chunkNum + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&I.selFrag.p, (size_t)nFrags + 4));
+    MXH_TRY(mx::dev_malloc(&I.usedCols.p, (size_t)chunkNum * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&I.nrefs.p, ((size_t)chunkNum + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&I.refStart.p, ((size_t)chunkNum + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&I.selPos.p, ((size_t)chunkNum + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&I.where.p, nKey * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&keyIn.p, nKey * 8));
+    MXH_TRY(mx::dev_malloc(&keyOut.p, nKey * 8));
+    MXH_TRY(mx::dev_malloc(&payIn.p, nKey * 4));
+    MXH_TRY(mx::dev_malloc(&payOut.p, nKey * 4));
+    MXH_TRY(mx::dev_malloc(&sortTmp.p, sortBytes + 256));
+    MXH_TRY(mx::dev_malloc(&scanTmp.p, scanBytes + 256));
+    MXH_TRY(mx::dev_malloc(&isSel.p, ((size_t)chunkNum + 1) * 4));
     MXH_TRY(hipMemsetAsync(I.nrefs.p, 0, ((size_t)chunkNum + 1) * 4, s));
     MXH_TRY(hipMemsetAsync(I.where.p, 0xff, nKey * 4 + 4, s));
     if (I.dtype == MX_F64)
@@ -1375,9 +1375,9 @@ int HybridDevice::tile_chunks(bool keepStrips, std::vector<int> &blocks)
     MXH_TRY(hipMemcpyAsync(&nSel, I.selPos.as<int>() + chunkNum, 4, hipMemcpyDeviceToHost, s));
     MXH_TRY(hipStreamSynchronize(s));
     if (nSel <= 0 || nRefs <= 0) return MX_OK;
-    MXH_TRY(hipMalloc(&I.sortedCol.p, (size_t)nRefs * 4 + 4));
-    MXH_TRY(hipMalloc(&I.selW.p, (size_t)nSel * 4 + 4));
-    MXH_TRY(hipMalloc(&selNb.p, (size_t)nSel * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&I.sortedCol.p, (size_t)nRefs * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&I.selW.p, (size_t)nSel * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&selNb.p, (size_t)nSel * 4 + 4));
     hipLaunchKernelGGL(ref_places_kernel, grid(nRefs), dim3(kBlock), 0, s, (const unsigned long long *)keyOut.p, (const int *)payOut.p,
                        (const int *)I.refStart.p, nRefs, I.sortedCol.as<int>(), I.where.as<int>());
     MXH_TRY(hipGetLastError());
@@ -1404,21 +1404,21 @@ int HybridDevice::tile_layout(bool keepStrips, const std::vector<int> &stepDesc,
     const size_t es = (size_t)mx::elem_size(I.dtype);
     const unsigned char *taken = keepStrips && I.nChunks > 0 ? (const unsigned char *)I.taken.p : nullptr;
     Buf dDesc;
-    MXH_TRY(hipMalloc(&dDesc.p, stepDesc.size() * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&dDesc.p, stepDesc.size() * 4 + 4));
     MXH_TRY(hipMemcpyAsync(dDesc.p, stepDesc.data(), stepDesc.size() * 4, hipMemcpyHostToDevice, s));
-    MXH_TRY(hipMalloc(&I.tileBlock0.p, ((size_t)I.nSel + 1) * 4));
+    MXH_TRY(mx::dev_malloc(&I.tileBlock0.p, ((size_t)I.nSel + 1) * 4));
     MXH_TRY(hipMemsetAsync(I.tileBlock0.p, 0, ((size_t)I.nSel + 1) * 4, s));
     MXH_TRY(hipMemcpyAsync(I.tileBlock0.p, chunkBlock0.data(), chunkBlock0.size() * 4, hipMemcpyHostToDevice, s));
     const size_t nWave = waveDesc.size() + 64, nHdr = (size_t)steps * kTileHdr + 256, nAtox = (size_t)steps * 64 + 256,
                  valBytes = (size_t)totalBlocks * 8 * K * es + 8192;
-    MXH_TRY(hipMalloc((void **)&T.waveDesc, nWave * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.waveDesc, nWave * 4));
     MXH_TRY(hipMemsetAsync(T.waveDesc, 0, nWave * 4, s));
     MXH_TRY(hipMemcpyAsync(T.waveDesc, waveDesc.data(), waveDesc.size() * 4, hipMemcpyHostToDevice, s));
-    MXH_TRY(hipMalloc((void **)&T.hdr, nHdr * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.hdr, nHdr * 4));
     MXH_TRY(hipMemsetAsync(T.hdr, 0, nHdr * 4, s));
-    MXH_TRY(hipMalloc((void **)&T.atox, nAtox * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.atox, nAtox * 4));
     MXH_TRY(hipMemsetAsync(T.atox, 0, nAtox * 4, s));
-    MXH_TRY(hipMalloc(&T.tcVal, valBytes));
+    MXH_TRY(mx::dev_malloc(&T.tcVal, valBytes));
     MXH_TRY(hipMemsetAsync(T.tcVal, 0, valBytes, s));
     if (I.dtype == MX_F64)
         hipLaunchKernelGGL(tile_steps_kernel<true>, dim3(steps), dim3(64), 0, s, (const int *)dDesc.p, (const int *)I.selW.p,
@@ -1443,21 +1443,21 @@ int HybridDevice::strip_layout(const std::vector<int> &stepDesc, const std::vect
     hipStream_t s = I.s;
     const int steps = (int)(stepDesc.size() / 8);
     Buf dDesc, dBlock0;
-    MXH_TRY(hipMalloc(&dDesc.p, stepDesc.size() * 4 + 4));
-    MXH_TRY(hipMalloc(&dBlock0.p, chunkBlock0.size() * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&dDesc.p, stepDesc.size() * 4 + 4));
+    MXH_TRY(mx::dev_malloc(&dBlock0.p, chunkBlock0.size() * 4 + 4));
     MXH_TRY(hipMemcpyAsync(dDesc.p, stepDesc.data(), stepDesc.size() * 4, hipMemcpyHostToDevice, s));
     MXH_TRY(hipMemcpyAsync(dBlock0.p, chunkBlock0.data(), chunkBlock0.size() * 4, hipMemcpyHostToDevice, s));
     // (sizes and zero padding as the host route uploads them)
     const size_t nWave = waveDesc.size() + 64, nHdr = (size_t)steps * kTileHdr + 256, nAtox = (size_t)steps * 64 + 256,
                  valBytes = (size_t)totalBlocks * 64 * 2 + 8192;
-    MXH_TRY(hipMalloc((void **)&T.waveDesc, nWave * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.waveDesc, nWave * 4));
     MXH_TRY(hipMemsetAsync(T.waveDesc, 0, nWave * 4, s));
     MXH_TRY(hipMemcpyAsync(T.waveDesc, waveDesc.data(), waveDesc.size() * 4, hipMemcpyHostToDevice, s));
-    MXH_TRY(hipMalloc((void **)&T.hdr, nHdr * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.hdr, nHdr * 4));
     MXH_TRY(hipMemsetAsync(T.hdr, 0, nHdr * 4, s));
-    MXH_TRY(hipMalloc((void **)&T.atox, nAtox * 4));
+    MXH_TRY(mx::dev_malloc((void **)&T.atox, nAtox * 4));
     MXH_TRY(hipMemsetAsync(T.atox, 0, nAtox * 4, s));
-    MXH_TRY(hipMalloc(&T.tcVal, valBytes));
+    MXH_TRY(mx::dev_malloc(&T.tcVal, valBytes));
     MXH_TRY(hipMemsetAsync(T.tcVal, 0, valBytes, s));
     hipLaunchKernelGGL(strip_steps_kernel, dim3(steps), dim3(64), 0, s, (const int *)dDesc.p, (const int *)I.chunkRows.p,
                        (const int *)I.chunkKey.p, steps, T.hdr, T.atox);

@@ -36,7 +36,7 @@ struct Buf {  // device memory released at scope exit unless taken
     ~Buf() { release(); }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p) (void)mx::dev_free(p);
         p = nullptr;
     }
     template <typename T>
@@ -495,7 +495,7 @@ static int device_value_dict(const V *val, int nnz, mxl::Buf &codes, std::vector
     *nDict = 0;
     Buf table;  // keys, codes of the slots, first places, flag
     const size_t keyB = kDictSlots * 8, codeB = 2048, firstB = (kDictSlots + 1) * 4;
-    MXL_TRY(hipMalloc(&table.p, keyB + codeB + firstB + 256));
+    MXL_TRY(mx::dev_malloc(&table.p, keyB + codeB + firstB + 256));
     unsigned long long *keys = table.as<unsigned long long>();
     unsigned char *codeOf = table.as<unsigned char>() + keyB;
     int *first = (int *)(codeOf + codeB), *flag = first + kDictSlots + 1;
@@ -529,7 +529,7 @@ static int device_value_dict(const V *val, int nnz, mxl::Buf &codes, std::vector
         std::memcpy(&dict[(size_t)c * sizeof(V)], &v, sizeof(V));  // little-endian: the low bytes are the value
     }
     MXL_TRY(hipMemcpyAsync(codeOf, h.codeOf, sizeof(h.codeOf), hipMemcpyHostToDevice, s));
-    MXL_TRY(hipMalloc(&codes.p, (size_t)nnz + codePad));
+    MXL_TRY(mx::dev_malloc(&codes.p, (size_t)nnz + codePad));
     if (codePad) MXL_TRY(hipMemsetAsync((unsigned char *)codes.p + nnz, 0, codePad, s));
     hipLaunchKernelGGL(value_codes_kernel<V>, dim3((unsigned)std::min<long long>(4096, ((long long)nnz + 1023) / 1024)), dim3(kBlock), 0, s, val, nnz,
                        (const unsigned long long *)keys, (const unsigned char *)codeOf, codes.as<unsigned char>());
@@ -570,9 +570,9 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     D.nnz = nnz;
     // ---- rows in ascending column order
     Buf row, ord, flag;
-    MXL_TRY(hipMalloc(&row.p, std::max<size_t>((size_t)nnz, 1) * 4));
-    MXL_TRY(hipMalloc(&ord.p, std::max<size_t>((size_t)nnz, 1) * 4));
-    MXL_TRY(hipMalloc(&flag.p, 256));
+    MXL_TRY(mx::dev_malloc(&row.p, std::max<size_t>((size_t)nnz, 1) * 4));
+    MXL_TRY(mx::dev_malloc(&ord.p, std::max<size_t>((size_t)nnz, 1) * 4));
+    MXL_TRY(mx::dev_malloc(&flag.p, 256));
     MXL_TRY(hipMemsetAsync(flag.p, 0, 256, s));
     int *over4 = flag.as<int>() + 1;
     Buf tmp;
@@ -581,7 +581,7 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     MXL_TRY(rocprim::inclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, nScan, MaxOp(), s));
     MXL_TRY(rocprim::exclusive_scan(nullptr, b2, (const int *)nullptr, (int *)nullptr, 0, nScan, rocprim::plus<int>(), s));
     scanBytes = std::max(scanBytes, b2);
-    MXL_TRY(hipMalloc(&tmp.p, scanBytes + 256));
+    MXL_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
     if (nnz > 0) {
         // (`ord` is free until the order of the entries is known: it holds the row heads meanwhile)
         MXL_TRY(hipMemsetAsync(ord.p, 0, (size_t)nnz * 4, s));
@@ -602,10 +602,10 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
         size_t sortBytes = 0;
         MXL_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
                                           (const int *)nullptr, (int *)nullptr, (size_t)nnz, 0u, (unsigned)(colBits + rowBits), s));
-        MXL_TRY(hipMalloc(&keyIn.p, (size_t)nnz * 8));
-        MXL_TRY(hipMalloc(&keyOut.p, (size_t)nnz * 8));
-        MXL_TRY(hipMalloc(&payIn.p, (size_t)nnz * 4));
-        MXL_TRY(hipMalloc(&tmp.p, sortBytes + 256));
+        MXL_TRY(mx::dev_malloc(&keyIn.p, (size_t)nnz * 8));
+        MXL_TRY(mx::dev_malloc(&keyOut.p, (size_t)nnz * 8));
+        MXL_TRY(mx::dev_malloc(&payIn.p, (size_t)nnz * 4));
+        MXL_TRY(mx::dev_malloc(&tmp.p, sortBytes + 256));
         hipLaunchKernelGGL(sort_keys_kernel, grid(nnz), dim3(kBlock), 0, s, (const int *)row.p, col, nnz, colBits,
                            keyIn.as<unsigned long long>(), payIn.as<int>());
         MXL_TRY(hipGetLastError());
@@ -618,10 +618,10 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     }
     // ---- virtual rows
     Buf runHead, runStart, start, vid;
-    MXL_TRY(hipMalloc(&runHead.p, ((size_t)nnz + 1) * 4));
-    MXL_TRY(hipMalloc(&runStart.p, ((size_t)nnz + 1) * 4));
-    MXL_TRY(hipMalloc(&start.p, ((size_t)nnz + 1) * 4));
-    MXL_TRY(hipMalloc(&vid.p, ((size_t)nnz + 1) * 4));
+    MXL_TRY(mx::dev_malloc(&runHead.p, ((size_t)nnz + 1) * 4));
+    MXL_TRY(mx::dev_malloc(&runStart.p, ((size_t)nnz + 1) * 4));
+    MXL_TRY(mx::dev_malloc(&start.p, ((size_t)nnz + 1) * 4));
+    MXL_TRY(mx::dev_malloc(&vid.p, ((size_t)nnz + 1) * 4));
     int nV = 0;
     if (nnz > 0) {
         hipLaunchKernelGGL(run_heads_kernel, grid(nnz), dim3(kBlock), 0, s, rowPtr, (const int *)row.p, col, (const int *)ord.p, nnz, SW,
@@ -641,16 +641,16 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     D.vrows = nV;
     Buf vStart, vRow, vSlice, vLen, segPtr, key, keyOut, pay, sorted, sliceCount;
     const size_t nv1 = (size_t)nV + 1;
-    MXL_TRY(hipMalloc(&vStart.p, nv1 * 4));
-    MXL_TRY(hipMalloc(&vRow.p, nv1 * 4));
-    MXL_TRY(hipMalloc(&vSlice.p, nv1 * 4));
-    MXL_TRY(hipMalloc(&vLen.p, nv1 * 4));
-    MXL_TRY(hipMalloc(&segPtr.p, ((size_t)rows + 2) * 4));
-    MXL_TRY(hipMalloc(&key.p, nv1 * 4));
-    MXL_TRY(hipMalloc(&keyOut.p, nv1 * 4));
-    MXL_TRY(hipMalloc(&pay.p, nv1 * 4));
-    MXL_TRY(hipMalloc(&sorted.p, nv1 * 4));
-    MXL_TRY(hipMalloc(&sliceCount.p, ((size_t)S + 2) * 4));
+    MXL_TRY(mx::dev_malloc(&vStart.p, nv1 * 4));
+    MXL_TRY(mx::dev_malloc(&vRow.p, nv1 * 4));
+    MXL_TRY(mx::dev_malloc(&vSlice.p, nv1 * 4));
+    MXL_TRY(mx::dev_malloc(&vLen.p, nv1 * 4));
+    MXL_TRY(mx::dev_malloc(&segPtr.p, ((size_t)rows + 2) * 4));
+    MXL_TRY(mx::dev_malloc(&key.p, nv1 * 4));
+    MXL_TRY(mx::dev_malloc(&keyOut.p, nv1 * 4));
+    MXL_TRY(mx::dev_malloc(&pay.p, nv1 * 4));
+    MXL_TRY(mx::dev_malloc(&sorted.p, nv1 * 4));
+    MXL_TRY(mx::dev_malloc(&sliceCount.p, ((size_t)S + 2) * 4));
     if (nnz > 0) {
         hipLaunchKernelGGL(vrow_records_kernel, grid(nnz), dim3(kBlock), 0, s, (const int *)start.p, (const int *)vid.p, (const int *)row.p,
                            col, (const int *)ord.p, nnz, SW, vStart.as<int>(), vRow.as<int>(), vSlice.as<int>());
@@ -695,7 +695,7 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
         MXL_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned *)nullptr, (unsigned *)nullptr, (const int *)nullptr,
                                           (int *)nullptr, (size_t)nV, 0u, keyBits, s));
         Buf sortTmp;
-        MXL_TRY(hipMalloc(&sortTmp.p, sortBytes + 256));
+        MXL_TRY(mx::dev_malloc(&sortTmp.p, sortBytes + 256));
         MXL_TRY(rocprim::radix_sort_pairs(sortTmp.p, sortBytes, (const unsigned *)key.p, keyOut.as<unsigned>(), (const int *)pay.p,
                                           sorted.as<int>(), (size_t)nV, 0u, keyBits, s));
         hipLaunchKernelGGL(slice_starts_kernel, grid((long long)S + 1), dim3(kBlock), 0, s, (const unsigned *)keyOut.p, nV, S,
@@ -723,8 +723,8 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     if (nChunk > 0 && !fusedTaken) {
         Buf dFirst, dLen;
         std::vector<int> len((size_t)nChunk);
-        MXL_TRY(hipMalloc(&dFirst.p, (size_t)nChunk * 4));
-        MXL_TRY(hipMalloc(&dLen.p, (size_t)nChunk * 4));
+        MXL_TRY(mx::dev_malloc(&dFirst.p, (size_t)nChunk * 4));
+        MXL_TRY(mx::dev_malloc(&dLen.p, (size_t)nChunk * 4));
         MXL_TRY(hipMemcpyAsync(dFirst.p, firstIdx.data(), (size_t)nChunk * 4, hipMemcpyHostToDevice, s));
         hipLaunchKernelGGL(gather_len_kernel, grid(nChunk), dim3(kBlock), 0, s, (const int *)sorted.p, (const int *)vLen.p,
                            (const int *)dFirst.p, nChunk, dLen.as<int>());
@@ -744,7 +744,7 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     D.steps = SP.totalSteps;
     D.chunks = SP.totalChunks;
     auto up = [&](void **dst, const void *src, size_t bytes) -> int {
-        MXL_TRY(hipMalloc(dst, std::max<size_t>(bytes, 4)));
+        MXL_TRY(mx::dev_malloc(dst, std::max<size_t>(bytes, 4)));
         if (bytes) MXL_TRY(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, s));
         return MX_OK;
     };
@@ -759,9 +759,9 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     if ((rc = up(&chunkStep0.p, SP.chunkStep0.data(), SP.chunkStep0.size() * 8))) return rc;
     // ---- the streams
     const size_t nEcol = ((size_t)SP.totalSteps + kSlicePadSteps) * 64 * E;
-    MXL_TRY(hipMalloc((void **)&D.ecol, nEcol * 2));
+    MXL_TRY(mx::dev_malloc((void **)&D.ecol, nEcol * 2));
     MXL_TRY(hipMemsetAsync(D.ecol, 0, nEcol * 2, s));
-    MXL_TRY(hipMalloc(&D.eval, nEcol * sizeof(V)));
+    MXL_TRY(mx::dev_malloc(&D.eval, nEcol * sizeof(V)));
     MXL_TRY(hipMemsetAsync(D.eval, 0, nEcol * sizeof(V), s));
     Buf codes;
     std::vector<unsigned char> dict;
@@ -771,13 +771,13 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
             if ((rc = device_value_dict<V>(val, nnz, codes, dict, &nDict, s))) return rc;
         }
         if (nDict > 0) {
-            MXL_TRY(hipMalloc((void **)&D.ecode, nEcol));
+            MXL_TRY(mx::dev_malloc((void **)&D.ecode, nEcol));
             MXL_TRY(hipMemsetAsync(D.ecode, 255, nEcol, s));
             if ((rc = up(&D.dict, dict.data(), dict.size()))) return rc;
             D.nDict = nDict;
         }
     }
-    MXL_TRY(hipMalloc((void **)&D.segIdx, nv1 * 4));
+    MXL_TRY(mx::dev_malloc((void **)&D.segIdx, nv1 * 4));
     MXL_TRY(hipMemsetAsync(D.segIdx, 0, nv1 * 4, s));
     if (SP.totalChunks > 0) {
         hipLaunchKernelGGL(vrow_places_kernel, grid(SP.totalChunks * 64), dim3(kBlock), 0, s, (const int *)sorted.p, (const int *)chunkFirst.p,
@@ -797,7 +797,7 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     }
     // ---- how the sums become y
     const size_t nInfo = ((size_t)rows + 3) / 4 * 4 + 4;
-    MXL_TRY(hipMalloc((void **)&D.rowInfo, nInfo * 4));
+    MXL_TRY(mx::dev_malloc((void **)&D.rowInfo, nInfo * 4));
     MXL_TRY(hipMemsetAsync(D.rowInfo, 0xfe, nInfo * 4, s));  // (overwritten below for the rows; the padding must read -2)
     {
         std::vector<int> fill(nInfo - (size_t)rows, -2);
@@ -806,10 +806,10 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     }
     Buf isLight, isHeavy, lightPos, heavyPos;
     const size_t r1 = (size_t)rows + 1;
-    MXL_TRY(hipMalloc(&isLight.p, r1 * 4));
-    MXL_TRY(hipMalloc(&isHeavy.p, r1 * 4));
-    MXL_TRY(hipMalloc(&lightPos.p, r1 * 4));
-    MXL_TRY(hipMalloc(&heavyPos.p, r1 * 4));
+    MXL_TRY(mx::dev_malloc(&isLight.p, r1 * 4));
+    MXL_TRY(mx::dev_malloc(&isHeavy.p, r1 * 4));
+    MXL_TRY(mx::dev_malloc(&lightPos.p, r1 * 4));
+    MXL_TRY(mx::dev_malloc(&heavyPos.p, r1 * 4));
     hipLaunchKernelGGL(row_info_kernel, grid((long long)rows + 1), dim3(kBlock), 0, s, (const int *)segPtr.p, (const int *)D.segIdx, elsewhere,
                        rows, kSliceLightSegs, D.rowInfo, isLight.as<int>(), isHeavy.as<int>(), over4, over4 + 1);
     MXL_TRY(hipGetLastError());
@@ -826,19 +826,19 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     D.mostVrows = std::max(mostVrows, nV > 0 ? 1 : 0);
     const int places = anyOver4 ? kSliceLightSegs : 4;
     D.lightQuads = places / 4;
-    MXL_TRY(hipMalloc((void **)&D.lightRow, ((size_t)nLight + 1) * 4));
+    MXL_TRY(mx::dev_malloc((void **)&D.lightRow, ((size_t)nLight + 1) * 4));
     MXL_TRY(hipMemsetAsync(D.lightRow, 0, ((size_t)nLight + 1) * 4, s));
-    MXL_TRY(hipMalloc((void **)&D.lightIdx, ((size_t)nLight * places + 8) * 4));
+    MXL_TRY(mx::dev_malloc((void **)&D.lightIdx, ((size_t)nLight * places + 8) * 4));
     MXL_TRY(hipMemsetAsync(D.lightIdx, 0xff, (size_t)nLight * places * 4, s));                    // -1 = no virtual row
     MXL_TRY(hipMemsetAsync(D.lightIdx + (size_t)nLight * places, 0, 8 * 4, s));                   // the spare entries read 0
-    MXL_TRY(hipMalloc((void **)&D.heavyInfo, ((size_t)nHeavy * 4 + 4) * 4));
+    MXL_TRY(mx::dev_malloc((void **)&D.heavyInfo, ((size_t)nHeavy * 4 + 4) * 4));
     MXL_TRY(hipMemsetAsync(D.heavyInfo, 0, ((size_t)nHeavy * 4 + 4) * 4, s));
     hipLaunchKernelGGL(row_lists_kernel, grid(rows), dim3(kBlock), 0, s, (const int *)segPtr.p, (const int *)D.segIdx, (const int *)isLight.p,
                        (const int *)isHeavy.p, (const int *)lightPos.p, (const int *)heavyPos.p, rows, places, D.lightRow, D.lightIdx,
                        D.heavyInfo);
     MXL_TRY(hipGetLastError());
     const size_t accBytes = dtype == MX_F64 ? 8 : 4;
-    MXL_TRY(hipMalloc(&D.partial, ((size_t)SP.totalChunks * 64 + 64) * accBytes));
+    MXL_TRY(mx::dev_malloc(&D.partial, ((size_t)SP.totalChunks * 64 + 64) * accBytes));
     MXL_TRY(hipMemsetAsync(D.partial, 0, ((size_t)SP.totalChunks * 64 + 64) * accBytes, s));
     if (fusedTaken) {
         // what the one-launch kernel needs beyond the two-launch arrays (which stay valid: the plan falls back on them)
@@ -852,16 +852,16 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
         if ((rc = up((void **)&D.wgGroups, SP.wgGroups.data(), SP.wgGroups.size() * 4))) return rc;
         if ((rc = up((void **)&D.groupNeed, SP.groupNeed.data(), SP.groupNeed.size() * 4))) return rc;
         const size_t nTarget = target.size() + 64;  // (64 spare entries, zero)
-        MXL_TRY(hipMalloc((void **)&D.fusedTarget, nTarget * 4));
+        MXL_TRY(mx::dev_malloc((void **)&D.fusedTarget, nTarget * 4));
         MXL_TRY(hipMemsetAsync(D.fusedTarget, 0, nTarget * 4, s));
         MXL_TRY(hipMemcpyAsync(D.fusedTarget, target.data(), target.size() * 4, hipMemcpyHostToDevice, s));
         const size_t nCount = (size_t)SP.nGroups + 1, nClaim = (size_t)SP.nWG + 1;
         const size_t sumBytes = ((size_t)SP.nGroups * fusedPlaces * kFusedGroupRows + 64) * accBytes;
-        MXL_TRY(hipMalloc((void **)&D.groupCount, nCount * 4));
+        MXL_TRY(mx::dev_malloc((void **)&D.groupCount, nCount * 4));
         MXL_TRY(hipMemsetAsync(D.groupCount, 0, nCount * 4, s));
-        MXL_TRY(hipMalloc((void **)&D.claim, nClaim * 4));
+        MXL_TRY(mx::dev_malloc((void **)&D.claim, nClaim * 4));
         MXL_TRY(hipMemsetAsync(D.claim, 0, nClaim * 4, s));
-        MXL_TRY(hipMalloc(&D.fusedSums, sumBytes));
+        MXL_TRY(mx::dev_malloc(&D.fusedSums, sumBytes));
         MXL_TRY(hipMemsetAsync(D.fusedSums, 0, sumBytes, s));
         MXL_TRY(hipStreamSynchronize(s));  // `target` leaves scope
         D.fused = true;
@@ -888,7 +888,7 @@ int check_csr_device(int rows, int cols, int nnz, const int *rowPtr_dev, const i
         return MX_ERR_ARG;
     }
     Buf bad;
-    MXL_TRY(hipMalloc(&bad.p, 256));
+    MXL_TRY(mx::dev_malloc(&bad.p, 256));
     MXL_TRY(hipMemsetAsync(bad.p, 0, 256, s));
     hipLaunchKernelGGL(check_csr_kernel, grid(std::max<long long>((long long)rows + 1, nnz)), dim3(kBlock), 0, s, rowPtr_dev, col_dev, rows,
                        cols, nnz, bad.as<int>());
@@ -910,7 +910,7 @@ int lines_per_gather_device(mx_dtype dtype, int nnz, const int *col_dev, hipStre
     *out = 1.0;
     if (sampled <= 0) return MX_OK;
     Buf sum;
-    MXL_TRY(hipMalloc(&sum.p, 256));
+    MXL_TRY(mx::dev_malloc(&sum.p, 256));
     MXL_TRY(hipMemsetAsync(sum.p, 0, 256, s));
     hipLaunchKernelGGL(window_lines_kernel, grid(sampled), dim3(kBlock), 0, s, col_dev, sampled, stride, 64 / elem_size(dtype),
                        sum.as<unsigned long long>());
@@ -936,18 +936,18 @@ int upload_csr_device(mx_dtype dtype, int rows, int cols, int nnz, const int *ro
     A.npt = csr_entries_per_lane(dtype);
     A.scan = scan;
     A.nBlocks = (int)desc.size() / 4;
-    MXL_TRY(hipMalloc((void **)&A.rowPtr, ((size_t)rows + 1) * 4));
+    MXL_TRY(mx::dev_malloc((void **)&A.rowPtr, ((size_t)rows + 1) * 4));
     MXL_TRY(hipMemcpyAsync(A.rowPtr, rowPtr_dev, ((size_t)rows + 1) * 4, hipMemcpyDeviceToDevice, s));
-    MXL_TRY(hipMalloc(&A.val, ((size_t)nnz + kCsrPad) * es));
+    MXL_TRY(mx::dev_malloc(&A.val, ((size_t)nnz + kCsrPad) * es));
     MXL_TRY(hipMemsetAsync((unsigned char *)A.val + (size_t)nnz * es, 0, (size_t)kCsrPad * es, s));
     if (nnz) MXL_TRY(hipMemcpyAsync(A.val, val_dev, (size_t)nnz * es, hipMemcpyDeviceToDevice, s));
-    MXL_TRY(hipMalloc((void **)&A.blockDesc, std::max<size_t>(desc.size(), 4) * 4));
+    MXL_TRY(mx::dev_malloc((void **)&A.blockDesc, std::max<size_t>(desc.size(), 4) * 4));
     if (!desc.empty()) MXL_TRY(hipMemcpyAsync(A.blockDesc, desc.data(), desc.size() * 4, hipMemcpyHostToDevice, s));
     bool narrow = mx::opt().csr_col16 && nnz > 0;
     Buf lo, wide;
     if (narrow) {
-        MXL_TRY(hipMalloc(&lo.p, std::max<size_t>((size_t)A.nBlocks, 1) * 4));
-        MXL_TRY(hipMalloc(&wide.p, 256));
+        MXL_TRY(mx::dev_malloc(&lo.p, std::max<size_t>((size_t)A.nBlocks, 1) * 4));
+        MXL_TRY(mx::dev_malloc(&wide.p, 256));
         MXL_TRY(hipMemsetAsync(wide.p, 0, 256, s));
         hipLaunchKernelGGL(block_ranges_kernel, grid((long long)A.nBlocks * 64), dim3(kBlock), 0, s, (const int4 *)A.blockDesc, col_dev,
                            A.nBlocks, lo.as<int>(), wide.as<int>());
@@ -958,7 +958,7 @@ int upload_csr_device(mx_dtype dtype, int rows, int cols, int nnz, const int *ro
         narrow = w == 0;
     }
     if (narrow) {
-        MXL_TRY(hipMalloc((void **)&A.col16, ((size_t)nnz + kCsrPad) * 2));
+        MXL_TRY(mx::dev_malloc((void **)&A.col16, ((size_t)nnz + kCsrPad) * 2));
         MXL_TRY(hipMemsetAsync(A.col16 + nnz, 0, (size_t)kCsrPad * 2, s));
         hipLaunchKernelGGL(narrow_columns_kernel, grid((long long)A.nBlocks * 64), dim3(kBlock), 0, s, (const int4 *)A.blockDesc, col_dev,
                            (const int *)lo.p, A.nBlocks, A.col16);
@@ -973,14 +973,14 @@ int upload_csr_device(mx_dtype dtype, int rows, int cols, int nnz, const int *ro
             if (rc) return rc;
             if (nd > 0) {
                 A.codes = (unsigned char *)codes.take();
-                MXL_TRY(hipMalloc(&A.dict, dict.size()));
+                MXL_TRY(mx::dev_malloc(&A.dict, dict.size()));
                 MXL_TRY(hipMemcpyAsync(A.dict, dict.data(), dict.size(), hipMemcpyHostToDevice, s));
                 MXL_TRY(hipStreamSynchronize(s));
                 A.nDict = nd;
             }
         }
     } else {
-        MXL_TRY(hipMalloc((void **)&A.col, ((size_t)nnz + kCsrPad) * 4));
+        MXL_TRY(mx::dev_malloc((void **)&A.col, ((size_t)nnz + kCsrPad) * 4));
         MXL_TRY(hipMemsetAsync(A.col + nnz, 0, (size_t)kCsrPad * 4, s));
         if (nnz) MXL_TRY(hipMemcpyAsync(A.col, col_dev, (size_t)nnz * 4, hipMemcpyDeviceToDevice, s));
     }

@@ -350,7 +350,7 @@ struct Buf {
     Buf &operator=(const Buf &) = delete;
     ~Buf()
     {
-        if (p) (void)hipFree(p);
+        if (p) (void)mx::dev_free(p);
     }
 };
 inline dim3 grid(long long n) { return dim3((unsigned)((std::max<long long>(n, 1) + kBlock - 1) / kBlock)); }
@@ -393,12 +393,12 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     Buf lists, count, units, unit0, totals, tmp;
     size_t scanBytes = 0;
     MXO_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, (size_t)nChunks + 1, rocprim::plus<int>(), s));
-    MXO_TRY(hipMalloc(&lists.p, (size_t)nChunks * kMaxOffsets * 4));
-    MXO_TRY(hipMalloc(&count.p, ((size_t)nChunks + 1) * 4));
-    MXO_TRY(hipMalloc(&units.p, ((size_t)nChunks + 1) * 4));
-    MXO_TRY(hipMalloc(&unit0.p, ((size_t)nChunks + 1) * 4));
-    MXO_TRY(hipMalloc(&totals.p, 256));
-    MXO_TRY(hipMalloc(&tmp.p, scanBytes + 256));
+    MXO_TRY(mx::dev_malloc(&lists.p, (size_t)nChunks * kMaxOffsets * 4));
+    MXO_TRY(mx::dev_malloc(&count.p, ((size_t)nChunks + 1) * 4));
+    MXO_TRY(mx::dev_malloc(&units.p, ((size_t)nChunks + 1) * 4));
+    MXO_TRY(mx::dev_malloc(&unit0.p, ((size_t)nChunks + 1) * 4));
+    MXO_TRY(mx::dev_malloc(&totals.p, 256));
+    MXO_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
     MXO_TRY(hipMemsetAsync(totals.p, 0, 256, s));
     int *tot = (int *)totals.p;
     hipLaunchKernelGGL(offset_lists_kernel, dim3(nChunks), dim3(64), 0, s, rowPtr_dev, col_dev, rows, chunkRows, (int *)lists.p, (int *)count.p, tot);
@@ -445,11 +445,11 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
         return code;
     };
     auto body = [&]() -> int {
-        MXO_TRY(hipMalloc((void **)&D.chunk, (size_t)nChunks * 16));
-        MXO_TRY(hipMalloc((void **)&D.offs, (size_t)D.nOffs * 4));
-        MXO_TRY(hipMalloc(&D.stream, (size_t)D.units * 64 * unitBytes));
+        MXO_TRY(mx::dev_malloc((void **)&D.chunk, (size_t)nChunks * 16));
+        MXO_TRY(mx::dev_malloc((void **)&D.offs, (size_t)D.nOffs * 4));
+        MXO_TRY(mx::dev_malloc(&D.stream, (size_t)D.units * 64 * unitBytes));
         if (D.nDict > 0) {
-            MXO_TRY(hipMalloc(&D.dict, dict.size()));
+            MXO_TRY(mx::dev_malloc(&D.dict, dict.size()));
             MXO_TRY(hipMemcpyAsync(D.dict, dict.data(), dict.size(), hipMemcpyHostToDevice, s));
         }
         int *bad = tot + 3;

@@ -72,9 +72,9 @@ static int cdspmv_any(mx_dtype dtype, const void *csrVal, const int *csrRowPtr, 
     };
     rc = body();
     free_csr(plan.csr);
-    (void)hipFree(dx);
-    (void)hipFree(dy);
-    (void)hipFree(dscratch);
+    (void)mx::dev_free(dx);
+    (void)mx::dev_free(dy);
+    (void)mx::dev_free(dscratch);
     if (plan.ev0) (void)hipEventDestroy(plan.ev0);
     if (plan.ev1) (void)hipEventDestroy(plan.ev1);
     if (plan.stream) (void)hipStreamDestroy(plan.stream);
@@ -154,9 +154,9 @@ static int du_any(mx_dtype dtype, const int *chunkPtr, const int *fragPtr, const
     };
     rc = body();
     free_tiles(T);
-    (void)hipFree(dx);
-    (void)hipFree(dy);
-    (void)hipFree(dscratch);
+    (void)mx::dev_free(dx);
+    (void)mx::dev_free(dy);
+    (void)mx::dev_free(dscratch);
     if (plan.ev0) (void)hipEventDestroy(plan.ev0);
     if (plan.ev1) (void)hipEventDestroy(plan.ev1);
     if (plan.stream) (void)hipStreamDestroy(plan.stream);
@@ -194,9 +194,9 @@ extern "C" int mx_probe_mfma_f64(const double *A, const double *B, double *D)
         return MX_OK;
     };
     rc = body();
-    (void)hipFree(dA);
-    (void)hipFree(dB);
-    (void)hipFree(dD);
+    (void)mx::dev_free(dA);
+    (void)mx::dev_free(dB);
+    (void)mx::dev_free(dD);
     return rc;
 }
 
@@ -217,9 +217,9 @@ extern "C" int mx_probe_mfma_f16(const uint16_t *A, const uint16_t *B, float *D)
         return MX_OK;
     };
     rc = body();
-    (void)hipFree(dA);
-    (void)hipFree(dB);
-    (void)hipFree(dD);
+    (void)mx::dev_free(dA);
+    (void)mx::dev_free(dB);
+    (void)mx::dev_free(dD);
     return rc;
 }
 

@@ -30,22 +30,23 @@ extern "C" int mx_device_count(void)
 
 void mx::free_offsets(mx::DeviceOffsets &D)
 {
-    (void)hipFree(D.chunk);
-    (void)hipFree(D.offs);
-    (void)hipFree(D.stream);
-    (void)hipFree(D.dict);
+    (void)mx::dev_free(D.chunk);
+    (void)mx::dev_free(D.offs);
+    (void)mx::dev_free(D.stream);
+    (void)mx::dev_free(D.dict);
     D = mx::DeviceOffsets();
 }
 
 extern "C" void mx_plan_destroy(mx_plan *plan)
 {
     if (!plan) return;
+    mx::IdleFrees idle;
     free_csr(plan->csr);
     free_slices(plan->slices);
     mx::free_offsets(plan->offsets);
     free_tiles(plan->tiles);
     free_tiles(plan->strips);
-    (void)hipFree(plan->ywide);
+    (void)mx::dev_free(plan->ywide);
     if (plan->ev0) (void)hipEventDestroy(plan->ev0);
     if (plan->ev1) (void)hipEventDestroy(plan->ev1);
     if (plan->stream) (void)hipStreamDestroy(plan->stream);
@@ -336,22 +337,21 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
         if (!e) e = upload(&ci, col, (size_t)nnz);
         if (!e) e = upload_bytes(&va, val, (size_t)nnz * es);
         if (!e) e = try_offsets(plan, nnz, rp, ci, va, flags, &took);
-        (void)hipFree(rp);
-        (void)hipFree(ci);
-        (void)hipFree(va);
+        (void)mx::dev_free(rp);
+        (void)mx::dev_free(ci);
+        (void)mx::dev_free(va);
         if (e || took) return e;
     }
-    hipDeviceProp_t prop;
-    int dev = 0;
-    MX_HIP(hipGetDevice(&dev));
-    MX_HIP(hipGetDeviceProperties(&prop, dev));
-    const int nCU = std::max(1, prop.multiProcessorCount);
+    int nCU = 1;
+    if (int e = compute_units(&nCU)) return e;
     const int S = slice_count(plan->dtype, rows, cols, nnz, nCU);
     CsrChoice pick = choose_csr_form(plan->dtype, rows, cols, rowPtr, col, val, flags, nCU, S, stripRows == nullptr);
     bool(&want)[3] = pick.want;
     plan->est_rows_us = pick.usRows;
     plan->est_slices_us = pick.usSlices;
     const bool autotune = plan_autotune();
+    if (autotune)
+        if (int e = plan_stream(plan)) return e;
     // the split: rows of at least split_length() entries, when they hold a good part of the matrix
     std::vector<char> longRow;
     int longNnz = 0, longRows = 0;
@@ -375,7 +375,7 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
         int e = upload_bytes(&tx, nullptr, 0, std::max<size_t>(cols * es, 16));
         if (e) return e;
         if ((e = upload_bytes(&ty, nullptr, 0, std::max<size_t>(rows * es, 16)))) {
-            (void)hipFree(tx);
+            (void)mx::dev_free(tx);
             tx = nullptr;
         }
         return e;
@@ -462,8 +462,8 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
         free_csr(C);
         free_slices(L);
     }
-    (void)hipFree(tx);
-    (void)hipFree(ty);
+    (void)mx::dev_free(tx);
+    (void)mx::dev_free(ty);
     if (!rc) decide_keep(plan, flags);
     return rc;
 }
@@ -909,6 +909,7 @@ static int create_plan(const mx_partition *P, int flags, mx_plan **out, bool noB
     *out = nullptr;
     int rc = need_device();
     if (rc) return rc;
+    mx::MemScope scope(nullptr);
     mx_plan *plan = new (std::nothrow) mx_plan();
     if (!plan) {
         set_error("mx_plan_create: out of memory");
@@ -928,11 +929,6 @@ static int create_plan(const mx_partition *P, int flags, mx_plan **out, bool noB
         mx_plan_destroy(plan);
         return code;
     };
-    if (hipStreamCreate(&plan->stream) != hipSuccess || hipEventCreate(&plan->ev0) != hipSuccess ||
-        hipEventCreate(&plan->ev1) != hipSuccess) {
-        set_error("mx_plan_create: could not create stream/events");
-        return fail(MX_ERR_DEVICE);
-    }
     {
         // set-up: the address of the fixed array of mx_spmv_static on this device (kept per device)
         void *fixed = nullptr;

@@ -30,11 +30,8 @@ static int setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, 
     const int rows = plan->rows, cols = plan->cols;
     int rc;
     plan->csr_nnz = nnz;
-    hipDeviceProp_t prop;
-    int dev = 0;
-    MX_HIP(hipGetDevice(&dev));
-    MX_HIP(hipGetDeviceProperties(&prop, dev));
-    const int nCU = std::max(1, prop.multiProcessorCount);
+    int nCU = 1;
+    if ((rc = compute_units(&nCU))) return rc;
     const int S = rows > 0 ? slice_count(dtype, rows, cols, nnz, nCU) : 0;
     if (alone && may_look_for_form(flags)) {
         bool took = false;
@@ -135,6 +132,7 @@ extern "C" int mx_plan_create_device_csr(mx_dtype dtype, int rows, int cols, int
     *out = nullptr;
     int rc = need_device();
     if (rc) return rc;
+    mx::MemScope scope(nullptr);
     if ((rc = mx::check_csr_device(rows, cols, nnz, rowPtr_dev, colInd_dev, nullptr, "mx_plan_create_device_csr"))) return rc;
     mx_plan *plan = new (std::nothrow) mx_plan();
     if (!plan) {
@@ -151,11 +149,6 @@ extern "C" int mx_plan_create_device_csr(mx_dtype dtype, int rows, int cols, int
         mx_plan_destroy(plan);
         return code;
     };
-    if (hipStreamCreate(&plan->stream) != hipSuccess || hipEventCreate(&plan->ev0) != hipSuccess ||
-        hipEventCreate(&plan->ev1) != hipSuccess) {
-        set_error("mx_plan_create_device_csr: could not create stream/events");
-        return fail(MX_ERR_DEVICE);
-    }
     {
         void *fixed = nullptr;
         if (mx::static_scratch(&fixed) != hipSuccess) {
@@ -311,6 +304,7 @@ int mxp::create_plan_device(mx_dtype dtype, int rows, int cols, int nnz, const i
 {
     const char *who = twin ? "mx_plan_create" : "mx_plan_create_device";
     int rc;
+    mx::MemScope scope(nullptr);
     if (!twin) {
         if (!out || (dtype != MX_F64 && dtype != MX_F16) || rows < 1 || cols < 1 || nnz < 0 || !rowPtr_dev ||
             (nnz > 0 && (!colInd_dev || !val_dev)) || !(tau_c >= 0.0f && tau_c <= 1.0f) || !(tau_r >= 0.0f && tau_r <= 1.0f)) {
@@ -332,10 +326,10 @@ int mxp::create_plan_device(mx_dtype dtype, int rows, int cols, int nnz, const i
     void *partVal = nullptr;
     char *stripRows = nullptr;
     auto fail = [&](int code) {
-        (void)hipFree(partPtr);
-        (void)hipFree(partCol);
-        (void)hipFree(partVal);
-        (void)hipFree(stripRows);
+        (void)mx::dev_free(partPtr);
+        (void)mx::dev_free(partCol);
+        (void)mx::dev_free(partVal);
+        (void)mx::dev_free(stripRows);
         partPtr = partCol = nullptr;
         partVal = nullptr;
         stripRows = nullptr;
@@ -344,11 +338,8 @@ int mxp::create_plan_device(mx_dtype dtype, int rows, int cols, int nnz, const i
         return code;
     };
     try {
-        hipDeviceProp_t prop;
-        int dev = 0;
-        MX_HIP(hipGetDevice(&dev));
-        MX_HIP(hipGetDeviceProperties(&prop, dev));
-        const int nCU = std::max(1, prop.multiProcessorCount);
+        int nCU = 1;
+        if ((rc = compute_units(&nCU))) return rc;
         const int fragM = mx::kFragM, fragK = mx::frag_k(dtype);
         const bool noTiles = (flags & MX_PLAN_NO_TILES) != 0, allTiles = !noTiles && (flags & MX_PLAN_ALL_TILES) != 0;
         const bool wantStrips = dtype == MX_F16 && !noTiles && !allTiles && !mx::opt().no_strips;
@@ -392,11 +383,6 @@ int mxp::create_plan_device(mx_dtype dtype, int rows, int cols, int nnz, const i
         plan->ext_dRows = cnt.dRows;
         plan->ext_nnzRowD = cnt.nnzRowD;
         plan->ext_frags = cnt.frags;
-        if (hipStreamCreate(&plan->stream) != hipSuccess || hipEventCreate(&plan->ev0) != hipSuccess ||
-            hipEventCreate(&plan->ev1) != hipSuccess) {
-            set_error(std::string(who) + ": could not create stream/events");
-            return fail(MX_ERR_DEVICE);
-        }
         {
             void *fixed = nullptr;
             if (mx::static_scratch(&fixed) != hipSuccess) {
@@ -501,10 +487,10 @@ int mxp::create_plan_device(mx_dtype dtype, int rows, int cols, int nnz, const i
             // (general tiles share rows with the CSR part: its sums stay binary32 until the tile kernel has added its own)
             if ((rc = upload_bytes(&plan->ywide, nullptr, 0, (size_t)std::max(rows, 1) * sizeof(float)))) return fail(rc);
         }
-        (void)hipFree(partPtr);
-        (void)hipFree(partCol);
-        (void)hipFree(partVal);
-        (void)hipFree(stripRows);
+        (void)mx::dev_free(partPtr);
+        (void)mx::dev_free(partCol);
+        (void)mx::dev_free(partVal);
+        (void)mx::dev_free(stripRows);
         decide_keep(plan, flags);  // (again, now that the tile part is known: it counts towards what a product touches)
         *out = plan;
         return MX_OK;

@@ -37,12 +37,14 @@ inline int upload(T **dst, const T *src, size_t n, size_t pad = 0)
 {
     *dst = nullptr;
     const size_t total = std::max<size_t>(n + pad, 1);
-    MX_HIP(hipMalloc((void **)dst, total * sizeof(T)));
+    MX_HIP(mx::dev_malloc((void **)dst, total * sizeof(T)));
     if (pad || n == 0) MX_HIP(hipMemset(*dst, 0, total * sizeof(T)));
     if (n) MX_HIP(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
     return MX_OK;
 }
 int upload_bytes(void **dst, const void *src, size_t n, size_t pad = 0);
+// Compute units of the current device (asked for once per device).
+int compute_units(int *n);
 void pack_rows(const int *rowPtr, int rows, int npt, std::vector<int> &desc);
 void free_csr(mx::DeviceCsr &A);
 void free_tiles(mx::DeviceTiles &T);
@@ -154,11 +156,22 @@ struct mx_plan {
     // the fill a fragment needed); the product looks at these, never at the environment
     int opt_flags = mxp::plan_opt_flags();
     double opt_tile_gate = mx::opt().tile_gate >= 0.0 ? mx::opt().tile_gate : 0.5;
+    // made when something is first timed or run on them (mxp::plan_stream)
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 
 namespace mxp {
+
+// The plan's own stream and its two events: a plan that only ever runs on its callers' streams does without them
+// (making them costs as much as a small plan).
+inline int plan_stream(mx_plan *plan)
+{
+    if (!plan->stream) MX_HIP(hipStreamCreate(&plan->stream));
+    if (!plan->ev0) MX_HIP(hipEventCreate(&plan->ev0));
+    if (!plan->ev1) MX_HIP(hipEventCreate(&plan->ev1));
+    return MX_OK;
+}
 
 // Mean milliseconds per iteration of `body` over `iters` back-to-back runs after `warm`
 // untimed ones, by events on the stream the kernels run on.

@@ -356,9 +356,12 @@ __global__ __launch_bounds__(kBlock) void narrow_bits_kernel(const unsigned long
 
 struct Scratch {
     void *p = nullptr;
+    Scratch() = default;
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
     ~Scratch()
     {
-        if (p) (void)hipFree(p);
+        if (p) (void)mx::dev_free(p);
     }
 };
 
@@ -389,6 +392,7 @@ extern "C" int mx_transpose_device(mx_dtype dtype, int outer, int inner, int nnz
         return MX_ERR_ARG;
     }
     hipStream_t s = (hipStream_t)stream;
+    mx::MemScope scope(s);
     const int pblocks = (int)(((long long)nnz + 1 + kBlock - 1) / kBlock);
     if (nnz == 0) {
         hipLaunchKernelGGL(line_pointers_kernel, dim3(pblocks), dim3(kBlock), 0, s, (const int *)nullptr, 0, inner, tPtr_dev);
@@ -404,7 +408,7 @@ extern "C" int mx_transpose_device(mx_dtype dtype, int outer, int inner, int nnz
                                       (int *)nullptr, (size_t)nnz, 0u, (unsigned)bits, s));
     const size_t n4 = ((size_t)nnz * sizeof(int) + 255) & ~(size_t)255;
     Scratch scratch;
-    MXP_TRY(hipMalloc(&scratch.p, 4 * n4 + 256 + sortBytes));
+    MXP_TRY(mx::dev_malloc(&scratch.p, 4 * n4 + 256 + sortBytes));
     unsigned char *base = (unsigned char *)scratch.p;
     int *line = (int *)base, *payIn = (int *)(base + n4), *payOut = (int *)(base + 2 * n4), *keyOut = (int *)(base + 3 * n4);
     int *bad = (int *)(base + 4 * n4);
@@ -487,6 +491,7 @@ extern "C" int mx_select_device(int rows, int cols, int nnz, const int *rowPtr_d
         return MX_ERR_ARG;
     }
     hipStream_t s = (hipStream_t)stream;
+    mx::MemScope scope(s);
     *out = mx_selection{0, 0, 0, 0};
     const size_t n = (size_t)std::max(rows, cols);
     size_t sortBytes = 0, scanBytes = 0;
@@ -500,7 +505,7 @@ extern "C" int mx_select_device(int rows, int cols, int nnz, const int *rowPtr_d
     const size_t cntB = (n * sizeof(int) + 255) & ~(size_t)255, workB = ((3 * n + 4) * sizeof(int) + 255) & ~(size_t)255;
     const size_t denseB = ((size_t)cols + 255) & ~(size_t)255;
     Scratch scratch;
-    MXP_TRY(hipMalloc(&scratch.p, cntB + workB + 256 + denseB + sortBytes + scanBytes + 256));
+    MXP_TRY(mx::dev_malloc(&scratch.p, cntB + workB + 256 + denseB + sortBytes + scanBytes + 256));
     unsigned char *base = (unsigned char *)scratch.p;
     int *cnt = (int *)base, *work = (int *)(base + cntB), *bad = (int *)(base + cntB + workB);
     unsigned char *dense = base + cntB + workB + 256;
@@ -562,6 +567,7 @@ extern "C" int mx_split_device(mx_dtype dtype, int rows, int cols, int nnz, cons
         return MX_ERR_ARG;
     }
     hipStream_t s = (hipStream_t)stream;
+    mx::MemScope scope(s);
     const int dCols = sel->dCols, dRows = sel->dRows, nDD = sel->nnzRowD;
     int colBits = 1, rowBits = 1;
     while (colBits < 31 && (1ll << colBits) < (long long)cols) ++colBits;
@@ -579,7 +585,7 @@ extern "C" int mx_split_device(mx_dtype dtype, int rows, int cols, int nnz, cons
     const size_t denseB = al((size_t)cols + 1), keyB = al((size_t)nnz * 8), payB = al((size_t)nnz * 4);
     // newCol, notSel, pos [cols+1]; rowRank, rcnt, cdLen, ddLen [rows+1]; dense; keys and payloads in and out
     Scratch scratch;
-    MXP_TRY(hipMalloc(&scratch.p, 3 * colB + 4 * rowB + denseB + 2 * keyB + 2 * payB + sortBytes + scanBytes + 256));
+    MXP_TRY(mx::dev_malloc(&scratch.p, 3 * colB + 4 * rowB + denseB + 2 * keyB + 2 * payB + sortBytes + scanBytes + 256));
     unsigned char *b = (unsigned char *)scratch.p;
     int *newCol = (int *)b, *notSel = (int *)(b + colB), *pos = (int *)(b + 2 * colB);
     b += 3 * colB;
@@ -671,7 +677,7 @@ extern "C" int mx_split_device(mx_dtype dtype, int rows, int cols, int nnz, cons
 extern "C" void mx_tiles_device_free(mx_device_tiles *t)
 {
     if (!t) return;
-    if (t->base) (void)hipFree(t->base);
+    if (t->base) (void)mx::dev_free(t->base);
     *t = mx_device_tiles{};
 }
 
@@ -690,6 +696,7 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
         return MX_ERR_ARG;
     }
     hipStream_t s = (hipStream_t)stream;
+    mx::MemScope scope(s);
     *out = mx_device_tiles{};
     const int fragK = mx::frag_k(dtype), n = nnzRowD, chunkNum = (dRows + mx::kFragM - 1) / mx::kFragM;
     const size_t es = (size_t)mx::elem_size(dtype);
@@ -716,7 +723,7 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
     // scratch: keys and payloads in and out, heads, their running count, ecr, per-chunk fragments
     const size_t keyB = al((size_t)n * 8), intB = al(((size_t)n + 1) * 4), chB = al(((size_t)chunkNum + 1) * 4);
     Scratch scratch;
-    MXP_TRY(hipMalloc(&scratch.p, 2 * keyB + 5 * intB + 2 * chB + sortBytes + scanBytes + 256));
+    MXP_TRY(mx::dev_malloc(&scratch.p, 2 * keyB + 5 * intB + 2 * chB + sortBytes + scanBytes + 256));
     unsigned char *b = (unsigned char *)scratch.p;
     unsigned long long *keyIn = (unsigned long long *)b, *keyOut = (unsigned long long *)(b + keyB);
     b += 2 * keyB;
@@ -766,7 +773,7 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
     const size_t cpB = al(((size_t)chunkNum + 1) * 4), axB = al((size_t)totalTcFrags * fragK * 4 + 4),
                  fpB = al(((size_t)totalTcFrags + 1) * 4), fbB = al((size_t)totalTcFrags * 8 + 8), tvB = al((size_t)n * es + 8);
     Scratch outBlock;
-    MXP_TRY(hipMalloc(&outBlock.p, cpB + axB + fpB + fbB + tvB));
+    MXP_TRY(mx::dev_malloc(&outBlock.p, cpB + axB + fpB + fbB + tvB));
     unsigned char *o = (unsigned char *)outBlock.p;
     int *chunkPtr = (int *)o, *atox = (int *)(o + cpB), *fragPtr = (int *)(o + cpB + axB);
     unsigned long long *bits = (unsigned long long *)(o + cpB + axB + fpB);
@@ -836,8 +843,9 @@ void twin_free(void *w)
 {
     mx::PartitionTwin *W = (mx::PartitionTwin *)w;
     if (!W) return;
-    (void)hipFree(W->order);
-    (void)hipFree(W->split);
+    mx::IdleFrees idle;
+    (void)mx::dev_free(W->order);
+    (void)mx::dev_free(W->split);
     mx_tiles_device_free(&W->T);
     delete W;
 }
@@ -917,6 +925,7 @@ extern "C" int mx_partition_create_device(const mx_csr *A, float tau_c, float ta
         return MX_ERR_DEVICE;
     }
     (void)who;
+    mx::MemScope scope(nullptr);
     const int rows = A->rows, cols = A->cols, nnz = A->nnz;
     const size_t es = (size_t)mx::elem_size(A->dtype);
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -937,11 +946,11 @@ extern "C" int mx_partition_create_device(const mx_csr *A, float tau_c, float ta
     const size_t rpB = al(((size_t)rows + 1) * 4), ciB = al((size_t)nnz * 4 + 4), vaB = al((size_t)nnz * es + 8),
                  dcB = al((size_t)cols * 4 + 4), drB = al((size_t)rows * 4 + 4);
     Scratch in;
-    MXP_TRY(hipMalloc(&in.p, rpB + ciB + vaB));
+    MXP_TRY(mx::dev_malloc(&in.p, rpB + ciB + vaB));
     unsigned char *b = (unsigned char *)in.p;
     int *rp = (int *)b, *ci = (int *)(b + rpB);
     void *va = b + rpB + ciB;
-    MXP_TRY(hipMalloc(&W->order, dcB + drB));
+    MXP_TRY(mx::dev_malloc(&W->order, dcB + drB));
     W->dc = (int *)W->order;
     W->dr = (int *)((unsigned char *)W->order + dcB);
     int *dc = W->dc, *dr = W->dr;
@@ -956,7 +965,7 @@ extern "C" int mx_partition_create_device(const mx_csr *A, float tau_c, float ta
     const int nDD = sel.nnzRowD, nCD = nnz - nDD;
     const size_t ddpB = al(((size_t)sel.dRows + 1) * 4), ddcB = al((size_t)nDD * 4 + 4), ddvB = al((size_t)nDD * es + 8),
                  cdpB = al(((size_t)rows + 1) * 4), cdcB = al((size_t)nCD * 4 + 4), cdvB = al((size_t)nCD * es + 8);
-    MXP_TRY(hipMalloc(&W->split, ddpB + ddcB + ddvB + cdpB + cdcB + cdvB));
+    MXP_TRY(mx::dev_malloc(&W->split, ddpB + ddcB + ddvB + cdpB + cdcB + cdvB));
     b = (unsigned char *)W->split;
     W->ddp = (int *)b;
     W->ddc = (int *)(b + ddpB);

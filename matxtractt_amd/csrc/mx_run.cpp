@@ -182,10 +182,12 @@ extern "C" int mx_spmv_host(mx_plan *plan, const void *x_host, void *y_host)
         return MX_ERR_ARG;
     }
     const size_t es = (size_t)mx::elem_size(plan->dtype);
+    if (int bad = plan_stream(plan)) return bad;
+    mx::MemScope scope(plan->stream);
     void *dx = nullptr, *dy = nullptr;
-    MX_HIP(hipMalloc(&dx, std::max<size_t>(plan->cols * es, 1)));
-    if (hipMalloc(&dy, std::max<size_t>(plan->rows * es, 1)) != hipSuccess) {
-        (void)hipFree(dx);
+    MX_HIP(mx::dev_malloc(&dx, std::max<size_t>(plan->cols * es, 1)));
+    if (mx::dev_malloc(&dy, std::max<size_t>(plan->rows * es, 1)) != hipSuccess) {
+        (void)mx::dev_free(dx);
         set_error("mx_spmv_host: hipMalloc failed");
         return MX_ERR_DEVICE;
     }
@@ -199,8 +201,8 @@ extern "C" int mx_spmv_host(mx_plan *plan, const void *x_host, void *y_host)
         return MX_OK;
     };
     rc = body();
-    (void)hipFree(dx);
-    (void)hipFree(dy);
+    (void)mx::dev_free(dx);
+    (void)mx::dev_free(dy);
     return rc;
 }
 
@@ -210,6 +212,7 @@ extern "C" int mx_time_csr_main(mx_plan *plan, const void *x_dev, void *y_dev, i
         set_error("mx_time_csr_main: bad argument");
         return MX_ERR_ARG;
     }
+    if (int bad = plan_stream(plan)) return bad;
     hipStream_t s = plan->stream;
     if (int bad = check_x(plan, x_dev, "mx_time_csr_main")) return bad;
     int rc = time_loop(plan, warm, iters, [&]() -> int {
@@ -236,6 +239,7 @@ extern "C" int mx_time(mx_plan *plan, const void *x_dev, void *y_dev, int warm, 
         set_error("mx_time: bad argument");
         return MX_ERR_ARG;
     }
+    if (int bad = plan_stream(plan)) return bad;
     hipStream_t s = plan->stream;
     int rc;
     double t = 0.0;
@@ -311,6 +315,7 @@ extern "C" int mx_time_rotate(mx_plan *const *plans, const void *const *x_dev, v
             return MX_ERR_ARG;
         }
     mx_plan *first = plans[0];
+    if (int bad = plan_stream(first)) return bad;
     hipStream_t s = first->stream;
     int turn = 0;
     return time_loop(first, warm, iters, [&]() -> int {
@@ -332,6 +337,7 @@ extern "C" int mx_time_kernels(mx_plan *plan, const void *x_dev, void *y_dev, in
         set_error("mx_time_kernels: bad argument");
         return MX_ERR_ARG;
     }
+    if (int bad = plan_stream(plan)) return bad;
     hipStream_t s = plan->stream;
     const double es = mx::elem_size(plan->dtype);
     const char *vt = plan->dtype == MX_F64 ? "f64" : "f16";

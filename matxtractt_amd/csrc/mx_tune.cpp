@@ -36,7 +36,7 @@ extern "C" int mx_tune_tau(const mx_csr *A, int levels, int flags, int warm, int
         mx_init_vec(A->dtype, hx.data(), A->cols);
         if ((rc = upload_bytes(&dx, hx.data(), hx.size()))) return rc;
         if ((rc = upload_bytes(&dy, nullptr, 0, std::max<size_t>((size_t)A->rows * es, 16)))) {
-            (void)hipFree(dx);
+            (void)mx::dev_free(dx);
             return rc;
         }
     }
@@ -47,11 +47,11 @@ extern "C" int mx_tune_tau(const mx_csr *A, int levels, int flags, int warm, int
     int *dRowPtr = nullptr, *dColInd = nullptr;
     void *dVal = nullptr;
     auto release = [&]() {
-        (void)hipFree(dx);
-        (void)hipFree(dy);
-        (void)hipFree(dRowPtr);
-        (void)hipFree(dColInd);
-        (void)hipFree(dVal);
+        (void)mx::dev_free(dx);
+        (void)mx::dev_free(dy);
+        (void)mx::dev_free(dRowPtr);
+        (void)mx::dev_free(dColInd);
+        (void)mx::dev_free(dVal);
     };
     if (onDevice) {
         rc = upload(&dRowPtr, A->rowPtr, (size_t)A->rows + 1);
@@ -135,9 +135,9 @@ extern "C" int mx_estimate_tau(const mx_csr *A, int levels, float *tau_c, float 
     int *dRowPtr = nullptr, *dColInd = nullptr;
     void *dVal = nullptr;
     auto release = [&]() {
-        (void)hipFree(dRowPtr);
-        (void)hipFree(dColInd);
-        (void)hipFree(dVal);
+        (void)mx::dev_free(dRowPtr);
+        (void)mx::dev_free(dColInd);
+        (void)mx::dev_free(dVal);
     };
     rc = upload(&dRowPtr, A->rowPtr, (size_t)A->rows + 1);
     if (!rc) rc = upload(&dColInd, A->colInd, (size_t)A->nnz);

@@ -1,8 +1,13 @@
-// Error text and binary16 conversions shared by the host code.
+// Error text, binary16 conversions and the device memory kept between calls, shared by the host code.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <mutex>
+#include <unordered_map>
+#include <vector>
 
+#include "mx_device.h"
 #include "mx_internal.h"
 
 namespace mx {
@@ -107,3 +112,214 @@ extern "C" const char *mx_last_error(void) { return mx::g_error.c_str(); }
 
 extern "C" uint16_t mx_f32_to_f16(float f) { return mx::f64_to_f16_bits((double)f); }
 extern "C" float mx_f16_to_f32(uint16_t h) { return mx::f16_bits_to_f32(h); }
+
+// ---- device memory kept from one call to the next --------------------------------------------------------
+namespace mx {
+namespace {
+
+// A block of at least this many bytes is handed out for a request when it is not more than an eighth (and
+// 64 KB) larger.
+size_t block_bytes(size_t n)
+{
+    if (n < 512) return 512;
+    size_t step = 256;  // an eighth of the largest power of two in n, at least 256 bytes, at most 2 MB
+    while (step * 16 <= n && step < ((size_t)2 << 20)) step *= 2;
+    return (n + step - 1) / step * step;
+}
+
+struct Block {
+    size_t bytes;
+    int dev;
+};
+struct Idle {
+    void *p;
+    uint64_t stamp;  // number of the call that gave it back
+};
+constexpr int kPoolDevices = 64;
+constexpr uint64_t kPoolCalls = 64;   // a block nobody has asked for in so many calls goes back to the device
+constexpr size_t kPoolShare = 128;    // idle blocks hold at most this fraction of a device's memory (2.25 GB of 288)
+
+struct Pool {
+    std::mutex mu;
+    std::unordered_map<void *, Block> blocks;            // every block made here, in use or idle
+    std::multimap<size_t, Idle> idle[kPoolDevices];      // by size; no work on the device touches them any more
+    size_t idleBytes[kPoolDevices] = {}, limit[kPoolDevices] = {};
+    uint64_t calls = 0;
+};
+Pool &pool()
+{
+    static Pool *p = new Pool();  // (never destroyed: plans may be released by destructors that run after this file's)
+    return *p;
+}
+
+// What the calling thread has given back inside its current MemScope.
+struct ThreadScope {
+    int depth = 0, idleFrees = 0;
+    hipStream_t stream = nullptr;
+    std::multimap<size_t, void *> freed;
+};
+thread_local ThreadScope t_scope;
+
+// (with the lock held) blocks beyond the bound, and blocks nobody has asked for in a while, oldest first
+void trim(Pool &P, int dev, std::vector<void *> &out, bool all)
+{
+    auto &I = P.idle[dev];
+    for (;;) {
+        auto oldest = I.end();
+        for (auto it = I.begin(); it != I.end(); ++it)
+            if (oldest == I.end() || it->second.stamp < oldest->second.stamp) oldest = it;
+        if (oldest == I.end() || !(all || P.idleBytes[dev] > P.limit[dev] || oldest->second.stamp + kPoolCalls < P.calls)) return;
+        P.idleBytes[dev] -= oldest->first;
+        P.blocks.erase(oldest->second.p);
+        out.push_back(oldest->second.p);
+        I.erase(oldest);
+    }
+}
+void put_idle(Pool &P, void *p, const Block &b)
+{
+    P.idle[b.dev].emplace(b.bytes, Idle{p, P.calls});
+    P.idleBytes[b.dev] += b.bytes;
+}
+bool fits(size_t have, size_t need) { return have <= need + need / 8 + 65536; }
+
+}  // namespace
+
+hipError_t dev_malloc(void **out, size_t bytes)
+{
+    *out = nullptr;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kPoolDevices) return hipMalloc(out, bytes);
+    const size_t need = block_bytes(bytes);
+    Pool &P = pool();
+    ThreadScope &T = t_scope;
+    if (T.depth > 0) {
+        auto it = T.freed.lower_bound(need);
+        if (it != T.freed.end() && fits(it->first, need)) {
+            *out = it->second;
+            T.freed.erase(it);
+            return hipSuccess;
+        }
+    }
+    {
+        std::lock_guard<std::mutex> hold(P.mu);
+        auto it = P.idle[dev].lower_bound(need);
+        if (it != P.idle[dev].end() && fits(it->first, need)) {
+            *out = it->second.p;
+            P.idleBytes[dev] -= it->first;
+            P.idle[dev].erase(it);
+            return hipSuccess;
+        }
+    }
+    void *p = nullptr;
+    e = hipMalloc(&p, need);
+    if (e == hipErrorOutOfMemory) {  // what lies idle here may be what is missing
+        (void)hipGetLastError();
+        release_idle_memory();
+        e = hipMalloc(&p, need);
+    }
+    if (e != hipSuccess) return e;
+    std::lock_guard<std::mutex> hold(P.mu);
+    if (P.limit[dev] == 0) {
+        size_t freeB = 0, total = 0;
+        if (hipMemGetInfo(&freeB, &total) != hipSuccess) {
+            (void)hipGetLastError();
+            total = (size_t)16 << 30;
+        }
+        P.limit[dev] = std::max<size_t>(total / kPoolShare, 1);
+    }
+    P.blocks[p] = Block{need, dev};
+    *out = p;
+    return hipSuccess;
+}
+
+hipError_t dev_free(void *p)
+{
+    if (!p) return hipSuccess;
+    Pool &P = pool();
+    ThreadScope &T = t_scope;
+    Block b{};
+    {
+        std::lock_guard<std::mutex> hold(P.mu);
+        auto it = P.blocks.find(p);
+        int dev = -1;
+        if (it == P.blocks.end() || hipGetDevice(&dev) != hipSuccess || dev != it->second.dev) {
+            // not made here, or on another device than the current one: the plain way
+            if (it != P.blocks.end()) P.blocks.erase(it);
+            b.bytes = 0;
+        } else {
+            b = it->second;
+            if (T.idleFrees > 0) {
+                put_idle(P, p, b);
+                return hipSuccess;
+            }
+        }
+    }
+    if (b.bytes == 0) return hipFree(p);
+    if (T.depth > 0) {
+        T.freed.emplace(b.bytes, p);
+        return hipSuccess;
+    }
+    const hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess) return e;
+    std::lock_guard<std::mutex> hold(P.mu);
+    put_idle(P, p, b);
+    return hipSuccess;
+}
+
+void release_idle_memory()
+{
+    Pool &P = pool();
+    std::vector<void *> out;
+    {
+        std::lock_guard<std::mutex> hold(P.mu);
+        for (int d = 0; d < kPoolDevices; ++d) trim(P, d, out, true);
+    }
+    for (void *p : out) (void)hipFree(p);
+}
+
+MemScope::MemScope(hipStream_t s)
+{
+    ThreadScope &T = t_scope;
+    // (a call inside another one works on the same stream -- every caller here hands its own on -- or is done with
+    // the memory it gave back when it returns)
+    if (T.depth++ == 0) T.stream = s;
+}
+MemScope::~MemScope()
+{
+    ThreadScope &T = t_scope;
+    if (--T.depth > 0 || T.freed.empty()) return;
+    const bool idle = hipStreamSynchronize(T.stream) == hipSuccess;
+    Pool &P = pool();
+    std::vector<void *> out;
+    {
+        std::lock_guard<std::mutex> hold(P.mu);
+        ++P.calls;
+        int dev = -1;
+        for (auto &f : T.freed) {
+            auto it = P.blocks.find(f.second);
+            if (idle && it != P.blocks.end()) {
+                dev = it->second.dev;
+                put_idle(P, f.second, it->second);
+            } else {
+                if (it != P.blocks.end()) P.blocks.erase(it);
+                out.push_back(f.second);
+            }
+        }
+        if (dev >= 0) trim(P, dev, out, false);
+    }
+    T.freed.clear();
+    for (void *p : out) (void)hipFree(p);
+}
+
+IdleFrees::IdleFrees()
+{
+    (void)hipDeviceSynchronize();
+    ++t_scope.idleFrees;
+}
+IdleFrees::~IdleFrees() { --t_scope.idleFrees; }
+
+}  // namespace mx
+
+extern "C" void mx_release_memory(void) { mx::release_idle_memory(); }

@@ -114,3 +114,47 @@ def test_value_dictionary_of_a_device_layout(mx, dtype, values):
     assert H["nDict"] == D["nDict"]
     for k in ("ecode", "dict", "eval"):
         assert np.array_equal(H[k].view(np.uint8), D[k].view(np.uint8)), k
+
+
+def test_memory_kept_between_calls_is_bounded_and_given_back(mx):
+    """Plans made and dropped one after the other, from two threads with streams of their own, leave products
+    right while the library keeps what they gave back; release_memory() returns it to the device."""
+    import threading
+
+    import torch
+    rng = np.random.default_rng(3)
+    mats = []
+    for rows in (20000, 90000):
+        ptr = (np.arange(rows + 1) * 12).astype(np.int32)
+        mats.append(mx.Csr(rows, rows, ptr, rng.integers(0, rows, ptr[-1]).astype(np.int32), rng.integers(-3, 4, ptr[-1]).astype(np.float64)))
+    wrong = []
+
+    def work(A, seed):
+        g = np.random.default_rng(seed)
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            dev = [torch.from_numpy(a).cuda() for a in (A.rowPtr, A.colInd, A.val)]
+            for k in range(12):
+                x = g.integers(-2, 3, A.cols).astype(np.float64)
+                want = np.add.reduceat(A.val * x[A.colInd], A.rowPtr[:-1])
+                s.synchronize()
+                plan = mx.Plan.from_device(*dev, A.cols, *((0.0, 0.0) if k % 2 else (0.5, 0.25)))
+                y = plan.spmv(torch.from_numpy(x).cuda())
+                plan.close()                     # while the product may still run
+                t = mx.transpose_device(*dev, A.cols)
+                if not np.array_equal(y.cpu().numpy(), want):
+                    wrong.append((seed, k))
+                if int(t[0][-1]) != A.nnz:
+                    wrong.append((seed, k, "transpose"))
+    threads = [threading.Thread(target=work, args=(A, i)) for i, A in enumerate(mats)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free0, total = torch.cuda.mem_get_info()
+    mx.release_memory()
+    free1 = torch.cuda.mem_get_info()[0]
+    assert free0 <= free1 <= free0 + total // 128 + (64 << 20)
