@@ -52,13 +52,29 @@ struct Buf {  // device memory released at scope exit unless taken
     }
 };
 
-// sum over the grid of one count per lane (every lane of a wave must arrive here)
-__device__ __forceinline__ void add_total(unsigned long long v, unsigned long long *dst)
+// dst[0] += a, dst[1] += b, summed over the workgroup first (every thread must arrive here): atomics on one word
+// take about 8 ns each whoever issues them, so the kernels that count go over their input with at most
+// kCountBlocks workgroups.
+constexpr int kCountBlocks = 1024;
+__device__ __forceinline__ void add_totals(unsigned long long a, unsigned long long b, unsigned long long *dst)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if ((threadIdx.x & 63) == 0 && v) atomicAdd(dst, v);
+    __shared__ unsigned long long part[2][kBlock / 64];
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_xor(a, off);
+        b += __shfl_xor(b, off);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        part[0][threadIdx.x >> 6] = a;
+        part[1][threadIdx.x >> 6] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned long long v = 0;
+        for (int w = 0; w < kBlock / 64; ++w) v += part[threadIdx.x][w];
+        if (v) atomicAdd(dst + threadIdx.x, v);
+    }
 }
+inline dim3 count_grid(long long n) { return dim3((unsigned)std::min<long long>(kCountBlocks, (std::max<long long>(n, 1) + kBlock - 1) / kBlock)); }
 
 __global__ __launch_bounds__(kBlock) void mark_kernel(const int *__restrict__ list, int n, unsigned char *__restrict__ flag)
 {
@@ -247,21 +263,22 @@ __global__ __launch_bounds__(kBlock) void chunk_members_kernel(const int *__rest
     }
 }
 
-// The fill gate on what the taken rows leave of every fragment (binary16: one thread per chunk of
-// the reference's numbering): fragments and entries that pass, summed.
+// The fill gate on what the taken rows leave of every fragment (binary16: one wave per chunk of the reference's
+// numbering, chunk after chunk): fragments and entries that pass, summed.  The chunks in front hold the longest rows,
+// thousands of fragments each; with a thread per chunk those few threads were the kernel's time (1.34 ms for
+// 131072 chunks of a matrix with rows of up to 4096 entries; a wave per chunk takes 0.05).
 __global__ __launch_bounds__(kBlock) void gate_f16_kernel(const int *__restrict__ chunkPtr, const unsigned long long *__restrict__ fragBit,
                                                           const unsigned char *__restrict__ taken, int chunkNum, int dRows, int minVals,
                                                           unsigned long long *__restrict__ totals)
 {
-    const int w = blockIdx.x * kBlock + threadIdx.x;
+    const int lane = threadIdx.x & 63;
     unsigned long long frags = 0, entries = 0;
-    if (w < chunkNum) {
+    for (int w = (blockIdx.x * kBlock + threadIdx.x) >> 6; w < chunkNum; w += gridDim.x * (kBlock / 64)) {
+        const int i = w * 8 + (lane & 7);
+        const unsigned left = (unsigned)__ballot(i < dRows && !(taken && taken[i])) & 0xffu;  // bit r: row r of the chunk
         unsigned long long rowsLeft = 0;
-        for (int r = 0; r < 8; ++r) {
-            const int i = w * 8 + r;
-            if (i < dRows && !(taken && taken[i])) rowsLeft |= 0xffull << (r * 8);
-        }
-        for (int f = chunkPtr[w]; f < chunkPtr[w + 1]; ++f) {
+        for (int r = 0; r < 8; ++r) rowsLeft |= ((left >> r) & 1u) ? 0xffull << (r * 8) : 0ull;
+        for (int f = chunkPtr[w] + lane; f < chunkPtr[w + 1]; f += 64) {
             const int vals = __popcll(fragBit[f] & rowsLeft);
             if (vals > 0 && vals >= minVals) {
                 ++frags;
@@ -269,23 +286,20 @@ __global__ __launch_bounds__(kBlock) void gate_f16_kernel(const int *__restrict_
             }
         }
     }
-    add_total(frags, totals);
-    add_total(entries, totals + 1);
+    add_totals(frags, entries, totals);
 }
 __global__ __launch_bounds__(kBlock) void gate_counts_kernel(const int *__restrict__ fragPtr, int nFrags, int minVals,
                                                              unsigned long long *__restrict__ totals)
 {
-    const int f = blockIdx.x * kBlock + threadIdx.x;
     unsigned long long frags = 0, entries = 0;
-    if (f < nFrags) {
+    for (int f = blockIdx.x * kBlock + threadIdx.x; f < nFrags; f += gridDim.x * kBlock) {
         const int vals = fragPtr[f + 1] - fragPtr[f];
         if (vals > 0 && vals >= minVals) {
-            frags = 1;
-            entries = (unsigned)vals;
+            ++frags;
+            entries += (unsigned)vals;
         }
     }
-    add_total(frags, totals);
-    add_total(entries, totals + 1);
+    add_totals(frags, entries, totals);
 }
 
 // binary64: (block row, block column) of every entry of A_dd that is not followed by a twin
@@ -308,19 +322,20 @@ __global__ __launch_bounds__(kBlock) void block_keys_kernel(const int *__restric
 __global__ __launch_bounds__(kBlock) void block_runs_kernel(const unsigned long long *__restrict__ key, int n, int need, int cols,
                                                             unsigned long long *__restrict__ totals)
 {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
     unsigned long long blocks = 0, entries = 0;
-    if (p < n && key[p] != ~0ull && (p == 0 || key[p - 1] != key[p])) {
-        int e = p + 1;
-        while (e < n && e - p < 64 && key[e] == key[p]) ++e;  // (a block holds at most 64 entries that are not twins)
+    for (int p = blockIdx.x * kBlock + threadIdx.x; p < n; p += gridDim.x * kBlock) {
+        if (key[p] == ~0ull || (p > 0 && key[p - 1] == key[p])) continue;
+        // (a block holds at most 64 entries that are not twins; most runs are short of `need`, which one look tells)
+        if (p + need > n || key[p + need - 1] != key[p]) continue;
+        int e = p + need;
+        while (e < n && e - p < 64 && key[e] == key[p]) ++e;
         const int bc = (int)(unsigned)key[p];
-        if (e - p >= need && bc + 1 <= cols / 8) {
-            blocks = 1;
-            entries = (unsigned)(e - p);
+        if (bc + 1 <= cols / 8) {
+            ++blocks;
+            entries += (unsigned)(e - p);
         }
     }
-    add_total(blocks, totals);
-    add_total(entries, totals + 1);
+    add_totals(blocks, entries, totals);
 }
 
 // ---- the CSR part: every row's residual entries, then the entries of A_dd that stay
@@ -632,9 +647,7 @@ __global__ __launch_bounds__(kBlock) void block_heads_kernel(const unsigned long
     if (p > n) return;
     int h = 0;
     if (p < n && key[p] != ~0ull && (p == 0 || key[p - 1] != key[p])) {
-        int e = p + 1;
-        while (e < n && e - p < 64 && key[e] == key[p]) ++e;
-        h = e - p >= need && (int)(unsigned)key[p] + 1 <= cols / 8 ? 1 : 0;
+        h = p + need <= n && key[p + need - 1] == key[p] && (int)(unsigned)key[p] + 1 <= cols / 8 ? 1 : 0;
     }
     selHead[p] = h;
 }
@@ -1082,18 +1095,18 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         MXH_TRY(hipGetLastError());
         MXH_TRY(rocprim::radix_sort_pairs(sortTmp.p, sortBytes, (const unsigned long long *)keyIn.p, I.blkKey.as<unsigned long long>(),
                                           (const int *)payIn.p, I.blkPay.as<int>(), n, 0u, 64u, s));
-        hipLaunchKernelGGL(block_runs_kernel, grid(I.nDD), dim3(kBlock), 0, s, (const unsigned long long *)I.blkKey.p, I.nDD, 48, cols, tot + 2);
+        hipLaunchKernelGGL(block_runs_kernel, count_grid(I.nDD), dim3(kBlock), 0, s, (const unsigned long long *)I.blkKey.p, I.nDD, 48, cols, tot + 2);
         MXH_TRY(hipGetLastError());
     }
     // ---- the fill gate of the reference's fragments
     const int nFrags = I.T.totalTcFrags;
     if (wantGeneral && nFrags > 0) {
         if (dtype == MX_F16)
-            hipLaunchKernelGGL(gate_f16_kernel, grid(I.T.chunkNum), dim3(kBlock), 0, s, (const int *)I.T.chunkPtr,
+            hipLaunchKernelGGL(gate_f16_kernel, count_grid((long long)I.T.chunkNum * 64), dim3(kBlock), 0, s, (const int *)I.T.chunkPtr,
                                (const unsigned long long *)I.T.fragBit, I.nChunks > 0 ? (const unsigned char *)I.taken.p : nullptr, I.T.chunkNum,
                                I.dRows, minVals, tot);
         else
-            hipLaunchKernelGGL(gate_counts_kernel, grid(nFrags), dim3(kBlock), 0, s, (const int *)I.T.fragPtr, nFrags, minVals, tot);
+            hipLaunchKernelGGL(gate_counts_kernel, count_grid(nFrags), dim3(kBlock), 0, s, (const int *)I.T.fragPtr, nFrags, minVals, tot);
         MXH_TRY(hipGetLastError());
     }
     unsigned long long h[4] = {0, 0, 0, 0};
