@@ -22,6 +22,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include "mx_device.h"
+#include "mx_entry_rows.h"
 #include "mx_internal.h"
 
 namespace mxh {
@@ -319,16 +320,17 @@ __global__ __launch_bounds__(kBlock) void block_keys_kernel(const int *__restric
                                                             const int *__restrict__ descColId, const int *__restrict__ rId, int dRows,
                                                             int nDD, unsigned long long *__restrict__ key)
 {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= nDD) return;
-    int lo = 0, hi = dRows - 1;
-    while (lo < hi) {  // last i with ddRowPtr[i] <= p
-        const int mid = (lo + hi + 1) >> 1;
-        if (ddRowPtr[mid] <= p) lo = mid;
-        else hi = mid - 1;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(ddRowPtr, dRows, nDD, t0, T);
+#pragma unroll
+    for (int k = 0; k < mxr::kPer; ++k) {
+        const int i = k * kBlock + threadIdx.x, p = t0 + i;
+        if (i >= nDD - t0) break;
+        const int row = T.row[i];
+        const bool twin = p + 1 < ddRowPtr[row + 1] && ddCol[p + 1] == ddCol[p];
+        key[p] = twin ? ~0ull : ((unsigned long long)(unsigned)(rId[row] >> 3) << 32) | (unsigned)(descColId[ddCol[p]] >> 3);
     }
-    const bool twin = p + 1 < ddRowPtr[lo + 1] && ddCol[p + 1] == ddCol[p];
-    key[p] = twin ? ~0ull : ((unsigned long long)(unsigned)(rId[lo] >> 3) << 32) | (unsigned)(descColId[ddCol[p]] >> 3);
 }
 // runs of one key at least `need` long whose block lies inside x: blocks and entries, summed
 __global__ __launch_bounds__(kBlock) void block_runs_kernel(const unsigned long long *__restrict__ key, int n, int need, int cols,
@@ -374,17 +376,17 @@ __global__ __launch_bounds__(kBlock) void part_residual_kernel(const int *__rest
                                                                const int *__restrict__ outPtr, int rows, int nCD, int *__restrict__ col,
                                                                V *__restrict__ val)
 {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= nCD) return;
-    int lo = 0, hi = rows - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (cdRowPtr[mid] <= p) lo = mid;
-        else hi = mid - 1;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(cdRowPtr, rows, nCD, t0, T);
+#pragma unroll
+    for (int k = 0; k < mxr::kPer; ++k) {
+        const int i = k * kBlock + threadIdx.x, p = t0 + i;
+        if (i >= nCD - t0) break;
+        const int row = T.row[i], q = outPtr[row] + (p - cdRowPtr[row]);
+        col[q] = colOrig[cdCol[p]];
+        val[q] = cdVal[p];
     }
-    const int q = outPtr[lo] + (p - cdRowPtr[lo]);
-    col[q] = colOrig[cdCol[p]];
-    val[q] = cdVal[p];
 }
 template <typename V>
 __global__ __launch_bounds__(kBlock) void part_dense_kernel(const int *__restrict__ ddRowPtr, const int *__restrict__ ddCol,
@@ -393,19 +395,19 @@ __global__ __launch_bounds__(kBlock) void part_dense_kernel(const int *__restric
                                                             const int *__restrict__ cdRowPtr, const int *__restrict__ outPtr, int dRows,
                                                             int nDD, int *__restrict__ col, V *__restrict__ val)
 {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= nDD) return;
-    int lo = 0, hi = dRows - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ddRowPtr[mid] <= p) lo = mid;
-        else hi = mid - 1;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(ddRowPtr, dRows, nDD, t0, T);
+#pragma unroll
+    for (int k = 0; k < mxr::kPer; ++k) {
+        const int i = k * kBlock + threadIdx.x, p = t0 + i;
+        if (i >= nDD - t0) break;
+        const int row = T.row[i];
+        if (taken && taken[row]) continue;
+        const int r = rId[row], q = outPtr[r] + (cdRowPtr[r + 1] - cdRowPtr[r]) + (p - ddRowPtr[row]);
+        col[q] = descColId[ddCol[p]];
+        val[q] = ddVal[p];
     }
-    if (taken && taken[lo]) return;
-    const int r = rId[lo];
-    const int q = outPtr[r] + (cdRowPtr[r + 1] - cdRowPtr[r]) + (p - ddRowPtr[lo]);
-    col[q] = descColId[ddCol[p]];
-    val[q] = ddVal[p];
 }
 
 // ---- the strips' steps.  stepDesc[s] = {chunk of half 0, chunk of half 1 (-1 none, -2 the same chunk
@@ -748,18 +750,18 @@ __global__ __launch_bounds__(kBlock) void block_values_kernel(const int *__restr
                                                               const double *__restrict__ ddVal, const int *__restrict__ descColId,
                                                               const int *__restrict__ rId, int dRows, int nDD, double *__restrict__ tcVal)
 {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= nDD) return;
-    const int g = entryBlock[p];
-    if (g < 0) return;
-    int lo = 0, hi = dRows - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ddRowPtr[mid] <= p) lo = mid;
-        else hi = mid - 1;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(ddRowPtr, dRows, nDD, t0, T);
+#pragma unroll
+    for (int k = 0; k < mxr::kPer; ++k) {
+        const int i = k * kBlock + threadIdx.x, p = t0 + i;
+        if (i >= nDD - t0) break;
+        const int g = entryBlock[p];
+        if (g < 0) continue;
+        const int chunk = chunkIdIncl[g] - 1, r = rId[T.row[i]], c = descColId[ddCol[p]];
+        tcVal[((size_t)chunkBlock0[chunk] + (g - chunkStart[chunk])) * 64 + (r & 7) * 8 + (c & 7)] = ddVal[p];
     }
-    const int chunk = chunkIdIncl[g] - 1, r = rId[lo], c = descColId[ddCol[p]];
-    tcVal[((size_t)chunkBlock0[chunk] + (g - chunkStart[chunk])) * 64 + (r & 7) * 8 + (c & 7)] = ddVal[p];
 }
 // the CSR part beside blocks: an entry stays unless a block took it
 __global__ __launch_bounds__(kBlock) void block_keep_kernel(const int *__restrict__ entryBlock, int nDD, int *__restrict__ keep)
@@ -788,18 +790,19 @@ __global__ __launch_bounds__(kBlock) void part_dense_scan_kernel(const int *__re
                                                                  const int *__restrict__ outPtr, int dRows, int nDD, int *__restrict__ col,
                                                                  V *__restrict__ val)
 {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= nDD || entryBlock[p] >= 0) return;
-    int lo = 0, hi = dRows - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ddRowPtr[mid] <= p) lo = mid;
-        else hi = mid - 1;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(ddRowPtr, dRows, nDD, t0, T);
+#pragma unroll
+    for (int k = 0; k < mxr::kPer; ++k) {
+        const int i = k * kBlock + threadIdx.x, p = t0 + i;
+        if (i >= nDD - t0) break;
+        if (entryBlock[p] >= 0) continue;
+        const int row = T.row[i], r = rId[row];
+        const int q = outPtr[r] + (cdRowPtr[r + 1] - cdRowPtr[r]) + (keptBefore[p] - keptBefore[ddRowPtr[row]]);
+        col[q] = descColId[ddCol[p]];
+        val[q] = ddVal[p];
     }
-    const int r = rId[lo];
-    const int q = outPtr[r] + (cdRowPtr[r + 1] - cdRowPtr[r]) + (keptBefore[p] - keptBefore[ddRowPtr[lo]]);
-    col[q] = descColId[ddCol[p]];
-    val[q] = ddVal[p];
 }
 
 }  // namespace mxh
@@ -1090,7 +1093,7 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         MXH_TRY(mx::dev_malloc(&I.blkKey.p, n * 8));
         MXH_TRY(mx::dev_malloc(&I.blkPay.p, n * 4));
         MXH_TRY(mx::dev_malloc(&sortTmp.p, sortBytes + 256));
-        hipLaunchKernelGGL(block_keys_kernel, grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const int *)I.dc,
+        hipLaunchKernelGGL(block_keys_kernel, mxr::tile_grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const int *)I.dc,
                            (const int *)I.dr, I.dRows, I.nDD, keyIn.as<unsigned long long>());
         MXH_TRY(hipGetLastError());
         hipLaunchKernelGGL(iota_kernel, grid(I.nDD), dim3(kBlock), 0, s, payIn.as<int>(), I.nDD);
@@ -1191,12 +1194,12 @@ static int csr_part_t(HybridDevice::Impl &I, bool keepStrips, bool keepGeneral, 
     MXH_TRY(mx::dev_malloc(&col.p, (size_t)n * 4 + 4));
     MXH_TRY(mx::dev_malloc(&val.p, (size_t)n * sizeof(V) + 8));
     if (I.nCD > 0) {
-        hipLaunchKernelGGL(part_residual_kernel<V>, grid(I.nCD), dim3(kBlock), 0, s, (const int *)I.cdp, (const int *)I.cdc, (const V *)I.cdv,
+        hipLaunchKernelGGL(part_residual_kernel<V>, mxr::tile_grid(I.nCD), dim3(kBlock), 0, s, (const int *)I.cdp, (const int *)I.cdc, (const V *)I.cdv,
                            (const int *)I.colOrig.p, (const int *)ptr.p, rows, I.nCD, col.as<int>(), val.as<V>());
         MXH_TRY(hipGetLastError());
     }
     if (blocks) {
-        hipLaunchKernelGGL(part_dense_scan_kernel<V>, grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const V *)I.ddv,
+        hipLaunchKernelGGL(part_dense_scan_kernel<V>, mxr::tile_grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const V *)I.ddv,
                            (const int *)I.dc, (const int *)I.dr, (const int *)I.entryBlock.p, (const int *)keptBefore.p, (const int *)I.cdp,
                            (const int *)ptr.p, I.dRows, I.nDD, col.as<int>(), val.as<V>());
         MXH_TRY(hipGetLastError());
@@ -1208,7 +1211,7 @@ static int csr_part_t(HybridDevice::Impl &I, bool keepStrips, bool keepGeneral, 
                            (const int *)I.selPos.p, (const int *)I.tileBlock0.p, (V *)I.tileVal);
         MXH_TRY(hipGetLastError());
     } else if (I.nDD > 0) {
-        hipLaunchKernelGGL(part_dense_kernel<V>, grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const V *)I.ddv,
+        hipLaunchKernelGGL(part_dense_kernel<V>, mxr::tile_grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const V *)I.ddv,
                            (const int *)I.dc, (const int *)I.dr, taken, (const int *)I.cdp, (const int *)ptr.p, I.dRows, I.nDD, col.as<int>(),
                            val.as<V>());
         MXH_TRY(hipGetLastError());
@@ -1322,7 +1325,7 @@ int HybridDevice::block_layout(const std::vector<int> &stepDesc, const std::vect
     hipLaunchKernelGGL(block_steps_kernel, dim3(steps), dim3(64), 0, s, (const int *)dDesc.p, (const int *)I.blkChunkStart.p,
                        (const int *)I.blkChunkBr.p, (const int *)I.blkBc.p, I.rows, steps, T.hdr, T.atox);
     MXH_TRY(hipGetLastError());
-    hipLaunchKernelGGL(block_values_kernel, grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.entryBlock.p, (const int *)I.blkChunkIdIncl.p,
+    hipLaunchKernelGGL(block_values_kernel, mxr::tile_grid(I.nDD), dim3(kBlock), 0, s, (const int *)I.entryBlock.p, (const int *)I.blkChunkIdIncl.p,
                        (const int *)I.blkChunkStart.p, (const int *)dBlock0.p, (const int *)I.ddp, (const int *)I.ddc, (const double *)I.ddv,
                        (const int *)I.dc, (const int *)I.dr, I.dRows, I.nDD, (double *)T.tcVal);
     MXH_TRY(hipGetLastError());

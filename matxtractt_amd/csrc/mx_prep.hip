@@ -13,7 +13,7 @@
 // gets the key ind[e] and the payload e; source order is ascending (r, e), so a stable sort by
 // key alone gives ascending (ind, r, e).  rocPRIM's radix sort is stable and sorts only the
 // ceil(log2(inner)) bits the keys can have.  Three small kernels around it: the source line of
-// every entry (binary search in ptr), the output line pointers from the sorted keys (every
+// every entry (tile_rows), the output line pointers from the sorted keys (every
 // thread writes the pointers of the lines that start at its position), and the gather of
 // source lines and values through the sorted payload.
 #include <hip/hip_runtime.h>
@@ -28,6 +28,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include "mx_device.h"
+#include "mx_entry_rows.h"
 #include "mx_internal.h"
 
 namespace mxp {
@@ -37,23 +38,24 @@ constexpr int kBlock = 256;
 constexpr int kMaxCount = 2147483647 - 2 * kBlock;
 
 // line[e] = r with ptr[r] <= e < ptr[r+1]; bad |= 1 where ind[e] lies outside [0, inner).
+// (7 million entries in 700001 lines: 0.13 ms with a search per entry, 0.04 so)
 __global__ __launch_bounds__(kBlock) void entry_lines_kernel(const int *__restrict__ ptr, const int *__restrict__ ind,
                                                              int outer, int inner, int nnz, int *__restrict__ line,
                                                              int *__restrict__ payload, int *__restrict__ bad)
 {
-    const int e = blockIdx.x * kBlock + threadIdx.x;
-    if (e >= nnz) return;
-    // last r in [0, outer) with ptr[r] <= e  (empty lines repeat a pointer: the last one wins,
-    // and it is the only one whose range holds e)
-    int lo = 0, hi = outer - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ptr[mid] <= e) lo = mid;
-        else hi = mid - 1;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(ptr, outer, nnz, t0, T);
+    bool out = false;
+#pragma unroll
+    for (int k = 0; k < mxr::kPer; ++k) {
+        const int i = k * kBlock + threadIdx.x;
+        if (i >= nnz - t0) break;
+        line[t0 + i] = T.row[i];
+        payload[t0 + i] = t0 + i;
+        out |= (unsigned)ind[t0 + i] >= (unsigned)inner;
     }
-    line[e] = lo;
-    payload[e] = e;
-    if ((unsigned)ind[e] >= (unsigned)inner) atomicOr(bad, 1);
+    if (__any(out) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
 }
 
 // tPtr[c] = number of sorted keys below c, for c in [0, inner].  Thread k owns the lines
@@ -159,22 +161,27 @@ __global__ __launch_bounds__(kBlock) void dense_row_counts_kernel(const int *__r
                                                                   const unsigned char *__restrict__ dense, int rows, int nnz,
                                                                   int *__restrict__ rcnt)
 {
-    // The lanes of a wave hold consecutive entries, so their rows ascend: the first lane of every run
-    // of equal rows adds the run's count in one atomic (a row of thousands of entries would otherwise
-    // take thousands of atomics on one address).
-    const int e = blockIdx.x * kBlock + threadIdx.x;
-    const bool in = e < nnz;
-    const int r = in ? line_of(rowPtr, rows, e) : -1;
-    const bool d = in && dense[col[e]];
-    const int lane = threadIdx.x & 63;
-    const int rPrev = __shfl_up(r, 1);
-    const unsigned long long heads = __ballot(lane == 0 || r != rPrev), hits = __ballot(d);
-    if (!in || !((heads >> lane) & 1)) return;
-    const unsigned long long above = lane == 63 ? 0ull : heads >> (lane + 1);
-    const int next = above ? lane + 1 + __builtin_ctzll(above) : 64;
-    const unsigned long long run = (next == 64 ? ~0ull : (1ull << next) - 1) & ~((1ull << lane) - 1);
-    const int c = __popcll(hits & run);
-    if (c) atomicAdd(&rcnt[r], c);
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile, lane = threadIdx.x & 63;
+    mxr::tile_rows(rowPtr, rows, nnz, t0, T);
+#pragma unroll
+    for (int k = 0; k < mxr::kPer; ++k) {
+        // The lanes of a wave hold consecutive entries, so their rows ascend: the first lane of every run
+        // of equal rows adds the run's count in one atomic (a row of thousands of entries would otherwise
+        // take thousands of atomics on one address).
+        const int i = k * kBlock + threadIdx.x;
+        const bool in = i < nnz - t0;
+        const int r = in ? T.row[i] : -1;
+        const bool d = in && dense[col[t0 + i]];
+        const int rPrev = __shfl_up(r, 1);
+        const unsigned long long heads = __ballot(lane == 0 || r != rPrev), hits = __ballot(d);
+        if (!in || !((heads >> lane) & 1)) continue;
+        const unsigned long long above = lane == 63 ? 0ull : heads >> (lane + 1);
+        const int next = above ? lane + 1 + __builtin_ctzll(above) : 64;
+        const unsigned long long run = (next == 64 ? ~0ull : (1ull << next) - 1) & ~((1ull << lane) - 1);
+        const int c = __popcll(hits & run);
+        if (c) atomicAdd(&rcnt[r], c);
+    }
 }
 
 // ---- split --------------------------------------------------------------------------------
@@ -415,7 +422,7 @@ extern "C" int mx_transpose_device(mx_dtype dtype, int outer, int inner, int nnz
     void *sortTmp = base + 4 * n4 + 256;
     const int eblocks = (nnz + kBlock - 1) / kBlock;
     MXP_TRY(hipMemsetAsync(bad, 0, sizeof(int), s));
-    hipLaunchKernelGGL(entry_lines_kernel, dim3(eblocks), dim3(kBlock), 0, s, ptr_dev, ind_dev, outer, inner, nnz, line,
+    hipLaunchKernelGGL(entry_lines_kernel, mxr::tile_grid(nnz), dim3(kBlock), 0, s, ptr_dev, ind_dev, outer, inner, nnz, line,
                        payIn, bad);
     MXP_TRY(hipGetLastError());
     // an index outside [0, inner) must not reach the pointer kernel: look before going on
@@ -537,7 +544,7 @@ extern "C" int mx_select_device(int rows, int cols, int nnz, const int *rowPtr_d
         MXP_TRY(hipGetLastError());
     }
     if (nnz > 0) {
-        hipLaunchKernelGGL(dense_row_counts_kernel, dim3(eblocks), dim3(kBlock), 0, s, rowPtr_dev, colInd_dev,
+        hipLaunchKernelGGL(dense_row_counts_kernel, mxr::tile_grid(nnz), dim3(kBlock), 0, s, rowPtr_dev, colInd_dev,
                            (const unsigned char *)dense, rows, nnz, cnt);
         MXP_TRY(hipGetLastError());
     }
@@ -638,7 +645,7 @@ extern "C" int mx_split_device(mx_dtype dtype, int rows, int cols, int nnz, cons
     // rows: rank of the selected ones, counts inside the selected columns, lengths, pointers
     if (dRows > 0) hipLaunchKernelGGL(scatter_rank_kernel, grid(dRows), dim3(kBlock), 0, s, descRowId_dev, dRows, rowRank);
     if (nnz > 0)
-        hipLaunchKernelGGL(dense_row_counts_kernel, grid(nnz), dim3(kBlock), 0, s, rowPtr_dev, colInd_dev,
+        hipLaunchKernelGGL(dense_row_counts_kernel, mxr::tile_grid(nnz), dim3(kBlock), 0, s, rowPtr_dev, colInd_dev,
                            (const unsigned char *)dense, rows, nnz, rcnt);
     hipLaunchKernelGGL(split_lengths_kernel, grid((long long)rows + 1), dim3(kBlock), 0, s, rowPtr_dev, (const int *)rcnt,
                        (const int *)rowRank, descRowId_dev, rows, dRows, cdLen, ddLen);
