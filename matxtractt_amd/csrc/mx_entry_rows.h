@@ -38,6 +38,21 @@ __device__ __forceinline__ void tile_rows(const int *__restrict__ ptr, int rows,
     for (int k = 0; k < kPer; ++k) T.row[k * kBlock + tid] = 0;
     __syncthreads();
     const int size = min(n - t0, kTile);
+    // Where nearly all rows are without entries, walking them takes longer than a search per entry: the row
+    // 8 * kTile further on begins inside the tile.
+    if (rows - lo > 8 * kTile && (long long)ptr[lo + 8 * kTile] < (long long)t0 + size) {
+        for (int i = tid; i < size; i += kBlock) {
+            int a = lo, b = rows - 1;
+            while (a < b) {
+                const int mid = a + (b - a + 1) / 2;
+                if ((long long)ptr[mid] - t0 <= i) a = mid;
+                else b = mid - 1;
+            }
+            T.row[i] = a;
+        }
+        __syncthreads();
+        return;
+    }
     for (int r = lo + 1 + tid; r < rows; r += kBlock) {
         const long long at = (long long)ptr[r] - t0;
         if (at >= size) break;
