@@ -24,6 +24,7 @@
 #include "mx_device.h"
 #include "mx_entry_rows.h"
 #include "mx_internal.h"
+#include "mx_row_sort.h"
 
 namespace mxl {
 
@@ -75,6 +76,14 @@ __global__ __launch_bounds__(kBlock) void entry_rows_kernel(const int *__restric
     // put one per entry on the same word, and half a million of them take four milliseconds)
     if (__any(descends) && (threadIdx.x & 63) == 0 && *(volatile int *)flag == 0) atomicOr(flag, 1);
 }
+
+// The order of a row's entries by column, made inside their workgroups.
+struct RowColumns {
+    const int *col;
+    int *ord;
+    __device__ __forceinline__ unsigned key(int, int e) const { return (unsigned)col[e]; }
+    __device__ __forceinline__ void put(int, int, unsigned, int e, int k) const { ord[k] = e; }
+};
 
 __global__ __launch_bounds__(kBlock) void sort_keys_kernel(const int *__restrict__ row, const int *__restrict__ col, int nnz,
                                                            int colBits, unsigned long long *__restrict__ key, int *__restrict__ pay)
@@ -600,23 +609,35 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     MXL_TRY(hipMemcpyAsync(&unsorted, flag.p, 4, hipMemcpyDeviceToHost, s));
     MXL_TRY(hipStreamSynchronize(s));
     if (unsorted) {
-        int colBits = 1, rowBits = 1;
-        while (colBits < 31 && (1ll << colBits) < (long long)cols) ++colBits;
-        while (rowBits < 31 && (1ll << rowBits) < (long long)rows) ++rowBits;
-        Buf keyIn, keyOut, payIn, tmp;
-        size_t sortBytes = 0;
-        MXL_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
-                                          (const int *)nullptr, (int *)nullptr, (size_t)nnz, 0u, (unsigned)(colBits + rowBits), s));
-        MXL_TRY(mx::dev_malloc(&keyIn.p, (size_t)nnz * 8));
-        MXL_TRY(mx::dev_malloc(&keyOut.p, (size_t)nnz * 8));
-        MXL_TRY(mx::dev_malloc(&payIn.p, (size_t)nnz * 4));
-        MXL_TRY(mx::dev_malloc(&tmp.p, sortBytes + 256));
-        hipLaunchKernelGGL(sort_keys_kernel, grid(nnz), dim3(kBlock), 0, s, (const int *)row.p, col, nnz, colBits,
-                           keyIn.as<unsigned long long>(), payIn.as<int>());
-        MXL_TRY(hipGetLastError());
-        MXL_TRY(rocprim::radix_sort_pairs(tmp.p, sortBytes, (const unsigned long long *)keyIn.p, keyOut.as<unsigned long long>(),
-                                          (const int *)payIn.p, ord.as<int>(), (size_t)nnz, 0u, (unsigned)(colBits + rowBits), s));
+        // inside a workgroup per row or group of rows, where there is no row too long for that
+        // (15.8 million entries in a million rows: keys and radix sort 0.91 ms, so 0.39)
+        Buf list;
+        mxs::RowClasses classes{};
+        int *count = flag.as<int>() + 8;
+        MXL_TRY(mx::dev_malloc(&list.p, mxs::list_ints(nnz) * 4));
+        MXL_TRY(mxs::classify_rows(rowPtr, rows, nnz, list.as<int>(), count, s));
+        MXL_TRY(hipMemcpyAsync(classes.n, count, sizeof(classes.n), hipMemcpyDeviceToHost, s));
         MXL_TRY(hipStreamSynchronize(s));
+        if (classes.n[mxs::kClasses] == 0) {
+            MXL_TRY(mxs::sort_rows(rowPtr, rows, nnz, list.as<int>(), classes, RowColumns{col, ord.as<int>()}, s));
+        } else {
+            int colBits = 1, rowBits = 1;
+            while (colBits < 31 && (1ll << colBits) < (long long)cols) ++colBits;
+            while (rowBits < 31 && (1ll << rowBits) < (long long)rows) ++rowBits;
+            Buf keyIn, keyOut, payIn, tmp;
+            size_t sortBytes = 0;
+            MXL_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
+                                              (const int *)nullptr, (int *)nullptr, (size_t)nnz, 0u, (unsigned)(colBits + rowBits), s));
+            MXL_TRY(mx::dev_malloc(&keyIn.p, (size_t)nnz * 8));
+            MXL_TRY(mx::dev_malloc(&keyOut.p, (size_t)nnz * 8));
+            MXL_TRY(mx::dev_malloc(&payIn.p, (size_t)nnz * 4));
+            MXL_TRY(mx::dev_malloc(&tmp.p, sortBytes + 256));
+            hipLaunchKernelGGL(sort_keys_kernel, grid(nnz), dim3(kBlock), 0, s, (const int *)row.p, col, nnz, colBits,
+                               keyIn.as<unsigned long long>(), payIn.as<int>());
+            MXL_TRY(hipGetLastError());
+            MXL_TRY(rocprim::radix_sort_pairs(tmp.p, sortBytes, (const unsigned long long *)keyIn.p, keyOut.as<unsigned long long>(),
+                                              (const int *)payIn.p, ord.as<int>(), (size_t)nnz, 0u, (unsigned)(colBits + rowBits), s));
+        }
     }
     // ---- virtual rows
     Buf runHead, runStart, start, vid;

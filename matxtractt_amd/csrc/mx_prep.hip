@@ -30,6 +30,7 @@
 #include "mx_device.h"
 #include "mx_entry_rows.h"
 #include "mx_internal.h"
+#include "mx_row_sort.h"
 
 namespace mxp {
 
@@ -83,18 +84,6 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(const int *__restrict__ 
 }
 
 // ---- selection ---------------------------------------------------------------------------
-// The line of entry e, as in entry_lines_kernel.
-__device__ __forceinline__ int line_of(const int *__restrict__ ptr, int outer, int e)
-{
-    int lo = 0, hi = outer - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ptr[mid] <= e) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
 // cnt[ind[e]] += 1 for every entry (integer atomics: the result does not depend on the order).
 __global__ __launch_bounds__(kBlock) void index_histogram_kernel(const int *__restrict__ ind, int nnz, int inner,
                                                                  int *__restrict__ cnt, int *__restrict__ bad)
@@ -222,23 +211,63 @@ __global__ __launch_bounds__(kBlock) void split_lengths_kernel(const int *__rest
 // Sort key of an entry: [which matrix][its row there][residual only: selected column?][new column].
 // A_dd (matrix 0) sorts in front of the residual (matrix 1); inside a residual row the entries in
 // unselected columns come first, then those in selected ones; equal keys keep source order.
+// (Only for matrices with rows too long to be put in order by a workgroup; SplitRows is the other way.)
 __global__ __launch_bounds__(kBlock) void split_keys_kernel(const int *__restrict__ rowPtr, const int *__restrict__ col,
                                                             const int *__restrict__ newCol, const int *__restrict__ rowRank,
                                                             int rows, int nnz, int dCols, int colBits, int rowBits,
                                                             unsigned long long *__restrict__ key, int *__restrict__ payload)
 {
-    const int e = blockIdx.x * kBlock + threadIdx.x;
-    if (e >= nnz) return;
-    const int r = line_of(rowPtr, rows, e), nc = newCol[col[e]], rank = rowRank[r];
-    const bool sel = nc < dCols;
-    unsigned long long k;
-    if (sel && rank >= 0) k = ((unsigned long long)rank << (colBits + 1)) | (unsigned long long)nc;
-    else
-        k = (1ull << (rowBits + colBits + 1)) | ((unsigned long long)r << (colBits + 1)) |
-            ((unsigned long long)sel << colBits) | (unsigned long long)nc;
-    key[e] = k;
-    payload[e] = e;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(rowPtr, rows, nnz, t0, T);
+#pragma unroll
+    for (int j = 0; j < mxr::kPer; ++j) {
+        const int i = j * kBlock + threadIdx.x, e = t0 + i;
+        if (i >= nnz - t0) break;
+        const int r = T.row[i], nc = newCol[col[e]], rank = rowRank[r];
+        const bool sel = nc < dCols;
+        unsigned long long k;
+        if (sel && rank >= 0) k = ((unsigned long long)rank << (colBits + 1)) | (unsigned long long)nc;
+        else
+            k = (1ull << (rowBits + colBits + 1)) | ((unsigned long long)r << (colBits + 1)) |
+                ((unsigned long long)sel << colBits) | (unsigned long long)nc;
+        key[e] = k;
+        payload[e] = e;
+    }
 }
+
+// The split of a row inside its workgroup: by {selected column?, new column}, so that the entries in unselected columns
+// come first; those behind them are A_dd's where the row was selected, too.
+// (15.8 million binary16 entries in a million rows: keys, radix sort and gather 1.31 ms, so 0.44)
+template <typename V>
+struct SplitRows {
+    const int *ptr, *col, *newCol, *rowRank, *rcnt, *ddPtr, *cdPtr;
+    const V *val;
+    int dCols, colBits;
+    int *ddInd;
+    V *ddVal;
+    int *cdInd;
+    V *cdVal;
+    __device__ __forceinline__ unsigned key(int, int e) const
+    {
+        const int nc = newCol[col[e]];
+        return ((unsigned)(nc < dCols) << colBits) | (unsigned)nc;
+    }
+    __device__ __forceinline__ void put(int r, int place, unsigned key, int e, int) const
+    {
+        const int nc = (int)(key & ((1u << colBits) - 1)), rank = rowRank[r], rest = ptr[r + 1] - ptr[r] - rcnt[r];
+        const V v = val[e];
+        if (rank >= 0 && place >= rest) {
+            const int at = ddPtr[rank] + place - rest;
+            ddInd[at] = nc;
+            ddVal[at] = v;
+        } else {
+            const int at = cdPtr[r] + place;
+            cdInd[at] = nc;
+            cdVal[at] = v;
+        }
+    }
+};
 
 template <typename V>
 __global__ __launch_bounds__(kBlock) void split_gather_kernel(const unsigned long long *__restrict__ key, const int *__restrict__ payload,
@@ -260,17 +289,54 @@ __global__ __launch_bounds__(kBlock) void split_gather_kernel(const unsigned lon
 }
 
 // ---- tile encoding ------------------------------------------------------------------------
-// key = [chunk of the entry's row][column] for every entry of A_dd; payload = the entry
-__global__ __launch_bounds__(kBlock) void tile_keys_kernel(const int *__restrict__ ddRowPtr, const int *__restrict__ ddCol,
-                                                           int dRows, int n, int colBits, unsigned long long *__restrict__ key,
+// first[w] = where the entries of chunk w begin
+__global__ __launch_bounds__(kBlock) void chunk_starts_kernel(const int *__restrict__ ddRowPtr, int dRows, int chunkNum, int *__restrict__ first)
+{
+    const int w = blockIdx.x * kBlock + threadIdx.x;
+    if (w <= chunkNum) first[w] = ddRowPtr[min(w * mx::kFragM, dRows)];
+}
+
+// reach[0] = where the last chunk ends that is too long for a workgroup
+__global__ __launch_bounds__(kBlock) void long_chunks_kernel(const int *__restrict__ first, int chunkNum, int *__restrict__ reach)
+{
+    const int w = blockIdx.x * kBlock + threadIdx.x;
+    const bool big = w < chunkNum && first[w + 1] - first[w] > mxs::kLongest;
+    const unsigned long long m = __ballot(big);
+    if (m && (threadIdx.x & 63) == 63 - __builtin_clzll(m)) atomicMax(reach, first[w + 1]);
+}
+
+// key = [chunk of the entry's row][column], payload = the entry, for the first n entries of A_dd: those of the chunks up to
+// the last one that a workgroup has no room for.  (A_dd's rows stand in order of their length, so these are few chunks.)
+__global__ __launch_bounds__(kBlock) void tile_keys_kernel(const int *__restrict__ first, const int *__restrict__ ddCol,
+                                                           int chunkNum, int n, int colBits, unsigned long long *__restrict__ key,
                                                            int *__restrict__ payload)
 {
-    const int e = blockIdx.x * kBlock + threadIdx.x;
-    if (e >= n) return;
-    const int w = line_of(ddRowPtr, dRows, e) / mx::kFragM;
-    key[e] = ((unsigned long long)w << colBits) | (unsigned long long)ddCol[e];
-    payload[e] = e;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(first, chunkNum, n, t0, T);
+#pragma unroll
+    for (int j = 0; j < mxr::kPer; ++j) {
+        const int i = j * kBlock + threadIdx.x, e = t0 + i;
+        if (i >= n - t0) break;
+        key[e] = ((unsigned long long)T.row[i] << colBits) | (unsigned long long)ddCol[e];
+        payload[e] = e;
+    }
 }
+
+// The same order for the chunks that a workgroup has room for.
+// (15.8 million entries, of which 5.6 lie in chunks up to the last of more than 8192: keys and radix sort 1.05 ms, so 0.69, 0.38 of them for those 5.6)
+struct ChunkColumns {
+    const int *ddCol;
+    int colBits;
+    unsigned long long *keyOut;
+    int *payload;
+    __device__ __forceinline__ unsigned key(int, int e) const { return (unsigned)ddCol[e]; }
+    __device__ __forceinline__ void put(int chunk, int, unsigned col, int e, int k) const
+    {
+        keyOut[k] = ((unsigned long long)(unsigned)chunk << colBits) | col;
+        payload[k] = e;
+    }
+};
 
 // head[k] = 1 where sorted position k holds the first occurrence of its (chunk, column)
 __global__ __launch_bounds__(kBlock) void tile_heads_kernel(const unsigned long long *__restrict__ key, int n, int *__restrict__ head)
@@ -313,7 +379,9 @@ __global__ __launch_bounds__(kBlock) void tile_rank_kernel(const unsigned long l
         ecr[e] = rank;
         const int f0 = chunkPtr[w];
         if (head[k]) atox[(size_t)f0 * fragK + rank] = c;
-        const int r = line_of(ddRowPtr, dRows, e) - w * mx::kFragM;
+        int r = 0;  // the row inside the chunk
+#pragma unroll
+        for (int i = 1; i < mx::kFragM; ++i) r += ddRowPtr[min(w * mx::kFragM + i, dRows)] <= e;
         f = f0 + rank / fragK;
         v = 1ull << (r * fragK + rank % fragK);
     }
@@ -346,13 +414,19 @@ __global__ __launch_bounds__(kBlock) void tile_values_kernel(const int *__restri
                                                              const unsigned long long *__restrict__ bits, int dRows, int n, int fragK,
                                                              V *__restrict__ tcVal)
 {
-    const int e = blockIdx.x * kBlock + threadIdx.x;
-    if (e >= n) return;
-    const int i = line_of(ddRowPtr, dRows, e);
-    if (e + 1 < ddRowPtr[i + 1] && ddCol[e + 1] == ddCol[e]) return;  // a later twin wins
-    const int w = i / mx::kFragM, rank = ecr[e], f = chunkPtr[w] + rank / fragK;
-    const int bit = (i - w * mx::kFragM) * fragK + rank % fragK;
-    tcVal[fragPtr[f] + __popcll(bits[f] & ((1ull << bit) - 1))] = ddVal[e];
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(ddRowPtr, dRows, n, t0, T);
+#pragma unroll
+    for (int j = 0; j < mxr::kPer; ++j) {
+        const int k = j * kBlock + threadIdx.x, e = t0 + k;
+        if (k >= n - t0) break;
+        const int i = T.row[k];
+        if (e + 1 < ddRowPtr[i + 1] && ddCol[e + 1] == ddCol[e]) continue;  // a later twin wins
+        const int w = i / mx::kFragM, rank = ecr[e], f = chunkPtr[w] + rank / fragK;
+        const int bit = (i - w * mx::kFragM) * fragK + rank % fragK;
+        tcVal[fragPtr[f] + __popcll(bits[f] & ((1ull << bit) - 1))] = ddVal[e];
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void narrow_bits_kernel(const unsigned long long *__restrict__ bits, int nf, unsigned *__restrict__ out)
@@ -581,18 +655,14 @@ extern "C" int mx_split_device(mx_dtype dtype, int rows, int cols, int nnz, cons
     while (rowBits < 31 && (1ll << rowBits) < (long long)rows) ++rowBits;
     const unsigned keyBits = (unsigned)(colBits + rowBits + 2);
     const size_t nScan = (size_t)std::max(rows, cols) + 1;
-    size_t sortBytes = 0, scanBytes = 0;
-    if (nnz > 0)
-        MXP_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
-                                          (const int *)nullptr, (int *)nullptr, (size_t)nnz, 0u, keyBits, s));
+    size_t scanBytes = 0;
     MXP_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, nScan, rocprim::plus<int>(), s));
-    sortBytes = (sortBytes + 255) & ~(size_t)255;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t colB = al(((size_t)cols + 1) * sizeof(int)), rowB = al(((size_t)rows + 1) * sizeof(int));
-    const size_t denseB = al((size_t)cols + 1), keyB = al((size_t)nnz * 8), payB = al((size_t)nnz * 4);
-    // newCol, notSel, pos [cols+1]; rowRank, rcnt, cdLen, ddLen [rows+1]; dense; keys and payloads in and out
+    const size_t denseB = al((size_t)cols + 1), listB = al(mxs::list_ints(nnz) * sizeof(int));
+    // newCol, notSel, pos [cols+1]; rowRank, rcnt, cdLen, ddLen [rows+1]; dense; the lists of long rows
     Scratch scratch;
-    MXP_TRY(mx::dev_malloc(&scratch.p, 3 * colB + 4 * rowB + denseB + 2 * keyB + 2 * payB + sortBytes + scanBytes + 256));
+    MXP_TRY(mx::dev_malloc(&scratch.p, 3 * colB + 4 * rowB + denseB + listB + scanBytes + 512));
     unsigned char *b = (unsigned char *)scratch.p;
     int *newCol = (int *)b, *notSel = (int *)(b + colB), *pos = (int *)(b + 2 * colB);
     b += 3 * colB;
@@ -600,26 +670,28 @@ extern "C" int mx_split_device(mx_dtype dtype, int rows, int cols, int nnz, cons
     b += 4 * rowB;
     unsigned char *dense = b;
     b += denseB;
-    unsigned long long *keyIn = (unsigned long long *)b, *keyOut = (unsigned long long *)(b + keyB);
-    b += 2 * keyB;
-    int *payIn = (int *)b, *payOut = (int *)(b + payB);
-    b += 2 * payB;
-    void *sortTmp = b, *scanTmp = b + sortBytes;
-    int *bad = (int *)((unsigned char *)sortTmp + sortBytes + scanBytes);  // in the 256 spare bytes at the end
+    int *list = (int *)b;
+    b += listB;
+    void *scanTmp = b;
+    int *bad = (int *)(b + al(scanBytes)), *classCount = bad + 1;  // in the spare bytes at the end
     auto grid = [](long long n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); };
 
     // the caller's arrays become addresses below: row pointers, column ids and both orders are
     // looked at first (1 = rowPtr, 2 = colInd, 4 = descColId, 8 = descRowId)
-    MXP_TRY(hipMemsetAsync(bad, 0, sizeof(int), s));
+    MXP_TRY(hipMemsetAsync(bad, 0, (2 + mxs::kClasses) * sizeof(int), s));
     hipLaunchKernelGGL(pointer_check_kernel, grid((long long)rows + 1), dim3(kBlock), 0, s, rowPtr_dev, rows, nnz, 1, bad);
     if (nnz > 0) hipLaunchKernelGGL(range_check_kernel, grid(nnz), dim3(kBlock), 0, s, colInd_dev, nnz, cols, 2, bad);
     if (dCols > 0) hipLaunchKernelGGL(range_check_kernel, grid(dCols), dim3(kBlock), 0, s, descColId_dev, dCols, cols, 4, bad);
     if (dRows > 0) hipLaunchKernelGGL(range_check_kernel, grid(dRows), dim3(kBlock), 0, s, descRowId_dev, dRows, rows, 8, bad);
     MXP_TRY(hipGetLastError());
+    MXP_TRY(mxs::classify_rows(rowPtr_dev, rows, nnz, list, classCount, s));
+    mxs::RowClasses classes{};
     {
-        int badHost = 0;
-        MXP_TRY(hipMemcpyAsync(&badHost, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+        int got[2 + mxs::kClasses] = {};
+        MXP_TRY(hipMemcpyAsync(got, bad, sizeof(got), hipMemcpyDeviceToHost, s));
         MXP_TRY(hipStreamSynchronize(s));
+        const int badHost = got[0];
+        std::copy(got + 1, got + 2 + mxs::kClasses, classes.n);
         if (badHost) {
             mx::set_error(std::string("mx_split_device: ") + ((badHost & 1) ? "rowPtr does not rise from 0 to nnz" :
                           (badHost & 2) ? "column index out of range" : (badHost & 4) ? "descColId entry out of range" :
@@ -652,8 +724,36 @@ extern "C" int mx_split_device(mx_dtype dtype, int rows, int cols, int nnz, cons
     MXP_TRY(hipGetLastError());
     MXP_TRY(rocprim::exclusive_scan(scanTmp, scanBytes, (const int *)cdLen, cdRowPtr_dev, 0, (size_t)rows + 1, rocprim::plus<int>(), s));
     MXP_TRY(rocprim::exclusive_scan(scanTmp, scanBytes, (const int *)ddLen, ddRowPtr_dev, 0, (size_t)dRows + 1, rocprim::plus<int>(), s));
-    if (nnz > 0) {
-        hipLaunchKernelGGL(split_keys_kernel, grid(nnz), dim3(kBlock), 0, s, rowPtr_dev, colInd_dev, (const int *)newCol,
+    // the totals must be what the caller sized the outputs for
+    int totals[2] = {0, 0};
+    MXP_TRY(hipMemcpyAsync(&totals[0], ddRowPtr_dev + dRows, sizeof(int), hipMemcpyDeviceToHost, s));
+    MXP_TRY(hipMemcpyAsync(&totals[1], cdRowPtr_dev + rows, sizeof(int), hipMemcpyDeviceToHost, s));
+    MXP_TRY(hipStreamSynchronize(s));
+    if (totals[0] != nDD || totals[1] != nnz - nDD) {
+        mx::set_error("mx_split_device: the selection does not belong to this matrix (entry totals differ)");
+        return MX_ERR_ARG;
+    }
+    if (nnz > 0 && classes.n[mxs::kClasses] == 0) {
+        auto split = [&](auto *ddVal, auto *cdVal, auto *val) -> hipError_t {
+            typedef typename std::remove_pointer<decltype(ddVal)>::type V;
+            const SplitRows<V> io{rowPtr_dev, colInd_dev, newCol, rowRank, rcnt, ddRowPtr_dev, cdRowPtr_dev, val, dCols, colBits,
+                                  ddColInd_dev, ddVal, cdColInd_dev, cdVal};
+            return mxs::sort_rows(rowPtr_dev, rows, nnz, list, classes, io, s);
+        };
+        if (dtype == MX_F64) MXP_TRY(split((double *)ddVal_dev, (double *)cdVal_dev, (const double *)val_dev));
+        else MXP_TRY(split((uint16_t *)ddVal_dev, (uint16_t *)cdVal_dev, (const uint16_t *)val_dev));
+    } else if (nnz > 0) {
+        size_t sortBytes = 0;
+        MXP_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
+                                          (const int *)nullptr, (int *)nullptr, (size_t)nnz, 0u, keyBits, s));
+        const size_t keyB = al((size_t)nnz * 8), payB = al((size_t)nnz * 4);
+        Scratch sort;
+        MXP_TRY(mx::dev_malloc(&sort.p, 2 * keyB + 2 * payB + sortBytes + 256));
+        b = (unsigned char *)sort.p;
+        unsigned long long *keyIn = (unsigned long long *)b, *keyOut = (unsigned long long *)(b + keyB);
+        int *payIn = (int *)(b + 2 * keyB), *payOut = (int *)(b + 2 * keyB + payB);
+        void *sortTmp = b + 2 * keyB + 2 * payB;
+        hipLaunchKernelGGL(split_keys_kernel, mxr::tile_grid(nnz), dim3(kBlock), 0, s, rowPtr_dev, colInd_dev, (const int *)newCol,
                            (const int *)rowRank, rows, nnz, dCols, colBits, rowBits, keyIn, payIn);
         MXP_TRY(hipGetLastError());
         MXP_TRY(rocprim::radix_sort_pairs(sortTmp, sortBytes, (const unsigned long long *)keyIn, keyOut, (const int *)payIn, payOut,
@@ -668,16 +768,7 @@ extern "C" int mx_split_device(mx_dtype dtype, int rows, int cols, int nnz, cons
                                (uint16_t *)ddVal_dev, cdColInd_dev, (uint16_t *)cdVal_dev);
         MXP_TRY(hipGetLastError());
     }
-    // the totals must be what the caller sized the outputs for
-    int totals[2] = {0, 0};
-    MXP_TRY(hipMemcpyAsync(&totals[0], ddRowPtr_dev + dRows, sizeof(int), hipMemcpyDeviceToHost, s));
-    MXP_TRY(hipMemcpyAsync(&totals[1], cdRowPtr_dev + rows, sizeof(int), hipMemcpyDeviceToHost, s));
-    MXP_TRY(hipStreamSynchronize(s));
-    if (totals[0] != nDD || totals[1] != nnz - nDD) {
-        mx::set_error("mx_split_device: the selection does not belong to this matrix (entry totals differ)");
-        return MX_ERR_ARG;
-    }
-    return MX_OK;
+    return MX_OK;  // (the scope waits for the stream before it hands the scratch on)
 }
 
 
@@ -713,10 +804,7 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
     const unsigned keyBits = (unsigned)(colBits + chunkBits);
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     auto grid = [](long long m) { return dim3((unsigned)((m + kBlock - 1) / kBlock)); };
-    size_t sortBytes = 0, scanBytes = 0;
-    if (n > 0)
-        MXP_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
-                                          (const int *)nullptr, (int *)nullptr, (size_t)n, 0u, keyBits, s));
+    size_t scanBytes = 0;
     MXP_TRY(rocprim::inclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr,
                                     (size_t)std::max(n, chunkNum) + 1, rocprim::plus<int>(), s));
     {   // the exclusive form may ask for a different amount: take the larger
@@ -725,31 +813,40 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
                                         rocprim::plus<int>(), s));
         scanBytes = std::max(scanBytes, b2);
     }
-    sortBytes = al(sortBytes);
     scanBytes = al(scanBytes);
-    // scratch: keys and payloads in and out, heads, their running count, ecr, per-chunk fragments
+    // scratch: sorted keys and payloads, heads, their running count, ecr, per-chunk fragments and first entries, lists
     const size_t keyB = al((size_t)n * 8), intB = al(((size_t)n + 1) * 4), chB = al(((size_t)chunkNum + 1) * 4);
+    const size_t listB = al(mxs::list_ints(n) * 4);
     Scratch scratch;
-    MXP_TRY(mx::dev_malloc(&scratch.p, 2 * keyB + 5 * intB + 2 * chB + sortBytes + scanBytes + 256));
+    MXP_TRY(mx::dev_malloc(&scratch.p, keyB + 4 * intB + 3 * chB + listB + scanBytes + 256));
     unsigned char *b = (unsigned char *)scratch.p;
-    unsigned long long *keyIn = (unsigned long long *)b, *keyOut = (unsigned long long *)(b + keyB);
-    b += 2 * keyB;
-    int *payIn = (int *)b, *payOut = (int *)(b + intB), *head = (int *)(b + 2 * intB), *run = (int *)(b + 3 * intB),
-        *ecr = (int *)(b + 4 * intB);
-    b += 5 * intB;
-    int *frags = (int *)b, *chunkPtrTmp = (int *)(b + chB);
-    b += 2 * chB;
-    void *sortTmp = b, *scanTmp = b + sortBytes;
+    unsigned long long *keyOut = (unsigned long long *)b;
+    b += keyB;
+    int *payOut = (int *)b, *head = (int *)(b + intB), *run = (int *)(b + 2 * intB), *ecr = (int *)(b + 3 * intB);
+    b += 4 * intB;
+    int *frags = (int *)b, *chunkPtrTmp = (int *)(b + chB), *chunkFirst = (int *)(b + 2 * chB);
+    b += 3 * chB;
+    int *list = (int *)b;
+    b += listB;
+    void *scanTmp = b;
+    mxs::RowClasses classes{};
+    int nLong = 0;  // entries up to the end of the last chunk that a workgroup has no room for
     {
         // the caller's A_dd is about to be used for addressing: pointers and column ids are looked at first
-        int *bad = (int *)((unsigned char *)sortTmp + sortBytes + scanBytes);  // in the 256 spare bytes at the end
-        MXP_TRY(hipMemsetAsync(bad, 0, sizeof(int), s));
+        int *bad = (int *)((unsigned char *)scanTmp + scanBytes);  // in the 256 spare bytes at the end
+        MXP_TRY(hipMemsetAsync(bad, 0, (3 + mxs::kClasses) * sizeof(int), s));
         hipLaunchKernelGGL(pointer_check_kernel, grid((long long)dRows + 1), dim3(kBlock), 0, s, ddRowPtr_dev, dRows, n, 1, bad);
         if (n > 0) hipLaunchKernelGGL(range_check_kernel, grid(n), dim3(kBlock), 0, s, ddColInd_dev, n, dCols, 2, bad);
+        hipLaunchKernelGGL(chunk_starts_kernel, grid((long long)chunkNum + 1), dim3(kBlock), 0, s, ddRowPtr_dev, dRows, chunkNum, chunkFirst);
+        hipLaunchKernelGGL(long_chunks_kernel, grid((long long)chunkNum + 1), dim3(kBlock), 0, s, (const int *)chunkFirst, chunkNum, bad + 1);
         MXP_TRY(hipGetLastError());
-        int badHost = 0;
-        MXP_TRY(hipMemcpyAsync(&badHost, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+        MXP_TRY(mxs::classify_rows(chunkFirst, chunkNum, n, list, bad + 2, s));
+        int got[3 + mxs::kClasses] = {};
+        MXP_TRY(hipMemcpyAsync(got, bad, sizeof(got), hipMemcpyDeviceToHost, s));
         MXP_TRY(hipStreamSynchronize(s));
+        const int badHost = got[0];
+        nLong = got[1];
+        std::copy(got + 2, got + 3 + mxs::kClasses, classes.n);
         if (badHost) {
             mx::set_error((badHost & 1) ? "mx_tiles_device: ddRowPtr does not rise from 0 to nnzRowD"
                                         : "mx_tiles_device: column index out of range");
@@ -759,10 +856,22 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
 
     // distinct columns per chunk: sort by (chunk, column), mark first occurrences, count them
     if (n > 0) {
-        hipLaunchKernelGGL(tile_keys_kernel, grid(n), dim3(kBlock), 0, s, ddRowPtr_dev, ddColInd_dev, dRows, n, colBits, keyIn, payIn);
-        MXP_TRY(hipGetLastError());
-        MXP_TRY(rocprim::radix_sort_pairs(sortTmp, sortBytes, (const unsigned long long *)keyIn, keyOut, (const int *)payIn, payOut,
-                                          (size_t)n, 0u, keyBits, s));
+        MXP_TRY(mxs::sort_rows(chunkFirst, chunkNum, n, list, classes, ChunkColumns{ddColInd_dev, colBits, keyOut, payOut}, s));
+        if (nLong > 0) {
+            size_t sortBytes = 0;
+            MXP_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
+                                              (const int *)nullptr, (int *)nullptr, (size_t)nLong, 0u, keyBits, s));
+            Scratch sort;
+            const size_t inB = al((size_t)nLong * 8), payB = al((size_t)nLong * 4);
+            MXP_TRY(mx::dev_malloc(&sort.p, inB + payB + sortBytes + 256));
+            unsigned long long *keyIn = (unsigned long long *)sort.p;
+            int *payIn = (int *)((unsigned char *)sort.p + inB);
+            hipLaunchKernelGGL(tile_keys_kernel, mxr::tile_grid(nLong), dim3(kBlock), 0, s, (const int *)chunkFirst, ddColInd_dev, chunkNum, nLong,
+                               colBits, keyIn, payIn);
+            MXP_TRY(hipGetLastError());
+            MXP_TRY(rocprim::radix_sort_pairs((unsigned char *)sort.p + inB + payB, sortBytes, (const unsigned long long *)keyIn, keyOut,
+                                              (const int *)payIn, payOut, (size_t)nLong, 0u, keyBits, s));
+        }
         hipLaunchKernelGGL(tile_heads_kernel, grid(n), dim3(kBlock), 0, s, (const unsigned long long *)keyOut, n, head);
         MXP_TRY(hipGetLastError());
         MXP_TRY(rocprim::inclusive_scan(scanTmp, scanBytes, (const int *)head, run, (size_t)n, rocprim::plus<int>(), s));
@@ -805,11 +914,11 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
     MXP_TRY(rocprim::exclusive_scan(scanTmp, scanBytes, (const int *)head, fragPtr, 0, (size_t)totalTcFrags + 1, rocprim::plus<int>(), s));
     if (n > 0) {
         if (dtype == MX_F64)
-            hipLaunchKernelGGL(tile_values_kernel<double>, grid(n), dim3(kBlock), 0, s, ddRowPtr_dev, ddColInd_dev,
+            hipLaunchKernelGGL(tile_values_kernel<double>, mxr::tile_grid(n), dim3(kBlock), 0, s, ddRowPtr_dev, ddColInd_dev,
                                (const double *)ddVal_dev, (const int *)ecr, (const int *)chunkPtr, (const int *)fragPtr,
                                (const unsigned long long *)bits, dRows, n, fragK, (double *)tcVal);
         else
-            hipLaunchKernelGGL(tile_values_kernel<uint16_t>, grid(n), dim3(kBlock), 0, s, ddRowPtr_dev, ddColInd_dev,
+            hipLaunchKernelGGL(tile_values_kernel<uint16_t>, mxr::tile_grid(n), dim3(kBlock), 0, s, ddRowPtr_dev, ddColInd_dev,
                                (const uint16_t *)ddVal_dev, (const int *)ecr, (const int *)chunkPtr, (const int *)fragPtr,
                                (const unsigned long long *)bits, dRows, n, fragK, (uint16_t *)tcVal);
         MXP_TRY(hipGetLastError());

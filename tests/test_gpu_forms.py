@@ -158,3 +158,36 @@ def test_memory_kept_between_calls_is_bounded_and_given_back(mx):
     mx.release_memory()
     free1 = torch.cuda.mem_get_info()[0]
     assert free0 <= free1 <= free0 + total // 128 + (64 << 20)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float16])
+@pytest.mark.parametrize("lens", [
+    [511, 512, 513, 1, 0, 1535, 1536, 1537, 2, 2047, 2048, 2049, 3],  # a workgroup's share of short rows, the first long class
+    [4095, 4096, 4097, 7, 8191, 8192, 0, 5, 512, 512, 512, 512],      # the other two classes
+    [20, 8193, 3000, 1, 700, 0, 0, 9],                                # a row that no workgroup has room for
+    [1] * 1536 + [512] * 4 + [1] * 511 + [513] + [0] * 40 + [2] * 700,
+    [0] * 20000 + [3] + [0] * 9000 + [600, 0, 2] + [0] * 40000,       # nearly all rows empty
+], ids=["short", "long", "beyond", "packed", "empty"])
+def test_rows_put_in_order(mx, dtype, lens):
+    """Split, tile encoding and slice layout made on the device from rows in any order that name columns twice, with
+    rows at the edges of what a workgroup puts in order: byte for byte the host's."""
+    import torch
+    rng = np.random.default_rng(len(lens))
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    n, cols = int(ptr[-1]), 9000
+    A = mx.Csr(len(lens), cols, ptr, rng.integers(0, cols, n).astype(np.int32), (rng.integers(1, 2000, n) / 64.0).astype(dtype))
+    rp, ci, va = (torch.from_numpy(a).cuda() for a in (A.rowPtr, A.colInd, A.val))
+    for tau in [(0.5, 0.25), (1.0, 1.0), (0.1, 0.02)]:
+        P = mx.Partition(A, *tau)
+        dc, dr, sel = mx.select_device(rp, ci, cols, *tau)
+        got = mx.split_device(rp, ci, va, cols, sel, dc, dr)
+        T = mx.tiles_device(got[0], got[1], got[2], sel["dCols"])
+        pairs = list(zip(got, ("ddRowPtr", "ddColInd", "ddVal", "cdRowPtr", "cdColInd", "cdVal")))
+        pairs += [(T[k], k) for k in ("chunkPtr", "sparse_AToX_index", "fragPtr", "fragBit", "tcVal")]
+        for g, name in pairs:
+            want = np.ascontiguousarray(getattr(P, name))
+            assert np.array_equal(g.cpu().numpy().view(np.uint8), want.view(np.uint8)), (tau, name)
+        P.close()
+    H, D = mx.slice_layout(A, nCU=16), mx.slice_layout(A, nCU=16, device=True)
+    for k in ("chunkEnd", "segPtr", "segIdx", "rowInfo", "ecol", "eval"):
+        assert np.array_equal(H[k].view(np.uint8), D[k].view(np.uint8)), k
