@@ -4,7 +4,7 @@
 // workgroup, in registers and LDS, and the matrix is read once and written once.  (A radix sort of all entries by
 // {row, key} moves 24 bytes an entry through memory for every eight bits of the two together, six times for a million
 // rows and columns: 0.83 ms for 15.8 million entries, and 28 bytes an entry of working memory; this takes 0.31 to 0.44 ms and none.  Without that
-memory the plan of such a matrix stays inside what is kept from one call to the next: 15.4 -> 7.2 ms, 5.7 of them hipFree.)
+// memory the plan of such a matrix stays inside what is kept from one call to the next: 15.4 -> 7.2 ms, 5.7 of them hipFree.)
 //
 //   rows of at most kShort entries   several to a workgroup, 1536 entries and the rest of the last row at a time
 //   rows of at most 2048/4096/8192   one to a workgroup of 256/512/1024 threads, from lists made on the device
