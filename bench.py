@@ -361,7 +361,7 @@ def run_workload(mx, torch, ora, cfg, steps, warmup, mode, traffic, only_tau=Non
         ("" if scale == 1.0 else ", at %g of the benchmark's rows" % scale),
         "dtype": dtype, "rows": A.rows, "nnz": A.nnz,
         "tau_c": tau[0], "tau_r": tau[1], "plan": plan_kind, "plan_flags": "MX_PLAN_DEFAULT" if FLAGS == mx.MX_PLAN_DEFAULT else "MX_PLAN_KEEP_TILES" if FLAGS == mx.MX_PLAN_KEEP_TILES else int(FLAGS),
-        "csr_variant": ("rows", "slices", "split", "offsets")[info["csr_variant"]], "csr_one_launch": bool(info["csr_fused"]),
+        "csr_variant": ("rows", "slices", "split", "offsets", "windows")[info["csr_variant"]], "csr_one_launch": bool(info["csr_fused"]),
         "csr_entries_kept_in_cache": bool(info["csr_keep"]),
         "tile_nnz": info["tile_nnz"], "csr_nnz": info["csr_nnz"],
         "ms_per_step": wall_ms, "ms_per_step_events": ev_total,

@@ -480,12 +480,14 @@ typedef struct mx_plan_info {
     int csr_blocks;      /* workgroups of the CSR kernel */
     int csr_variant;     /* 0 = row tiles (csr_rows_kernel), 1 = column slices (csr_slice_kernel),
                             2 = row tiles for the short rows, then column slices for the long ones, 3 = rows that
-                            repeat a pattern of column offsets (csr_offsets_kernel): a stencil, a few diagonals.  A
-                            plan that keeps no tiles looks for 3 unless a flag or the environment names another form */
+                            repeat a pattern of column offsets (csr_offsets_kernel): a stencil, a few diagonals,
+                            4 = neighbouring rows that reach into one window of x (csr_window_kernel): a mesh of small
+                            bandwidth.  A plan that keeps no tiles looks for 3 and then 4 unless a flag or the environment names another form */
     double tile_bytes;   /* bytes the tile kernel must read+write per launch */
     double csr_bytes;    /* bytes the CSR kernel must read+write per launch */
     int csr_main_kernel; /* the CSR-part kernel that holds most entries (the one mx_time_csr_main times):
-                            0 = csr_rows_kernel, 1 = csr_slice_kernel, 2 = csr_offsets_kernel */
+                            0 = csr_rows_kernel, 1 = csr_slice_kernel, 2 = csr_offsets_kernel,
+                            3 = csr_window_kernel */
     int csr_main_nnz;    /* entries that kernel holds */
     int tile_variant;    /* 1 when part of the tiles runs through tile_dense_kernel: binary16 rows whose columns
                             fill at most 8 blocks of 8 consecutive columns at least half (a row of a dense strip in
@@ -623,7 +625,7 @@ typedef struct mx_plan_layout_view {
     mx_tile_layout_view tiles[2];
     int csr_variant;     /* the form mx_plan_create would give the CSR part on a device with nCU compute units:
                             0 row tiles, 1 slices, 2 split; -1 when MX_PLAN_AUTOTUNE=1 leaves it to a timed trial.  (A
-                            matrix in form 3 of mx_plan_info.csr_variant is recognised on the device; here it reads as
+                            matrix in form 3 or 4 of mx_plan_info.csr_variant is recognised on the device; here it reads as
                             the form it would have otherwise) */
     double est_rows_us, est_slices_us; /* the estimates behind that choice (mx_plan_info) */
 } mx_plan_layout_view;

@@ -236,6 +236,44 @@ __attribute__((weak)) int build_offsets_device(mx_dtype dtype, int rows, int col
                                                const void *val_dev, DeviceOffsets &D, hipStream_t s);
 __attribute__((weak)) hipError_t launch_offsets(mx_dtype dtype, const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s);
 
+// The CSR part of a matrix whose neighbouring rows reach into one stretch of x (a mesh numbered for a small bandwidth):
+// chunks of 64 consecutive rows, a row per lane, kWindowWaves of them to a workgroup, which puts the window of x that its rows
+// reach into LDS.  Per chunk and unit four entries of every row: their places in the window (16 bits) and their values; a
+// place that no entry owns is zeroPlace, where the kernel puts a zero, with the value zero.  Entries outside the
+// window are kept with their columns and gathered from memory.
+struct DeviceWindows {
+    int rows = 0, cols = 0, nnz = 0, nChunks = 0, nWG = 0;
+    int units = 0, unitBytes = 0;      // units of all chunks; bytes of a wave's unit
+    int zeroPlace = 0, ldsBytes = 0;   // elements of the widest window; LDS of a workgroup
+    int *window = nullptr;             // [nWG][2] {first element of x, vectors of 16 bytes}
+    int farSteps = 0;                  // of all chunks: a step is one entry outside the window per row
+    int nApart = 0;                    // chunks that a workgroup of its own gathers from memory
+    int *chunk = nullptr;              // [nChunks][4] {first unit, units (-1: a chunk apart), first far step, far steps}
+    int *apart = nullptr;              // [nApart] chunks, ascending
+    unsigned char *stream = nullptr;   // [units + 1][unitBytes]
+    int *farCol = nullptr;             // [farSteps + 1][64] columns, -1 for none
+    void *farVal = nullptr;            // [farSteps + 1][64] values
+    bool keep = false;                 // the units are read with plain loads (they may stay in the caches), not streamed
+};
+constexpr int kWindowUnit = 4;                // entries of a row in a unit
+constexpr int kWindowWaves = 8;               // chunks (and waves) of a workgroup
+constexpr int kWindowRowsLeast = 32768;       // fewest rows of a matrix that takes the form (33 thousand of 40 entries, binary16: 4.3 us, row tiles 5.3)
+constexpr int kWindowEntriesLeast = 600000;   // binary64: fewest entries (0.33 million: 4.0 us, row tiles 3.8; 0.9 million: 4.2, 4.7)
+constexpr int kWindowMeanLeast = 4;           // fewest entries a row on average
+constexpr double kWindowFill = 1.5;           // most bytes stored per byte of the entries
+constexpr double kWindowFarMost = 0.12;       // most entries outside the windows, of all
+constexpr int kWindowFarSteps = 3;            // most entries of a row outside the window, but for chunks apart
+constexpr int kWindowTrim = 32;               // bytes that a far entry is worth: an end of the window with fewer entries is left out
+constexpr int kWindowLongest = 1024;          // most entries of a row
+constexpr double kWindowShare = 0.6;          // most bytes of a window per byte of its workgroup's entries
+constexpr int kWindowBytesMost = 80 << 10;    // of a window: two workgroups share the LDS of a CU
+constexpr int window_unit_bytes(bool f64) { return 64 * kWindowUnit * (f64 ? 10 : 4); }
+void free_windows(DeviceWindows &D);
+// As build_offsets_device and launch_offsets.
+__attribute__((weak)) int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev,
+                                               const void *val_dev, DeviceWindows &D, hipStream_t s);
+__attribute__((weak)) hipError_t launch_windows(mx_dtype dtype, const DeviceWindows &D, const void *x, void *y, int accumulate, hipStream_t s);
+
 // The sums of the virtual rows (DeviceSlices::partial) of mx_spmv_static live in a fixed array
 // in device memory instead of the plan's own buffer: static_scratch gives the address of the
 // current device's copy (looked up once per device, no allocation).

@@ -37,6 +37,17 @@ void mx::free_offsets(mx::DeviceOffsets &D)
     D = mx::DeviceOffsets();
 }
 
+void mx::free_windows(mx::DeviceWindows &D)
+{
+    (void)mx::dev_free(D.window);
+    (void)mx::dev_free(D.chunk);
+    (void)mx::dev_free(D.farCol);
+    (void)mx::dev_free(D.farVal);
+    (void)mx::dev_free(D.apart);
+    (void)mx::dev_free(D.stream);
+    D = mx::DeviceWindows();
+}
+
 extern "C" void mx_plan_destroy(mx_plan *plan)
 {
     if (!plan) return;
@@ -44,6 +55,7 @@ extern "C" void mx_plan_destroy(mx_plan *plan)
     free_csr(plan->csr);
     free_slices(plan->slices);
     mx::free_offsets(plan->offsets);
+    mx::free_windows(plan->windows);
     free_tiles(plan->tiles);
     free_tiles(plan->strips);
     (void)mx::dev_free(plan->ywide);
@@ -222,6 +234,7 @@ double mxp::touched_bytes(const mx_plan *plan)
         const mx::DeviceOffsets &D = plan->offsets;
         b += (double)D.units * 64 * D.unitBytes + (double)D.nOffs * 4 + (double)D.nChunks * 16;
     }
+    if (plan->csr_variant == 4) b += (double)plan->windows.units * plan->windows.unitBytes + (double)plan->windows.farSteps * 64 * (4 + es) + (double)plan->windows.nChunks * 16;
     if (plan->csr_variant == 0 || plan->csr_variant == 2) b += (double)plan->csr.nnz * ((plan->csr.useDict ? 1.0 : es) + 4.0) + ((double)plan->rows + 1) * 4;
     if (plan->csr_variant == 1 || plan->csr_variant == 2) b += (double)slice_entry_bytes(plan) + (double)slice_handoff_bytes(plan) - (double)plan->rows * es;
     if (plan->tiles.steps)
@@ -245,11 +258,12 @@ void mxp::decide_keep(mx_plan *plan, int flags)
 {
     mx::DeviceSlices &L = plan->slices;
     L.keep = false;
-    if (plan->csr_variant == 3) {
+    if (plan->csr_variant == 3 || plan->csr_variant == 4) {
         const int env = mx::opt().csr_keep;
-        if ((flags & MX_PLAN_STREAM) || env == 0) plan->offsets.keep = false;
-        else if ((flags & MX_PLAN_KEEP) || env == 1) plan->offsets.keep = true;
-        else plan->offsets.keep = touched_bytes(plan) <= (double)mx::kOffsetsKeepBytes;
+        bool &keep = plan->csr_variant == 3 ? plan->offsets.keep : plan->windows.keep;
+        if ((flags & MX_PLAN_STREAM) || env == 0) keep = false;
+        else if ((flags & MX_PLAN_KEEP) || env == 1) keep = true;
+        else keep = touched_bytes(plan) <= (double)mx::kOffsetsKeepBytes;
         return;
     }
     if (plan->csr_variant == 0) return;
@@ -295,12 +309,20 @@ bool mxp::may_look_for_form(int flags)
     const mx::Options &o = mx::opt();
     return !(flags & (MX_PLAN_CSR_ROWS | MX_PLAN_CSR_SLICES | MX_PLAN_FUSE)) && o.csr_kernel == 0 && o.csr_fused != 1 && !o.autotune;
 }
-int mxp::try_offsets(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took)
+int mxp::try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took)
 {
     *took = false;
     const int rc = mx::build_offsets_device(plan->dtype, plan->rows, plan->cols, nnz, rowPtr_dev, colInd_dev, val_dev, plan->offsets, nullptr);
-    if (rc || plan->offsets.nChunks == 0) return rc;
+    if (rc) return rc;
     plan->csr_variant = 3;
+    if (plan->offsets.nChunks == 0) {
+        const int rcw = mx::build_windows_device(plan->dtype, plan->rows, plan->cols, nnz, rowPtr_dev, colInd_dev, val_dev, plan->windows, nullptr);
+        plan->csr_variant = 4;
+        if (rcw || plan->windows.nChunks == 0) {
+            plan->csr_variant = 0;
+            return rcw;
+        }
+    }
     plan->csr_nnz = nnz;
     decide_keep(plan, flags);
     *took = true;
@@ -329,14 +351,14 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
     const size_t es = (size_t)mx::elem_size(plan->dtype);
     plan->csr_nnz = nnz;
     if (alone && may_look_for_form(flags)) {
-        // (the offset form is found and laid out on the device, whatever MX_LAYOUT says)
+        // (the offset and window forms are found and laid out on the device, whatever MX_LAYOUT says)
         int *rp = nullptr, *ci = nullptr;
         void *va = nullptr;
         bool took = false;
         int e = upload(&rp, rowPtr, (size_t)rows + 1);
         if (!e) e = upload(&ci, col, (size_t)nnz);
         if (!e) e = upload_bytes(&va, val, (size_t)nnz * es);
-        if (!e) e = try_offsets(plan, nnz, rp, ci, va, flags, &took);
+        if (!e) e = try_forms(plan, nnz, rp, ci, va, flags, &took);
         (void)mx::dev_free(rp);
         (void)mx::dev_free(ci);
         (void)mx::dev_free(va);

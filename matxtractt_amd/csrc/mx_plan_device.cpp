@@ -35,7 +35,7 @@ static int setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, 
     const int S = rows > 0 ? slice_count(dtype, rows, cols, nnz, nCU) : 0;
     if (alone && may_look_for_form(flags)) {
         bool took = false;
-        if ((rc = try_offsets(plan, nnz, rowPtr_dev, colInd_dev, val_dev, flags, &took))) return rc;
+        if ((rc = try_forms(plan, nnz, rowPtr_dev, colInd_dev, val_dev, flags, &took))) return rc;
         if (took) return MX_OK;
     }
     bool want[2] = {true, S > 0};

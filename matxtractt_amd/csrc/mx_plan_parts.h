@@ -138,8 +138,9 @@ struct mx_plan {
     mx::DeviceCsr csr;        // CSR part (or its short rows), row-tile form (csr_rows_kernel)
     mx::DeviceSlices slices;  // CSR part (or its long rows), x-resident-in-LDS form (csr_slice_kernel)
     mx::DeviceOffsets offsets; // CSR part, offset form (csr_offsets_kernel)
+    mx::DeviceWindows windows; // CSR part, window form (csr_window_kernel)
     int csr_variant = 0;      // 0 = row tiles, 1 = slices, 2 = row tiles for the short rows, then slices for the long ones,
-                              // 3 = rows that repeat a pattern of column offsets
+                              // 3 = rows that repeat a pattern of column offsets, 4 = a window of x per workgroup
     bool fused = false;       // slices in the one-launch form (slices.fused), until a misplaced workgroup is reported
     unsigned fused_seq = 0;   // one-launch products queued so far
     int csr_nnz = 0;
@@ -254,11 +255,11 @@ void decide_keep(mx_plan *plan, int flags);
 double touched_bytes(const mx_plan *plan);
 CsrChoice choose_csr_form(mx_dtype dtype, int rows, int cols, const int *rowPtr, const int *col, const void *val, int flags, int nCU,
                           int S, bool mayFuse = false);
-// Whether a plan that keeps no tiles may take a form that is looked for in the matrix itself (the offset form): no flag
+// Whether a plan that keeps no tiles may take a form that is looked for in the matrix itself (the offset and window forms): no flag
 // and nothing in the environment asks for another form or for a timed choice.
 bool may_look_for_form(int flags);
-// Tries the offset form on a CSR part in device memory; *took says whether the plan has its CSR part now.
-int try_offsets(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took);
+// Tries the offset form, then the window form, on a CSR part in device memory; *took says whether the plan has its CSR part now.
+int try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took);
 int setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const void *val, int flags, const char *stripRows = nullptr,
                    std::pair<std::vector<int>, std::vector<int>> *segOut = nullptr, bool alone = true);
 int tiles_worth(mx_dtype dtype, int fragM, int fragK, bool blocks64, double generalEntries, double generalFrags, double stripEntries,

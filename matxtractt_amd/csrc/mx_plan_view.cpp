@@ -63,6 +63,15 @@ extern "C" int mx_plan_arrays(const mx_plan *plan, mx_plan_array *out, int cap, 
         add("offsets.stream", D.stream, (size_t)D.units * 64 * D.unitBytes);
         add("offsets.dict", D.dict, 256 * es);
     }
+    if (plan->csr_variant == 4) {
+        const mx::DeviceWindows &D = plan->windows;
+        add("windows.window", D.window, (size_t)D.nWG * 8);
+        add("windows.chunk", D.chunk, (size_t)D.nChunks * 16);
+        add("windows.stream", D.stream, (size_t)D.units * D.unitBytes);
+        add("windows.farCol", D.farCol, (size_t)D.farSteps * 64 * 4);
+        add("windows.apart", D.apart, (size_t)D.nApart * 4);
+        add("windows.farVal", D.farVal, (size_t)D.farSteps * 64 * es);
+    }
     if (plan->csr_variant == 0 || plan->csr_variant == 2) {
         const mx::DeviceCsr &A = plan->csr;
         add("csr.rowPtr", A.rowPtr, ((size_t)A.rows + 1) * 4);
@@ -241,7 +250,7 @@ extern "C" int mx_plan_get_info(const mx_plan *plan, mx_plan_info *info)
     info->tile_frags = plan->tiles.frags + plan->strips.frags;
     info->tile_nnz = plan->tile_nnz;
     info->csr_nnz = plan->csr_nnz;
-    info->csr_blocks = plan->csr_variant == 3 ? plan->offsets.nChunks : plan->csr_variant == 1 ? plan->slices.nWG : plan->csr.nBlocks;
+    info->csr_blocks = plan->csr_variant == 4 ? plan->windows.nWG : plan->csr_variant == 3 ? plan->offsets.nChunks : plan->csr_variant == 1 ? plan->slices.nWG : plan->csr.nBlocks;
     info->csr_variant = plan->csr_variant;
     // what each kernel has to move at least once: its arrays, x once, its y rows
     info->csr_bytes = (double)plan->csr_nnz * (es + 4) + ((double)plan->rows + 1) * 4 + (double)plan->cols * es +
@@ -257,11 +266,11 @@ extern "C" int mx_plan_get_info(const mx_plan *plan, mx_plan_info *info)
                             (double)plan->strips.frags * 8 * es + (double)plan->strips.chunkNum * 8 * es;
     (void)bitBytes;
     const bool sliceMain = plan->csr_variant == 1 || (plan->csr_variant == 2 && plan->slices.nnz > plan->csr.nnz);
-    info->csr_main_kernel = plan->csr_variant == 3 ? 2 : sliceMain ? 1 : 0;
+    info->csr_main_kernel = plan->csr_variant >= 3 ? plan->csr_variant - 1 : sliceMain ? 1 : 0;
     info->csr_main_nnz = plan->csr_variant == 2 ? (sliceMain ? plan->slices.nnz : plan->csr.nnz) : plan->csr_nnz;
     info->tile_variant = plan->strips.steps > 0 ? (plan->dtype == MX_F64 ? 2 : 1) : 0;
     info->tile_strip_nnz = plan->strips.vals;
-    info->csr_value_dict = plan->csr_variant == 3 ? plan->offsets.nDict : plan->csr_variant == 1 ? (plan->slices.useDict ? plan->slices.nDict : 0)
+    info->csr_value_dict = plan->csr_variant == 4 ? 0 : plan->csr_variant == 3 ? plan->offsets.nDict : plan->csr_variant == 1 ? (plan->slices.useDict ? plan->slices.nDict : 0)
                                                   : (plan->csr.useDict ? plan->csr.nDict : 0);
     info->est_rows_us = plan->est_rows_us;
     info->est_slices_us = plan->est_slices_us;
@@ -273,7 +282,7 @@ extern "C" int mx_plan_get_info(const mx_plan *plan, mx_plan_info *info)
     info->csr_fused = plan->csr_variant == 1 && plan->fused ? 1 : 0;
     info->opt_flags = plan->opt_flags;
     info->opt_tile_gate = plan->opt_tile_gate;
-    info->csr_keep = (plan->csr_variant == 3 ? plan->offsets.keep : plan->csr_variant != 0 && plan->slices.keep) ? 1 : 0;
+    info->csr_keep = (plan->csr_variant == 4 ? plan->windows.keep : plan->csr_variant == 3 ? plan->offsets.keep : plan->csr_variant != 0 && plan->slices.keep) ? 1 : 0;
     info->touched_bytes = mxp::touched_bytes(plan);
     return MX_OK;
 }

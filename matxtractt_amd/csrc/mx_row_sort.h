@@ -36,7 +36,7 @@ struct RowClasses {
 inline size_t list_ints(long long entries) { return (size_t)(entries / kShort + entries / 2048 + entries / 4096 + 3); }
 
 // count[c] rows of class c, in list + list_at(c, entries)
-__global__ __launch_bounds__(256) inline void row_classes_kernel(const int *__restrict__ ptr, int rows, int entries, int *__restrict__ list,
+static __global__ __launch_bounds__(256) void row_classes_kernel(const int *__restrict__ ptr, int rows, int entries, int *__restrict__ list,
                                                                  int *__restrict__ count)
 {
     __shared__ int here[kClasses + 1], first[kClasses + 1];  // (one atomic per workgroup and class)

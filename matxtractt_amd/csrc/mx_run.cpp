@@ -50,6 +50,10 @@ extern "C" int mx_debug_fused_misplaced(int set)
 int mxp::launch_csr_part(mx_plan *plan, const void *x, void *y, int accumulate, hipStream_t s, const mx::DeviceTiles *strips, void *partial,
                          void *ywide)
 {
+    if (plan->csr_variant == 4) {
+        MX_HIP(mx::launch_windows(plan->dtype, plan->windows, x, y, accumulate, s));
+        return MX_OK;
+    }
     if (plan->csr_variant == 3) {
         MX_HIP(mx::launch_offsets(plan->dtype, plan->offsets, x, y, accumulate, s));
         return MX_OK;
@@ -217,7 +221,7 @@ extern "C" int mx_time_csr_main(mx_plan *plan, const void *x_dev, void *y_dev, i
     if (int bad = check_x(plan, x_dev, "mx_time_csr_main")) return bad;
     int rc = time_loop(plan, warm, iters, [&]() -> int {
         // the kernel that holds most of the entries
-        if (plan->csr_variant == 3 || (plan->csr_variant == 1 && plan->fused))
+        if (plan->csr_variant >= 3 || (plan->csr_variant == 1 && plan->fused))
             return launch_csr_part(plan, x_dev, y_dev, 0, s);
         if (plan->csr_variant == 1 || (plan->csr_variant == 2 && plan->slices.nnz > plan->csr.nnz))
             MX_HIP(mx::launch_slices(plan->dtype, plan->slices, x_dev, y_dev, 0, s, 1));
@@ -363,7 +367,10 @@ extern "C" int mx_time_kernels(mx_plan *plan, const void *x_dev, void *y_dev, in
         add(std::string("csr_offsets_kernel<") + vt + (plan->offsets.nDict > 0 ? ",dict" : "") + (plan->offsets.keep ? ",keep>" : ">"),
             (double)plan->csr_nnz * (es + 4) + xBytes + yBytes, plan->csr_nnz,
             [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, 0, s); });
-    if (plan->csr_variant != 1 && plan->csr_variant != 3 && plan->csr.nBlocks > 0) {
+    if (plan->csr_variant == 4)
+        add(std::string("csr_window_kernel<") + vt + (plan->windows.keep ? ",keep>" : ">"), (double)plan->csr_nnz * (es + 4) + xBytes + yBytes,
+            plan->csr_nnz, [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, 0, s); });
+    if ((plan->csr_variant == 0 || plan->csr_variant == 2) && plan->csr.nBlocks > 0) {
         const bool last = plan->csr_variant == 0;  // writes y for good
         add(std::string("csr_rows_kernel<") + vt + (plan->csr.useDict ? ",dict>" : ">"),
             (double)plan->csr.nnz * (es + 4) + xBytes + (last ? yBytes : 0.0), plan->csr.nnz, [&]() -> int {

@@ -191,3 +191,57 @@ def test_rows_put_in_order(mx, dtype, lens):
     H, D = mx.slice_layout(A, nCU=16), mx.slice_layout(A, nCU=16, device=True)
     for k in ("chunkEnd", "segPtr", "segIdx", "rowInfo", "ecol", "eval"):
         assert np.array_equal(H[k].view(np.uint8), D[k].view(np.uint8)), k
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float16])
+@pytest.mark.parametrize("rows,cols,half,far", [
+    (40000, 40000, 300, 0),      # nothing outside the windows
+    (40001, 40000, 300, 300),    # one row beyond whole chunks; a few rows that reach elsewhere
+    (65600, 30011, 900, 2000),   # fewer columns, an odd number: the last windows end at the end of x
+    (40007, 90005, 2000, 40007), # more columns; an entry outside for every row
+])
+def test_window_form(mx, ora, dtype, rows, cols, half, far):
+    """Matrices whose neighbouring rows reach into one window of x, with entries outside it, chunks taken apart for a
+    row with many of those, empty rows and whole empty chunks, rows in any order that name a column twice: the product
+    from both routes equals the oracle's (integers: every sum is exact), entries kept or streamed, with x at any element;
+    a row's sum is not touched by an infinite x that the row does not name."""
+    import torch
+    rng = np.random.default_rng(rows + far)
+    lens = rng.integers(14, 21, rows)
+    lens[5], lens[640:704], lens[1000:1003], lens[-1] = 90, 0, 0, 1
+    r = np.repeat(np.arange(rows), lens)
+    c = np.clip(r * cols // rows + rng.integers(-half, half + 1, r.size), 0, cols - 1)
+    lo = np.concatenate([[0], np.cumsum(lens)])
+    for i in rng.choice(rows, far, replace=False) if far else []:
+        if lens[i] > 1:
+            c[lo[i] + rng.integers(0, lens[i])] = rng.integers(0, cols)
+    if far:
+        c[lo[2000]:lo[2000] + 12] = rng.integers(0, cols, 12)   # more than a lane takes beside its window
+    c[lo[3000] + 1] = c[lo[3000]]
+    val = rng.integers(1, 4, r.size) * rng.choice([-1, 1], r.size)
+    if dtype == np.float64:
+        val = val * rng.integers(1, 1000, r.size)  # (few distinct binary64 values would send it to another form)
+    A = mx.Csr(rows, cols, lo.astype(np.int32), c.astype(np.int32), val.astype(dtype))
+    x = rng.integers(-2, 3, cols).astype(dtype)
+    ref = _exact(ora, A, x)
+    dev = [torch.from_numpy(a).cuda() for a in (A.rowPtr, A.colInd, A.val)]
+    xd = torch.zeros(cols + 1, dtype=torch.from_numpy(x).dtype, device="cuda")[1:]  # not at a multiple of 16 bytes
+    xd.copy_(torch.from_numpy(x))
+    arrays = None
+    for plan in (mx.Plan(mx.Partition(A, 0.0, 0.0)), mx.Plan.from_device(*dev, cols, 0.0, 0.0),
+                 mx.Plan.from_device(*dev, cols, 0.0, 0.0, mx.MX_PLAN_STREAM)):
+        assert plan.info["csr_variant"] == 4 and plan.info["csr_main_kernel"] == 3, plan.info
+        got = plan.arrays()
+        assert len(got["windows.apart"]) > 0 or not far
+        assert arrays is None or got == arrays
+        arrays = got
+        y = torch.full((rows,), 7.0, dtype=xd.dtype, device="cuda")
+        plan.spmv(xd, y)
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy(), ref)
+    bad = x.copy()
+    bad[[0, cols // 2, cols - 1]] = np.inf
+    touched = np.zeros(rows, bool)
+    touched[r[~np.isfinite(bad[A.colInd])]] = True
+    got = plan.spmv(torch.from_numpy(bad).cuda()).cpu().numpy()
+    assert np.array_equal(~np.isfinite(got), touched)
