@@ -251,14 +251,25 @@ __global__ __launch_bounds__(kBlock) void row_info_kernel(const int *__restrict_
         const bool listed = n > 1 && !fetched;
         isLight[r] = listed && n <= lightSegs;
         isHeavy[r] = listed && n > lightSegs;
-        if (listed && n <= lightSegs && n > 4) atomicOr(over4, 1);
+        if (listed && n <= lightSegs && n > 4 && *(volatile int *)over4 == 0) atomicOr(over4, 1);
     } else if (r == rows) {  // the scans run over rows + 1 elements
         isLight[r] = isHeavy[r] = 0;
     }
-    // the most virtual rows of any row: one atomic per wave
+    // the most virtual rows of any row: one atomic per wave that brings more than there is already (a wave's every time
+    // is 16 thousand on one word for a million rows, 0.24 ms; so 0.13)
     int m = n;
     for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
-    if ((threadIdx.x & 63) == 0 && m > 1) atomicMax(most, m);
+    if ((threadIdx.x & 63) == 0 && m > 1 && m > *(volatile int *)most) atomicMax(most, m);
+}
+
+// What the host asks for after the row marks and their running counts, in one place: one copy instead of four.
+__global__ void row_totals_kernel(const int *__restrict__ over4, const int *__restrict__ lightPos, const int *__restrict__ heavyPos, int rows,
+                                  int *__restrict__ out)
+{
+    out[0] = over4[0];
+    out[1] = over4[1];
+    out[2] = lightPos[rows];
+    out[3] = heavyPos[rows];
 }
 
 __global__ __launch_bounds__(kBlock) void row_lists_kernel(const int *__restrict__ segPtr, const int *__restrict__ segIdx,
@@ -838,12 +849,13 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     MXL_TRY(hipGetLastError());
     MXL_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)isLight.p, lightPos.as<int>(), 0, r1, rocprim::plus<int>(), s));
     MXL_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)isHeavy.p, heavyPos.as<int>(), 0, r1, rocprim::plus<int>(), s));
-    int nLight = 0, nHeavy = 0, anyOver4 = 0, mostVrows = 0;
-    MXL_TRY(hipMemcpyAsync(&mostVrows, over4 + 1, 4, hipMemcpyDeviceToHost, s));
-    MXL_TRY(hipMemcpyAsync(&nLight, lightPos.as<int>() + rows, 4, hipMemcpyDeviceToHost, s));
-    MXL_TRY(hipMemcpyAsync(&nHeavy, heavyPos.as<int>() + rows, 4, hipMemcpyDeviceToHost, s));
-    MXL_TRY(hipMemcpyAsync(&anyOver4, over4, 4, hipMemcpyDeviceToHost, s));
+    int got[4] = {0, 0, 0, 0};
+    hipLaunchKernelGGL(row_totals_kernel, dim3(1), dim3(1), 0, s, (const int *)over4, (const int *)lightPos.p, (const int *)heavyPos.p, rows,
+                       flag.as<int>() + 16);
+    MXL_TRY(hipGetLastError());
+    MXL_TRY(hipMemcpyAsync(got, flag.as<int>() + 16, sizeof(got), hipMemcpyDeviceToHost, s));
     MXL_TRY(hipStreamSynchronize(s));
+    const int anyOver4 = got[0], mostVrows = got[1], nLight = got[2], nHeavy = got[3];
     D.nLight = nLight;
     D.nHeavy = nHeavy;
     D.mostVrows = std::max(mostVrows, nV > 0 ? 1 : 0);
