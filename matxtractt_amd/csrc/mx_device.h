@@ -13,7 +13,7 @@ namespace mx {
 //    request at once, in the order of that stream, and becomes anybody's when the scope ends, after the stream has
 //    been waited for;
 //  * inside IdleFrees, which waits for the device first, it is anybody's at once (plans that are destroyed: their
-//    streams are the callers');
+//    streams are the callers'); where that wait is refused the block goes back by hipFree;
 //  * elsewhere dev_free waits for the device, as hipFree does.
 // Idle blocks hold at most 1/128 of the device's memory, go back to the device after 64 calls in which nobody asked
 // for them, all of them when an allocation fails, and on mx_release_memory.

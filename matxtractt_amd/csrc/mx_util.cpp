@@ -155,6 +155,7 @@ Pool &pool()
 // What the calling thread has given back inside its current MemScope.
 struct ThreadScope {
     int depth = 0, idleFrees = 0;
+    bool waited = false;  // the last IdleFrees' wait for the device was granted and ended
     hipStream_t stream = nullptr;
     std::multimap<size_t, void *> freed;
 };
@@ -246,8 +247,9 @@ hipError_t dev_free(void *p)
         std::lock_guard<std::mutex> hold(P.mu);
         auto it = P.blocks.find(p);
         int dev = -1;
-        if (it == P.blocks.end() || hipGetDevice(&dev) != hipSuccess || dev != it->second.dev) {
-            // not made here, or on another device than the current one: the plain way
+        if (it == P.blocks.end() || hipGetDevice(&dev) != hipSuccess || dev != it->second.dev || (T.idleFrees > 0 && !T.waited)) {
+            // not made here, on another device than the current one, or still read by work that could not be waited for (a plan
+            // dropped while a stream is captured): the plain way
             if (it != P.blocks.end()) P.blocks.erase(it);
             b.bytes = 0;
         } else {
@@ -317,7 +319,7 @@ MemScope::~MemScope()
 
 IdleFrees::IdleFrees()
 {
-    (void)hipDeviceSynchronize();
+    t_scope.waited = hipDeviceSynchronize() == hipSuccess;
     ++t_scope.idleFrees;
 }
 IdleFrees::~IdleFrees() { --t_scope.idleFrees; }

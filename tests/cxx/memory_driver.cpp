@@ -1,0 +1,94 @@
+// The device memory that the library keeps between calls (mx_util.cpp), on a device that exists only here: the few HIP
+// functions it calls are defined below and count bytes.  Run with the name of one check; exit status 0 means it holds.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include "mx_device.h"
+#include "mx_internal.h"
+
+namespace {
+
+constexpr size_t GB = (size_t)1 << 30;
+
+struct Device {
+    std::mutex mu;
+    size_t total = 256 * GB, used = 0, most = 0;
+    std::map<void *, size_t> blocks;
+    uintptr_t next = 0x10000;
+    int frees = 0;
+    bool refuse = false;  // waits for the device
+} device;
+
+#define CHECK(x)                                                     \
+    do {                                                             \
+        if (!(x)) {                                                  \
+            std::printf("line %d: %s does not hold\n", __LINE__, #x); \
+            std::exit(1);                                            \
+        }                                                            \
+    } while (0)
+
+void *take(size_t bytes)
+{
+    void *p = nullptr;
+    CHECK(mx::dev_malloc(&p, bytes) == hipSuccess && p);
+    return p;
+}
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    if (device.used + n > device.total) return hipErrorOutOfMemory;
+    *p = (void *)device.next;
+    device.next += (n + 4095) / 4096 * 4096;
+    device.blocks[*p] = n;
+    device.used += n;
+    device.most = std::max(device.most, device.used);
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    auto it = device.blocks.find(p);
+    if (it == device.blocks.end()) std::abort();  // (freed twice)
+    device.used -= it->second;
+    device.blocks.erase(it);
+    ++device.frees;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
+hipError_t hipMemGetInfo(size_t *f, size_t *t) { return *f = device.total - device.used, *t = device.total, hipSuccess; }
+hipError_t hipDeviceSynchronize() { return device.refuse ? hipErrorStreamCaptureUnsupported : hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+}
+
+// Where the wait for the device is refused, no block becomes anybody's.
+static void wait_refused()
+{
+    void *p = take(GB);
+    device.refuse = true;
+    {
+        mx::IdleFrees idle;
+        CHECK(mx::dev_free(p) == hipSuccess);
+    }
+    device.refuse = false;
+    CHECK(device.frees == 1 && device.used == 0);
+    CHECK(take(GB) != p);
+}
+
+int main(int argc, char **argv)
+{
+    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}};
+    const auto it = checks.find(argc > 1 ? argv[1] : "");
+    if (it == checks.end()) return 2;
+    it->second();
+    return 0;
+}

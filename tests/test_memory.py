@@ -1,0 +1,28 @@
+"""The device memory that the library keeps between calls, on a device that exists only in the test (no GPU)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SRC = os.path.join(ROOT, "matxtractt_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    exe = str(tmp_path_factory.mktemp("memory") / "memory_driver")
+    cmd = ["g++", "-O1", "-g", "-std=c++17", "-pthread", "-Wall", "-Wextra", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROOT, "include"),
+           "-I" + SRC, "-I/opt/rocm/include", os.path.join(ROOT, "tests", "cxx", "memory_driver.cpp"), os.path.join(SRC, "mx_util.cpp"), "-o", exe]
+    b = subprocess.run(cmd, capture_output=True, text=True)
+    assert b.returncode == 0, b.stderr[-2000:]
+    return exe
+
+
+@pytest.mark.parametrize("check", ["wait_refused"])
+def test_memory_kept_between_calls(driver, check):
+    """tests/cxx/memory_driver.cpp, one check at a time."""
+    r = subprocess.run([driver, check], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
