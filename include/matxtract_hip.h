@@ -463,9 +463,9 @@ typedef struct mx_tau_estimate {
 } mx_tau_estimate;
 int mx_estimate_tau(const mx_csr *A, int levels, float *tau_c, float *tau_r, mx_tau_estimate *table, int cap, int *n_points);
 
-/* Making plans and partitions takes and gives back device memory by the hundred arrays; what was given back is kept
- * for the next call (at most 1/128 of a device's memory, and nothing for longer than 64 such calls).  This gives all
- * of it back to the device now.  No counterpart in the reference, which allocates and frees on every call
+/* Making and destroying plans and partitions takes and gives back device memory by the hundred arrays; what was given
+ * back is kept for the next call (at most 1/128 of a device's memory once a call has returned, and nothing for longer than 64 such
+ * calls).  This gives all of it back to the device now.  No counterpart in the reference, which allocates and frees on every call
  * (src/spmv_kernel/cdSpMV.cu:407-418). */
 void mx_release_memory(void);
 

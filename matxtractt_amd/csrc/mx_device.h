@@ -14,9 +14,9 @@ namespace mx {
 //    been waited for;
 //  * inside IdleFrees, which waits for the device first, it is anybody's at once (plans that are destroyed: their
 //    streams are the callers'); where that wait is refused the block goes back by hipFree;
-//  * elsewhere dev_free waits for the device, as hipFree does.
-// Idle blocks hold at most 1/128 of the device's memory, go back to the device after 64 calls in which nobody asked
-// for them, all of them when an allocation fails, and on mx_release_memory.
+//  * elsewhere dev_free waits for the device, as hipFree does (an IdleFrees of its own).
+// Idle blocks hold at most 1/128 of the device's memory whenever a scope or an IdleFrees ends, go back to the device after 64 of
+// those in which nobody asked for them, all of them when an allocation fails, and on mx_release_memory.
 hipError_t dev_malloc(void **out, size_t bytes);
 hipError_t dev_free(void *p);
 void release_idle_memory();

@@ -1368,6 +1368,7 @@ extern "C" int mx_slice_layout_device(const mx_csr *A, int nCU, mx_slice_layout_
     const size_t es = (size_t)mx::elem_size(A->dtype);
     int *dRowPtr = nullptr, *dCol = nullptr;
     void *dVal = nullptr;
+    mx::MemScope scope(nullptr);
     mx::DeviceSlices D;
     std::vector<int> segPtr, segIdx;
     rc = upload(&dRowPtr, A->rowPtr, (size_t)A->rows + 1);

@@ -71,6 +71,7 @@ static int cdspmv_any(mx_dtype dtype, const void *csrVal, const int *csrRowPtr, 
         return MX_OK;
     };
     rc = body();
+    mx::IdleFrees idle;
     free_csr(plan.csr);
     (void)mx::dev_free(dx);
     (void)mx::dev_free(dy);
@@ -153,6 +154,7 @@ static int du_any(mx_dtype dtype, const int *chunkPtr, const int *fragPtr, const
         return MX_OK;
     };
     rc = body();
+    mx::IdleFrees idle;
     free_tiles(T);
     (void)mx::dev_free(dx);
     (void)mx::dev_free(dy);
@@ -194,6 +196,7 @@ extern "C" int mx_probe_mfma_f64(const double *A, const double *B, double *D)
         return MX_OK;
     };
     rc = body();
+    mx::IdleFrees idle;
     (void)mx::dev_free(dA);
     (void)mx::dev_free(dB);
     (void)mx::dev_free(dD);
@@ -217,6 +220,7 @@ extern "C" int mx_probe_mfma_f16(const uint16_t *A, const uint16_t *B, float *D)
         return MX_OK;
     };
     rc = body();
+    mx::IdleFrees idle;
     (void)mx::dev_free(dA);
     (void)mx::dev_free(dB);
     (void)mx::dev_free(dD);

@@ -47,6 +47,7 @@ extern "C" int mx_tune_tau(const mx_csr *A, int levels, int flags, int warm, int
     int *dRowPtr = nullptr, *dColInd = nullptr;
     void *dVal = nullptr;
     auto release = [&]() {
+        mx::IdleFrees idle;
         (void)mx::dev_free(dx);
         (void)mx::dev_free(dy);
         (void)mx::dev_free(dRowPtr);
@@ -131,6 +132,7 @@ extern "C" int mx_estimate_tau(const mx_csr *A, int levels, float *tau_c, float 
     }
     int rc = need_device();
     if (rc) return rc;
+    mx::MemScope scope(nullptr);
     const size_t es = (size_t)mx::elem_size(A->dtype);
     int *dRowPtr = nullptr, *dColInd = nullptr;
     void *dVal = nullptr;

@@ -161,22 +161,28 @@ struct ThreadScope {
 };
 thread_local ThreadScope t_scope;
 
-// (with the lock held) blocks beyond the bound, and blocks nobody has asked for in a while, oldest first, of equally old ones the
-// largest: a call that passes the bound gives back a few large blocks, not dozens of small ones (plan and first product of
-// 45 million binary16 entries 27.0 -> 15.8 ms)
-void trim(Pool &P, int dev, std::vector<void *> &out, bool all)
+// Blocks beyond the bound, and blocks nobody has asked for in a while (`all`: every block), go back to the device, oldest first,
+// of equally old ones the largest: a call that passes the bound gives back a few large blocks, not dozens of small ones (plan
+// and first product of 45 million binary16 entries 27.0 -> 15.8 ms)
+void trim(Pool &P, bool all)
 {
-    auto &I = P.idle[dev];
-    for (;;) {
-        auto oldest = I.end();
-        for (auto it = I.begin(); it != I.end(); ++it)
-            if (oldest == I.end() || it->second.stamp <= oldest->second.stamp) oldest = it;  // (of equally old ones the largest)
-        if (oldest == I.end() || !(all || P.idleBytes[dev] > P.limit[dev] || oldest->second.stamp + kPoolCalls < P.calls)) return;
-        P.idleBytes[dev] -= oldest->first;
-        P.blocks.erase(oldest->second.p);
-        out.push_back(oldest->second.p);
-        I.erase(oldest);
-    }
+    for (int dev = 0; dev < kPoolDevices; ++dev)
+        for (;;) {
+            void *p;
+            {
+                std::lock_guard<std::mutex> hold(P.mu);
+                auto &I = P.idle[dev];
+                auto oldest = I.end();
+                for (auto it = I.begin(); it != I.end(); ++it)
+                    if (oldest == I.end() || it->second.stamp <= oldest->second.stamp) oldest = it;
+                if (oldest == I.end() || !(all || P.idleBytes[dev] > P.limit[dev] || oldest->second.stamp + kPoolCalls < P.calls)) break;
+                P.idleBytes[dev] -= oldest->first;
+                p = oldest->second.p;
+                P.blocks.erase(p);
+                I.erase(oldest);
+            }
+            (void)hipFree(p);
+        }
 }
 void put_idle(Pool &P, void *p, const Block &b)
 {
@@ -242,6 +248,10 @@ hipError_t dev_free(void *p)
     if (!p) return hipSuccess;
     Pool &P = pool();
     ThreadScope &T = t_scope;
+    if (T.depth == 0 && T.idleFrees == 0) {
+        IdleFrees one;
+        return dev_free(p);
+    }
     Block b{};
     {
         std::lock_guard<std::mutex> hold(P.mu);
@@ -261,27 +271,11 @@ hipError_t dev_free(void *p)
         }
     }
     if (b.bytes == 0) return hipFree(p);
-    if (T.depth > 0) {
-        T.freed.emplace(b.bytes, p);
-        return hipSuccess;
-    }
-    const hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> hold(P.mu);
-    put_idle(P, p, b);
+    T.freed.emplace(b.bytes, p);
     return hipSuccess;
 }
 
-void release_idle_memory()
-{
-    Pool &P = pool();
-    std::vector<void *> out;
-    {
-        std::lock_guard<std::mutex> hold(P.mu);
-        for (int d = 0; d < kPoolDevices; ++d) trim(P, d, out, true);
-    }
-    for (void *p : out) (void)hipFree(p);
-}
+void release_idle_memory() { trim(pool(), true); }
 
 MemScope::MemScope(hipStream_t s)
 {
@@ -293,28 +287,26 @@ MemScope::MemScope(hipStream_t s)
 MemScope::~MemScope()
 {
     ThreadScope &T = t_scope;
-    if (--T.depth > 0 || T.freed.empty()) return;
-    const bool idle = hipStreamSynchronize(T.stream) == hipSuccess;
+    if (--T.depth > 0) return;
+    const bool idle = T.freed.empty() || hipStreamSynchronize(T.stream) == hipSuccess;
     Pool &P = pool();
     std::vector<void *> out;
     {
         std::lock_guard<std::mutex> hold(P.mu);
         ++P.calls;
-        int dev = -1;
         for (auto &f : T.freed) {
             auto it = P.blocks.find(f.second);
             if (idle && it != P.blocks.end()) {
-                dev = it->second.dev;
                 put_idle(P, f.second, it->second);
             } else {
                 if (it != P.blocks.end()) P.blocks.erase(it);
                 out.push_back(f.second);
             }
         }
-        if (dev >= 0) trim(P, dev, out, false);
     }
     T.freed.clear();
     for (void *p : out) (void)hipFree(p);
+    trim(P, false);
 }
 
 IdleFrees::IdleFrees()
@@ -322,7 +314,16 @@ IdleFrees::IdleFrees()
     t_scope.waited = hipDeviceSynchronize() == hipSuccess;
     ++t_scope.idleFrees;
 }
-IdleFrees::~IdleFrees() { --t_scope.idleFrees; }
+IdleFrees::~IdleFrees()
+{
+    if (--t_scope.idleFrees > 0) return;
+    Pool &P = pool();
+    {
+        std::lock_guard<std::mutex> hold(P.mu);
+        ++P.calls;
+    }
+    trim(P, false);
+}
 
 }  // namespace mx
 

@@ -84,9 +84,45 @@ static void wait_refused()
     CHECK(take(GB) != p);
 }
 
+// What lies idle is at most 1/128 of the device after every way of giving memory back.
+static void bound()
+{
+    const size_t limit = device.total / 128;
+    std::vector<void *> plan;
+    for (int k = 0; k < 20; ++k) plan.push_back(take(GB));
+    {
+        mx::IdleFrees idle;  // a plan is destroyed
+        for (void *p : plan) CHECK(mx::dev_free(p) == hipSuccess);
+    }
+    CHECK(device.used > 0 && device.used <= limit);
+    for (int k = 1; k <= 40; ++k) {  // calls without a scope, each on a larger matrix
+        void *p = take((size_t)k * 300 << 20);
+        CHECK(mx::dev_free(p) == hipSuccess);
+        CHECK(device.used <= limit);
+    }
+    for (int k = 0; k < 6; ++k) plan[k] = take(GB);
+    {
+        mx::MemScope scope(nullptr);
+        for (int k = 0; k < 6; ++k) CHECK(mx::dev_free(plan[k]) == hipSuccess);
+    }
+    CHECK(device.used <= limit);
+    mx::release_idle_memory();
+    CHECK(device.used == 0);
+}
+
+// A block that nobody asks for is given back after 64 calls, also where those calls give nothing back themselves.
+static void age()
+{
+    void *p = take(GB);
+    CHECK(mx::dev_free(p) == hipSuccess);
+    CHECK(device.used >= GB);
+    for (int k = 0; k < 70; ++k) mx::MemScope scope(nullptr);
+    CHECK(device.used == 0);
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}};
+    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}, {"bound", bound}, {"age", age}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();

@@ -160,6 +160,41 @@ def test_memory_kept_between_calls_is_bounded_and_given_back(mx):
     assert free0 <= free1 <= free0 + total // 128 + (64 << 20)
 
 
+def test_memory_of_destroyed_plans_is_bounded(mx):
+    """Plans of more than 1/128 of the device's memory, alive side by side and then destroyed: what the library keeps of
+    them stays within that bound, and release_memory() gives back what it kept."""
+    import torch
+    rows, offs = 6000000, torch.arange(-4, 4, device="cuda", dtype=torch.int32) * 1000
+    r = torch.arange(rows, device="cuda", dtype=torch.int32)
+    c = r[:, None] + offs[None, :]
+    ok = (c >= 0) & (c < rows)
+    ptr = torch.zeros(rows + 1, dtype=torch.int32, device="cuda")
+    ptr[1:] = torch.cumsum(ok.sum(1), 0)
+    c = c[ok]
+    v = torch.rand(c.numel(), dtype=torch.float64, device="cuda")
+    del ok, r
+    slack = 64 << 20  # (of the runtime's own)
+
+    def free():
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        return torch.cuda.mem_get_info()[0]
+
+    mx.Plan.from_device(ptr, c, v, rows, 0.0, 0.0).close()  # (code objects and the like are there from here on)
+    mx.release_memory()
+    total, before = torch.cuda.mem_get_info()[1], free()
+    plans = []
+    while before - free() < total // 128 + (1 << 30):
+        plans.append(mx.Plan.from_device(ptr, c, v, rows, 0.0, 0.0))
+        assert len(plans) < 32
+    for p in plans:
+        p.close()
+    kept = before - free()
+    assert 256 << 20 < kept <= total // 128 + slack, kept
+    mx.release_memory()
+    assert before - free() <= slack
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float16])
 @pytest.mark.parametrize("lens", [
     [511, 512, 513, 1, 0, 1535, 1536, 1537, 2, 2047, 2048, 2049, 3],  # a workgroup's share of short rows, the first long class
