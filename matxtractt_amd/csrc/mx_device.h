@@ -16,7 +16,8 @@ namespace mx {
 //    streams are the callers'); where that wait is refused the block goes back by hipFree;
 //  * elsewhere dev_free waits for the device, as hipFree does (an IdleFrees of its own).
 // Idle blocks hold at most 1/128 of the device's memory whenever a scope or an IdleFrees ends, go back to the device after 64 of
-// those in which nobody asked for them, all of them when an allocation fails, and on mx_release_memory.
+// those in which nobody asked for them, all of them when an allocation fails, and on mx_release_memory.  What a thread has
+// given back inside a scope holds at most 1/16, and goes back to the device as well when an allocation of its own fails.
 hipError_t dev_malloc(void **out, size_t bytes);
 hipError_t dev_free(void *p);
 void release_idle_memory();

@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <unordered_map>
@@ -138,6 +139,7 @@ struct Idle {
 constexpr int kPoolDevices = 64;
 constexpr uint64_t kPoolCalls = 64;   // a block nobody has asked for in so many calls goes back to the device
 constexpr size_t kPoolShare = 128;    // idle blocks hold at most this fraction of a device's memory (2.25 GB of 288)
+constexpr size_t kScopeShare = 16;    // what a thread has given back inside its scope, at most (18 GB)
 
 struct Pool {
     std::mutex mu;
@@ -158,6 +160,7 @@ struct ThreadScope {
     bool waited = false;  // the last IdleFrees' wait for the device was granted and ended
     hipStream_t stream = nullptr;
     std::multimap<size_t, void *> freed;
+    size_t freedBytes = 0;
 };
 thread_local ThreadScope t_scope;
 
@@ -189,6 +192,23 @@ void put_idle(Pool &P, void *p, const Block &b)
     P.idle[b.dev].emplace(b.bytes, Idle{p, P.calls});
     P.idleBytes[b.dev] += b.bytes;
 }
+// What the thread has given back inside its scope goes back to the device, the largest block first, until at most `keep` bytes
+// are left -- after a wait for the scope's stream; nothing does where that fails.
+void shrink_scope(Pool &P, ThreadScope &T, size_t keep)
+{
+    if (T.freedBytes <= keep || hipStreamSynchronize(T.stream) != hipSuccess) return;
+    while (T.freedBytes > keep) {
+        const auto it = std::prev(T.freed.end());
+        void *p = it->second;
+        T.freedBytes -= it->first;
+        T.freed.erase(it);
+        {
+            std::lock_guard<std::mutex> hold(P.mu);
+            P.blocks.erase(p);
+        }
+        (void)hipFree(p);
+    }
+}
 bool fits(size_t have, size_t need) { return have <= need + need / 8 + 65536; }
 
 }  // namespace
@@ -207,6 +227,7 @@ hipError_t dev_malloc(void **out, size_t bytes)
         auto it = T.freed.lower_bound(need);
         if (it != T.freed.end() && fits(it->first, need)) {
             *out = it->second;
+            T.freedBytes -= it->first;
             T.freed.erase(it);
             return hipSuccess;
         }
@@ -223,12 +244,16 @@ hipError_t dev_malloc(void **out, size_t bytes)
     }
     void *p = nullptr;
     e = hipMalloc(&p, need);
-    if (e == hipErrorOutOfMemory) {  // what lies idle here may be what is missing
+    if (e == hipErrorOutOfMemory) {  // what lies idle here, or waits in this scope, may be what is missing
         (void)hipGetLastError();
+        shrink_scope(P, T, 0);
         release_idle_memory();
         e = hipMalloc(&p, need);
     }
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // (a caller that goes on without the memory must not meet the error at its next launch)
+        return e;
+    }
     std::lock_guard<std::mutex> hold(P.mu);
     if (P.limit[dev] == 0) {
         size_t freeB = 0, total = 0;
@@ -253,6 +278,7 @@ hipError_t dev_free(void *p)
         return dev_free(p);
     }
     Block b{};
+    size_t scopeLimit = 0;
     {
         std::lock_guard<std::mutex> hold(P.mu);
         auto it = P.blocks.find(p);
@@ -264,6 +290,7 @@ hipError_t dev_free(void *p)
             b.bytes = 0;
         } else {
             b = it->second;
+            scopeLimit = P.limit[b.dev] * (kPoolShare / kScopeShare);
             if (T.idleFrees > 0) {
                 put_idle(P, p, b);
                 return hipSuccess;
@@ -272,6 +299,8 @@ hipError_t dev_free(void *p)
     }
     if (b.bytes == 0) return hipFree(p);
     T.freed.emplace(b.bytes, p);
+    T.freedBytes += b.bytes;
+    shrink_scope(P, T, scopeLimit);
     return hipSuccess;
 }
 
@@ -305,6 +334,7 @@ MemScope::~MemScope()
         }
     }
     T.freed.clear();
+    T.freedBytes = 0;
     for (void *p : out) (void)hipFree(p);
     trim(P, false);
 }

@@ -22,6 +22,7 @@ struct Device {
     uintptr_t next = 0x10000;
     int frees = 0;
     bool refuse = false;  // waits for the device
+    hipError_t last = hipSuccess;
 } device;
 
 #define CHECK(x)                                                     \
@@ -45,7 +46,7 @@ extern "C" {
 hipError_t hipMalloc(void **p, size_t n)
 {
     std::lock_guard<std::mutex> hold(device.mu);
-    if (device.used + n > device.total) return hipErrorOutOfMemory;
+    if (device.used + n > device.total) return device.last = hipErrorOutOfMemory;
     *p = (void *)device.next;
     device.next += (n + 4095) / 4096 * 4096;
     device.blocks[*p] = n;
@@ -67,7 +68,12 @@ hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) { return *f = device.total - device.used, *t = device.total, hipSuccess; }
 hipError_t hipDeviceSynchronize() { return device.refuse ? hipErrorStreamCaptureUnsupported : hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError()
+{
+    const hipError_t e = device.last;
+    device.last = hipSuccess;
+    return e;
+}
 }
 
 // Where the wait for the device is refused, no block becomes anybody's.
@@ -120,9 +126,41 @@ static void age()
     CHECK(device.used == 0);
 }
 
+// A request that the device has room for once the scope's own blocks are given back is granted, and what a scope keeps for
+// itself stays within its share.
+static void scope_full()
+{
+    device.total = 10 * GB;
+    {
+        mx::MemScope scope(nullptr);
+        std::vector<void *> part;
+        for (int k = 0; k < 6; ++k) part.push_back(take(GB));
+        for (void *p : part) CHECK(mx::dev_free(p) == hipSuccess);
+        void *large = take(9 * GB);
+        CHECK(mx::dev_free(large) == hipSuccess);
+        void *none = nullptr;
+        CHECK(mx::dev_malloc(&none, 11 * GB) == hipErrorOutOfMemory && !none);
+        CHECK(hipGetLastError() == hipSuccess);
+    }
+    CHECK(device.used <= device.total / 128);
+}
+static void scope_share()
+{
+    const size_t share = device.total / 16;
+    {
+        mx::MemScope scope(nullptr);
+        for (int k = 1; k <= 60; ++k) {
+            void *p = take((size_t)k * 600 << 20);
+            CHECK(mx::dev_free(p) == hipSuccess);
+            CHECK(device.used <= share);
+        }
+    }
+    CHECK(device.used <= device.total / 128);
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}, {"bound", bound}, {"age", age}};
+    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}, {"bound", bound}, {"age", age}, {"scope_full", scope_full}, {"scope_share", scope_share}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();
