@@ -312,17 +312,20 @@ bool mxp::may_look_for_form(int flags)
 int mxp::try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took)
 {
     *took = false;
-    const int rc = mx::build_offsets_device(plan->dtype, plan->rows, plan->cols, nnz, rowPtr_dev, colInd_dev, val_dev, plan->offsets, nullptr);
-    if (rc) return rc;
-    plan->csr_variant = 3;
-    if (plan->offsets.nChunks == 0) {
-        const int rcw = mx::build_windows_device(plan->dtype, plan->rows, plan->cols, nnz, rowPtr_dev, colInd_dev, val_dev, plan->windows, nullptr);
-        plan->csr_variant = 4;
-        if (rcw || plan->windows.nChunks == 0) {
-            plan->csr_variant = 0;
-            return rcw;
-        }
+    plan->csr_variant = 0;
+    // (a form that there is no memory for is not taken: the others need less beside the matrix, and what is looked for here is not needed at all)
+    int rc = mx::build_offsets_device(plan->dtype, plan->rows, plan->cols, nnz, rowPtr_dev, colInd_dev, val_dev, plan->offsets, nullptr);
+    if (rc == MX_ERR_ALLOC) mx::free_offsets(plan->offsets);
+    else if (rc) return rc;
+    int variant = plan->offsets.nChunks > 0 ? 3 : 0;
+    if (!variant) {
+        rc = mx::build_windows_device(plan->dtype, plan->rows, plan->cols, nnz, rowPtr_dev, colInd_dev, val_dev, plan->windows, nullptr);
+        if (rc == MX_ERR_ALLOC) mx::free_windows(plan->windows);
+        else if (rc) return rc;
+        if (plan->windows.nChunks > 0) variant = 4;
     }
+    if (!variant) return MX_OK;
+    plan->csr_variant = variant;
     plan->csr_nnz = nnz;
     decide_keep(plan, flags);
     *took = true;
@@ -355,10 +358,9 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
         int *rp = nullptr, *ci = nullptr;
         void *va = nullptr;
         bool took = false;
-        int e = upload(&rp, rowPtr, (size_t)rows + 1);
-        if (!e) e = upload(&ci, col, (size_t)nnz);
-        if (!e) e = upload_bytes(&va, val, (size_t)nnz * es);
-        if (!e) e = try_forms(plan, nnz, rp, ci, va, flags, &took);
+        // (nor is a matrix that does not get there a failure: what the plan needs of it goes up below, in its form)
+        const bool up = !upload(&rp, rowPtr, (size_t)rows + 1) && !upload(&ci, col, (size_t)nnz) && !upload_bytes(&va, val, (size_t)nnz * es);
+        const int e = up ? try_forms(plan, nnz, rp, ci, va, flags, &took) : MX_OK;
         (void)mx::dev_free(rp);
         (void)mx::dev_free(ci);
         (void)mx::dev_free(va);

@@ -1,0 +1,79 @@
+// How a plan looks for the forms of its CSR part that are made on the device (mxp::try_forms), with the two makers
+// replaced by what the check says.  No GPU call.  Run with the name of one check; exit status 0 means it holds.
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include <string>
+
+#include "mx_plan_parts.h"
+
+#define CHECK(x)                                                     \
+    do {                                                             \
+        if (!(x)) {                                                  \
+            std::printf("line %d: %s does not hold\n", __LINE__, #x); \
+            std::exit(1);                                            \
+        }                                                            \
+    } while (0)
+
+namespace {
+int offsets_rc = MX_OK, windows_rc = MX_OK, offsets_asked = 0, windows_asked = 0;
+bool offsets_suit = false, windows_suit = false;
+}  // namespace
+
+namespace mx {
+int build_offsets_device(mx_dtype, int, int, int, const int *, const int *, const void *, DeviceOffsets &D, hipStream_t)
+{
+    ++offsets_asked;
+    D = DeviceOffsets();
+    if (offsets_suit) D.nChunks = 5;
+    return offsets_rc;
+}
+int build_windows_device(mx_dtype, int, int, int, const int *, const int *, const void *, DeviceWindows &D, hipStream_t)
+{
+    ++windows_asked;
+    D = DeviceWindows();
+    if (windows_suit) D.nChunks = 7;
+    return windows_rc;
+}
+hipError_t launch_offsets(mx_dtype, const DeviceOffsets &, const void *, void *, int, hipStream_t) { return hipErrorUnknown; }
+hipError_t launch_windows(mx_dtype, const DeviceWindows &, const void *, void *, int, hipStream_t) { return hipErrorUnknown; }
+}  // namespace mx
+
+// No memory for a form is a reason to go on without it (the forms behind it need less beside the matrix), any other
+// failure is the plan's.
+static void no_memory()
+{
+    const struct {
+        int orc, wrc;
+        bool osuit, wsuit;
+        int rc, variant;
+    } cases[] = {
+        {MX_OK, MX_OK, true, true, MX_OK, 3},
+        {MX_OK, MX_OK, false, true, MX_OK, 4},
+        {MX_OK, MX_OK, false, false, MX_OK, 0},
+        {MX_ERR_ALLOC, MX_OK, true, true, MX_OK, 4},
+        {MX_ERR_ALLOC, MX_OK, true, false, MX_OK, 0},
+        {MX_OK, MX_ERR_ALLOC, false, true, MX_OK, 0},
+        {MX_ERR_ALLOC, MX_ERR_ALLOC, true, true, MX_OK, 0},
+        {MX_ERR_DEVICE, MX_OK, true, true, MX_ERR_DEVICE, 0},
+        {MX_OK, MX_ERR_DEVICE, false, true, MX_ERR_DEVICE, 0},
+    };
+    for (const auto &c : cases) {
+        offsets_rc = c.orc, windows_rc = c.wrc, offsets_suit = c.osuit, windows_suit = c.wsuit;
+        mx_plan plan;
+        plan.rows = plan.cols = 100000;
+        bool took = false;
+        CHECK(mxp::try_forms(&plan, 1000000, nullptr, nullptr, nullptr, MX_PLAN_DEFAULT, &took) == c.rc);
+        CHECK(plan.csr_variant == c.variant && took == (c.rc == MX_OK && c.variant != 0));
+        if (c.rc == MX_OK) CHECK((plan.offsets.nChunks > 0) == (c.variant == 3) && (plan.windows.nChunks > 0) == (c.variant == 4));
+    }
+}
+
+int main(int argc, char **argv)
+{
+    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}};
+    const auto it = checks.find(argc > 1 ? argv[1] : "");
+    if (it == checks.end()) return 2;
+    it->second();
+    return 0;
+}
