@@ -422,7 +422,7 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     D = DeviceWindows();
     const bool f64 = dtype == MX_F64;
     const int es = elem_size(dtype), epv = 16 / es;
-    if (rows < kWindowRowsLeast || cols < 64 || (long long)nnz < (long long)rows * kWindowMeanLeast || nnz > 1500000000 ||
+    if (rows < kWindowRowsLeast || cols < 64 || !window_mean_ok(f64, rows, nnz) || nnz > 1500000000 ||
         (f64 && nnz < kWindowEntriesLeast))
         return MX_OK;
     const int nChunks = (rows + 63) / 64, waves = kWindowWaves, nWG = (nChunks + waves - 1) / waves;
@@ -461,7 +461,10 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
         MXW_TRY(hipMemcpyAsync(h, totals.p, sizeof(h), hipMemcpyDeviceToHost, s));
         MXW_TRY(hipStreamSynchronize(s));
         const double stored = (double)h[1] * window_unit_bytes(f64) + (double)h[2] * 64 * (4 + es);
-        if (h[0] || h[1] <= 0 || h[4] > kWindowFarMost * (double)nnz || stored > kWindowFill * (double)nnz * (2 + es) + 65536) return fail(MX_OK);
+        int dev = 0, nCU = 0;
+        MXW_TRY(hipGetDevice(&dev));
+        MXW_TRY(hipDeviceGetAttribute(&nCU, hipDeviceAttributeMultiprocessorCount, dev));
+        if (h[0] || h[1] <= 0 || h[4] > kWindowFarMost * (double)nnz || !window_form_pays(f64, nnz, stored, nWG, nCU)) return fail(MX_OK);
         if (f64 && nnz >= 65536 && mx::opt().csr_dict != 0) {
             // few distinct binary64 values: slices with a byte a value move a third of what this form would
             void *codes = nullptr;
