@@ -262,27 +262,29 @@ constexpr int kWindowRowsLeast = 32768;       // fewest rows of a matrix that ta
 constexpr int kWindowEntriesLeast = 600000;   // binary64: fewest entries (0.33 million: 4.0 us, row tiles 3.8; 0.9 million: 4.2, 4.7)
 constexpr double kWindowFill = 1.5;           // most bytes stored per byte of the entries
 // Fewest entries a row on average: a wave waits for its window whatever it has to add, and with two units a row that is most of its
-// time (binary64, 6 a row: 260 thousand rows 7.1 us, row tiles 5.5; 1.5 million 42, slices 29.5; binary16, 7 a row: 3.2 million
-// rows 37, slices 29).  In binary16 it still beats row tiles and slices while there are few rows (130 thousand of 6: 2.9, 4.0; 260 thousand 3.5, 4.6; 600
-// thousand 7.3, 7.9 back to back and 9.0, 8.4 in a rotation of three).
-constexpr int kWindowMean = 8, kWindowMeanFewRows = 4, kWindowFewRows = 300000;
+// time (binary64, 6 a row: 260 thousand rows 7.1 us, row tiles 5.5; 1.5 million 42, slices 29.5).  In binary16 a row has fewer bytes:
+// over a million rows more of them are needed (2.2 million of 11.5: 34.5, slices 28.3; 3.2 million of 7: 37, 29; 1.5 million of 16: 21.4, 24.5), and
+// few rows beat row tiles and slices with less (130 thousand of 6: 2.9, 4.0; 260 thousand 3.5, 4.6; 600 thousand 7.3, 7.9 back to back and 9.0, 8.4
+// in a rotation of three).
+constexpr int kWindowMean = 8, kWindowMeanFewRows = 4, kWindowFewRows = 300000, kWindowMeanManyRows = 14, kWindowManyRows = 1000000;
 inline bool window_mean_ok(bool f64, int rows, int nnz)
 {
-    return (long long)nnz >= (long long)rows * (f64 || rows > kWindowFewRows ? kWindowMean : kWindowMeanFewRows);
+    const int least = f64 ? kWindowMean : rows <= kWindowFewRows ? kWindowMeanFewRows : rows <= kWindowManyRows ? kWindowMean : kWindowMeanManyRows;
+    return (long long)nnz >= (long long)rows * least;
 }
 // Whether a matrix laid out in `stored` bytes by nWG workgroups is better off in this form than in slices (or row tiles).  The
-// one launch saves about 4 us, some 20 MB's worth; padding beyond that (rows of uneven length) costs more than it
+// one launch saves about 4 us, some 18 MB's worth; padding beyond that (rows of uneven length) costs more than it
 // (binary64, 600 thousand rows of 28 to 52 entries, 314 MB instead of 238: 55 us, slices 48; of 34 to 46, 290 MB: 48.6, 48.1).
 // Slices spread any matrix over all CUs, a window's rows stay with one, which takes in 50 to 80 bytes a nanosecond
 // (33 thousand rows of 300, 65 workgroups of 1.5 MB, binary64: 20 to 44 us, slices 20; binary16, 0.6 MB: 11 to 14.8, one-launch slices 11.2 to 12;
 // 66 thousand rows of 300, 129 workgroups: binary16, 0.6 MB, 13.8, slices 18.5, binary64, 1.5 MB, 36.5, 34.6).  Among the smallest
 // binary64 matrices row tiles are close (33 thousand rows of 40: 5.1 at a fill of 1.06, 5.9 at 1.36, row tiles 5.5).
 // Over 296 bands of 33 thousand to 3.2 million rows and 4 to 300 entries a row that pass the limits above, the form was more than 3 % slower than the one
-// before it 80 times, at worst 2.2 times as slow; none of the 187 that this lets through was.
+// before it 80 times, at worst 2.2 times as slow; none of the 184 that this lets through was.
 inline bool window_form_pays(bool f64, int nnz, double stored, int nWG, int nCU)
 {
     const double entries = (double)nnz * (f64 ? 10 : 4);
-    if (stored > kWindowFill * entries + 65536 || stored > 1.1 * entries + 20e6) return false;
+    if (stored > kWindowFill * entries + 65536 || stored > 1.1 * entries + 18e6) return false;
     if (f64 && nnz < 1300000 && stored > 1.3 * entries) return false;
     const double most = f64 ? 0.8e6 : nWG * 8 < nCU * 3 ? 0.3e6 : 0.7e6;  // of a workgroup, where there are fewer than CUs
     return nWG * 16 >= nCU * 15 || stored <= most * nWG;
