@@ -296,6 +296,11 @@ constexpr int kWindowLongest = 1024;          // most entries of a row
 constexpr double kWindowShare = 0.6;          // most bytes of a window per byte of its workgroup's entries
 constexpr int kWindowBytesMost = 80 << 10;    // of a window: two workgroups share the LDS of a CU
 constexpr int window_unit_bytes(bool f64) { return 64 * kWindowUnit * (f64 ? 10 : 4); }
+// What a product may touch for its units to be read with plain loads.  Plain / streaming loads, us, back to back | three plans in
+// turn: binary16, 51 MB 11.3 / 12.0 | 11.2 / 12.6; 76 MB 14.2 / 14.2 | 14.2 / 14.9; 99 MB 16.7 / 16.2 | 18.6 / 17.2; 108 MB 18.9 / 21.7 | 23.1 /
+// 22.7; 126 MB 19.5 / 19.1 | 23.3 / 20.3; binary64, 79 MB 14.7 / 15.7 | 14.8 / 16.7; 100 MB 16.5 / 17.6 | 18.4 / 18.6; 120 MB 18.8 / 19.2 | 23.3 / 20.0;
+// 132 MB 20.5 / 21.2 | 25.1 / 22.6.
+constexpr long long kWindowKeepBytes = 112LL << 20;
 void free_windows(DeviceWindows &D);
 // As build_offsets_device and launch_offsets.
 __attribute__((weak)) int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev,

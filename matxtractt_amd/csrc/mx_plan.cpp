@@ -263,7 +263,7 @@ void mxp::decide_keep(mx_plan *plan, int flags)
         bool &keep = plan->csr_variant == 3 ? plan->offsets.keep : plan->windows.keep;
         if ((flags & MX_PLAN_STREAM) || env == 0) keep = false;
         else if ((flags & MX_PLAN_KEEP) || env == 1) keep = true;
-        else keep = touched_bytes(plan) <= (double)mx::kOffsetsKeepBytes;
+        else keep = touched_bytes(plan) <= (double)(plan->csr_variant == 3 ? mx::kOffsetsKeepBytes : mx::kWindowKeepBytes);
         return;
     }
     if (plan->csr_variant == 0) return;

@@ -99,9 +99,30 @@ static void window_rule()
     }
 }
 
+// Plain or streaming loads, by what the form itself was measured at.
+static void keep_rule()
+{
+    mx_plan plan;
+    plan.dtype = MX_F16;
+    plan.rows = plan.cols = 1000000;
+    const struct {
+        int variant;
+        double mb;
+        bool keep;
+    } cases[] = {{3, 100, true}, {3, 130, true}, {3, 140, false}, {4, 100, true}, {4, 115, true}, {4, 126, false}};
+    for (const auto &c : cases) {
+        plan.csr_variant = c.variant;
+        const double rest = c.mb * 1e6 - 4e6;  // (x and y)
+        plan.offsets.units = (int)(rest / (64 * 16)), plan.offsets.unitBytes = 16;
+        plan.windows.units = (int)(rest / 1024), plan.windows.unitBytes = 1024;
+        mxp::decide_keep(&plan, MX_PLAN_DEFAULT);
+        CHECK((c.variant == 3 ? plan.offsets.keep : plan.windows.keep) == c.keep);
+    }
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}};
+    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();
