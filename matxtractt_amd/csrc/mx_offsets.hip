@@ -490,13 +490,10 @@ static hipError_t launch_offsets_t(const DeviceOffsets &D, const void *x, void *
 hipError_t launch_offsets(mx_dtype dtype, const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s)
 {
     if (D.nChunks <= 0) return hipSuccess;
-    // Four waves a chunk: a wave's trips to memory are fewer and more of them are in flight on a matrix of few chunks
-    // (one / two / four waves, us, binary64: 22 thousand rows 6.3 / 4.2 / 3.2; 717 thousand 33.1 / 31.2 / 28.6; 1.2 million
-    // 52.9 / 51.3 / 48.3).  With one byte per binary64 value the kernel is bound by what a wave computes and the sum of
-    // the parts costs more than it gives from about two thousand chunks on (290 thousand rows 6.5 / 6.1 / 6.4, 717
-    // thousand 10.9 / 10.5 / 11.7, a million 13.1 / 13.7 / 14.8).
-    if (dtype == MX_F16) return launch_offsets_t<_Float16, 4>(D, x, y, accumulate, s);
-    return D.nDict > 0 && D.nChunks >= 2048 ? launch_offsets_t<double, 2>(D, x, y, accumulate, s) : launch_offsets_t<double, 4>(D, x, y, accumulate, s);
+    const int waves = offsets_waves(dtype == MX_F64, D.nDict > 0, D.nOffs, D.nChunks);
+    if (dtype == MX_F16) return waves == 1 ? launch_offsets_t<_Float16, 1>(D, x, y, accumulate, s) : launch_offsets_t<_Float16, 4>(D, x, y, accumulate, s);
+    if (waves == 1) return launch_offsets_t<double, 1>(D, x, y, accumulate, s);
+    return waves == 2 ? launch_offsets_t<double, 2>(D, x, y, accumulate, s) : launch_offsets_t<double, 4>(D, x, y, accumulate, s);
 }
 
 }  // namespace mx

@@ -120,9 +120,19 @@ static void keep_rule()
     }
 }
 
+// Waves that share a chunk of the offset form: one where its list is one round.
+static void offset_waves()
+{
+    CHECK(mx::offsets_waves(true, false, 11719, 11719) == 1 && mx::offsets_waves(true, false, 8 * 11719, 11719) == 1);
+    CHECK(mx::offsets_waves(true, false, 9 * 11719, 11719) == 4 && mx::offsets_waves(true, true, 12 * 11719, 11719) == 2);
+    CHECK(mx::offsets_waves(true, true, 8 * 11719, 11719) == 1 && mx::offsets_waves(true, true, 12 * 300, 300) == 4);
+    CHECK(mx::offsets_waves(false, false, 8 * 5860, 5860) == 1 && mx::offsets_waves(false, true, 28 * 5860, 5860) == 4);
+    CHECK(mx::offsets_waves(true, false, 8ll << 28, 1 << 28) == 1);
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}};
+    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();

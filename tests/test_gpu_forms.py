@@ -33,7 +33,10 @@ def _diagonals(mx, rng, rows, cols, offs, dtype, few, holes=0.0):
     (30011, 30011, list(range(-32, 32))),                # as many offsets as a chunk may have
     (30011, 30011, list(range(-32, 33))),                # one more: another form takes the matrix
     (40000, 40000, sorted({dx + 20 * (dy + 50 * dz) for dx in (-1, 0, 1) for dy in (-1, 0, 1) for dz in (-1, 0, 1)})),
-    (270000, 270000, [-700, -3, -2, 0, 2, 3, 700]),      # more than 2048 chunks of binary64 rows
+    (270000, 270000, [-700, -3, -2, 0, 2, 3, 700]),      # more than 2048 chunks of binary64 rows, a wave each
+    (270000, 270000, list(range(-6, 6))),                # ... a list of more than one round: two or four waves a chunk
+    (5001, 5001, list(range(0, 16, 2))),                 # as long a list as one wave takes, a row beyond whole chunks
+    (5001, 5001, list(range(0, 18, 2))),                 # one more
 ])
 def test_offset_form(mx, ora, dtype, few, rows, cols, offs):
     """Matrices whose rows repeat a pattern of column offsets: the product from both routes equals the oracle's
