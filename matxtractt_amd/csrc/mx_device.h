@@ -275,10 +275,10 @@ constexpr int kWindowEntriesLeast = 600000;   // binary64: fewest entries (0.33 
 constexpr double kWindowFill = 1.5;           // most bytes stored per byte of the entries
 // Fewest entries a row on average: a wave waits for its window whatever it has to add, and with two units a row that is most of its
 // time (binary64, 6 a row: 260 thousand rows 7.1 us, row tiles 5.5; 1.5 million 42, slices 29.5).  In binary16 a row has fewer bytes:
-// over a million rows more of them are needed (2.2 million of 11.5: 34.5, slices 28.3; 3.2 million of 7: 37, 29; 1.5 million of 16: 21.4, 24.5), and
+// over a million rows more of them are needed (2.2 million of 11.5: 34.5, slices 28.3; 3.2 million of 7: 37, 29; 1.5 million of 14: 19.5, 22.8), and
 // few rows beat row tiles and slices with less (130 thousand of 6: 2.9, 4.0; 260 thousand 3.5, 4.6; 600 thousand 7.3, 7.9 back to back and 9.0, 8.4
 // in a rotation of three).
-constexpr int kWindowMean = 8, kWindowMeanFewRows = 4, kWindowFewRows = 300000, kWindowMeanManyRows = 14, kWindowManyRows = 1000000;
+constexpr int kWindowMean = 8, kWindowMeanFewRows = 4, kWindowFewRows = 300000, kWindowMeanManyRows = 13, kWindowManyRows = 1000000;
 inline bool window_mean_ok(bool f64, int rows, int nnz)
 {
     const int least = f64 ? kWindowMean : rows <= kWindowFewRows ? kWindowMeanFewRows : rows <= kWindowManyRows ? kWindowMean : kWindowMeanManyRows;
@@ -311,8 +311,10 @@ constexpr int window_unit_bytes(bool f64) { return 64 * kWindowUnit * (f64 ? 10 
 // What a product may touch for its units to be read with plain loads.  Plain / streaming loads, us, back to back | three plans in
 // turn: binary16, 51 MB 11.3 / 12.0 | 11.2 / 12.6; 76 MB 14.2 / 14.2 | 14.2 / 14.9; 99 MB 16.7 / 16.2 | 18.6 / 17.2; 108 MB 18.9 / 21.7 | 23.1 /
 // 22.7; 126 MB 19.5 / 19.1 | 23.3 / 20.3; binary64, 79 MB 14.7 / 15.7 | 14.8 / 16.7; 100 MB 16.5 / 17.6 | 18.4 / 18.6; 120 MB 18.8 / 19.2 | 23.3 / 20.0;
-// 132 MB 20.5 / 21.2 | 25.1 / 22.6.
-constexpr long long kWindowKeepBytes = 112LL << 20;
+// 132 MB 20.5 / 21.2 | 25.1 / 22.6.  Beyond 110 MB that is a trade, and against the slices these matrices had before plain loads come out
+// ahead (127 MB, binary16: 1.5 million rows of 16, plain 22.9 | 29.7, streaming 26.8 | 27.2, slices 25.1 | 29.6; 600 thousand of 40, 20.3 | 25.9,
+// 23.4 | 24.3, 22.2 | 25.4).
+constexpr long long kWindowKeepBytes = 128LL << 20;
 void free_windows(DeviceWindows &D);
 // As build_offsets_device and launch_offsets.
 __attribute__((weak)) int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev,

@@ -82,7 +82,7 @@ static void window_rule()
         {true, 66000, 2640000, 26.5, true},    {true, 33000, 3300000, 32.5, true},   {true, 130000, 39000000, 385.9, true},
         {true, 260000, 26000000, 299.9, true}, {true, 600000, 9600000, 123.6, true}, {true, 130000, 2080000, 30.0, true},
         {false, 250007, 10000280, 42.0, true}, {false, 130000, 780000, 4.3, true},   {false, 66000, 19800000, 77.4, true},
-        {false, 600000, 23844517, 115.4, true}, {false, 1000000, 8000000, 33.0, true}, {false, 1500000, 23940000, 97.4, true},
+        {false, 600000, 23844517, 115.4, true}, {false, 1000000, 8000000, 33.0, true}, {false, 1500000, 23940000, 97.4, true}, {false, 1500000, 20990000, 96.0, true},
         // (slower)
         {true, 33000, 9228706, 136.4, false},   {true, 33000, 9253352, 95.6, false},   {true, 66000, 18793119, 193.7, false},
         {true, 600000, 23840358, 314.4, false}, {true, 260000, 1549859, 21.1, false},  {true, 1500000, 8943723, 122.5, false},
@@ -109,7 +109,7 @@ static void keep_rule()
         int variant;
         double mb;
         bool keep;
-    } cases[] = {{3, 100, true}, {3, 130, true}, {3, 140, false}, {4, 100, true}, {4, 115, true}, {4, 126, false}};
+    } cases[] = {{3, 100, true}, {3, 130, true}, {3, 140, false}, {4, 100, true}, {4, 130, true}, {4, 140, false}};
     for (const auto &c : cases) {
         plan.csr_variant = c.variant;
         const double rest = c.mb * 1e6 - 4e6;  // (x and y)
