@@ -223,6 +223,16 @@ struct DeviceOffsets {
 };
 constexpr int kOffsetsMost = 64;           // most offsets of a chunk
 constexpr int kOffsetsRowsLeast = 1024;    // fewest rows of a matrix that takes the form (2431 rows: 3.3 us, row tiles 3.3)
+// A chunk's list of more than 40 offsets (binary16: 48) is two rounds of its four waves, one after the other, and a small matrix has
+// nothing else to do meanwhile: 1100 rows of 60, binary64, 4.3 us, row tiles 3.1; 5000 4.4, 3.4; 10 thousand 4.4, 3.9; 20 thousand 4.4, 5.0; of 48, 5000
+// 3.8, 3.4; 10 thousand 3.8, 3.6; 20 thousand 3.9, 4.6; of 40, 3000 3.5, 3.4; 10 thousand 3.5, 3.8; binary16, of 60, 5000 4.7, 4.0; 10
+// thousand 4.7, 4.3; 20 thousand 4.7, 4.6; of 48, 5000 4.0, 4.3.  With one byte per binary64 value the second round is half as long
+// (5000 rows of 60: 3.6, 3.6).
+inline bool offsets_lists_pay(bool f64, bool dict, int longest, int nnz)
+{
+    if (f64 && dict) return true;
+    return longest <= (f64 ? 40 : 48) || nnz >= (f64 ? 700000 : 1300000);
+}
 constexpr double kOffsetsFill = 1.2;       // most places per entry: 9.6 bytes per binary64 entry, as much as with a column offset of two bytes
 // What a product may touch for its units to be read with plain loads.  Plain / streaming loads, us, back to back | three
 // plans in turn: 67 MB 11.9 / 12.2 | 11.8 / 13.1; 98 MB 15.6 / 16.7 | 17.4 / 17.6; 142 MB 21.3 / 23.0 | 28.8 / 25.1;

@@ -425,6 +425,10 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
         if ((rc = value_dict_device(dtype, val_dev, nnz, 255, &codes, dict, &D.nDict, s))) return rc;
     Buf codesHold;
     codesHold.p = codes;
+    if (!offsets_lists_pay(dtype == MX_F64, D.nDict > 0, h[2], nnz)) {
+        D = DeviceOffsets();
+        return MX_OK;
+    }
     int unitBytes = 16;
     if (D.nDict > 0) {
         unitBytes = offsets_unit_bytes(true);

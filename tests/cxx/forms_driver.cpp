@@ -130,9 +130,19 @@ static void offset_waves()
     CHECK(mx::offsets_waves(true, false, 8ll << 28, 1 << 28) == 1);
 }
 
+// Long lists on small matrices, where row tiles were measured to be the faster ones.
+static void offset_lists()
+{
+    CHECK(!mx::offsets_lists_pay(true, false, 60, 65100) && !mx::offsets_lists_pay(true, false, 48, 480000));
+    CHECK(mx::offsets_lists_pay(true, false, 27, 27000) && mx::offsets_lists_pay(true, false, 60, 1200000));
+    CHECK(mx::offsets_lists_pay(true, true, 60, 299100) && mx::offsets_lists_pay(true, false, 48, 960000));
+    CHECK(!mx::offsets_lists_pay(false, false, 60, 600000) && !mx::offsets_lists_pay(false, true, 60, 299100));
+    CHECK(mx::offsets_lists_pay(false, false, 48, 240000) && mx::offsets_lists_pay(false, true, 60, 1800000));
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}};
+    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();

@@ -37,6 +37,7 @@ def _diagonals(mx, rng, rows, cols, offs, dtype, few, holes=0.0):
     (270000, 270000, list(range(-6, 6))),                # ... a list of more than one round: two or four waves a chunk
     (5001, 5001, list(range(0, 16, 2))),                 # as long a list as one wave takes, a row beyond whole chunks
     (5001, 5001, list(range(0, 18, 2))),                 # one more
+    (1100, 1100, list(range(-30, 30))),                  # a small matrix with a long list: row tiles are the faster ones
 ])
 def test_offset_form(mx, ora, dtype, few, rows, cols, offs):
     """Matrices whose rows repeat a pattern of column offsets: the product from both routes equals the oracle's
@@ -47,7 +48,8 @@ def test_offset_form(mx, ora, dtype, few, rows, cols, offs):
     A = _diagonals(mx, rng, rows, cols, np.array(offs), dtype, few, holes=0.05 if len(offs) > 8 else 0.0)
     small = few or dtype == np.float64
     x = rng.integers(-2, 3, cols).astype(dtype) if small else rng.choice([-1, 0, 0, 0, 0, 0, 0, 0, 0, 1], cols).astype(dtype)
-    takes = len(offs) <= 64
+    long = 48 if dtype == np.float16 else 40
+    takes = len(offs) <= 64 and (len(offs) <= long or rows >= 30000)
     xd = torch.from_numpy(x).cuda()
     dev = [torch.from_numpy(a).cuda() for a in (A.rowPtr, A.colInd, A.val)]
     ref = _exact(ora, A, x)
