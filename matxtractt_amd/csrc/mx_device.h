@@ -252,6 +252,12 @@ inline int offsets_waves(bool f64, bool dict, long long nOffs, int nChunks)
     if (nOffs <= 8ll * nChunks) return 1;
     return f64 && dict && nChunks >= 2048 ? 2 : 4;
 }
+// Workgroups of a product: four waves each.
+inline int offsets_blocks(bool f64, const DeviceOffsets &D)
+{
+    const int chunks = 4 / offsets_waves(f64, D.nDict > 0, D.nOffs, D.nChunks);
+    return (D.nChunks + chunks - 1) / chunks;
+}
 void free_offsets(DeviceOffsets &D);
 // Lays the matrix out in this form if it suits it (D.nChunks > 0 then); otherwise D stays empty and MX_OK is returned.
 // (weak: a host-only link of the library's C++ files has no device code to call)

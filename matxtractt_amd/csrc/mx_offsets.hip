@@ -25,6 +25,7 @@ typedef int v4i32 __attribute__((ext_vector_type(4)));
 typedef int v2i32 __attribute__((ext_vector_type(2)));
 
 constexpr int kBlock = 256;
+static_assert(kBlock == 4 * 64, "mx::offsets_blocks counts workgroups of four waves");
 constexpr int kMaxOffsets = mx::kOffsetsMost;  // most distinct offsets of a chunk
 constexpr int kTable = 2 * kMaxOffsets;        // slots of the table the offsets of a chunk are collected in
 constexpr int kFree = (int)0x80000000;         // no offset: columns and rows are not negative
@@ -477,10 +478,11 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     return MX_OK;
 }
 
+// (W as offsets_waves gives it for D: the grid is made from the same rule)
 template <typename VT, int W>
 static hipError_t launch_offsets_t(const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s)
 {
-    const int perWG = mxo::kBlock / 64 / W, wgs = (D.nChunks + perWG - 1) / perWG;
+    const int wgs = offsets_blocks(sizeof(VT) == 8, D);
 #define MX_LAUNCH_OFFSETS(DICT, KEEP)                                                                                                    \
     hipLaunchKernelGGL((mxo::csr_offsets_kernel<VT, DICT, KEEP, W>), dim3(wgs), dim3(mxo::kBlock), 0, s, (const int4 *)D.chunk, D.offs,    \
                        (const void *)D.stream, (const VT *)D.dict, (const VT *)x, (VT *)y, D.rows, D.cols, D.nChunks, accumulate)

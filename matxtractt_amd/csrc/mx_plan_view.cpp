@@ -250,7 +250,9 @@ extern "C" int mx_plan_get_info(const mx_plan *plan, mx_plan_info *info)
     info->tile_frags = plan->tiles.frags + plan->strips.frags;
     info->tile_nnz = plan->tile_nnz;
     info->csr_nnz = plan->csr_nnz;
-    info->csr_blocks = plan->csr_variant == 4 ? plan->windows.nWG : plan->csr_variant == 3 ? plan->offsets.nChunks : plan->csr_variant == 1 ? plan->slices.nWG : plan->csr.nBlocks;
+    info->csr_blocks = plan->csr_variant == 4 ? plan->windows.nWG + plan->windows.nApart
+                     : plan->csr_variant == 3 ? mx::offsets_blocks(plan->dtype == MX_F64, plan->offsets)
+                     : plan->csr_variant == 1 ? plan->slices.nWG : plan->csr.nBlocks;
     info->csr_variant = plan->csr_variant;
     // what each kernel has to move at least once: its arrays, x once, its y rows
     info->csr_bytes = (double)plan->csr_nnz * (es + 4) + ((double)plan->rows + 1) * 4 + (double)plan->cols * es +

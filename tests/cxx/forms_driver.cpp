@@ -140,9 +140,30 @@ static void offset_lists()
     CHECK(mx::offsets_lists_pay(false, false, 48, 240000) && mx::offsets_lists_pay(false, true, 60, 1800000));
 }
 
+// What a plan says of the workgroups of its CSR kernel is what the launch has.
+static void csr_blocks()
+{
+    mx_plan plan;
+    mx_plan_info info;
+    plan.rows = plan.cols = 1500000;
+    plan.csr_variant = 3;
+    plan.offsets.nChunks = 11719;
+    const struct {
+        int perChunk, nDict, blocks;
+    } cases[] = {{3, 0, 2930}, {27, 0, 11719}, {28, 2, 5860}};
+    for (const auto &c : cases) {
+        plan.offsets.nOffs = (long long)c.perChunk * plan.offsets.nChunks;
+        plan.offsets.nDict = c.nDict;
+        CHECK(mx_plan_get_info(&plan, &info) == MX_OK && info.csr_blocks == c.blocks);
+    }
+    plan.csr_variant = 4;
+    plan.windows.nWG = 489, plan.windows.nApart = 11;
+    CHECK(mx_plan_get_info(&plan, &info) == MX_OK && info.csr_blocks == 500);
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}};
+    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}, {"csr_blocks", csr_blocks}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();
