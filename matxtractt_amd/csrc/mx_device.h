@@ -263,7 +263,7 @@ void free_offsets(DeviceOffsets &D);
 // (weak: a host-only link of the library's C++ files has no device code to call)
 __attribute__((weak)) int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev,
                                                const void *val_dev, DeviceOffsets &D, hipStream_t s);
-__attribute__((weak)) hipError_t launch_offsets(mx_dtype dtype, const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s);
+__attribute__((weak)) hipError_t launch_offsets(mx_dtype dtype, const DeviceOffsets &D, const void *x, void *y, hipStream_t s);
 
 // The CSR part of a matrix whose neighbouring rows reach into one stretch of x (a mesh numbered for a small bandwidth):
 // chunks of 64 consecutive rows, a row per lane, kWindowWaves of them to a workgroup, which puts the window of x that its rows
@@ -335,7 +335,7 @@ void free_windows(DeviceWindows &D);
 // As build_offsets_device and launch_offsets.
 __attribute__((weak)) int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev,
                                                const void *val_dev, DeviceWindows &D, hipStream_t s);
-__attribute__((weak)) hipError_t launch_windows(mx_dtype dtype, const DeviceWindows &D, const void *x, void *y, int accumulate, hipStream_t s);
+__attribute__((weak)) hipError_t launch_windows(mx_dtype dtype, const DeviceWindows &D, const void *x, void *y, hipStream_t s);
 
 // The sums of the virtual rows (DeviceSlices::partial) of mx_spmv_static live in a fixed array
 // in device memory instead of the plan's own buffer: static_scratch gives the address of the

@@ -97,7 +97,7 @@ template <typename VT, bool DICT, bool KEEP, int W>
 __global__ __launch_bounds__(kBlock) void csr_offsets_kernel(const int4 *__restrict__ chunk, const int *__restrict__ offs,
                                                              const void *__restrict__ stream, const VT *__restrict__ dictG,
                                                              const VT *__restrict__ x, VT *__restrict__ y, int rows, int cols,
-                                                             int nChunks, int accumulate)
+                                                             int nChunks)
 {
     typedef Form<VT, DICT> F;
     typedef typename F::AT AT;
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kBlock) void csr_offsets_kernel(const int4 *__restr
             for (int i = 0; i < R; ++i) acc[i] += part[wave + k][i * 64 + lane];
     }
     if (!live) return;
-    if (r0 + R <= rows && !accumulate) {
+    if (r0 + R <= rows) {
         typename F::XV t;
 #pragma unroll
         for (int i = 0; i < R; ++i) t[i] = (VT)acc[i];
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(kBlock) void csr_offsets_kernel(const int4 *__restr
     } else {
 #pragma unroll
         for (int i = 0; i < R; ++i)
-            if (r0 + i < rows) y[r0 + i] = (VT)(acc[i] + (accumulate ? (AT)y[r0 + i] : (AT)0));
+            if (r0 + i < rows) y[r0 + i] = (VT)acc[i];
     }
 }
 
@@ -480,12 +480,12 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
 
 // (W as offsets_waves gives it for D: the grid is made from the same rule)
 template <typename VT, int W>
-static hipError_t launch_offsets_t(const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s)
+static hipError_t launch_offsets_t(const DeviceOffsets &D, const void *x, void *y, hipStream_t s)
 {
     const int wgs = offsets_blocks(sizeof(VT) == 8, D);
 #define MX_LAUNCH_OFFSETS(DICT, KEEP)                                                                                                    \
     hipLaunchKernelGGL((mxo::csr_offsets_kernel<VT, DICT, KEEP, W>), dim3(wgs), dim3(mxo::kBlock), 0, s, (const int4 *)D.chunk, D.offs,    \
-                       (const void *)D.stream, (const VT *)D.dict, (const VT *)x, (VT *)y, D.rows, D.cols, D.nChunks, accumulate)
+                       (const void *)D.stream, (const VT *)D.dict, (const VT *)x, (VT *)y, D.rows, D.cols, D.nChunks)
     if (D.nDict > 0 && D.keep) MX_LAUNCH_OFFSETS(true, true);
     else if (D.nDict > 0) MX_LAUNCH_OFFSETS(true, false);
     else if (D.keep) MX_LAUNCH_OFFSETS(false, true);
@@ -493,13 +493,13 @@ static hipError_t launch_offsets_t(const DeviceOffsets &D, const void *x, void *
 #undef MX_LAUNCH_OFFSETS
     return hipGetLastError();
 }
-hipError_t launch_offsets(mx_dtype dtype, const DeviceOffsets &D, const void *x, void *y, int accumulate, hipStream_t s)
+hipError_t launch_offsets(mx_dtype dtype, const DeviceOffsets &D, const void *x, void *y, hipStream_t s)
 {
     if (D.nChunks <= 0) return hipSuccess;
     const int waves = offsets_waves(dtype == MX_F64, D.nDict > 0, D.nOffs, D.nChunks);
-    if (dtype == MX_F16) return waves == 1 ? launch_offsets_t<_Float16, 1>(D, x, y, accumulate, s) : launch_offsets_t<_Float16, 4>(D, x, y, accumulate, s);
-    if (waves == 1) return launch_offsets_t<double, 1>(D, x, y, accumulate, s);
-    return waves == 2 ? launch_offsets_t<double, 2>(D, x, y, accumulate, s) : launch_offsets_t<double, 4>(D, x, y, accumulate, s);
+    if (dtype == MX_F16) return waves == 1 ? launch_offsets_t<_Float16, 1>(D, x, y, s) : launch_offsets_t<_Float16, 4>(D, x, y, s);
+    if (waves == 1) return launch_offsets_t<double, 1>(D, x, y, s);
+    return waves == 2 ? launch_offsets_t<double, 2>(D, x, y, s) : launch_offsets_t<double, 4>(D, x, y, s);
 }
 
 }  // namespace mx

@@ -456,18 +456,18 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
             std::swap(plan->slices, L);
             const int keepVariant = plan->csr_variant;
             plan->csr_variant = v;
-            rc = time_loop(plan, 3, 10, [&]() { return launch_csr_part(plan, tx, ty, 0, plan->stream); }, &ms);
+            rc = time_loop(plan, 3, 10, [&]() { return launch_csr_part(plan, tx, ty, plan->stream); }, &ms);
             if (!rc && v == 1 && plan->slices.ecode) {  // the same slices with one byte per value
                 double msDict = 0.0;
                 plan->slices.useDict = true;
-                rc = time_loop(plan, 3, 10, [&]() { return launch_csr_part(plan, tx, ty, 0, plan->stream); }, &msDict);
+                rc = time_loop(plan, 3, 10, [&]() { return launch_csr_part(plan, tx, ty, plan->stream); }, &msDict);
                 if (!rc && (msDict < ms || mx::opt().csr_dict == 2)) ms = msDict;
                 else plan->slices.useDict = false;
             }
             if (!rc && v == 0 && plan->csr.codes) {  // the same rows with one byte per value (MX_CSR_DICT=2: whatever the timing)
                 double msDict = 0.0;
                 plan->csr.useDict = true;
-                rc = time_loop(plan, 3, 10, [&]() { return launch_csr_part(plan, tx, ty, 0, plan->stream); }, &msDict);
+                rc = time_loop(plan, 3, 10, [&]() { return launch_csr_part(plan, tx, ty, plan->stream); }, &msDict);
                 if (!rc && (msDict < ms || mx::opt().csr_dict == 2)) ms = msDict;
                 else plan->csr.useDict = false;
             }

@@ -277,7 +277,7 @@ int create_plan_device(mx_dtype dtype, int rows, int cols, int nnz, const int *r
 extern std::atomic<bool> g_fused_off;
 // The CSR part of one product on stream `s`.  `strips`: tiles that ride in the combine kernel's launch;
 // `partial`: where the slice kernel puts the sums of the virtual rows, in place of the plan's own buffer.
-int launch_csr_part(mx_plan *plan, const void *x, void *y, int accumulate, hipStream_t s, const mx::DeviceTiles *strips = nullptr,
+int launch_csr_part(mx_plan *plan, const void *x, void *y, hipStream_t s, const mx::DeviceTiles *strips = nullptr,
                     void *partial = nullptr, void *ywide = nullptr);
 
 }  // namespace mxp

@@ -47,22 +47,22 @@ extern "C" int mx_debug_fused_misplaced(int set)
 
 // `partial` (optional): where the slice kernel puts the sums of the virtual rows, in place of the
 // plan's own buffer.
-int mxp::launch_csr_part(mx_plan *plan, const void *x, void *y, int accumulate, hipStream_t s, const mx::DeviceTiles *strips, void *partial,
+int mxp::launch_csr_part(mx_plan *plan, const void *x, void *y, hipStream_t s, const mx::DeviceTiles *strips, void *partial,
                          void *ywide)
 {
     if (plan->csr_variant == 4) {
-        MX_HIP(mx::launch_windows(plan->dtype, plan->windows, x, y, accumulate, s));
+        MX_HIP(mx::launch_windows(plan->dtype, plan->windows, x, y, s));
         return MX_OK;
     }
     if (plan->csr_variant == 3) {
-        MX_HIP(mx::launch_offsets(plan->dtype, plan->offsets, x, y, accumulate, s));
+        MX_HIP(mx::launch_offsets(plan->dtype, plan->offsets, x, y, s));
         return MX_OK;
     }
     if (plan->csr_variant != 0 && ((uintptr_t)x & 15)) {
         set_error("mx_spmv: x must be 16-byte aligned for this plan");
         return MX_ERR_ARG;
     }
-    if (plan->csr_variant != 1) MX_HIP(mx::launch_csr(plan->dtype, plan->csr, x, y, accumulate, s, ywide));
+    if (plan->csr_variant != 1) MX_HIP(mx::launch_csr(plan->dtype, plan->csr, x, y, 0, s, ywide));
     if (plan->csr_variant == 1 && plan->fused && !strips && !partial) {  // (sums in a caller's buffer: the two launches)
         // one launch.  A workgroup that found its share of the work taken already has said so in the
         // host-visible word: the products since the last look cannot be trusted, and from here on every
@@ -86,7 +86,7 @@ int mxp::launch_csr_part(mx_plan *plan, const void *x, void *y, int accumulate, 
                       "products since the previous call may be wrong; plans use the two-launch form from now on");
             return MX_ERR_DEVICE;
         } else {
-            MX_HIP(mx::launch_fused(plan->dtype, plan->slices, x, y, accumulate, s, ywide, word, plan->fused_seq++));
+            MX_HIP(mx::launch_fused(plan->dtype, plan->slices, x, y, 0, s, ywide, word, plan->fused_seq++));
             return MX_OK;
         }
     }
@@ -94,9 +94,9 @@ int mxp::launch_csr_part(mx_plan *plan, const void *x, void *y, int accumulate, 
         if (partial) {
             mx::DeviceSlices L = plan->slices;  // a view: same arrays, other sums
             L.partial = partial;
-            MX_HIP(mx::launch_slices(plan->dtype, L, x, y, accumulate, s, 0, strips, ywide));
+            MX_HIP(mx::launch_slices(plan->dtype, L, x, y, 0, s, 0, strips, ywide));
         } else {
-            MX_HIP(mx::launch_slices(plan->dtype, plan->slices, x, y, accumulate, s, 0, strips, ywide));
+            MX_HIP(mx::launch_slices(plan->dtype, plan->slices, x, y, 0, s, 0, strips, ywide));
         }
     }
     return MX_OK;
@@ -130,7 +130,7 @@ static int spmv_on(mx_plan *plan, const void *x, void *y, hipStream_t s, void *p
     // (a binary16 row that gets sums from both parts: the CSR part leaves its sum in binary32 as
     // well and the tile kernel adds to that, so that y is rounded once, not twice)
     void *wide = plan->tiles.nWaves > 0 ? plan->ywide : nullptr;
-    int rc = launch_csr_part(plan, x, y, 0, s, ride ? &plan->strips : nullptr, partial, wide);
+    int rc = launch_csr_part(plan, x, y, s, ride ? &plan->strips : nullptr, partial, wide);
     if (rc) return rc;
     MX_HIP(mx::launch_tiles(plan->dtype, plan->tiles, x, y, 1, s, wide));
     if (!ride) MX_HIP(mx::launch_tiles(plan->dtype, plan->strips, x, y, 1, s));
@@ -222,7 +222,7 @@ extern "C" int mx_time_csr_main(mx_plan *plan, const void *x_dev, void *y_dev, i
     int rc = time_loop(plan, warm, iters, [&]() -> int {
         // the kernel that holds most of the entries
         if (plan->csr_variant >= 3 || (plan->csr_variant == 1 && plan->fused))
-            return launch_csr_part(plan, x_dev, y_dev, 0, s);
+            return launch_csr_part(plan, x_dev, y_dev, s);
         if (plan->csr_variant == 1 || (plan->csr_variant == 2 && plan->slices.nnz > plan->csr.nnz))
             MX_HIP(mx::launch_slices(plan->dtype, plan->slices, x_dev, y_dev, 0, s, 1));
         else
@@ -264,12 +264,12 @@ extern "C" int mx_time(mx_plan *plan, const void *x_dev, void *y_dev, int warm, 
     const bool blocksApart = !ride && plan->dtype == MX_F64 && plan->strips.nWaves > 0;  // binary64 blocks in a launch of their own
     double tBare = 0.0;
     if (ms_csr || (ms_tile && (ride || blocksApart))) {
-        rc = time_loop(plan, warm, iters, [&]() { return launch_csr_part(plan, x_dev, y_dev, 0, s, ride ? &plan->strips : nullptr, nullptr, wide); }, &t);
+        rc = time_loop(plan, warm, iters, [&]() { return launch_csr_part(plan, x_dev, y_dev, s, ride ? &plan->strips : nullptr, nullptr, wide); }, &t);
         if (rc) return rc;
         if (ms_csr) *ms_csr = t;
         if (ms_tile && ride) {
             // (the rows of riders are left alone by the bare launch: nothing is added to them, y stays bounded)
-            rc = time_loop(plan, warm, iters, [&]() { return launch_csr_part(plan, x_dev, y_dev, 0, s, nullptr, nullptr, wide); }, &tBare);
+            rc = time_loop(plan, warm, iters, [&]() { return launch_csr_part(plan, x_dev, y_dev, s, nullptr, nullptr, wide); }, &tBare);
             if (rc) return rc;
         }
     }
@@ -291,7 +291,7 @@ extern "C" int mx_time(mx_plan *plan, const void *x_dev, void *y_dev, int warm, 
             // CSR part rewrites y before every launch of the blocks
             double pair = 0.0;
             rc = time_loop(plan, warm, iters, [&]() -> int {
-                int r = launch_csr_part(plan, x_dev, y_dev, 0, s, nullptr, nullptr, wide);
+                int r = launch_csr_part(plan, x_dev, y_dev, s, nullptr, nullptr, wide);
                 if (r) return r;
                 MX_HIP(mx::launch_tiles(plan->dtype, plan->strips, x_dev, y_dev, 1, s));
                 return MX_OK;
@@ -366,10 +366,10 @@ extern "C" int mx_time_kernels(mx_plan *plan, const void *x_dev, void *y_dev, in
     if (plan->csr_variant == 3)
         add(std::string("csr_offsets_kernel<") + vt + (plan->offsets.nDict > 0 ? ",dict" : "") + (plan->offsets.keep ? ",keep>" : ">"),
             (double)plan->csr_nnz * (es + 4) + xBytes + yBytes, plan->csr_nnz,
-            [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, 0, s); });
+            [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, s); });
     if (plan->csr_variant == 4)
         add(std::string("csr_window_kernel<") + vt + (plan->windows.keep ? ",keep>" : ">"), (double)plan->csr_nnz * (es + 4) + xBytes + yBytes,
-            plan->csr_nnz, [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, 0, s); });
+            plan->csr_nnz, [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, s); });
     if ((plan->csr_variant == 0 || plan->csr_variant == 2) && plan->csr.nBlocks > 0) {
         const bool last = plan->csr_variant == 0;  // writes y for good
         add(std::string("csr_rows_kernel<") + vt + (plan->csr.useDict ? ",dict>" : ">"),
@@ -383,7 +383,7 @@ extern "C" int mx_time_kernels(mx_plan *plan, const void *x_dev, void *y_dev, in
         // the one-launch form: one kernel multiplies, adds up and writes y
         add(std::string("csr_slice_kernel<") + vt + (plan->slices.useDict ? ",dict" : "") + ",fused" + (plan->slices.keep ? ",keep>" : ">"),
             (double)plan->slices.nnz * (es + 4) + xBytes + yBytes, plan->slices.nnz,
-            [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, 0, s, nullptr, nullptr, wide); });
+            [&]() -> int { return launch_csr_part(plan, x_dev, y_dev, s, nullptr, nullptr, wide); });
     } else if (plan->csr_variant == 1 || plan->csr_variant == 2) {
         add(std::string("csr_slice_kernel<") + vt + (plan->slices.useDict ? ",dict" : "") + (plan->slices.keep ? ",keep>" : ">"),
             (double)plan->slices.nnz * (es + 4) + (xCounted ? 0.0 : xBytes), plan->slices.nnz, [&]() -> int {

@@ -89,8 +89,7 @@ template <typename VT, bool KEEP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void csr_window_kernel(const int2 *__restrict__ window, const int4 *__restrict__ chunk,
                                                                 const unsigned char *__restrict__ stream, const int *__restrict__ farCol,
                                                                 const VT *__restrict__ farVal, const int *__restrict__ apart, const VT *__restrict__ x,
-                                                                VT *__restrict__ y, int rows, int cols, int nChunks, int nApart, int zeroPlace,
-                                                                int accumulate)
+                                                                VT *__restrict__ y, int rows, int cols, int nChunks, int nApart, int zeroPlace)
 {
     typedef typename std::conditional<sizeof(VT) == 8, double, float>::type AT;
     constexpr int EPV = 16 / (int)sizeof(VT), THREADS = 64 * WAVES, NB = sizeof(VT) == 8 ? 6 : 10, XR = 4, NF = mx::kWindowFarSteps;
@@ -129,7 +128,7 @@ __global__ __launch_bounds__(64 * WAVES) void csr_window_kernel(const int2 *__re
 #pragma unroll
         for (int k = 1; k < WAVES; ++k) acc += part[k * 64 + lane];
         const int r = c * 64 + lane;
-        if (r < rows) y[r] = (VT)(acc + (accumulate ? (AT)y[r] : (AT)0));
+        if (r < rows) y[r] = (VT)acc;
         return;
     }
     // every XCD walks one contiguous range of rows: the x of neighbouring windows lives in one L2
@@ -200,7 +199,7 @@ __global__ __launch_bounds__(64 * WAVES) void csr_window_kernel(const int2 *__re
     for (int k = 0; k < NF; ++k)
         if (k < nf && farC[k] >= 0) acc += (AT)farV[k] * (AT)farX[k];
     const int r = c * 64 + lane;
-    if (c < nChunks && d.y >= 0 && r < rows) y[r] = (VT)(acc + (accumulate ? (AT)y[r] : (AT)0));
+    if (c < nChunks && d.y >= 0 && r < rows) y[r] = (VT)acc;
 }
 
 // ---- laying a matrix out ----------------------------------------------------------------------------------
@@ -518,14 +517,14 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     return rc ? fail(rc) : rc;
 }
 
-hipError_t launch_windows(mx_dtype dtype, const DeviceWindows &D, const void *x, void *y, int accumulate, hipStream_t s)
+hipError_t launch_windows(mx_dtype dtype, const DeviceWindows &D, const void *x, void *y, hipStream_t s)
 {
     if (D.nChunks <= 0) return hipSuccess;
 #define MX_LAUNCH_WINDOWS(VT, KEEP)                                                                                                          \
     hipLaunchKernelGGL((mxw::csr_window_kernel<VT, KEEP, kWindowWaves>), dim3(D.nWG + D.nApart), dim3(64 * kWindowWaves), D.ldsBytes, s,                  \
                        (const int2 *)D.window, (const int4 *)D.chunk, (const unsigned char *)D.stream, (const int *)D.farCol,                  \
                        (const VT *)D.farVal, (const int *)D.apart, (const VT *)x, (VT *)y, D.rows, D.cols, D.nChunks, D.nApart,               \
-                       D.zeroPlace, accumulate)
+                       D.zeroPlace)
     if (dtype == MX_F64) {
         if (D.keep) MX_LAUNCH_WINDOWS(double, true);
         else MX_LAUNCH_WINDOWS(double, false);

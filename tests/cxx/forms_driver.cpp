@@ -35,8 +35,8 @@ int build_windows_device(mx_dtype, int, int, int, const int *, const int *, cons
     if (windows_suit) D.nChunks = 7;
     return windows_rc;
 }
-hipError_t launch_offsets(mx_dtype, const DeviceOffsets &, const void *, void *, int, hipStream_t) { return hipErrorUnknown; }
-hipError_t launch_windows(mx_dtype, const DeviceWindows &, const void *, void *, int, hipStream_t) { return hipErrorUnknown; }
+hipError_t launch_offsets(mx_dtype, const DeviceOffsets &, const void *, void *, hipStream_t) { return hipErrorUnknown; }
+hipError_t launch_windows(mx_dtype, const DeviceWindows &, const void *, void *, hipStream_t) { return hipErrorUnknown; }
 }  // namespace mx
 
 // No memory for a form is a reason to go on without it (the forms behind it need less beside the matrix), any other
