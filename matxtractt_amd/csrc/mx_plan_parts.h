@@ -8,6 +8,7 @@
 #include <chrono>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -157,7 +158,8 @@ struct mx_plan {
     // the fill a fragment needed); the product looks at these, never at the environment
     int opt_flags = mxp::plan_opt_flags();
     double opt_tile_gate = mx::opt().tile_gate >= 0.0 ? mx::opt().tile_gate : 0.5;
-    // made when something is first timed or run on them (mxp::plan_stream)
+    // made when something is first timed or run on them (mxp::plan_stream), and the same from then on
+    std::mutex stream_mu;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -165,9 +167,10 @@ struct mx_plan {
 namespace mxp {
 
 // The plan's own stream and its two events: a plan that only ever runs on its callers' streams does without them
-// (making them costs as much as a small plan).
+// (making them costs as much as a small plan).  Threads may share a plan: whoever comes first makes them.
 inline int plan_stream(mx_plan *plan)
 {
+    std::lock_guard<std::mutex> hold(plan->stream_mu);
     if (!plan->stream) MX_HIP(hipStreamCreate(&plan->stream));
     if (!plan->ev0) MX_HIP(hipEventCreate(&plan->ev0));
     if (!plan->ev1) MX_HIP(hipEventCreate(&plan->ev1));

@@ -187,7 +187,8 @@ extern "C" int mx_spmv_host(mx_plan *plan, const void *x_host, void *y_host)
     }
     const size_t es = (size_t)mx::elem_size(plan->dtype);
     if (int bad = plan_stream(plan)) return bad;
-    mx::MemScope scope(plan->stream);
+    const hipStream_t s = plan->stream;
+    mx::MemScope scope(s);
     void *dx = nullptr, *dy = nullptr;
     MX_HIP(mx::dev_malloc(&dx, std::max<size_t>(plan->cols * es, 1)));
     if (mx::dev_malloc(&dy, std::max<size_t>(plan->rows * es, 1)) != hipSuccess) {
@@ -197,11 +198,11 @@ extern "C" int mx_spmv_host(mx_plan *plan, const void *x_host, void *y_host)
     }
     int rc = MX_OK;
     auto body = [&]() -> int {
-        MX_HIP(hipMemcpyAsync(dx, x_host, plan->cols * es, hipMemcpyHostToDevice, plan->stream));
-        int r = spmv_on(plan, dx, dy, plan->stream);
+        MX_HIP(hipMemcpyAsync(dx, x_host, plan->cols * es, hipMemcpyHostToDevice, s));
+        int r = spmv_on(plan, dx, dy, s);
         if (r) return r;
-        MX_HIP(hipMemcpyAsync(y_host, dy, plan->rows * es, hipMemcpyDeviceToHost, plan->stream));
-        MX_HIP(hipStreamSynchronize(plan->stream));
+        MX_HIP(hipMemcpyAsync(y_host, dy, plan->rows * es, hipMemcpyDeviceToHost, s));
+        MX_HIP(hipStreamSynchronize(s));
         return MX_OK;
     };
     rc = body();

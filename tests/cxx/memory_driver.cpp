@@ -1,15 +1,17 @@
 // The device memory that the library keeps between calls (mx_util.cpp), on a device that exists only here: the few HIP
 // functions it calls are defined below and count bytes.  Run with the name of one check; exit status 0 means it holds.
+#include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
-#include "mx_device.h"
-#include "mx_internal.h"
+#include "mx_plan_parts.h"
 
 namespace {
 
@@ -21,6 +23,7 @@ struct Device {
     std::map<void *, size_t> blocks;
     uintptr_t next = 0x10000;
     int frees = 0;
+    std::atomic<int> streams{0};
     bool refuse = false;  // waits for the device
     hipError_t last = hipSuccess;
 } device;
@@ -68,6 +71,14 @@ hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) { return *f = device.total - device.used, *t = device.total, hipSuccess; }
 hipError_t hipDeviceSynchronize() { return device.refuse ? hipErrorStreamCaptureUnsupported : hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t *s)
+{
+    std::this_thread::sleep_for(std::chrono::milliseconds(2));
+    *s = (hipStream_t)(uintptr_t)++device.streams;
+    return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t *e) { return *e = (hipEvent_t)(uintptr_t)1, hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return ""; }
 hipError_t hipGetLastError()
 {
     const hipError_t e = device.last;
@@ -158,9 +169,27 @@ static void scope_share()
     CHECK(device.used <= device.total / 128);
 }
 
+// Threads that meet in the first call of a plan that needs a stream of its own get one and the same.
+static void one_stream()
+{
+    for (int round = 0; round < 20; ++round) {
+        mx_plan plan;
+        device.streams = 0;
+        std::vector<std::thread> threads;
+        std::vector<hipStream_t> got(8, nullptr);
+        for (int t = 0; t < 8; ++t)
+            threads.emplace_back([&, t]() {
+                if (!mxp::plan_stream(&plan)) got[t] = plan.stream;
+            });
+        for (auto &t : threads) t.join();
+        CHECK(device.streams == 1 && plan.ev0 && plan.ev1);
+        for (hipStream_t s : got) CHECK(s && s == plan.stream);
+    }
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}, {"bound", bound}, {"age", age}, {"scope_full", scope_full}, {"scope_share", scope_share}};
+    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}, {"bound", bound}, {"age", age}, {"scope_full", scope_full}, {"scope_share", scope_share}, {"one_stream", one_stream}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();
