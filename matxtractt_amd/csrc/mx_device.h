@@ -34,6 +34,16 @@ struct IdleFrees {
     IdleFrees &operator=(const IdleFrees &) = delete;
 };
 
+// The next of the places p, p + stride, .. below n; n where there is none (p + stride may be more than an int holds).
+__host__ __device__ inline int next_of(int p, int n, int stride) { return n - p > stride ? p + stride : n; }
+// Rows, columns and entries that the kernels of the offset and window forms can number: a chunk reaches past the last row by fewer
+// rows than this leaves.  (The other routes on the device refuse more than that; from host arrays row tiles take it.)
+inline bool forms_can_number(int rows, int cols, int nnz)
+{
+    constexpr int most = 2147483647 - 512;
+    return rows <= most && cols <= most && nnz <= most;
+}
+
 // CSR matrix resident on the device, plus the row ranges of the CSR kernel's workgroups.
 // col/val carry kCsrPad extra zero entries so that a wave's aligned 128-bit loads may overrun.
 struct DeviceCsr {

@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kBlock) void gate_counts_kernel(const int *__restri
                                                              unsigned long long *__restrict__ totals)
 {
     unsigned long long frags = 0, entries = 0;
-    for (int f = blockIdx.x * kBlock + threadIdx.x; f < nFrags; f += gridDim.x * kBlock) {
+    for (int f = blockIdx.x * kBlock + threadIdx.x; f < nFrags; f = mx::next_of(f, nFrags, gridDim.x * kBlock)) {
         const int vals = fragPtr[f + 1] - fragPtr[f];
         if (vals > 0 && vals >= minVals) {
             ++frags;
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kBlock) void block_runs_kernel(const unsigned long 
                                                             unsigned long long *__restrict__ totals)
 {
     unsigned long long blocks = 0, entries = 0;
-    for (int p = blockIdx.x * kBlock + threadIdx.x; p < n; p += gridDim.x * kBlock) {
+    for (int p = blockIdx.x * kBlock + threadIdx.x; p < n; p = mx::next_of(p, n, gridDim.x * kBlock)) {
         if (key[p] == ~0ull || (p > 0 && key[p - 1] == key[p])) continue;
         // (a block holds at most 64 entries that are not twins; most runs are short of `need`, which one look tells)
         if (p + need > n || key[p + need - 1] != key[p]) continue;

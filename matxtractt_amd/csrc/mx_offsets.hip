@@ -389,7 +389,7 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     using namespace mxo;
     D = DeviceOffsets();
     // (what cannot pass is not looked at: too few rows to fill a chunk, more entries a row than a chunk has offsets)
-    if (rows < kOffsetsRowsLeast || nnz < rows || (long long)nnz > (long long)rows * kMaxOffsets) return MX_OK;
+    if (!forms_can_number(rows, cols, nnz) || rows < kOffsetsRowsLeast || nnz < rows || (long long)nnz > (long long)rows * kMaxOffsets) return MX_OK;
     const int R = dtype == MX_F64 ? 2 : 4, chunkRows = 64 * R, nChunks = (rows + chunkRows - 1) / chunkRows;
     Buf lists, count, units, unit0, totals, tmp;
     size_t scanBytes = 0;

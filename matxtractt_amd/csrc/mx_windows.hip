@@ -421,7 +421,7 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     D = DeviceWindows();
     const bool f64 = dtype == MX_F64;
     const int es = elem_size(dtype), epv = 16 / es;
-    if (rows < kWindowRowsLeast || cols < 64 || !window_mean_ok(f64, rows, nnz) || nnz > 1500000000 ||
+    if (!forms_can_number(rows, cols, nnz) || rows < kWindowRowsLeast || cols < 64 || !window_mean_ok(f64, rows, nnz) || nnz > 1500000000 ||
         (f64 && nnz < kWindowEntriesLeast))
         return MX_OK;
     const int nChunks = (rows + 63) / 64, waves = kWindowWaves, nWG = (nChunks + waves - 1) / waves;

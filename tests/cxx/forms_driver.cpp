@@ -161,9 +161,27 @@ static void csr_blocks()
     CHECK(mx_plan_get_info(&plan, &info) == MX_OK && info.csr_blocks == 500);
 }
 
+// The entries that one thread of a counting kernel looks at: all below n and n at the end, also where n is close to what an int
+// holds (2^31 - 513 entries are accepted).
+static void strides()
+{
+    const int n = 2147483647 - 512, stride = 1024 * 256;
+    for (const int first : {0, stride - 1, n - 1, n - stride - 1, n - stride}) {
+        int p = first, steps = 0;
+        for (; p < n; p = mx::next_of(p, n, stride)) {
+            CHECK(p >= 0);
+            CHECK(++steps <= n / stride + 2);
+        }
+        CHECK(p == n && steps == (n - 1 - first) / stride + 1);
+    }
+    CHECK(mx::next_of(5, 3, 2) == 3 && mx::next_of(0, 1, 262144) == 1);
+    // ... and matrices whose last chunk would not be numbered in an int do not take the forms
+    CHECK(mx::forms_can_number(n, n, n) && !mx::forms_can_number(n + 1, 5, 5) && !mx::forms_can_number(5, n + 1, 5) && !mx::forms_can_number(5, 5, n + 1));
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}, {"csr_blocks", csr_blocks}};
+    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}, {"csr_blocks", csr_blocks}, {"strides", strides}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();
