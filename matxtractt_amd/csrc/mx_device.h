@@ -243,6 +243,11 @@ inline bool offsets_lists_pay(bool f64, bool dict, int longest, int nnz)
     if (f64 && dict) return true;
     return longest <= (f64 ? 40 : 48) || nnz >= (f64 ? 700000 : 1300000);
 }
+inline bool offsets_size_ok(int rows, int cols, int nnz)
+{
+    return forms_can_number(rows, cols, nnz) && rows >= kOffsetsRowsLeast && nnz >= rows && (long long)nnz <= (long long)rows * kOffsetsMost;
+}
+constexpr int offsets_chunk_rows(bool f64) { return f64 ? 128 : 256; }
 constexpr double kOffsetsFill = 1.2;       // most places per entry: 9.6 bytes per binary64 entry, as much as with a column offset of two bytes
 // What a product may touch for its units to be read with plain loads.  Plain / streaming loads, us, back to back | three
 // plans in turn: 67 MB 11.9 / 12.2 | 11.8 / 13.1; 98 MB 15.6 / 16.7 | 17.4 / 17.6; 142 MB 21.3 / 23.0 | 28.8 / 25.1;
@@ -310,6 +315,11 @@ inline bool window_mean_ok(bool f64, int rows, int nnz)
     const int least = f64 ? kWindowMean : rows <= kWindowFewRows ? kWindowMeanFewRows : rows <= kWindowManyRows ? kWindowMean : kWindowMeanManyRows;
     return (long long)nnz >= (long long)rows * least;
 }
+inline bool window_size_ok(bool f64, int rows, int cols, int nnz)
+{
+    return forms_can_number(rows, cols, nnz) && rows >= kWindowRowsLeast && cols >= 64 && window_mean_ok(f64, rows, nnz) && nnz <= 1500000000 &&
+           !(f64 && nnz < kWindowEntriesLeast);
+}
 // Whether a matrix laid out in `stored` bytes by nWG workgroups is better off in this form than in slices (or row tiles).  The
 // one launch saves about 4 us, some 18 MB's worth; padding beyond that (rows of uneven length) costs more than it
 // (binary64, 600 thousand rows of 28 to 52 entries, 314 MB instead of 238: 55 us, slices 48; of 34 to 46, 290 MB: 48.6, 48.1).
@@ -333,6 +343,18 @@ constexpr int kWindowTrim = 32;               // bytes that a far entry is worth
 constexpr int kWindowLongest = 1024;          // most entries of a row
 constexpr double kWindowShare = 0.6;          // most bytes of a window per byte of its workgroup's entries
 constexpr int kWindowBytesMost = 80 << 10;    // of a window: two workgroups share the LDS of a CU
+constexpr int kWindowBuckets = 2048;          // of columns, to find the windows with
+// Elements of x in a window, at most: it costs its workgroup as much intake as entries do -- at most kWindowShare of their bytes, and what
+// fits in LDS.
+inline int window_widest(bool f64, int nnz, int nWG)
+{
+    const int es = f64 ? 8 : 2;
+    return (int)std::min<double>(kWindowBytesMost, kWindowShare * ((double)nnz / nWG * (es + 2))) / es;
+}
+// Columns of a bucket, a multiple of a vector of x (cols >= 1; no sum here leaves the range of an int).
+__host__ __device__ inline int window_bucket(int cols, int epv) { return ((cols - 1) / kWindowBuckets + epv) / epv * epv; }
+// Whether a workgroup with `outside` of its n entries outside its window is one of a matrix of another kind.
+__host__ __device__ inline bool window_scattered(int outside, int n) { return (long long)outside * 4 > (long long)n * 3 + 256; }
 constexpr int window_unit_bytes(bool f64) { return 64 * kWindowUnit * (f64 ? 10 : 4); }
 // What a product may touch for its units to be read with plain loads.  Plain / streaming loads, us, back to back | three plans in
 // turn: binary16, 51 MB 11.3 / 12.0 | 11.2 / 12.6; 76 MB 14.2 / 14.2 | 14.2 / 14.9; 99 MB 16.7 / 16.2 | 18.6 / 17.2; 108 MB 18.9 / 21.7 | 23.1 /
@@ -354,6 +376,7 @@ constexpr size_t kStaticScratchBytes = (size_t)32 << 20;  // the largest benchma
 hipError_t static_scratch(void **ptr);
 
 }  // namespace mx
+#include <algorithm>
 #include <vector>
 namespace mx {
 // One chunk of a slice on its way into the layout: `first` = index of its first virtual row in

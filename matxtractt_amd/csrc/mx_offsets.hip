@@ -36,6 +36,7 @@ struct Form {
     static constexpr int kUnitBytes = mx::offsets_unit_bytes(DICT);                // what a lane loads at a time
     static constexpr int U = kUnitBytes / (R * (DICT ? 1 : (int)sizeof(VT)));      // offsets those bytes cover
     static constexpr int kRows = 64 * R;                                           // rows of a chunk, one chunk per wave
+    static_assert(kRows == mx::offsets_chunk_rows(sizeof(VT) == 8), "the host looks at chunks of as many rows");
     typedef VT XV __attribute__((ext_vector_type(R), aligned(sizeof(VT))));        // R consecutive x, at any element
     typedef typename std::conditional<DICT, v2i32, v4i32>::type Unit;
     typedef typename std::conditional<sizeof(VT) == 8, double, float>::type AT;
@@ -389,7 +390,7 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     using namespace mxo;
     D = DeviceOffsets();
     // (what cannot pass is not looked at: too few rows to fill a chunk, more entries a row than a chunk has offsets)
-    if (!forms_can_number(rows, cols, nnz) || rows < kOffsetsRowsLeast || nnz < rows || (long long)nnz > (long long)rows * kMaxOffsets) return MX_OK;
+    if (!offsets_size_ok(rows, cols, nnz)) return MX_OK;
     const int R = dtype == MX_F64 ? 2 : 4, chunkRows = 64 * R, nChunks = (rows + chunkRows - 1) / chunkRows;
     Buf lists, count, units, unit0, totals, tmp;
     size_t scanBytes = 0;

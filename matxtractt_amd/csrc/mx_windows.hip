@@ -204,7 +204,7 @@ __global__ __launch_bounds__(64 * WAVES) void csr_window_kernel(const int2 *__re
 
 // ---- laying a matrix out ----------------------------------------------------------------------------------
 
-constexpr int kBuckets = 2048;  // of columns, to find the windows with
+constexpr int kBuckets = mx::kWindowBuckets;
 
 // totals[0] = 1 where a row has more than kWindowLongest entries: a matrix with a tail of long rows is not looked at any
 // further (16 million entries in a million rows: 0.28 ms of counting columns)
@@ -237,8 +237,7 @@ __global__ __launch_bounds__(kBlock) void window_find_kernel(const int *__restri
     }
     __syncthreads();
     if (over) return;
-    // buckets of a multiple of epv columns
-    const int size = max(epv, ((cols + kBuckets - 1) / kBuckets + epv - 1) / epv * epv), wide = max(widest / size, 1);
+    const int size = mx::window_bucket(cols, epv), wide = max(widest / size, 1);
     const int c0 = blockIdx.x * waves, c1 = min(c0 + waves, nChunks);
     const int r0 = c0 * 64, r1 = min(c1 * 64, rows), p0 = rowPtr[r0], p1 = rowPtr[r1];
     for (int i = tid; i < kBuckets; i += kBlock) hist[i] = 0;
@@ -276,7 +275,7 @@ __global__ __launch_bounds__(kBlock) void window_find_kernel(const int *__restri
     const int vecs = max((behind - first + epv - 1) / epv, 1);
     const int outside = p1 - p0 - (hist[hi] - (lo ? hist[lo - 1] : 0));
     // (before a lane walks its row: a matrix of another kind is found out by its first workgroups)
-    if (size > widest || (long long)outside * 4 > (long long)(p1 - p0) * 3 + 256) {
+    if (size > widest || mx::window_scattered(outside, p1 - p0)) {
         if (tid == 0) *(volatile int *)totals = 1;
         return;
     }
@@ -421,13 +420,9 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     D = DeviceWindows();
     const bool f64 = dtype == MX_F64;
     const int es = elem_size(dtype), epv = 16 / es;
-    if (!forms_can_number(rows, cols, nnz) || rows < kWindowRowsLeast || cols < 64 || !window_mean_ok(f64, rows, nnz) || nnz > 1500000000 ||
-        (f64 && nnz < kWindowEntriesLeast))
-        return MX_OK;
+    if (!window_size_ok(f64, rows, cols, nnz)) return MX_OK;
     const int nChunks = (rows + 63) / 64, waves = kWindowWaves, nWG = (nChunks + waves - 1) / waves;
-    // a window costs its workgroup as much intake as entries do: at most kWindowShare of their bytes, and what fits in LDS
-    const double entryBytes = (double)nnz / nWG * (es + 2);
-    const int widest = (int)std::min<double>(kWindowBytesMost, kWindowShare * entryBytes) / es;
+    const int widest = window_widest(f64, nnz, nWG);
     Buf units, farSteps, alone, unit0, far0, apart0, totals, tmp;
     size_t scanBytes = 0;
     const size_t chunkB = ((size_t)nChunks + 1) * 4;

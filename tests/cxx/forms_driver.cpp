@@ -179,9 +179,20 @@ static void strides()
     CHECK(mx::forms_can_number(n, n, n) && !mx::forms_can_number(n + 1, 5, 5) && !mx::forms_can_number(5, n + 1, 5) && !mx::forms_can_number(5, 5, n + 1));
 }
 
+// Every column falls into one of the window form's buckets, of whole vectors of x.
+static void window_buckets()
+{
+    for (const int epv : {2, 8})
+        for (const int cols : {64, 2047, 2048, 2049, 16384, 16385, 30011, 1000003, 2147483647 - 2048, 2147483647 - 2047, 2147483647 - 512}) {
+            const int size = mx::window_bucket(cols, epv);
+            CHECK(size >= epv && size % epv == 0 && (cols - 1) / size < mx::kWindowBuckets);
+            CHECK(size == epv || (long long)(size - epv) * mx::kWindowBuckets < cols);  // (no larger than it has to be)
+        }
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}, {"csr_blocks", csr_blocks}, {"strides", strides}};
+    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}, {"csr_blocks", csr_blocks}, {"strides", strides}, {"window_buckets", window_buckets}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();
