@@ -309,6 +309,58 @@ bool mxp::may_look_for_form(int flags)
     const mx::Options &o = mx::opt();
     return !(flags & (MX_PLAN_CSR_ROWS | MX_PLAN_CSR_SLICES | MX_PLAN_FUSE)) && o.csr_kernel == 0 && o.csr_fused != 1 && !o.autotune;
 }
+// Whether a matrix in host memory may take the offset or the window form: false only where build_offsets_device and
+// build_windows_device would both leave it.  They refuse a matrix for one row, chunk or workgroup of the wrong kind, so the rows' lengths
+// and a few chunks and workgroups tell most matrices apart before anything is sent up.
+bool mxp::forms_may_suit(mx_dtype dtype, int rows, int cols, const int *rowPtr, const int *col)
+{
+    const bool f64 = dtype == MX_F64;
+    const int nnz = rows > 0 ? rowPtr[rows] : 0;
+    bool offsets = mx::offsets_size_ok(rows, cols, nnz), windows = mx::window_size_ok(f64, rows, cols, nnz);
+    if (!offsets && !windows) return false;
+    int longest = 0;
+#pragma omp parallel for schedule(static) reduction(max : longest) if (rows > 100000)
+    for (int r = 0; r < rows; ++r) longest = std::max(longest, rowPtr[r + 1] - rowPtr[r]);
+    offsets = offsets && longest <= mx::kOffsetsMost;
+    windows = windows && longest <= mx::kWindowLongest;
+    constexpr int looks = 5;
+    const int chunkRows = mx::offsets_chunk_rows(f64), nChunks = (int)(((long long)rows + chunkRows - 1) / chunkRows);
+    for (int i = 0; i < looks && offsets; ++i) {
+        const int c = (int)((long long)(nChunks - 1) * i / (looks - 1)), r1 = (int)std::min<long long>((c + 1ll) * chunkRows, rows);
+        int list[mx::kOffsetsMost], n = 0;  // ascending
+        for (int r = c * chunkRows; r < r1 && offsets; ++r)
+            for (int p = rowPtr[r]; p < rowPtr[r + 1] && offsets; ++p) {
+                int *at = std::lower_bound(list, list + n, col[p] - r);
+                if (at < list + n && *at == col[p] - r) continue;
+                if (n == mx::kOffsetsMost) {
+                    offsets = false;
+                    break;
+                }
+                std::copy_backward(at, list + n, list + n + 1);
+                *at = col[p] - r;
+                ++n;
+            }
+    }
+    if (offsets || !windows) return offsets;
+    const int wgRows = 64 * mx::kWindowWaves, nWG = (int)(((long long)rows + wgRows - 1) / wgRows), epv = 16 / mx::elem_size(dtype);
+    const int size = mx::window_bucket(cols, epv), widest = mx::window_widest(f64, nnz, nWG), wide = std::max(widest / size, 1);
+    if (size > widest) return false;
+    std::vector<int> before(mx::kWindowBuckets + 1);  // entries in the buckets in front
+    for (int i = 0; i < looks; ++i) {
+        const int w = (int)((long long)(nWG - 1) * i / (looks - 1)), p0 = rowPtr[w * wgRows], p1 = rowPtr[(int)std::min<long long>((w + 1ll) * wgRows, rows)];
+        std::fill(before.begin(), before.end(), 0);
+        for (int p = p0; p < p1; ++p) ++before[col[p] / size + 1];
+        int most = 0;
+        for (int b = 0; b < mx::kWindowBuckets; ++b) {
+            before[b + 1] += before[b];
+            most = std::max(most, before[b + 1] - before[std::max(b + 1 - wide, 0)]);
+        }
+        // (the device may leave ends of the window out, which only puts more entries outside)
+        if (mx::window_scattered(p1 - p0 - most, p1 - p0)) return false;
+    }
+    return true;
+}
+
 int mxp::try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took)
 {
     *took = false;
@@ -353,7 +405,7 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
     const int nnz = rowPtr[rows];
     const size_t es = (size_t)mx::elem_size(plan->dtype);
     plan->csr_nnz = nnz;
-    if (alone && may_look_for_form(flags)) {
+    if (alone && may_look_for_form(flags) && forms_may_suit(plan->dtype, rows, cols, rowPtr, col)) {
         // (the offset and window forms are found and laid out on the device, whatever MX_LAYOUT says)
         int *rp = nullptr, *ci = nullptr;
         void *va = nullptr;

@@ -261,6 +261,8 @@ CsrChoice choose_csr_form(mx_dtype dtype, int rows, int cols, const int *rowPtr,
 // Whether a plan that keeps no tiles may take a form that is looked for in the matrix itself (the offset and window forms): no flag
 // and nothing in the environment asks for another form or for a timed choice.
 bool may_look_for_form(int flags);
+// Whether it is worth sending a matrix up to look for them.
+bool forms_may_suit(mx_dtype dtype, int rows, int cols, const int *rowPtr, const int *col);
 // Tries the offset form, then the window form, on a CSR part in device memory; *took says whether the plan has its CSR part now.
 int try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took);
 int setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const void *val, int flags, const char *stripRows = nullptr,

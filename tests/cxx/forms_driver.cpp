@@ -1,9 +1,11 @@
 // How a plan looks for the forms of its CSR part that are made on the device (mxp::try_forms), with the two makers
 // replaced by what the check says.  No GPU call.  Run with the name of one check; exit status 0 means it holds.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <map>
 #include <string>
+#include <vector>
 
 #include "mx_plan_parts.h"
 
@@ -190,9 +192,57 @@ static void window_buckets()
         }
 }
 
+// What the host can tell of a matrix before it is sent up for the forms: never "no" to one that a form takes.
+static void host_look()
+{
+    struct Matrix {
+        int rows, cols;
+        std::vector<int> ptr{0}, col;
+        Matrix(int r, int c) : rows(r), cols(c) {}
+        void end_row() { ptr.push_back((int)col.size()); }
+        bool may(mx_dtype t) const { return mxp::forms_may_suit(t, rows, cols, ptr.data(), col.data()); }
+    };
+    unsigned seed = 1;
+    auto random = [&](int n) { return (int)((seed = seed * 1664525u + 1013904223u) >> 8) % n; };
+    auto uniform = [&](int rows, int cols, int per) {
+        Matrix A(rows, cols);
+        for (int r = 0; r < rows; ++r, A.end_row())
+            for (int k = 0; k < per; ++k) A.col.push_back(random(cols));
+        return A;
+    };
+    auto band = [&](int rows, int per, int half) {
+        Matrix A(rows, rows);
+        for (int r = 0; r < rows; ++r, A.end_row())
+            for (int k = 0; k < per; ++k) A.col.push_back(std::min(std::max(r + random(2 * half + 1) - half, 0), rows - 1));
+        return A;
+    };
+    auto diagonals = [&](int rows, int n) {
+        Matrix A(rows, rows);
+        for (int r = 0; r < rows; ++r, A.end_row())
+            for (int k = 0; k < n; ++k)
+                if (r + k - n / 2 >= 0 && r + k - n / 2 < rows) A.col.push_back(r + k - n / 2);
+        return A;
+    };
+    for (const mx_dtype t : {MX_F64, MX_F16}) {
+        CHECK(diagonals(5000, 64).may(t) && !diagonals(5000, 65).may(t) && diagonals(1024, 1).may(t) && !diagonals(1023, 1).may(t));
+        CHECK(band(40000, 20, 500).may(t) && band(40000, 20, 3000).may(t) && !band(30000, 20, 500).may(t));
+        CHECK(!uniform(4096, 4096, 16).may(t) && !uniform(65536, 65536, 16).may(t) && !uniform(40000, 300000, 30).may(t) && !uniform(2000, 50, 80).may(t));
+        Matrix far = band(40000, 20, 500);  // a few rows of another kind are no reason
+        for (int p = 0; p < 40000; p += 997) far.col[p] = random(40000);
+        CHECK(far.may(t));
+        Matrix longRow = band(40000, 20, 500);
+        for (int k = 0; k < 1025; ++k) longRow.col.push_back(k);
+        longRow.ptr.back() = (int)longRow.col.size();
+        CHECK(!longRow.may(t));
+        Matrix empty(50000, 50000);
+        for (int r = 0; r < 50000; ++r) empty.end_row();
+        CHECK(!empty.may(t));
+    }
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}, {"csr_blocks", csr_blocks}, {"strides", strides}, {"window_buckets", window_buckets}};
+    const std::map<std::string, void (*)()> checks = {{"no_memory", no_memory}, {"window_rule", window_rule}, {"keep_rule", keep_rule}, {"offset_waves", offset_waves}, {"offset_lists", offset_lists}, {"csr_blocks", csr_blocks}, {"strides", strides}, {"window_buckets", window_buckets}, {"host_look", host_look}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();

@@ -43,7 +43,7 @@ def forms(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["no_memory", "window_rule", "keep_rule", "offset_waves", "offset_lists", "csr_blocks", "strides", "window_buckets"])
+@pytest.mark.parametrize("check", ["no_memory", "window_rule", "keep_rule", "offset_waves", "offset_lists", "csr_blocks", "strides", "window_buckets", "host_look"])
 def test_forms_looked_for(forms, check):
     """tests/cxx/forms_driver.cpp, one check at a time."""
     r = subprocess.run([forms, check], capture_output=True, text=True, timeout=60)
