@@ -5,8 +5,8 @@
 #include <iterator>
 #include <map>
 #include <mutex>
+#include <new>
 #include <unordered_map>
-#include <vector>
 
 #include "mx_device.h"
 #include "mx_internal.h"
@@ -187,10 +187,16 @@ void trim(Pool &P, bool all)
             (void)hipFree(p);
         }
 }
-void put_idle(Pool &P, void *p, const Block &b)
+// (with the lock held) false where host memory has run out: the block goes back to the device then
+bool put_idle(Pool &P, void *p, const Block &b)
 {
-    P.idle[b.dev].emplace(b.bytes, Idle{p, P.calls});
+    try {
+        P.idle[b.dev].emplace(b.bytes, Idle{p, P.calls});
+    } catch (const std::bad_alloc &) {
+        return false;
+    }
     P.idleBytes[b.dev] += b.bytes;
+    return true;
 }
 // What the thread has given back inside its scope goes back to the device, the largest block first, until at most `keep` bytes
 // are left -- after a wait for the scope's stream; nothing does where that fails.
@@ -254,7 +260,7 @@ hipError_t dev_malloc(void **out, size_t bytes)
         (void)hipGetLastError();  // (a caller that goes on without the memory must not meet the error at its next launch)
         return e;
     }
-    std::lock_guard<std::mutex> hold(P.mu);
+    std::unique_lock<std::mutex> hold(P.mu);
     if (P.limit[dev] == 0) {
         size_t freeB = 0, total = 0;
         if (hipMemGetInfo(&freeB, &total) != hipSuccess) {
@@ -263,7 +269,13 @@ hipError_t dev_malloc(void **out, size_t bytes)
         }
         P.limit[dev] = std::max<size_t>(total / kPoolShare, 1);
     }
-    P.blocks[p] = Block{need, dev};
+    try {
+        P.blocks[p] = Block{need, dev};
+    } catch (const std::bad_alloc &) {
+        hold.unlock();
+        (void)hipFree(p);
+        return hipErrorOutOfMemory;
+    }
     *out = p;
     return hipSuccess;
 }
@@ -291,14 +303,24 @@ hipError_t dev_free(void *p)
         } else {
             b = it->second;
             scopeLimit = P.limit[b.dev] * (kPoolShare / kScopeShare);
+            bool kept = true;
             if (T.idleFrees > 0) {
-                put_idle(P, p, b);
-                return hipSuccess;
+                if (put_idle(P, p, b)) return hipSuccess;
+                kept = false;
+            } else {
+                try {
+                    T.freed.emplace(b.bytes, p);
+                } catch (const std::bad_alloc &) {
+                    kept = false;
+                }
+            }
+            if (!kept) {
+                P.blocks.erase(it);
+                b.bytes = 0;
             }
         }
     }
     if (b.bytes == 0) return hipFree(p);
-    T.freed.emplace(b.bytes, p);
     T.freedBytes += b.bytes;
     shrink_scope(P, T, scopeLimit);
     return hipSuccess;
@@ -319,23 +341,23 @@ MemScope::~MemScope()
     if (--T.depth > 0) return;
     const bool idle = T.freed.empty() || hipStreamSynchronize(T.stream) == hipSuccess;
     Pool &P = pool();
-    std::vector<void *> out;
     {
         std::lock_guard<std::mutex> hold(P.mu);
         ++P.calls;
-        for (auto &f : T.freed) {
+    }
+    for (auto &f : T.freed) {
+        {
+            std::lock_guard<std::mutex> hold(P.mu);
             auto it = P.blocks.find(f.second);
-            if (idle && it != P.blocks.end()) {
-                put_idle(P, f.second, it->second);
-            } else {
-                if (it != P.blocks.end()) P.blocks.erase(it);
-                out.push_back(f.second);
+            if (it != P.blocks.end()) {
+                if (idle && put_idle(P, f.second, it->second)) continue;
+                P.blocks.erase(it);
             }
         }
+        (void)hipFree(f.second);
     }
     T.freed.clear();
     T.freedBytes = 0;
-    for (void *p : out) (void)hipFree(p);
     trim(P, false);
 }
 

@@ -7,6 +7,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -45,9 +46,28 @@ void *take(size_t bytes)
 
 }  // namespace
 
+// (of the library only: the device's own bookkeeping does not count)
+static thread_local long allocations_left = -1, own_business = 0;
+void *operator new(size_t n)
+{
+    if (allocations_left >= 0 && own_business == 0 && allocations_left-- == 0) {
+        allocations_left = 0;
+        throw std::bad_alloc();
+    }
+    if (void *p = std::malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+struct OwnBusiness {
+    OwnBusiness() { ++own_business; }
+    ~OwnBusiness() { --own_business; }
+};
+
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n)
 {
+    OwnBusiness own;
     std::lock_guard<std::mutex> hold(device.mu);
     if (device.used + n > device.total) return device.last = hipErrorOutOfMemory;
     *p = (void *)device.next;
@@ -187,9 +207,31 @@ static void one_stream()
     }
 }
 
+// Host memory that runs out is an error of the allocation, or sends a block back to the device; nothing is thrown through
+// the library's C entry points or out of a destructor, and nothing is lost.
+static void host_memory()
+{
+    for (int after = 0; after < 12; ++after) {
+        void *p = nullptr, *q = take(GB), *r = take(2 * GB);
+        allocations_left = after;
+        {
+            mx::MemScope scope(nullptr);
+            const hipError_t e = mx::dev_malloc(&p, 3 * GB);
+            CHECK((e == hipSuccess) == (p != nullptr));
+            CHECK(mx::dev_free(q) == hipSuccess);
+            CHECK(mx::dev_free(p) == hipSuccess);
+        }
+        CHECK(mx::dev_free(r) == hipSuccess);
+        allocations_left = -1;
+        CHECK(device.used <= device.total / 128);
+        mx::release_idle_memory();
+        CHECK(device.used == 0 && device.blocks.empty());
+    }
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}, {"bound", bound}, {"age", age}, {"scope_full", scope_full}, {"scope_share", scope_share}, {"one_stream", one_stream}};
+    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}, {"bound", bound}, {"age", age}, {"scope_full", scope_full}, {"scope_share", scope_share}, {"one_stream", one_stream}, {"host_memory", host_memory}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();

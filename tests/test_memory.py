@@ -21,7 +21,7 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["wait_refused", "bound", "age", "scope_full", "scope_share", "one_stream"])
+@pytest.mark.parametrize("check", ["wait_refused", "bound", "age", "scope_full", "scope_share", "one_stream", "host_memory"])
 def test_memory_kept_between_calls(driver, check):
     """tests/cxx/memory_driver.cpp, one check at a time."""
     r = subprocess.run([driver, check], capture_output=True, text=True, timeout=60)
