@@ -1,4 +1,5 @@
-"""The device memory that the library keeps between calls, on a device that exists only in the test (no GPU)."""
+"""The device memory that the library keeps between calls, on a device that exists only in the test, and the rules by which a plan
+takes the forms that are made on the device (no GPU)."""
 import os
 import shutil
 import subprocess
