@@ -216,7 +216,7 @@ inline int slice_step_entries(mx_dtype) { return 1; }  // entries a lane takes p
 constexpr int kSliceLightSegs = 8;     // rows with at most this many virtual rows are summed by one lane
 
 // The CSR part of a matrix whose rows repeat a pattern of column offsets (a stencil, a few diagonals):
-// chunks of 64 * R consecutive rows (R = 2 binary64, 4 binary16), one per wave, each with the ascending
+// chunks of 64 * R consecutive rows (R = 2 binary64, 4 binary16), each of them one to four waves' (offsets_waves), with the ascending
 // list of the offsets (column - row) that its rows have.  Per chunk and unit -- unitBytes per lane, one
 // contiguous stretch per wave -- the values of U offsets for the R rows of every lane; a place that no
 // entry owns holds -0.0 (any binary64 whose upper half is 0x80000000) or code 255.
@@ -304,39 +304,48 @@ constexpr int kWindowWaves = 8;               // chunks (and waves) of a workgro
 constexpr int kWindowRowsLeast = 32768;       // fewest rows of a matrix that takes the form (33 thousand of 40 entries, binary16: 4.3 us, row tiles 5.3)
 constexpr int kWindowEntriesLeast = 600000;   // binary64: fewest entries (0.33 million: 4.0 us, row tiles 3.8; 0.9 million: 4.2, 4.7)
 constexpr double kWindowFill = 1.5;           // most bytes stored per byte of the entries
-// Fewest entries a row on average: a wave waits for its window whatever it has to add, and with two units a row that is most of its
-// time (binary64, 6 a row: 260 thousand rows 7.1 us, row tiles 5.5; 1.5 million 42, slices 29.5).  In binary16 a row has fewer bytes:
-// over a million rows more of them are needed (2.2 million of 11.5: 34.5, slices 28.3; 3.2 million of 7: 37, 29; 1.5 million of 14: 19.5, 22.8), and
-// few rows beat row tiles and slices with less (130 thousand of 6: 2.9, 4.0; 260 thousand 3.5, 4.6; 600 thousand 7.3, 7.9 back to back and 9.0, 8.4
-// in a rotation of three).
-constexpr int kWindowMean = 8, kWindowMeanFewRows = 4, kWindowFewRows = 300000, kWindowMeanManyRows = 13, kWindowManyRows = 1000000;
-inline bool window_mean_ok(bool f64, int rows, int nnz)
-{
-    const int least = f64 ? kWindowMean : rows <= kWindowFewRows ? kWindowMeanFewRows : rows <= kWindowManyRows ? kWindowMean : kWindowMeanManyRows;
-    return (long long)nnz >= (long long)rows * least;
-}
+constexpr int kWindowMeanLeast = 4;           // fewest entries a row on average
 inline bool window_size_ok(bool f64, int rows, int cols, int nnz)
 {
-    return forms_can_number(rows, cols, nnz) && rows >= kWindowRowsLeast && cols >= 64 && window_mean_ok(f64, rows, nnz) && nnz <= 1500000000 &&
+    return forms_can_number(rows, cols, nnz) && rows >= kWindowRowsLeast && cols >= 64 && (long long)nnz >= (long long)rows * kWindowMeanLeast && nnz <= 1500000000 &&
            !(f64 && nnz < kWindowEntriesLeast);
 }
-// Whether a matrix laid out in `stored` bytes by nWG workgroups is better off in this form than in slices (or row tiles).  The
-// one launch saves about 4 us, some 18 MB's worth; padding beyond that (rows of uneven length) costs more than it
-// (binary64, 600 thousand rows of 28 to 52 entries, 314 MB instead of 238: 55 us, slices 48; of 34 to 46, 290 MB: 48.6, 48.1).
-// Slices spread any matrix over all CUs, a window's rows stay with one, which takes in 50 to 80 bytes a nanosecond
-// (33 thousand rows of 300, 65 workgroups of 1.5 MB, binary64: 20 to 44 us, slices 20; binary16, 0.6 MB: 11 to 14.8, one-launch slices 11.2 to 12;
-// 66 thousand rows of 300, 129 workgroups: binary16, 0.6 MB, 13.8, slices 18.5, binary64, 1.5 MB, 36.5, 34.6).  Among the smallest
-// binary64 matrices row tiles are close (33 thousand rows of 40: 5.1 at a fill of 1.06, 5.9 at 1.36, row tiles 5.5).
-// Over 296 bands of 33 thousand to 3.2 million rows and 4 to 300 entries a row that pass the limits above, the form was more than 3 % slower than the one
-// before it 80 times, at worst 2.2 times as slow; none of the 184 that this lets through was.
-inline bool window_form_pays(bool f64, int nnz, double stored, int nWG, int nCU)
+// What a product may touch for its units to be read with plain loads.  Plain / streaming loads, us, back to back | three plans in
+// turn: binary16, 51 MB 11.3 / 12.0 | 11.2 / 12.6; 76 MB 14.2 / 14.2 | 14.2 / 14.9; 99 MB 16.7 / 16.2 | 18.6 / 17.2; 108 MB 18.9 / 21.7 | 23.1 /
+// 22.7; 126 MB 19.5 / 19.1 | 23.3 / 20.3; binary64, 79 MB 14.7 / 15.7 | 14.8 / 16.7; 100 MB 16.5 / 17.6 | 18.4 / 18.6; 120 MB 18.8 / 19.2 | 23.3 / 20.0;
+// 132 MB 20.5 / 21.2 | 25.1 / 22.6.  Beyond 110 MB that is a trade, and against the slices these matrices had before plain loads come out
+// ahead (127 MB, binary16: 1.5 million rows of 16, plain 22.9 | 29.7, streaming 26.8 | 27.2, slices 25.1 | 29.6; 600 thousand of 40, 20.3 | 25.9,
+// 23.4 | 24.3, 22.2 | 25.4).
+constexpr long long kWindowKeepBytes = 128LL << 20;
+// Estimated time of a product in this form, us: the launch, a wait for the window per round of workgroups over the CUs, and the stored
+// bytes, which come from the L2s, the memory-side cache (`touched` bytes have to fit) or memory -- or what one workgroup's CU takes in, 45 to 80
+// bytes a nanosecond, where there are few workgroups.  (Least squares over 647 bands of 33 thousand to 3.2 million rows of 4 to 300 entries, on
+// average 7 % off in binary64, 8 in binary16.)
+inline double window_estimate(bool f64, double stored, double touched, int nWG, int nCU)
 {
-    const double entries = (double)nnz * (f64 ? 10 : 4);
-    if (stored > kWindowFill * entries + 65536 || stored > 1.1 * entries + 18e6) return false;
-    if (f64 && nnz < 1300000 && stored > 1.3 * entries) return false;
-    const double most = f64 ? 0.8e6 : nWG * 8 < nCU * 3 ? 0.3e6 : 0.7e6;  // of a workgroup, where there are fewer than CUs
-    return nWG * 16 >= nCU * 15 || stored <= most * nWG;
+    const double MB = stored * 1e-6, own = MB / nWG * 1e3, rounds = (nWG + nCU - 1) / nCU, beyond = std::max(0.0, MB - 30.0);  // (own: KB of a workgroup)
+    if (touched <= (double)kWindowKeepBytes)
+        return f64 ? std::max(2.22 - 0.00146 * nWG + 1.3 * rounds + 0.084 * MB + 0.049 * beyond, 2.2 + own / 78)
+                   : std::max(2.06 - 0.00044 * nWG + 0.93 * rounds + 0.064 * MB + 0.109 * beyond, 2.2 + own / 58);
+    return f64 ? std::max(-2.59 + 0.00669 * nWG + 0.156 * MB, 2.2 + own / 44) : std::max(-1.65 + 0.0032 * nWG + 0.159 * MB, 2.2 + own / 45);
 }
+// Whether a matrix laid out in `stored` bytes by nWG workgroups is better off in this form than in the one it would have otherwise, which
+// takes `other` us (other_forms_us).  Of the 647 bands the form was more than 3 % slower than the one before it 100 times, at worst 2.2 times
+// as slow (33 thousand rows of 150 to 450 entries, binary64, 65 workgroups: 43.7 us, slices 20.2; 600 thousand of 28 to 52: 55, 48; 1.5
+// million of 6: 42, 29.5; 3.2 million of 9, binary16: 49, 33); where this takes it (508 of them), 5 times, by 0.25 us at most (80 thousand rows of 8, binary64:
+// 4.0, row tiles 3.8).  Few workgroups with more than so many bytes each also fall behind once the matrix shares the caches with
+// anything else (33 thousand rows of 300, binary64, 95 MB, three plans in turn: 31 us, slices 21), and in binary16 small matrices have the one-launch
+// slices (33 thousand of 300: 11.8 to 14.8, 11.2 to 11.5).
+inline bool window_form_pays(bool f64, int nnz, double stored, double touched, int nWG, int nCU, double other)
+{
+    if (stored > kWindowFill * (double)nnz * (f64 ? 10 : 4) + 65536) return false;
+    const double most = f64 ? 0.8e6 : nWG * 8 < nCU * 3 ? 0.3e6 : 0.7e6;
+    if (nWG * 16 < nCU * 15 && stored > most * nWG) return false;
+    return window_estimate(f64, stored, touched, nWG, nCU) <= other;
+}
+// What the row tiles or the slices of a matrix take whose neighbouring rows reach into one stretch of x, by csr_estimates: the estimate of
+// the one the plan would choose, brought to what these matrices were measured at (mx_plan.cpp).
+double other_forms_us(mx_dtype dtype, int rows, int cols, int nnz, double linesPerGather);
 constexpr double kWindowFarMost = 0.12;       // most entries outside the windows, of all
 constexpr int kWindowFarSteps = 3;            // most entries of a row outside the window, but for chunks apart
 constexpr int kWindowTrim = 32;               // bytes that a far entry is worth: an end of the window with fewer entries is left out
@@ -356,13 +365,6 @@ __host__ __device__ inline int window_bucket(int cols, int epv) { return ((cols 
 // Whether a workgroup with `outside` of its n entries outside its window is one of a matrix of another kind.
 __host__ __device__ inline bool window_scattered(int outside, int n) { return (long long)outside * 4 > (long long)n * 3 + 256; }
 constexpr int window_unit_bytes(bool f64) { return 64 * kWindowUnit * (f64 ? 10 : 4); }
-// What a product may touch for its units to be read with plain loads.  Plain / streaming loads, us, back to back | three plans in
-// turn: binary16, 51 MB 11.3 / 12.0 | 11.2 / 12.6; 76 MB 14.2 / 14.2 | 14.2 / 14.9; 99 MB 16.7 / 16.2 | 18.6 / 17.2; 108 MB 18.9 / 21.7 | 23.1 /
-// 22.7; 126 MB 19.5 / 19.1 | 23.3 / 20.3; binary64, 79 MB 14.7 / 15.7 | 14.8 / 16.7; 100 MB 16.5 / 17.6 | 18.4 / 18.6; 120 MB 18.8 / 19.2 | 23.3 / 20.0;
-// 132 MB 20.5 / 21.2 | 25.1 / 22.6.  Beyond 110 MB that is a trade, and against the slices these matrices had before plain loads come out
-// ahead (127 MB, binary16: 1.5 million rows of 16, plain 22.9 | 29.7, streaming 26.8 | 27.2, slices 25.1 | 29.6; 600 thousand of 40, 20.3 | 25.9,
-// 23.4 | 24.3, 22.2 | 25.4).
-constexpr long long kWindowKeepBytes = 128LL << 20;
 void free_windows(DeviceWindows &D);
 // As build_offsets_device and launch_offsets.
 __attribute__((weak)) int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev,

@@ -178,6 +178,20 @@ void mxp::csr_estimates(mx_dtype dtype, int cols, int nnz, const CsrStats &st, d
     *usSlices = 9.5 + bytes / (bytes <= 64.0e6 ? 9.0e6 : 5.8e6) + 2.0e-6 * st.vrows;
 }
 
+// (Least squares over 647 bands: row tiles 5 % off on average, slices 13 % in binary64 and 8 in binary16.  Row tiles are asked to be beaten by
+// a little more the longer they take; on the smallest matrices both forms are within a few tenths of a microsecond.)
+double mx::other_forms_us(mx_dtype dtype, int rows, int cols, int nnz, double linesPerGather)
+{
+    CsrStats st;
+    st.linesPerGather = linesPerGather;
+    st.vrows = rows;  // (a row rarely leaves its slice)
+    double usRows = 0.0, usSlices = 0.0;
+    csr_estimates(dtype, cols, nnz, st, &usRows, &usSlices);
+    const double M = 1e-6 * nnz, R = 1e-6 * rows;
+    if (usSlices <= usRows) return dtype == MX_F64 ? 1.6 + 0.81 * usSlices : 2.17 + 0.78 * usSlices;
+    return dtype == MX_F64 ? 0.6 + 0.88 * (2.49 + 0.176 * (usRows - 2.5) + 1.83 * M - 2.67 * R) : 0.95 * (3.5 + 0.14 * (usRows - 2.5) + 1.02 * M - 0.53 * R);
+}
+
 bool mxp::plan_autotune()
 {
     return mx::opt().autotune;
@@ -384,8 +398,9 @@ int mxp::try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *col
     return MX_OK;
 }
 
-// Puts the CSR part on the device.  Three executable forms exist: row tiles with direct x
-// gathers; column slices with x resident in LDS; and a split in which the long rows (most of
+// Puts the CSR part on the device.  A matrix whose rows repeat a pattern of offsets, or reach into one window of x, takes
+// the form made for that (try_forms) where no tiles are kept beside it and nothing asks for another.  Three executable
+// forms exist for any matrix: row tiles with direct x gathers; column slices with x resident in LDS; and a split in which the long rows (most of
 // the entries of a matrix with a heavy tail of row lengths) take the slices and the many short
 // ones the row tiles.  Unless a flag or MX_CSR_KERNEL=rows|slices|split forces one, the choice
 // between the first two is made from counts over the matrix (csr_stats, csr_estimates): the form

@@ -458,7 +458,11 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
         int dev = 0, nCU = 0;
         MXW_TRY(hipGetDevice(&dev));
         MXW_TRY(hipDeviceGetAttribute(&nCU, hipDeviceAttributeMultiprocessorCount, dev));
-        if (h[0] || h[1] <= 0 || h[4] > kWindowFarMost * (double)nnz || !window_form_pays(f64, nnz, stored, nWG, nCU)) return fail(MX_OK);
+        if (h[0] || h[1] <= 0 || h[4] > kWindowFarMost * (double)nnz) return fail(MX_OK);
+        double lines = 1.0;
+        if (const int rc = lines_per_gather_device(dtype, nnz, col_dev, s, &lines)) return rc;
+        if (!window_form_pays(f64, nnz, stored, stored + ((double)rows + cols) * es, nWG, nCU, other_forms_us(dtype, rows, cols, nnz, lines)))
+            return fail(MX_OK);
         if (f64 && nnz >= 65536 && mx::opt().csr_dict != 0) {
             // few distinct binary64 values: slices with a byte a value move a third of what this form would
             void *codes = nullptr;

@@ -71,32 +71,35 @@ static void no_memory()
     }
 }
 
-// The window form where it was measured to be faster than slices or row tiles, and not where it was slower.
+// The window form where it was measured to be faster than slices or row tiles, and not where it was slower.  `lines`: of x, per gather of
+// 64 entries, as such a band has them.
 static void window_rule()
 {
     const struct {
         bool f64;
         int rows, nnz;
         double stored;  // MB
+        double lines;
         bool pays;
     } cases[] = {
         // (faster)
-        {true, 66000, 2640000, 26.5, true},    {true, 33000, 3300000, 32.5, true},   {true, 130000, 39000000, 385.9, true},
-        {true, 260000, 26000000, 299.9, true}, {true, 600000, 9600000, 123.6, true}, {true, 130000, 2080000, 30.0, true},
-        {false, 250007, 10000280, 42.0, true}, {false, 130000, 780000, 4.3, true},   {false, 66000, 19800000, 77.4, true},
-        {false, 600000, 23844517, 115.4, true}, {false, 1000000, 8000000, 33.0, true}, {false, 1500000, 23940000, 97.4, true}, {false, 1500000, 20990000, 96.0, true},
+        {true, 66000, 2640000, 26.5, 55, true},     {true, 33000, 3300000, 32.5, 55, true},     {true, 130000, 39000000, 385.9, 60, true},
+        {true, 600000, 9600000, 99.7, 50, true},    {true, 600000, 4788000, 50.0, 50, true},    {true, 260000, 10400000, 105.5, 60, true},
+        {false, 250007, 10000280, 42.0, 55, true},  {false, 130000, 780000, 4.3, 25, true},     {false, 66000, 6600000, 26.2, 60, true},
+        {false, 600000, 23844517, 115.4, 50, true}, {false, 1500000, 23940000, 97.4, 45, true}, {false, 400000, 3188000, 13.0, 45, true},
         // (slower)
-        {true, 33000, 9228706, 136.4, false},   {true, 33000, 9253352, 95.6, false},   {true, 66000, 18793119, 193.7, false},
-        {true, 600000, 23840358, 314.4, false}, {true, 260000, 1549859, 21.1, false},  {true, 1500000, 8943723, 122.5, false},
-        {true, 800000, 9168242, 128.0, false},  {true, 33000, 1252319, 17.1, false},   {true, 260000, 25561141, 383.1, false},
-        {false, 33000, 8628000, 51.6, false},   {false, 3200000, 28679476, 156.0, false}, {false, 3200000, 22330908, 104.0, false},
-        {false, 130000, 37423087, 222.9, false}, {false, 1500000, 8943930, 48.9, false}, {false, 40000, 7568075, 33.9, false},
-        {false, 2200000, 19719164, 107.0, false}, {true, 800000, 6962243, 97.0, false},
+        {true, 33000, 9228706, 136.4, 60, false},   {true, 66000, 18793119, 193.7, 60, false},  {true, 600000, 23840358, 314.4, 58, false},
+        {true, 260000, 1549859, 21.1, 36, false},   {true, 1500000, 8943723, 122.5, 40, false}, {true, 400000, 2376000, 33.0, 28, false},
+        {true, 260000, 25561141, 383.1, 60, false}, {false, 33000, 8628000, 51.6, 60, false},   {false, 3200000, 28679476, 156.0, 40, false},
+        {false, 3200000, 22330908, 104.0, 40, false}, {false, 130000, 37423087, 222.9, 60, false},
     };
     for (const auto &c : cases) {
         const int nWG = ((c.rows + 63) / 64 + mx::kWindowWaves - 1) / mx::kWindowWaves;
-        const bool pays = mx::window_mean_ok(c.f64, c.rows, c.nnz) && mx::window_form_pays(c.f64, c.nnz, c.stored * 1e6, nWG, 256);
-        if (pays != c.pays) std::printf("binary%d, %d rows, %d entries, %.1f MB\n", c.f64 ? 64 : 16, c.rows, c.nnz, c.stored);
+        const double other = mx::other_forms_us(c.f64 ? MX_F64 : MX_F16, c.rows, c.rows, c.nnz, c.lines), touched = c.stored * 1e6 + 2.0 * c.rows * (c.f64 ? 8 : 2);
+        const bool pays = mx::window_form_pays(c.f64, c.nnz, c.stored * 1e6, touched, nWG, 256, other);
+        if (pays != c.pays)
+            std::printf("binary%d, %d rows, %d entries, %.1f MB: %.1f us, otherwise %.1f\n", c.f64 ? 64 : 16, c.rows, c.nnz, c.stored,
+                        mx::window_estimate(c.f64, c.stored * 1e6, touched, nWG, 256), other);
         CHECK(pays == c.pays);
     }
 }
