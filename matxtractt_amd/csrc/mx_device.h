@@ -259,12 +259,14 @@ constexpr int offsets_unit_bytes(bool dict) { return dict ? 8 : 16; }
 // (one / two / four waves, us, binary64, 27 offsets: 22 thousand rows 6.3 / 4.2 / 3.2; 717 thousand 33.1 / 31.2 / 28.6; 1.2 million
 // 52.9 / 51.3 / 48.3).  One where a chunk's list is a single round of a wave: the others would have nothing to ask for, and the
 // workgroups, which start at about one a nanosecond, are four times as many (1.5 million rows, binary64: one offset 6.7 / 8.5 / 12.4, three 10.3
-// / 11.6 / 17.0, eight 18.7 / 18.2 / 20.3, fourteen 35.8 / 32.7 / 30.9; binary16: two 3.7 / 4.1 / 5.5, eight 5.3 / 5.3 / 7.7; row tiles of the first two: 7.3, 14.4).
+// / 11.6 / 17.0, eight 18.7 / 18.2 / 20.3, fourteen 35.8 / 32.7 / 30.9; binary16: two 3.7 / 4.1 / 5.5, eight 5.3 / 5.3 / 7.7; row tiles of the first two: 7.3, 14.4); with more
+// than four offsets from the size on where the workgroups outweigh what four waves ask for sooner (four waves / one: binary16, eight offsets, 25 to 180 thousand rows 2.9 / 3.1 to
+// 3.2, 240 thousand 3.1 / 3.3, 358 thousand 3.55 / 3.5, 717 thousand 4.8 / 3.8; binary64, 90 thousand 3.0 / 3.0, 120 thousand 3.3 / 3.1).
 // With one byte per binary64 value the kernel is bound by what a wave computes and the sum of the parts costs more than
 // it gives from about two thousand chunks on (290 thousand rows 6.5 / 6.1 / 6.4, 717 thousand 10.9 / 10.5 / 11.7, a million 13.1 / 13.7 / 14.8).
 inline int offsets_waves(bool f64, bool dict, long long nOffs, int nChunks)
 {
-    if (nOffs <= 8ll * nChunks) return 1;
+    if (nOffs <= (nChunks < 1024 ? 4ll : 8ll) * nChunks) return 1;
     return f64 && dict && nChunks >= 2048 ? 2 : 4;
 }
 // Workgroups of a product: four waves each.

@@ -133,6 +133,8 @@ static void offset_waves()
     CHECK(mx::offsets_waves(true, true, 8 * 11719, 11719) == 1 && mx::offsets_waves(true, true, 12 * 300, 300) == 4);
     CHECK(mx::offsets_waves(false, false, 8 * 5860, 5860) == 1 && mx::offsets_waves(false, true, 28 * 5860, 5860) == 4);
     CHECK(mx::offsets_waves(true, false, 8ll << 28, 1 << 28) == 1);
+    CHECK(mx::offsets_waves(false, false, 8 * 470, 470) == 4 && mx::offsets_waves(true, true, 8 * 235, 235) == 4);
+    CHECK(mx::offsets_waves(false, false, 4 * 470, 470) == 1 && mx::offsets_waves(true, false, 8 * 1400, 1400) == 1);
 }
 
 // Long lists on small matrices, where row tiles were measured to be the faster ones.
