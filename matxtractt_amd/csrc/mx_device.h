@@ -433,9 +433,11 @@ int value_dict_device(mx_dtype dtype, const void *val_dev, int nnz, int most, vo
 
 // For plans made from a matrix that lives in device memory: the caller's arrays looked at before
 // they are used as addresses; the mean number of distinct lines of x per wave-wide gather (sampled
-// as on the host); the row-tile form from device arrays (`desc` = pack_rows of the row pointers).
+// as on the host; launch_lines_per_gather adds the lines of at most some 2 * `most` sampled windows to *sum and waits for
+// nothing); the row-tile form from device arrays (`desc` = pack_rows of the row pointers).
 int check_csr_device(int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev, hipStream_t s, const char *who);
 int lines_per_gather_device(mx_dtype dtype, int nnz, const int *col_dev, hipStream_t s, double *out);
+hipError_t launch_lines_per_gather(mx_dtype dtype, int nnz, const int *col_dev, int most, unsigned long long *sum, long long *sampled, hipStream_t s);
 int upload_csr_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev, const void *val_dev,
                       const std::vector<int> &desc, bool scan, DeviceCsr &A, hipStream_t s);
 

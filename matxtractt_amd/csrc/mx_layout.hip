@@ -938,18 +938,26 @@ int check_csr_device(int rows, int cols, int nnz, const int *rowPtr_dev, const i
     return MX_OK;
 }
 
+hipError_t launch_lines_per_gather(mx_dtype dtype, int nnz, const int *col_dev, int most, unsigned long long *sum, long long *sampled, hipStream_t s)
+{
+    using namespace mxl;
+    const long long windows = nnz / 64, stride = std::max<long long>(1, windows / most);
+    *sampled = windows / stride;
+    if (*sampled <= 0) return hipSuccess;
+    hipLaunchKernelGGL(window_lines_kernel, dim3((unsigned)std::min<long long>(kLinesBlocks, (*sampled + 3) / 4)), dim3(kBlock), 0, s, col_dev, *sampled, stride, 64 / elem_size(dtype),
+                       sum);
+    return hipGetLastError();
+}
 int lines_per_gather_device(mx_dtype dtype, int nnz, const int *col_dev, hipStream_t s, double *out)
 {
     using namespace mxl;
-    const long long windows = nnz / 64, stride = std::max<long long>(1, windows / 65536), sampled = windows / stride;
     *out = 1.0;
-    if (sampled <= 0) return MX_OK;
+    if (nnz < 64) return MX_OK;
     Buf sum;
     MXL_TRY(mx::dev_malloc(&sum.p, 256));
     MXL_TRY(hipMemsetAsync(sum.p, 0, 256, s));
-    hipLaunchKernelGGL(window_lines_kernel, dim3((unsigned)std::min<long long>(kLinesBlocks, (sampled + 3) / 4)), dim3(kBlock), 0, s, col_dev, sampled, stride, 64 / elem_size(dtype),
-                       sum.as<unsigned long long>());
-    MXL_TRY(hipGetLastError());
+    long long sampled = 0;
+    MXL_TRY(launch_lines_per_gather(dtype, nnz, col_dev, 65536, sum.as<unsigned long long>(), &sampled, s));
     unsigned long long h = 0;
     MXL_TRY(hipMemcpyAsync(&h, sum.p, 8, hipMemcpyDeviceToHost, s));
     MXL_TRY(hipStreamSynchronize(s));

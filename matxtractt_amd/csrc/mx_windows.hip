@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdint>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -423,17 +424,16 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     if (!window_size_ok(f64, rows, cols, nnz)) return MX_OK;
     const int nChunks = (rows + 63) / 64, waves = kWindowWaves, nWG = (nChunks + waves - 1) / waves;
     const int widest = window_widest(f64, nnz, nWG);
-    Buf units, farSteps, alone, unit0, far0, apart0, totals, tmp;
+    Buf counts, unit0, far0, apart0, tmp;
     size_t scanBytes = 0;
-    const size_t chunkB = ((size_t)nChunks + 1) * 4;
+    const size_t chunkB = ((size_t)nChunks + 1) * 4, countB = (chunkB + 255) & ~(size_t)255;
     MXW_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, (size_t)nChunks + 1, rocprim::plus<int>(), s));
-    MXW_TRY(mx::dev_malloc(&units.p, chunkB));
-    MXW_TRY(mx::dev_malloc(&farSteps.p, chunkB));
-    MXW_TRY(mx::dev_malloc(&alone.p, chunkB));
+    MXW_TRY(mx::dev_malloc(&counts.p, 256 + 3 * countB));  // (cleared together: 10 us for each of them apart)
+    int *const tot = (int *)counts.p, *const units = (int *)((char *)counts.p + 256), *const farSteps = (int *)((char *)units + countB),
+               *const alone = (int *)((char *)farSteps + countB);
     MXW_TRY(mx::dev_malloc(&unit0.p, chunkB));
     MXW_TRY(mx::dev_malloc(&far0.p, chunkB));
     MXW_TRY(mx::dev_malloc(&apart0.p, chunkB));
-    MXW_TRY(mx::dev_malloc(&totals.p, 256));
     MXW_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
     auto fail = [&](int code) {
         free_windows(D);
@@ -441,26 +441,26 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     };
     auto body = [&]() -> int {
         MXW_TRY(mx::dev_malloc((void **)&D.window, (size_t)nWG * 8));
-        MXW_TRY(hipMemsetAsync(totals.p, 0, 256, s));
-        MXW_TRY(hipMemsetAsync(units.p, 0, chunkB, s));
-        MXW_TRY(hipMemsetAsync(farSteps.p, 0, chunkB, s));
-        MXW_TRY(hipMemsetAsync(alone.p, 0, chunkB, s));
-        int *tot = (int *)totals.p;
+        MXW_TRY(hipMemsetAsync(counts.p, 0, 256 + 3 * countB, s));
         hipLaunchKernelGGL(window_rows_kernel, dim3((unsigned)(((long long)rows + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, rowPtr_dev, rows, tot);
         MXW_TRY(hipGetLastError());
         hipLaunchKernelGGL(window_find_kernel, dim3(nWG), dim3(kBlock), 0, s, rowPtr_dev, col_dev, rows, cols, nChunks, waves, epv, widest,
-                           (int2 *)D.window, (int *)units.p, (int *)farSteps.p, (int *)alone.p, tot);
+                           (int2 *)D.window, units, farSteps, alone, tot);
         MXW_TRY(hipGetLastError());
-        int h[6] = {0, 0, 0, 0, 0, 0};
-        MXW_TRY(hipMemcpyAsync(h, totals.p, sizeof(h), hipMemcpyDeviceToHost, s));
-        MXW_TRY(hipStreamSynchronize(s));
-        const double stored = (double)h[1] * window_unit_bytes(f64) + (double)h[2] * 64 * (4 + es);
+        // (for the estimate below, before anything is waited for; from 8192 windows instead of a thousand: 30 us)
+        long long sampled = 0;
+        MXW_TRY(launch_lines_per_gather(dtype, nnz, col_dev, 1024, (unsigned long long *)(tot + 8), &sampled, s));
         int dev = 0, nCU = 0;
         MXW_TRY(hipGetDevice(&dev));
         MXW_TRY(hipDeviceGetAttribute(&nCU, hipDeviceAttributeMultiprocessorCount, dev));
+        int h[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        MXW_TRY(hipMemcpyAsync(h, tot, sizeof(h), hipMemcpyDeviceToHost, s));
+        MXW_TRY(hipStreamSynchronize(s));
+        const double stored = (double)h[1] * window_unit_bytes(f64) + (double)h[2] * 64 * (4 + es);
         if (h[0] || h[1] <= 0 || h[4] > kWindowFarMost * (double)nnz) return fail(MX_OK);
-        double lines = 1.0;
-        if (const int rc = lines_per_gather_device(dtype, nnz, col_dev, s, &lines)) return rc;
+        unsigned long long lineSum = 0;
+        std::memcpy(&lineSum, h + 8, 8);
+        const double lines = sampled > 0 ? (double)lineSum / (double)sampled : 1.0;
         if (!window_form_pays(f64, nnz, stored, stored + ((double)rows + cols) * es, nWG, nCU, other_forms_us(dtype, rows, cols, nnz, lines)))
             return fail(MX_OK);
         if (f64 && nnz >= 65536 && mx::opt().csr_dict != 0) {
@@ -490,9 +490,9 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
         MXW_TRY(mx::dev_malloc(&D.farVal, ((size_t)D.farSteps + 1) * 64 * es));
         MXW_TRY(mx::dev_malloc((void **)&D.apart, ((size_t)D.nApart + 1) * 4));
         MXW_TRY(hipMemsetAsync(D.farCol + (size_t)D.farSteps * 64, 0xff, 64 * 4, s));  // the spare step: no entries
-        MXW_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)units.p, (int *)unit0.p, 0, (size_t)nChunks + 1, rocprim::plus<int>(), s));
-        MXW_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)farSteps.p, (int *)far0.p, 0, (size_t)nChunks + 1, rocprim::plus<int>(), s));
-        MXW_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)alone.p, (int *)apart0.p, 0, (size_t)nChunks + 1, rocprim::plus<int>(), s));
+        MXW_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)units, (int *)unit0.p, 0, (size_t)nChunks + 1, rocprim::plus<int>(), s));
+        MXW_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)farSteps, (int *)far0.p, 0, (size_t)nChunks + 1, rocprim::plus<int>(), s));
+        MXW_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)alone, (int *)apart0.p, 0, (size_t)nChunks + 1, rocprim::plus<int>(), s));
         const dim3 grid((unsigned)((nChunks + kBlock / 64 - 1) / (kBlock / 64)));
         const int *U0 = (const int *)unit0.p, *F0 = (const int *)far0.p, *A0 = (const int *)apart0.p;
         if (f64)
