@@ -12,19 +12,23 @@ constexpr int kPer = 4;                  // entries per thread
 constexpr int kTile = kBlock * kPer;     // entries per workgroup
 inline dim3 tile_grid(long long n) { return dim3((unsigned)((std::max<long long>(n, 1) + kTile - 1) / kTile)); }
 
-struct TileRows {
-    int row[kTile];
-    int top[kBlock / 64];
+template <int THREADS, int PER>
+struct TileRowsOf {
+    int row[THREADS * PER];
+    int top[THREADS / 64];
 };
+using TileRows = TileRowsOf<kBlock, kPer>;
 
-// The rows of the entries [t0, t0 + kTile) of a matrix with n entries, by a workgroup of kBlock threads:
+// The rows of the entries [t0, t0 + THREADS * PER) of a matrix with n entries, by a workgroup of THREADS threads:
 // T.row[i] is the row of entry t0 + i (the last r < rows with ptr[r] <= t0 + i).  A search of the row pointers per entry is
 // twenty dependent loads of its own for a matrix of a million rows, and the kernels that did so spent most of
 // their time on them; here a workgroup searches once, 64 pointers at a look, marks where the rows behind begin, and
 // a running maximum does the rest.  Whatever stands in ptr, the rows found lie in [0, rows) and no access outside ptr[0 .. rows]
 // is made (rows >= 1; entry points whose arrays are not looked at beforehand rely on that).  Every thread of the workgroup has to come here.
-__device__ __forceinline__ void tile_rows(const int *__restrict__ ptr, int rows, int n, int t0, TileRows &T)
+template <int THREADS, int PER>
+__device__ __forceinline__ void tile_rows(const int *__restrict__ ptr, int rows, int n, int t0, TileRowsOf<THREADS, PER> &T)
 {
+    constexpr int kBlock = THREADS, kPer = PER, kTile = THREADS * PER;
     const int tid = threadIdx.x, lane = tid & 63;
     int lo = 0, hi = rows;  // the row of entry t0 lies in [lo, hi)
     while (hi - lo > 1) {

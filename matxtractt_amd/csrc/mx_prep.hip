@@ -1,21 +1,5 @@
-// Device side of the preprocessing: the transposes, and the two selections of the cascaded
-// extraction (which columns, then which rows, are dense).
-//
-// The reference transposes on the GPU as well -- csr2csc / csc2csr copy the matrix to the
-// device, call cusparseCsr2cscEx2 and copy the result back (utilities/csr2csc.cpp:4-203), three
-// times per run (test/test_autotc_spmv.cpp:1119-1238).  Here the matrix stays where it is: the
-// entry point takes device arrays and leaves device arrays, so a caller that already holds the
-// matrix in HBM pays no PCIe traffic.  The order inside every output line is the one the host
-// transpose (mx_transpose) produces -- ascending source line, equal pairs in source order -- so
-// the two are interchangeable bit for bit.
-//
-// Route: a transpose is a stable sort of the entries by their index.  Entry e of source line r
-// gets the key ind[e] and the payload e; source order is ascending (r, e), so a stable sort by
-// key alone gives ascending (ind, r, e).  rocPRIM's radix sort is stable and sorts only the
-// ceil(log2(inner)) bits the keys can have.  Three small kernels around it: the source line of
-// every entry (tile_rows), the output line pointers from the sorted keys (every
-// thread writes the pointers of the lines that start at its position), and the gather of
-// source lines and values through the sorted payload.
+// Device side of the preprocessing: the two selections of the cascaded extraction (which columns, then which rows, are
+// dense), the split by them and the tile encoding.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,51 +21,6 @@ namespace mxp {
 constexpr int kBlock = 256;
 // Entry numbers are formed as blockIdx.x * kBlock + threadIdx.x in 32 bits: the last block must not pass 2^31.
 constexpr int kMaxCount = 2147483647 - 2 * kBlock;
-
-// line[e] = r with ptr[r] <= e < ptr[r+1]; bad |= 1 where ind[e] lies outside [0, inner).
-// (7 million entries in 700001 lines: 0.13 ms with a search per entry, 0.04 so)
-__global__ __launch_bounds__(kBlock) void entry_lines_kernel(const int *__restrict__ ptr, const int *__restrict__ ind,
-                                                             int outer, int inner, int nnz, int *__restrict__ line,
-                                                             int *__restrict__ payload, int *__restrict__ bad)
-{
-    __shared__ mxr::TileRows T;
-    const int t0 = blockIdx.x * mxr::kTile;
-    mxr::tile_rows(ptr, outer, nnz, t0, T);
-    bool out = false;
-#pragma unroll
-    for (int k = 0; k < mxr::kPer; ++k) {
-        const int i = k * kBlock + threadIdx.x;
-        if (i >= nnz - t0) break;
-        line[t0 + i] = T.row[i];
-        payload[t0 + i] = t0 + i;
-        out |= (unsigned)ind[t0 + i] >= (unsigned)inner;
-    }
-    if (__any(out) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
-}
-
-// tPtr[c] = number of sorted keys below c, for c in [0, inner].  Thread k owns the lines
-// (key[k-1], key[k]]; the thread behind the last key owns what is left, inner included.
-__global__ __launch_bounds__(kBlock) void line_pointers_kernel(const int *__restrict__ key, int nnz, int inner,
-                                                               int *__restrict__ tPtr)
-{
-    const long long k = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (k > nnz) return;
-    const int first = k == 0 ? 0 : key[k - 1] + 1;
-    const int last = k == nnz ? inner : key[k];
-    for (int c = first; c <= last; ++c) tPtr[c] = (int)k;
-}
-
-template <typename V>
-__global__ __launch_bounds__(kBlock) void gather_kernel(const int *__restrict__ payload, const int *__restrict__ line,
-                                                        const V *__restrict__ val, int nnz, int *__restrict__ tInd,
-                                                        V *__restrict__ tVal)
-{
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= nnz) return;
-    const int e = payload[k];
-    tInd[k] = line[e];
-    tVal[k] = val[e];
-}
 
 // ---- selection ---------------------------------------------------------------------------
 // cnt[ind[e]] += 1 for every entry (integer atomics: the result does not depend on the order).
@@ -457,71 +396,6 @@ struct Scratch {
             return e_ == hipErrorOutOfMemory ? MX_ERR_ALLOC : MX_ERR_DEVICE;                \
         }                                                                                   \
     } while (0)
-
-extern "C" int mx_transpose_device(mx_dtype dtype, int outer, int inner, int nnz, const int *ptr_dev, const int *ind_dev,
-                                   const void *val_dev, int *tPtr_dev, int *tInd_dev, void *tVal_dev, void *stream)
-{
-    static const char who[] = "mx_transpose_device";
-    using namespace mxp;
-    if ((dtype != MX_F64 && dtype != MX_F16) || outer < 0 || inner < 0 || nnz < 0 || !ptr_dev || !tPtr_dev ||
-        (nnz > 0 && (!ind_dev || !val_dev || !tInd_dev || !tVal_dev || outer == 0))) {
-        mx::set_error("mx_transpose_device: bad argument");
-        return MX_ERR_ARG;
-    }
-    if (nnz > kMaxCount || inner > kMaxCount || outer > kMaxCount) {
-        mx::set_error("mx_transpose_device: more than 2^31 - 513 entries or lines");
-        return MX_ERR_ARG;
-    }
-    hipStream_t s = (hipStream_t)stream;
-    mx::MemScope scope(s);
-    const int pblocks = (int)(((long long)nnz + 1 + kBlock - 1) / kBlock);
-    if (nnz == 0) {
-        hipLaunchKernelGGL(line_pointers_kernel, dim3(pblocks), dim3(kBlock), 0, s, (const int *)nullptr, 0, inner, tPtr_dev);
-        MXP_TRY(hipGetLastError());
-        MXP_TRY(hipStreamSynchronize(s));
-        return MX_OK;
-    }
-    int bits = 1;
-    while (bits < 31 && (1ll << bits) < (long long)inner) ++bits;
-    // one allocation: line[nnz], payload in/out [nnz] each, keys out [nnz], flag, sort storage
-    size_t sortBytes = 0;
-    MXP_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const int *)nullptr, (int *)nullptr, (const int *)nullptr,
-                                      (int *)nullptr, (size_t)nnz, 0u, (unsigned)bits, s));
-    const size_t n4 = ((size_t)nnz * sizeof(int) + 255) & ~(size_t)255;
-    Scratch scratch;
-    MXP_TRY(mx::dev_malloc(&scratch.p, 4 * n4 + 256 + sortBytes));
-    unsigned char *base = (unsigned char *)scratch.p;
-    int *line = (int *)base, *payIn = (int *)(base + n4), *payOut = (int *)(base + 2 * n4), *keyOut = (int *)(base + 3 * n4);
-    int *bad = (int *)(base + 4 * n4);
-    void *sortTmp = base + 4 * n4 + 256;
-    const int eblocks = (nnz + kBlock - 1) / kBlock;
-    MXP_TRY(hipMemsetAsync(bad, 0, sizeof(int), s));
-    hipLaunchKernelGGL(entry_lines_kernel, mxr::tile_grid(nnz), dim3(kBlock), 0, s, ptr_dev, ind_dev, outer, inner, nnz, line,
-                       payIn, bad);
-    MXP_TRY(hipGetLastError());
-    // an index outside [0, inner) must not reach the pointer kernel: look before going on
-    int badHost = 0;
-    MXP_TRY(hipMemcpyAsync(&badHost, bad, sizeof(int), hipMemcpyDeviceToHost, s));
-    MXP_TRY(hipStreamSynchronize(s));
-    if (badHost) {
-        mx::set_error("mx_transpose_device: index out of range");
-        return MX_ERR_ARG;
-    }
-    MXP_TRY(rocprim::radix_sort_pairs(sortTmp, sortBytes, ind_dev, keyOut, (const int *)payIn, payOut, (size_t)nnz, 0u,
-                                      (unsigned)bits, s));
-    hipLaunchKernelGGL(line_pointers_kernel, dim3(pblocks), dim3(kBlock), 0, s, (const int *)keyOut, nnz, inner, tPtr_dev);
-    MXP_TRY(hipGetLastError());
-    if (dtype == MX_F64)
-        hipLaunchKernelGGL(gather_kernel<double>, dim3(eblocks), dim3(kBlock), 0, s, (const int *)payOut, (const int *)line,
-                           (const double *)val_dev, nnz, tInd_dev, (double *)tVal_dev);
-    else
-        hipLaunchKernelGGL(gather_kernel<uint16_t>, dim3(eblocks), dim3(kBlock), 0, s, (const int *)payOut,
-                           (const int *)line, (const uint16_t *)val_dev, nnz, tInd_dev, (uint16_t *)tVal_dev);
-    MXP_TRY(hipGetLastError());
-    MXP_TRY(hipStreamSynchronize(s));  // the scratch is released on return
-    return MX_OK;
-}
-
 
 namespace mxp {
 

@@ -1,0 +1,587 @@
+// Transposes on the device.
+//
+// The reference transposes on the GPU as well -- csr2csc / csc2csr copy the matrix to the
+// device, call cusparseCsr2cscEx2 and copy the result back (utilities/csr2csc.cpp:4-203), three
+// times per run (test/test_autotc_spmv.cpp:1119-1238).  Here the matrix stays where it is: the
+// entry point takes device arrays and leaves device arrays, so a caller that already holds the
+// matrix in HBM pays no PCIe traffic.  The order inside every output line is the one the host
+// transpose (mx_transpose) produces -- ascending source line, equal pairs in source order -- so
+// the two are interchangeable bit for bit.
+//
+// A transpose is a stable sort of the entries by their index, and the lines and values travel with
+// the sort.  It is made in two steps, each of which reads and writes every entry once: the entries of a tile go
+// to buckets of consecutive output lines (bucket_entries_kernel), and a workgroup puts one bucket in order
+// in LDS (bucket_lines_kernel).  Both are counting sorts: an entry's place among those of its digit is
+// the number of lanes below it with the same digit, found with one ballot per bit of it, on top of what the waves and
+// tiles before it counted -- no atomics decide an order.  What it takes is bound by bytes: 28 an entry in and as many out in binary64 for the two
+// steps, and 4 to count them first.  (7.6 million entries of a power law, 700001 x 412345, binary64: 217 us;
+// three passes of a radix sort over index and entry number, with the lines and values gathered at the end, 448; 2 million lines, 4.1 million output lines, binary16: 287, 1046; 12000 x 9000 with nine a line: 63, 103.)
+//
+// One workgroup works on a bucket: a matrix with so many of its entries in one place that the others would wait for
+// that workgroup, or with more output lines than the buckets hold (kDigits each), takes the radix sort.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <cstring>
+#include <string>
+
+#include <rocprim/device/device_radix_sort.hpp>
+
+#include "mx_device.h"
+#include "mx_entry_rows.h"
+#include "mx_internal.h"
+
+namespace mxt {
+
+constexpr int kBlock = 256;
+// Entry numbers are formed as blockIdx.x * kBlock + threadIdx.x in 32 bits: the last block must not pass 2^31.
+constexpr int kMaxCount = 2147483647 - 2 * kBlock;
+
+// ---- the two steps ------------------------------------------------------------------------
+constexpr int kThreads = 1024, kPer = 8, kTile = kThreads * kPer;  // entries that a workgroup puts in order at a time
+constexpr int kWaves = kThreads / 64, kWave = 64 * kPer;
+constexpr int kDigitBits = 11, kDigits = 1 << kDigitBits;  // buckets, and lines of a bucket, at most
+constexpr int kBucketMean = 6800;     // entries of a bucket on average: nearly all then have at most kTile
+constexpr int kBucketsLeast = 64;     // but not so few buckets that most of the device has none
+// Entries of one bucket at most: its workgroup takes 11 us for every 8192 of them while the others are done, and the radix sort has
+// to be the slower way still (a million entries, 16 thousand of them in one line: 113 us, radix sort 231; 8 million, 60 thousand: 349, 620).
+inline int most_of_bucket(int nnz) { return 65536 + nnz / 64; }
+
+// The lanes of the wave whose digit is this lane's; `live` are those that have one.
+__device__ __forceinline__ unsigned long long same_digit(unsigned d, int bits, unsigned long long live)
+{
+    unsigned lo = (unsigned)live, hi = (unsigned)(live >> 32);
+#pragma unroll
+    for (int k = 0; k < kDigitBits; ++k)
+        if (k < bits) {
+            const unsigned set = (unsigned)((int)(d << (31 - k)) >> 31);  // all bits, or none
+            const unsigned long long b = __ballot(set != 0);
+            lo &= ~((unsigned)b ^ set);
+            hi &= ~((unsigned)(b >> 32) ^ set);
+        }
+    return ((unsigned long long)hi << 32) | lo;
+}
+__device__ __forceinline__ int lanes_below(unsigned long long m)
+{
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+}
+// The sum of v over the threads of the workgroup before this one; `part` has room for a wave each.
+__device__ __forceinline__ int sum_before(int v, int *part)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int run = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(run, off);
+        if (lane >= off) run += o;
+    }
+    if (lane == 63) part[w] = run;
+    __syncthreads();
+    int before = 0;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k)
+        if (k < w) before += part[k];
+    __syncthreads();
+    return before + run - v;
+}
+
+// The `size` entries of a workgroup in order of their digits, equal digits in order of their numbers: entry
+// i = w * kWave + j * 64 + lane belongs to thread (w, lane), digit(j) is its digit and at[j] becomes its place behind
+// start[digit].  SUM: start[k] is set to the entries of the digits before k, for every k up to kDigits; otherwise it is the
+// caller's.  D is free again on return.
+struct Digits {
+    unsigned short seen[kWaves][kDigits];
+};
+template <bool SUM, typename T, typename F>
+__device__ __forceinline__ void place_by_digit(const F &digit, int size, int bits, Digits &D, T *__restrict__ start, int *__restrict__ part,
+                                               int (&at)[kPer])
+{
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    for (int i = tid; i < kWaves * kDigits / 8; i += kThreads) ((int4 *)D.seen)[i] = make_int4(0, 0, 0, 0);
+    __syncthreads();
+    unsigned short *mine = D.seen[w];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const bool live = w * kWave + j * 64 + lane < size;
+        const int k = digit(j);
+        const unsigned long long m = same_digit((unsigned)k, bits, __ballot(live));
+        const int had = live ? mine[k] : 0, below = lanes_below(m);
+        // (a wave's LDS accesses happen in order; the fences keep the compiler from moving one over another)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (live && below == 0) mine[k] = (unsigned short)(had + __popcll(m));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        at[j] = had + below;
+    }
+    __syncthreads();
+    // a thread takes two digits, side by side in a word (no sum passes kTile)
+    unsigned n = 0;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) {
+        unsigned *word = (unsigned *)&D.seen[k][2 * tid];
+        const unsigned c = *word;
+        *word = n;
+        n += c;
+    }
+    if (SUM) {
+        const int n0 = (int)(n & 0xffff), n1 = (int)(n >> 16), s = sum_before(n0 + n1, part);
+        start[2 * tid] = (T)s;
+        start[2 * tid + 1] = (T)(s + n0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int k = digit(j);
+        if (w * kWave + j * 64 + lane < size) at[j] += start[k] + mine[k];
+    }
+    __syncthreads();
+}
+static_assert(kDigits == 2 * kThreads && kTile < 65536, "two digits to a thread, counts of 16 bits");
+
+// Buckets of `lines` output lines.  c / lines as a product: exact for c < kDigits * lines with lines <= kDigits, since the
+// error of `inverse`, below one, times c stays below 2^42 / lines.
+struct Buckets {
+    int n, bits, lines, lineBits;
+    unsigned long long inverse;  // 2^42 / lines, rounded up
+    __device__ __forceinline__ int of(int c) const { return (int)(((unsigned long long)(unsigned)c * inverse) >> 42); }
+};
+
+// The tile of a workgroup: every XCD takes one stretch of the tiles, so that the pieces that follow each other in a
+// bucket are written through one L2.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int tile_of_block(int tiles)
+{
+    const int per = (tiles + kXcds - 1) / kXcds, k = blockIdx.x / kXcds;
+    return k < per ? (int)(blockIdx.x % kXcds) * per + k : tiles;
+}
+inline dim3 tile_blocks(int tiles) { return dim3((unsigned)((tiles + kXcds - 1) / kXcds * kXcds)); }
+
+// count[tile][bucket] entries; bad[tile]: an index lies outside [0, inner)
+__global__ __launch_bounds__(kThreads) void bucket_counts_kernel(const int *__restrict__ ind, int inner, int nnz, Buckets B, int tiles,
+                                                                 int *__restrict__ count, int *__restrict__ bad)
+{
+    __shared__ int here[kDigits];
+    const int t = tile_of_block(tiles);
+    if (t >= tiles) return;
+    const int t0 = t * kTile, tid = threadIdx.x, lane = tid & 63;
+    here[tid] = here[tid + kThreads] = 0;
+    __syncthreads();
+    int b[kPer];
+    bool out = false;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int i = j * kThreads + tid;
+        b[j] = -1;
+        if (i >= nnz - t0) continue;
+        const int c = ind[t0 + i];
+        if ((unsigned)c < (unsigned)inner) b[j] = B.of(c);
+        else out = true;
+    }
+    // (neighbours often share a bucket, and an atomic takes as long as lanes want the same word: the first lane's bucket is counted at once)
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int first = __builtin_amdgcn_readfirstlane(b[j]);
+        const unsigned long long same = __ballot(b[j] == first);
+        if (first >= 0 && lane == __builtin_ctzll(same)) atomicAdd(&here[first], __popcll(same));
+        if (b[j] >= 0 && b[j] != first) atomicAdd(&here[b[j]], 1);
+    }
+    out = __syncthreads_or(out);
+    if (tid == 0) bad[t] = out;
+    for (int k = tid; k < B.n; k += kThreads) count[(size_t)t * B.n + k] = here[k];
+}
+
+// count[t][b] becomes the entries of bucket b in the tiles before t, total[b] those in all; a workgroup takes 16 buckets,
+// 64 stretches of tiles of each.
+__global__ __launch_bounds__(1024) void bucket_offsets_kernel(int *__restrict__ count, int buckets, int tiles, int *__restrict__ total)
+{
+    __shared__ int part[64][16];
+    const int k = threadIdx.x & 15, w = threadIdx.x >> 4, b = blockIdx.x * 16 + k, per = (tiles + 63) / 64;
+    const int a = min(tiles, w * per), z = min(tiles, a + per);
+    int sum = 0;
+    if (b < buckets)
+#pragma unroll 4
+        for (int t = a; t < z; ++t) sum += count[(size_t)t * buckets + b];
+    part[w][k] = sum;
+    __syncthreads();
+    if (b >= buckets) return;
+    int run = 0, all = 0;
+    for (int i = 0; i < 64; ++i) {
+        if (i < w) run += part[i][k];
+        all += part[i][k];
+    }
+    if (w == 0) total[b] = all;
+    for (int t = a; t < z; t += 4) {
+        int c[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[i] = t + i < z ? count[(size_t)(t + i) * buckets + b] : 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (t + i < z) count[(size_t)(t + i) * buckets + b] = run;
+            run += c[i];
+        }
+    }
+}
+// first[b] = entries of the buckets before b, first[buckets] = all; *flag = 1 when a tile is bad, + 2 when a bucket has more than `most`
+__global__ __launch_bounds__(kThreads) void bucket_starts_kernel(const int *__restrict__ total, int buckets, int most, const int *__restrict__ bad,
+                                                                 int tiles, int *__restrict__ first, int *__restrict__ flag)
+{
+    __shared__ int part[kWaves];
+    const int b = 2 * threadIdx.x, n0 = b < buckets ? total[b] : 0, n1 = b + 1 < buckets ? total[b + 1] : 0, at = sum_before(n0 + n1, part);
+    if (b <= buckets) first[b] = at;
+    if (b + 1 <= buckets) first[b + 1] = at + n0;
+    if (b + 2 == buckets) first[buckets] = at + n0 + n1;
+    bool out = false;
+    for (int t = threadIdx.x; t < tiles; t += kThreads) out |= bad[t] != 0;
+    out = __syncthreads_or(out);
+    const bool crowded = __syncthreads_or(max(n0, n1) > most);
+    if (b == 0) *flag = (int)out + 2 * (int)crowded;
+}
+
+// An entry between the two steps, in one piece: a store of a wave goes to as many places as it has lanes, whatever a lane
+// stores (line, source line and value in arrays of their own, put in order in LDS to be written side by side: 89 + 89 us
+// in the two steps for 7.6 million binary64 entries, so 92 + 65).
+template <typename V>
+struct Moved;
+template <>
+struct Moved<double> {
+    typedef int4 Word;
+    static __device__ __forceinline__ Word pack(int line, int source, double v)
+    {
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+        return make_int4((int)(unsigned)u, (int)(unsigned)(u >> 32), source, line);
+    }
+    static __device__ __forceinline__ int line(const Word &w) { return w.w; }
+    static __device__ __forceinline__ int source(const Word &w) { return w.z; }
+    static __device__ __forceinline__ double value(const Word &w)
+    {
+        return __builtin_bit_cast(double, ((unsigned long long)(unsigned)w.y << 32) | (unsigned)w.x);
+    }
+};
+template <>
+struct Moved<uint16_t> {
+    typedef int2 Word;
+    static __device__ __forceinline__ Word pack(int line, int source, uint16_t v) { return make_int2(source, line | (int)((unsigned)v << 16)); }
+    static __device__ __forceinline__ int line(const Word &w) { return w.y & 0xffff; }
+    static __device__ __forceinline__ int source(const Word &w) { return w.x; }
+    static __device__ __forceinline__ uint16_t value(const Word &w) { return (uint16_t)((unsigned)w.y >> 16); }
+};
+
+// The entries of a tile to their buckets, in source order.
+template <typename V>
+__global__ __launch_bounds__(kThreads, 8) void bucket_entries_kernel(const int *__restrict__ ptr, const int *__restrict__ ind, const V *__restrict__ val,
+                                                                     int outer, int nnz, Buckets B, int tiles, const int *__restrict__ before,
+                                                                     const int *__restrict__ first, const int *__restrict__ flag,
+                                                                     typename Moved<V>::Word *__restrict__ moved)
+{
+    __shared__ union {
+        mxr::TileRowsOf<kThreads, kPer> rows;
+        Digits digits;
+    } U;
+    __shared__ int start[kDigits];
+    const int t = tile_of_block(tiles);
+    if (t >= tiles || *flag) return;
+    const int t0 = t * kTile, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, size = min(kTile, nnz - t0);
+    mxr::tile_rows(ptr, outer, nnz, t0, U.rows);
+    int row[kPer], c[kPer], at[kPer];  // (c: bucket and line)
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int i = w * kWave + j * 64 + lane;
+        c[j] = i < size ? ind[t0 + i] : 0;
+        row[j] = i < size ? U.rows.row[i] : 0;
+    }
+    for (int k = tid; k < B.n; k += kThreads) start[k] = first[k] + before[(size_t)t * B.n + k];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int b = B.of(c[j]);
+        c[j] = b | (c[j] - b * B.lines) << 16;
+    }
+    __syncthreads();
+    place_by_digit<false>([&](int j) { return c[j] & 0xffff; }, size, B.bits, U.digits, start, (int *)nullptr, at);
+    V v[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) v[j] = val[t0 + min(w * kWave + j * 64 + lane, size - 1)];
+    __builtin_amdgcn_sched_barrier(0);  // (all values are asked for before the first is waited for)
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+        if (w * kWave + j * 64 + lane < size) moved[at[j]] = Moved<V>::pack(c[j] >> 16, row[j], v[j]);
+}
+
+// A bucket in order of its lines, and the pointers of its lines.  One of at most kTile entries is put in order in LDS
+// and written as it comes out; a larger one takes several rounds, whose entries go behind what the rounds before left of
+// their lines, each to its own place.
+template <typename V>
+__global__ __launch_bounds__(kThreads, 8) void bucket_lines_kernel(const typename Moved<V>::Word *__restrict__ moved, const int *__restrict__ first,
+                                                                   int inner, Buckets B, const int *__restrict__ flag, int *__restrict__ tPtr,
+                                                                   int *__restrict__ tInd, V *__restrict__ tVal)
+{
+    typedef Moved<V> M;
+    __shared__ union {
+        Digits digits;
+        V val[kTile];
+        int word[kTile];
+    } U;
+    __shared__ int next[kDigits], part[kWaves];
+    __shared__ unsigned short start[kDigits];
+    if (*flag) return;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, b = blockIdx.x;
+    const int c0 = b * B.lines, lines = min(B.lines, inner - c0), p0 = first[b], p1 = first[b + 1];
+    if (b == B.n - 1 && tid == 0) tPtr[inner] = p1;
+    int d[kPer], at[kPer], row[kPer];
+    V v[kPer];
+    auto load = [&](int q, int size) {
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const int i = w * kWave + j * 64 + lane;
+            const typename M::Word e = moved[q + min(i, size - 1)];
+            d[j] = M::line(e);
+            row[j] = M::source(e);
+            v[j] = M::value(e);
+        }
+    };
+    if (p1 - p0 <= kTile) {
+        const int size = p1 - p0;
+        if (size > 0) load(p0, size);
+        place_by_digit<true>([&](int j) { return d[j]; }, size, B.lineBits, U.digits, start, part, at);
+        for (int c = tid; c < lines; c += kThreads) tPtr[c0 + c] = p0 + start[c];
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+            if (w * kWave + j * 64 + lane < size) U.word[at[j]] = row[j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+            if (j * kThreads + tid < size) tInd[p0 + j * kThreads + tid] = U.word[j * kThreads + tid];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+            if (w * kWave + j * 64 + lane < size) U.val[at[j]] = v[j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+            if (j * kThreads + tid < size) tVal[p0 + j * kThreads + tid] = U.val[j * kThreads + tid];
+        return;
+    }
+    next[2 * tid] = next[2 * tid + 1] = 0;
+    __syncthreads();
+    for (int p = p0; p < p1; p += kThreads) {
+        const int c = p + tid < p1 ? M::line(moved[p + tid]) : -1, one = __builtin_amdgcn_readfirstlane(c);
+        const unsigned long long same = __ballot(c == one);  // (a crowded line)
+        if (one >= 0 && lane == __builtin_ctzll(same)) atomicAdd(&next[one], __popcll(same));
+        if (c >= 0 && c != one) atomicAdd(&next[c], 1);
+    }
+    __syncthreads();
+    {
+        const int n0 = next[2 * tid], n1 = next[2 * tid + 1], s = p0 + sum_before(n0 + n1, part);
+        next[2 * tid] = s;
+        next[2 * tid + 1] = s + n0;
+        if (2 * tid < lines) tPtr[c0 + 2 * tid] = s;
+        if (2 * tid + 1 < lines) tPtr[c0 + 2 * tid + 1] = s + n0;
+    }
+    for (int q = p0; q < p1; q += kTile) {
+        const int size = min(kTile, p1 - q);
+        load(q, size);
+        place_by_digit<true>([&](int j) { return d[j]; }, size, B.lineBits, U.digits, start, part, at);
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            if (w * kWave + j * 64 + lane >= size) continue;
+            const int to = next[d[j]] + at[j] - start[d[j]];
+            tInd[to] = row[j];
+            tVal[to] = v[j];
+        }
+        __syncthreads();
+        const int s0 = start[2 * tid], s1 = start[2 * tid + 1], s2 = tid + 1 < kThreads ? start[2 * tid + 2] : size;
+        next[2 * tid] += s1 - s0;
+        next[2 * tid + 1] += s2 - s1;
+    }
+}
+
+// ---- the radix sort's kernels ---------------------------------------------------------------
+// line[e] = r with ptr[r] <= e < ptr[r+1]; bad |= 1 where ind[e] lies outside [0, inner).
+// (7 million entries in 700001 lines: 0.13 ms with a search per entry, 0.04 so)
+__global__ __launch_bounds__(kBlock) void entry_lines_kernel(const int *__restrict__ ptr, const int *__restrict__ ind,
+                                                             int outer, int inner, int nnz, int *__restrict__ line,
+                                                             int *__restrict__ payload, int *__restrict__ bad)
+{
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(ptr, outer, nnz, t0, T);
+    bool out = false;
+#pragma unroll
+    for (int k = 0; k < mxr::kPer; ++k) {
+        const int i = k * kBlock + threadIdx.x;
+        if (i >= nnz - t0) break;
+        line[t0 + i] = T.row[i];
+        payload[t0 + i] = t0 + i;
+        out |= (unsigned)ind[t0 + i] >= (unsigned)inner;
+    }
+    if (__any(out) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
+}
+
+// tPtr[c] = number of sorted keys below c, for c in [0, inner].  Thread k owns the lines
+// (key[k-1], key[k]]; the thread behind the last key owns what is left, inner included.
+__global__ __launch_bounds__(kBlock) void line_pointers_kernel(const int *__restrict__ key, int nnz, int inner,
+                                                               int *__restrict__ tPtr)
+{
+    const long long k = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (k > nnz) return;
+    const int first = k == 0 ? 0 : key[k - 1] + 1;
+    const int last = k == nnz ? inner : key[k];
+    for (int c = first; c <= last; ++c) tPtr[c] = (int)k;
+}
+
+template <typename V>
+__global__ __launch_bounds__(kBlock) void gather_kernel(const int *__restrict__ payload, const int *__restrict__ line,
+                                                        const V *__restrict__ val, int nnz, int *__restrict__ tInd,
+                                                        V *__restrict__ tVal)
+{
+    const int k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= nnz) return;
+    const int e = payload[k];
+    tInd[k] = line[e];
+    tVal[k] = val[e];
+}
+
+struct Scratch {
+    void *p = nullptr;
+    Scratch() = default;
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
+    ~Scratch()
+    {
+        if (p) (void)mx::dev_free(p);
+    }
+};
+
+}  // namespace mxt
+
+#define MXT_TRY(call)                                                                                  \
+    do {                                                                                               \
+        hipError_t e_ = (call);                                                                        \
+        if (e_ != hipSuccess) {                                                                        \
+            mx::set_error(std::string("mx_transpose_device: ") + #call + ": " + hipGetErrorString(e_)); \
+            return e_ == hipErrorOutOfMemory ? MX_ERR_ALLOC : MX_ERR_DEVICE;                           \
+        }                                                                                              \
+    } while (0)
+
+namespace mxt {
+
+// By buckets; *done is false, and nothing is written, where the matrix does not suit it (*checked: its indices were looked at).
+template <typename V>
+static int transpose_by_buckets(int outer, int inner, int nnz, const int *ptr, const int *ind, const V *val, int *tPtr, int *tInd, V *tVal,
+                                bool *done, bool *checked, hipStream_t s)
+{
+    *done = *checked = false;
+    if (inner < 1 || inner > kDigits * kDigits) return MX_OK;
+    Buckets B;
+    const long long mean = ((long long)nnz + kBucketMean - 1) / kBucketMean, wide = ((long long)inner + kDigits - 1) / kDigits;
+    B.n = (int)std::min<long long>(kDigits, std::max<long long>(kBucketsLeast, std::max(mean, wide)));
+    B.lines = (inner + B.n - 1) / B.n;
+    B.n = (inner + B.lines - 1) / B.lines;
+    B.bits = B.lineBits = 0;
+    while ((1 << B.bits) < B.n) ++B.bits;
+    while ((1 << B.lineBits) < B.lines) ++B.lineBits;
+    B.inverse = ((1ull << 42) + B.lines - 1) / B.lines;
+    const int buckets = B.n, tiles = (int)(((long long)nnz + kTile - 1) / kTile);
+    typedef typename Moved<V>::Word Word;
+    auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const size_t countB = al((size_t)tiles * buckets * 4 + (size_t)tiles * 4), firstB = al((size_t)(2 * kDigits + 1) * 4);
+    Scratch scratch;
+    MXT_TRY(mx::dev_malloc(&scratch.p, countB + firstB + 256 + (size_t)nnz * sizeof(Word)));
+    unsigned char *b = (unsigned char *)scratch.p;
+    int *count = (int *)b, *bad = count + (size_t)tiles * buckets, *first = (int *)(b + countB), *total = first + kDigits + 1, *flag = (int *)(b + countB + firstB);
+    b += countB + firstB + 256;
+    Word *moved = (Word *)b;
+    hipLaunchKernelGGL(bucket_counts_kernel, tile_blocks(tiles), dim3(kThreads), 0, s, ind, inner, nnz, B, tiles, count, bad);
+    hipLaunchKernelGGL(bucket_offsets_kernel, dim3((unsigned)((buckets + 15) / 16)), dim3(1024), 0, s, count, buckets, tiles, total);
+    hipLaunchKernelGGL(bucket_starts_kernel, dim3(1), dim3(kThreads), 0, s, (const int *)total, buckets, most_of_bucket(nnz), (const int *)bad, tiles,
+                       first, flag);
+    hipLaunchKernelGGL(bucket_entries_kernel<V>, tile_blocks(tiles), dim3(kThreads), 0, s, ptr, ind, val, outer, nnz, B, tiles, (const int *)count,
+                       (const int *)first, (const int *)flag, moved);
+    hipLaunchKernelGGL(bucket_lines_kernel<V>, dim3((unsigned)buckets), dim3(kThreads), 0, s, (const Word *)moved, (const int *)first, inner, B, (const int *)flag, tPtr, tInd, tVal);
+    MXT_TRY(hipGetLastError());
+    int got = 0;
+    MXT_TRY(hipMemcpyAsync(&got, flag, 4, hipMemcpyDeviceToHost, s));
+    MXT_TRY(hipStreamSynchronize(s));
+    if (got & 1) {
+        mx::set_error("mx_transpose_device: index out of range");
+        return MX_ERR_ARG;
+    }
+    *done = got == 0;
+    *checked = true;
+    return MX_OK;
+}
+
+}  // namespace mxt
+
+extern "C" int mx_transpose_device(mx_dtype dtype, int outer, int inner, int nnz, const int *ptr_dev, const int *ind_dev,
+                                   const void *val_dev, int *tPtr_dev, int *tInd_dev, void *tVal_dev, void *stream)
+{
+    using namespace mxt;
+    if ((dtype != MX_F64 && dtype != MX_F16) || outer < 0 || inner < 0 || nnz < 0 || !ptr_dev || !tPtr_dev ||
+        (nnz > 0 && (!ind_dev || !val_dev || !tInd_dev || !tVal_dev || outer == 0))) {
+        mx::set_error("mx_transpose_device: bad argument");
+        return MX_ERR_ARG;
+    }
+    if (nnz > kMaxCount || inner > kMaxCount || outer > kMaxCount) {
+        mx::set_error("mx_transpose_device: more than 2^31 - 513 entries or lines");
+        return MX_ERR_ARG;
+    }
+    hipStream_t s = (hipStream_t)stream;
+    mx::MemScope scope(s);
+    const int pblocks = (int)(((long long)nnz + 1 + kBlock - 1) / kBlock);
+    if (nnz == 0) {
+        hipLaunchKernelGGL(line_pointers_kernel, dim3(pblocks), dim3(kBlock), 0, s, (const int *)nullptr, 0, inner, tPtr_dev);
+        MXT_TRY(hipGetLastError());
+        MXT_TRY(hipStreamSynchronize(s));
+        return MX_OK;
+    }
+    bool checked = false;
+    {
+        bool done = false;
+        const int rc = dtype == MX_F64 ? transpose_by_buckets(outer, inner, nnz, ptr_dev, ind_dev, (const double *)val_dev, tPtr_dev, tInd_dev,
+                                                              (double *)tVal_dev, &done, &checked, s)
+                                       : transpose_by_buckets(outer, inner, nnz, ptr_dev, ind_dev, (const uint16_t *)val_dev, tPtr_dev, tInd_dev,
+                                                              (uint16_t *)tVal_dev, &done, &checked, s);
+        if (rc != MX_OK || done) return rc;
+    }
+    int bits = 1;
+    while (bits < 31 && (1ll << bits) < (long long)inner) ++bits;
+    // one allocation: line[nnz], payload in/out [nnz] each, keys out [nnz], flag, sort storage
+    size_t sortBytes = 0;
+    MXT_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const int *)nullptr, (int *)nullptr, (const int *)nullptr,
+                                      (int *)nullptr, (size_t)nnz, 0u, (unsigned)bits, s));
+    const size_t n4 = ((size_t)nnz * sizeof(int) + 255) & ~(size_t)255;
+    Scratch scratch;
+    MXT_TRY(mx::dev_malloc(&scratch.p, 4 * n4 + 256 + sortBytes));
+    unsigned char *base = (unsigned char *)scratch.p;
+    int *line = (int *)base, *payIn = (int *)(base + n4), *payOut = (int *)(base + 2 * n4), *keyOut = (int *)(base + 3 * n4);
+    int *bad = (int *)(base + 4 * n4);
+    void *sortTmp = base + 4 * n4 + 256;
+    const int eblocks = (nnz + kBlock - 1) / kBlock;
+    MXT_TRY(hipMemsetAsync(bad, 0, sizeof(int), s));
+    hipLaunchKernelGGL(entry_lines_kernel, mxr::tile_grid(nnz), dim3(kBlock), 0, s, ptr_dev, ind_dev, outer, inner, nnz, line,
+                       payIn, bad);
+    MXT_TRY(hipGetLastError());
+    // an index outside [0, inner) must not reach the pointer kernel: look before going on
+    if (!checked) {
+        int badHost = 0;
+        MXT_TRY(hipMemcpyAsync(&badHost, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+        MXT_TRY(hipStreamSynchronize(s));
+        if (badHost) {
+            mx::set_error("mx_transpose_device: index out of range");
+            return MX_ERR_ARG;
+        }
+    }
+    MXT_TRY(rocprim::radix_sort_pairs(sortTmp, sortBytes, ind_dev, keyOut, (const int *)payIn, payOut, (size_t)nnz, 0u,
+                                      (unsigned)bits, s));
+    hipLaunchKernelGGL(line_pointers_kernel, dim3(pblocks), dim3(kBlock), 0, s, (const int *)keyOut, nnz, inner, tPtr_dev);
+    MXT_TRY(hipGetLastError());
+    if (dtype == MX_F64)
+        hipLaunchKernelGGL(gather_kernel<double>, dim3(eblocks), dim3(kBlock), 0, s, (const int *)payOut, (const int *)line,
+                           (const double *)val_dev, nnz, tInd_dev, (double *)tVal_dev);
+    else
+        hipLaunchKernelGGL(gather_kernel<uint16_t>, dim3(eblocks), dim3(kBlock), 0, s, (const int *)payOut,
+                           (const int *)line, (const uint16_t *)val_dev, nnz, tInd_dev, (uint16_t *)tVal_dev);
+    MXT_TRY(hipGetLastError());
+    MXT_TRY(hipStreamSynchronize(s));  // the scratch is released on return
+    return MX_OK;
+}
