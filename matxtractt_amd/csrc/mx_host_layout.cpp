@@ -1158,9 +1158,9 @@ int upload_csr(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr, c
 using namespace mxp;
 
 // The part of the slice layout that looks at chunks only (64 virtual rows each; a few per thousand
-// entries): which workgroup and wave streams which chunk, and where.  Shared by the host route and
-// the device route of the layout, which hand in the chunks of every slice (longest first, as the
-// sort leaves them) and fill the streams from what comes back.
+// entries): which workgroup and wave streams which chunk, and where.  Handed the chunks of every slice
+// (longest first, as the sort leaves them); the streams are filled from what comes back.  The device
+// route decides the same (plan_chunks_device).
 int mx::plan_slice_chunks(mx_dtype dtype, int budget, int S, const std::vector<std::vector<mx::SliceChunk>> &sliceChunks,
                           mx::SlicePlan &P)
 {
@@ -1200,7 +1200,8 @@ int mx::plan_slice_chunks(mx_dtype dtype, int budget, int S, const std::vector<s
         }
     }
     // workgroups: a slice's chunks, longest first, each to the workgroup of the slice with the
-    // fewest steps so far; then the same inside the workgroup for its waves
+    // fewest steps so far, those of one length dealt together so that a workgroup's share of them is
+    // consecutive (the device route works out the shares, not the dealing); then the same inside the workgroup for its waves
     std::vector<mxp::SliceWg> wgs;
     for (int q = 0; q < S; ++q) {
         const int g0 = (int)wgs.size(), G = Gq[q];
@@ -1211,12 +1212,20 @@ int mx::plan_slice_chunks(mx_dtype dtype, int budget, int S, const std::vector<s
         std::priority_queue<Load, std::vector<Load>, std::greater<Load>> heap;
         for (int g = 0; g < G; ++g) heap.push({0, g});
         const auto &ch = sliceChunks[q];
-        for (int c = 0; c < (int)ch.size(); ++c) {
-            Load top = heap.top();
-            heap.pop();
-            mine[top.second].push_back(c);
-            top.first += ch[c].steps + mx::kSliceChunkCost;
-            if ((int)mine[top.second].size() < mx::kSliceWgChunks) heap.push(top);
+        std::vector<int> take(G);
+        for (int c = 0, e; c < (int)ch.size(); c = e) {
+            e = c;
+            std::fill(take.begin(), take.end(), 0);
+            for (; e < (int)ch.size() && ch[e].steps == ch[c].steps; ++e) {
+                Load top = heap.top();
+                heap.pop();
+                ++take[top.second];
+                top.first += ch[c].steps + mx::kSliceChunkCost;
+                if ((int)mine[top.second].size() + take[top.second] < mx::kSliceWgChunks) heap.push(top);
+            }
+            int at = c;
+            for (int g = 0; g < G; ++g)
+                for (int k = 0; k < take[g]; ++k) mine[g].push_back(at++);
         }
         for (int g = 0; g < G; ++g) deal_to_waves(wgs[g0 + g], q, mine[g], ch, SPB);
     }

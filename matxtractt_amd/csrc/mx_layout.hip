@@ -8,8 +8,8 @@
 // order (a stable sort by (row, column) when some row is not), virtual rows cut at slice borders
 // and at the cap, their stable sort by (slice, length descending, kind of row), the entries
 // placed into the lanes' streams, the lists the combine kernel walks.  What depends on chunks
-// only (64 virtual rows each) -- which workgroup and wave streams which chunk -- is decided on the
-// host by the routine both routes share (plan_slice_chunks), from the chunks' lengths.
+// only (64 virtual rows each) -- which workgroup and wave streams which chunk -- is decided by
+// plan_chunks_device (mx_chunks.hip) as plan_slice_chunks decides it on the host.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -21,38 +21,13 @@
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
+#include "mx_chunks.h"
 #include "mx_device.h"
 #include "mx_entry_rows.h"
 #include "mx_internal.h"
 #include "mx_row_sort.h"
 
 namespace mxl {
-
-constexpr int kBlock = 256;
-
-struct Buf {  // device memory released at scope exit unless taken
-    void *p = nullptr;
-    Buf() = default;
-    Buf(const Buf &) = delete;
-    Buf &operator=(const Buf &) = delete;
-    ~Buf() { release(); }
-    void release()
-    {
-        if (p) (void)mx::dev_free(p);
-        p = nullptr;
-    }
-    template <typename T>
-    T *as() const
-    {
-        return (T *)p;
-    }
-    void *take()
-    {
-        void *q = p;
-        p = nullptr;
-        return q;
-    }
-};
 
 // The row and, for now, the place in the order of every entry; flag |= 1 when some row's columns are not ascending.
 // (13 million entries in a million rows: 0.11 ms; row heads, a running maximum over them and a pass that compared, 0.35 ms)
@@ -154,29 +129,6 @@ __global__ __launch_bounds__(kBlock) void vrow_keys_kernel(const int *__restrict
     key[t] = ((unsigned)vSlice[t] * (unsigned)(cap + 1) + (unsigned)(cap - len)) * 3u + (unsigned)kind;
     pay[t] = t;
     vLen[t] = len;
-}
-
-// sliceStart[q] = number of sorted keys that belong to slices before q, for q in [0, S]
-__global__ __launch_bounds__(kBlock) void slice_starts_kernel(const unsigned *__restrict__ sortedKey, int nV, int S, unsigned perSlice,
-                                                              int *__restrict__ sliceStart)
-{
-    const int q = blockIdx.x * kBlock + threadIdx.x;
-    if (q > S) return;
-    const unsigned long long want = (unsigned long long)q * perSlice;
-    int lo = 0, hi = nV;
-    while (lo < hi) {  // first position whose key is not below `want`
-        const int mid = (lo + hi) >> 1;
-        if ((unsigned long long)sortedKey[mid] < want) lo = mid + 1;
-        else hi = mid;
-    }
-    sliceStart[q] = lo;
-}
-
-__global__ __launch_bounds__(kBlock) void gather_len_kernel(const int *__restrict__ sorted, const int *__restrict__ vLen,
-                                                            const int *__restrict__ first, int n, int *__restrict__ out)
-{
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) out[i] = vLen[sorted[first[i]]];
 }
 
 // segIdx[t] = 64 * chunk + lane of every virtual row
@@ -498,18 +450,7 @@ __global__ __launch_bounds__(kBlock) void narrow_columns_kernel(const int4 *__re
     for (int p = d.z + lane; p < d.w; p += 64) c16[p] = (unsigned short)(col[p] - base);
 }
 
-inline dim3 grid(long long n) { return dim3((unsigned)((std::max<long long>(n, 1) + kBlock - 1) / kBlock)); }
-
 }  // namespace mxl
-
-#define MXL_TRY(call)                                                                                 \
-    do {                                                                                              \
-        hipError_t e_ = (call);                                                                       \
-        if (e_ != hipSuccess) {                                                                       \
-            mx::set_error(std::string("slice layout on the device: ") + #call + ": " + hipGetErrorString(e_)); \
-            return e_ == hipErrorOutOfMemory ? MX_ERR_ALLOC : MX_ERR_DEVICE;                          \
-        }                                                                                             \
-    } while (0)
 
 namespace mx {
 
@@ -673,7 +614,7 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     }
     runHead.release();
     D.vrows = nV;
-    Buf vStart, vRow, vSlice, vLen, segPtr, key, keyOut, pay, sorted, sliceCount;
+    Buf vStart, vRow, vSlice, vLen, segPtr, key, keyOut, pay, sorted;
     const size_t nv1 = (size_t)nV + 1;
     MXL_TRY(mx::dev_malloc(&vStart.p, nv1 * 4));
     MXL_TRY(mx::dev_malloc(&vRow.p, nv1 * 4));
@@ -684,7 +625,6 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     MXL_TRY(mx::dev_malloc(&keyOut.p, nv1 * 4));
     MXL_TRY(mx::dev_malloc(&pay.p, nv1 * 4));
     MXL_TRY(mx::dev_malloc(&sorted.p, nv1 * 4));
-    MXL_TRY(mx::dev_malloc(&sliceCount.p, ((size_t)S + 2) * 4));
     if (nnz > 0) {
         hipLaunchKernelGGL(vrow_records_kernel, grid(nnz), dim3(kBlock), 0, s, (const int *)start.p, (const int *)vid.p, (const int *)row.p,
                            col, (const int *)ord.p, nnz, SW, vStart.as<int>(), vRow.as<int>(), vSlice.as<int>());
@@ -693,7 +633,6 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     hipLaunchKernelGGL(seg_ptr_kernel, grid((long long)rows + 1), dim3(kBlock), 0, s, rowPtr, (const int *)vid.p, rows, nnz, nV,
                        segPtr.as<int>());
     MXL_TRY(hipGetLastError());
-    std::vector<int> sliceCnt((size_t)S, 0);
     if (nV > 0) {
         hipLaunchKernelGGL(vrow_keys_kernel, grid(nV), dim3(kBlock), 0, s, (const int *)vStart.p, (const int *)vRow.p, (const int *)vSlice.p,
                            (const int *)segPtr.p, nV, nnz, cap, kSliceLightSegs, key.as<unsigned>(), pay.as<int>(), vLen.as<int>());
@@ -732,67 +671,45 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
         MXL_TRY(mx::dev_malloc(&sortTmp.p, sortBytes + 256));
         MXL_TRY(rocprim::radix_sort_pairs(sortTmp.p, sortBytes, (const unsigned *)key.p, keyOut.as<unsigned>(), (const int *)pay.p,
                                           sorted.as<int>(), (size_t)nV, 0u, keyBits, s));
-        hipLaunchKernelGGL(slice_starts_kernel, grid((long long)S + 1), dim3(kBlock), 0, s, (const unsigned *)keyOut.p, nV, S,
-                           (unsigned)(cap + 1) * 3u, sliceCount.as<int>());
-        MXL_TRY(hipGetLastError());
-        std::vector<int> sliceStart((size_t)S + 1, 0);
-        MXL_TRY(hipMemcpyAsync(sliceStart.data(), sliceCount.p, ((size_t)S + 1) * 4, hipMemcpyDeviceToHost, s));
-        MXL_TRY(hipStreamSynchronize(s));
-        for (int q = 0; q < S; ++q) sliceCnt[q] = sliceStart[q + 1] - sliceStart[q];
     }
-    // ---- chunks: their lengths come down, the plan of the streams goes up
-    std::vector<std::vector<SliceChunk>> sliceChunks((size_t)S);
-    std::vector<int> firstIdx;
-    if (!fusedTaken) {
-        int at = 0;
-        for (int q = 0; q < S; ++q) {
-            for (int f = at; f < at + sliceCnt[q]; f += 64) {
-                sliceChunks[q].push_back({f, std::min(64, at + sliceCnt[q] - f), 0});
-                firstIdx.push_back(f);
-            }
-            at += sliceCnt[q];
-        }
-    }
-    const int nChunk = (int)firstIdx.size();
-    if (nChunk > 0 && !fusedTaken) {
-        Buf dFirst, dLen;
-        std::vector<int> len((size_t)nChunk);
-        MXL_TRY(mx::dev_malloc(&dFirst.p, (size_t)nChunk * 4));
-        MXL_TRY(mx::dev_malloc(&dLen.p, (size_t)nChunk * 4));
-        MXL_TRY(hipMemcpyAsync(dFirst.p, firstIdx.data(), (size_t)nChunk * 4, hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(gather_len_kernel, grid(nChunk), dim3(kBlock), 0, s, (const int *)sorted.p, (const int *)vLen.p,
-                           (const int *)dFirst.p, nChunk, dLen.as<int>());
-        MXL_TRY(hipGetLastError());
-        MXL_TRY(hipMemcpyAsync(len.data(), dLen.p, (size_t)nChunk * 4, hipMemcpyDeviceToHost, s));
-        MXL_TRY(hipStreamSynchronize(s));
-        int i = 0;
-        for (int q = 0; q < S; ++q)
-            for (SliceChunk &c : sliceChunks[q]) c.steps = (len[i++] + E - 1) / E;
-    }
-    if (!fusedTaken) {
-        const int rc = plan_slice_chunks(dtype, budget, S, sliceChunks, SP);
-        if (rc) return rc;
-    }
-    D.nWG = SP.nWG;
-    D.maxWgChunks = SP.maxWgChunks;
-    D.steps = SP.totalSteps;
-    D.chunks = SP.totalChunks;
+    // ---- chunks: which workgroup and wave streams which
+    ChunkPlan C;
     auto up = [&](void **dst, const void *src, size_t bytes) -> int {
         MXL_TRY(mx::dev_malloc(dst, std::max<size_t>(bytes, 4)));
         if (bytes) MXL_TRY(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, s));
         return MX_OK;
     };
     int rc;
-    if ((rc = up((void **)&D.wgDesc, SP.wgDesc.data(), SP.wgDesc.size() * 4))) return rc;
-    if ((rc = up((void **)&D.waveDesc, SP.waveDesc.data(), SP.waveDesc.size() * 4))) return rc;
-    if ((rc = up((void **)&D.chunkEnd, SP.chunkEnd.data(), SP.chunkEnd.size() * 4))) return rc;
     Buf chunkFirst, chunkN, chunkSteps, chunkStep0;
-    if ((rc = up(&chunkFirst.p, SP.chunkFirst.data(), SP.chunkFirst.size() * 4))) return rc;
-    if ((rc = up(&chunkN.p, SP.chunkN.data(), SP.chunkN.size() * 4))) return rc;
-    if ((rc = up(&chunkSteps.p, SP.chunkSteps.data(), SP.chunkSteps.size() * 4))) return rc;
-    if ((rc = up(&chunkStep0.p, SP.chunkStep0.data(), SP.chunkStep0.size() * 8))) return rc;
+    if (fusedTaken) {
+        C.nWG = SP.nWG;
+        C.maxWgChunks = SP.maxWgChunks;
+        C.totalSteps = SP.totalSteps;
+        C.totalChunks = SP.totalChunks;
+        if ((rc = up(&C.wgDesc.p, SP.wgDesc.data(), SP.wgDesc.size() * 4))) return rc;
+        if ((rc = up(&C.waveDesc.p, SP.waveDesc.data(), SP.waveDesc.size() * 4))) return rc;
+        if ((rc = up(&C.chunkEnd.p, SP.chunkEnd.data(), SP.chunkEnd.size() * 4))) return rc;
+        if ((rc = up(&chunkFirst.p, SP.chunkFirst.data(), SP.chunkFirst.size() * 4))) return rc;
+        if ((rc = up(&chunkN.p, SP.chunkN.data(), SP.chunkN.size() * 4))) return rc;
+        if ((rc = up(&chunkSteps.p, SP.chunkSteps.data(), SP.chunkSteps.size() * 4))) return rc;
+        if ((rc = up(&chunkStep0.p, SP.chunkStep0.data(), SP.chunkStep0.size() * 8))) return rc;
+        C.chunkFirst = chunkFirst.as<int>();
+        C.chunkN = chunkN.as<int>();
+        C.chunkSteps = chunkSteps.as<int>();
+        C.chunkStep0 = chunkStep0.as<long long>();
+    } else {
+        if ((rc = plan_chunks_device(dtype, budget, S, nV, (const unsigned *)keyOut.p, (unsigned)(cap + 1) * 3u, (const int *)sorted.p, (const int *)vLen.p, C, s)))
+            return rc;
+    }
+    D.wgDesc = (int *)C.wgDesc.take();
+    D.waveDesc = (int *)C.waveDesc.take();
+    D.chunkEnd = (int *)C.chunkEnd.take();
+    D.nWG = C.nWG;
+    D.maxWgChunks = C.maxWgChunks;
+    D.steps = C.totalSteps;
+    D.chunks = C.totalChunks;
     // ---- the streams
-    const size_t nEcol = ((size_t)SP.totalSteps + kSlicePadSteps) * 64 * E;
+    const size_t nEcol = ((size_t)C.totalSteps + kSlicePadSteps) * 64 * E;
     MXL_TRY(mx::dev_malloc((void **)&D.ecol, nEcol * 2));
     MXL_TRY(hipMemsetAsync(D.ecol, 0, nEcol * 2, s));
     MXL_TRY(mx::dev_malloc(&D.eval, nEcol * sizeof(V)));
@@ -813,19 +730,19 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     }
     MXL_TRY(mx::dev_malloc((void **)&D.segIdx, nv1 * 4));
     MXL_TRY(hipMemsetAsync(D.segIdx, 0, nv1 * 4, s));
-    if (SP.totalChunks > 0) {
-        hipLaunchKernelGGL(vrow_places_kernel, grid(SP.totalChunks * 64), dim3(kBlock), 0, s, (const int *)sorted.p, (const int *)chunkFirst.p,
-                           (const int *)chunkN.p, SP.totalChunks, D.segIdx);
+    if (C.totalChunks > 0) {
+        hipLaunchKernelGGL(vrow_places_kernel, grid(C.totalChunks * 64), dim3(kBlock), 0, s, (const int *)sorted.p, C.chunkFirst,
+                           C.chunkN, C.totalChunks, D.segIdx);
         MXL_TRY(hipGetLastError());
     }
     if (nnz > 0) {
         hipLaunchKernelGGL(place_entries_kernel<V>, grid(nnz), dim3(kBlock), 0, s, (const int *)start.p, (const int *)vid.p,
-                           (const int *)vStart.p, (const int *)vSlice.p, (const int *)D.segIdx, (const long long *)chunkStep0.p,
+                           (const int *)vStart.p, (const int *)vSlice.p, (const int *)D.segIdx, C.chunkStep0,
                            (const int *)ord.p, col, val, (const unsigned char *)codes.p, nnz, SW, D.ecol, (V *)D.eval,
                            nDict > 0 ? D.ecode : nullptr);
         MXL_TRY(hipGetLastError());
         hipLaunchKernelGGL(pad_columns_kernel, grid(nV), dim3(kBlock), 0, s, (const int *)vStart.p, (const int *)vLen.p, (const int *)vSlice.p,
-                           (const int *)D.segIdx, (const long long *)chunkStep0.p, (const int *)chunkSteps.p, (const int *)ord.p, col, nV, SW,
+                           (const int *)D.segIdx, C.chunkStep0, C.chunkSteps, (const int *)ord.p, col, nV, SW,
                            D.ecol);
         MXL_TRY(hipGetLastError());
     }
@@ -873,14 +790,14 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
                        D.heavyInfo);
     MXL_TRY(hipGetLastError());
     const size_t accBytes = dtype == MX_F64 ? 8 : 4;
-    MXL_TRY(mx::dev_malloc(&D.partial, ((size_t)SP.totalChunks * 64 + 64) * accBytes));
-    MXL_TRY(hipMemsetAsync(D.partial, 0, ((size_t)SP.totalChunks * 64 + 64) * accBytes, s));
+    MXL_TRY(mx::dev_malloc(&D.partial, ((size_t)C.totalChunks * 64 + 64) * accBytes));
+    MXL_TRY(hipMemsetAsync(D.partial, 0, ((size_t)C.totalChunks * 64 + 64) * accBytes, s));
     if (fusedTaken) {
         // what the one-launch kernel needs beyond the two-launch arrays (which stay valid: the plan falls back on them)
         std::vector<int> hSegIdx(nv1, 0), target;
         MXL_TRY(hipMemcpyAsync(hSegIdx.data(), D.segIdx, nv1 * 4, hipMemcpyDeviceToHost, s));
         MXL_TRY(hipStreamSynchronize(s));
-        fused_targets(rows, SP.nGroups, fusedPlaces, SP.totalChunks, hSegPtr.data(), hSegIdx.data(), target);
+        fused_targets(rows, SP.nGroups, fusedPlaces, C.totalChunks, hSegPtr.data(), hSegIdx.data(), target);
         D.nGroups = SP.nGroups;
         D.maxWgGroups = SP.maxWgGroups;
         D.placesPerRow = fusedPlaces;
