@@ -51,6 +51,21 @@ struct ChunkPlan {
 int plan_chunks_device(mx_dtype dtype, int budget, int S, int nV, const unsigned *sortedKey, unsigned perSlice, const int *sorted,
                        const int *vLen, ChunkPlan &P, hipStream_t s);
 
+// The one-launch form's part of a plan.
+struct FusedPlan {
+    int nGroups = 0, maxWgGroups = 0, places = 0;
+    Buf wgGroups, groupNeed;
+};
+// Whether plan_fused_device can make the plan: (XCD, slice) and a length are one digit each.
+bool fused_plan_on_device(int S, int cap);
+// plan_fused_records on the device: *taken, with `sorted` (the order in which the virtual rows are laid out), P and F filled, when the form is taken;
+// otherwise nothing is to be used.  vRow, vSlice, vLen: the virtual rows in the order of the rows.  One wait.
+int plan_fused_device(mx_dtype dtype, int budget, int S, int rows, int nnz, int cap, int nV, int mode, const int *rowPtr, const int *segPtr,
+                      const int *vRow, const int *vSlice, const int *vLen, int *sorted, ChunkPlan &P, FusedPlan &F, bool *taken, hipStream_t s);
+// fused_targets on the device: target [totalChunks * 64 + 64]
+int fused_targets_device(int nGroups, int places, long long totalChunks, const int *segPtr, const int *segIdx, const int *vRow, int nV, int *target,
+                         hipStream_t s);
+
 }  // namespace mxl
 
 #define MXL_TRY(call)                                                                                 \

@@ -638,11 +638,25 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
                            (const int *)segPtr.p, nV, nnz, cap, kSliceLightSegs, key.as<unsigned>(), pay.as<int>(), vLen.as<int>());
         MXL_TRY(hipGetLastError());
     }
-    // ---- the one-launch form, where it is wanted and the matrix suits it: the records of the virtual rows come
-    // down, the host plans (plan_fused_records: the same plan as the host route's), the order goes up
+    // ---- the one-launch form, where it is wanted and the matrix suits it (on the host where its digits are too many for the device:
+    // the records of the virtual rows come down, the plan goes up)
+    ChunkPlan C;
+    FusedPlan F;
+    if (fused && nV > 0 && !elsewhere && fused_plan_on_device(S, cap)) {
+        bool taken = false;
+        const int rc = plan_fused_device(dtype, budget, S, rows, nnz, cap, nV, fused, rowPtr, (const int *)segPtr.p, (const int *)vRow.p, (const int *)vSlice.p,
+                                         (const int *)vLen.p, sorted.as<int>(), C, F, &taken, s);
+        if (rc) return rc;
+        if (!taken) {
+            C.made.release();
+            F.wgGroups.release();
+        }
+        D.fused = taken;
+        fused = 0;
+    }
     SlicePlan SP;
     int fusedPlaces = 0;
-    bool fusedTaken = false;
+    bool fusedTaken = false;  // (by the host's plan; D.fused: by the device's)
     std::vector<int> hSegPtr;
     if (fused && nV > 0 && !elsewhere) {
         std::vector<int> hRowPtr((size_t)rows + 1), hSlice((size_t)nV), hLen((size_t)nV), hSorted;
@@ -661,7 +675,7 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
             MXL_TRY(hipStreamSynchronize(s));  // `hSorted` leaves scope
         }
     }
-    if (nV > 0 && !fusedTaken) {
+    if (nV > 0 && !fusedTaken && !D.fused) {
         unsigned keyBits = 1;
         while (keyBits < 32 && (1ull << keyBits) < (unsigned long long)S * (unsigned long long)(cap + 1) * 3ull) ++keyBits;
         size_t sortBytes = 0;
@@ -673,7 +687,6 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
                                           sorted.as<int>(), (size_t)nV, 0u, keyBits, s));
     }
     // ---- chunks: which workgroup and wave streams which
-    ChunkPlan C;
     auto up = [&](void **dst, const void *src, size_t bytes) -> int {
         MXL_TRY(mx::dev_malloc(dst, std::max<size_t>(bytes, 4)));
         if (bytes) MXL_TRY(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, s));
@@ -697,7 +710,7 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
         C.chunkN = chunkN.as<int>();
         C.chunkSteps = chunkSteps.as<int>();
         C.chunkStep0 = chunkStep0.as<long long>();
-    } else {
+    } else if (!D.fused) {
         if ((rc = plan_chunks_device(dtype, budget, S, nV, (const unsigned *)keyOut.p, (unsigned)(cap + 1) * 3u, (const int *)sorted.p, (const int *)vLen.p, C, s)))
             return rc;
     }
@@ -792,30 +805,41 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     const size_t accBytes = dtype == MX_F64 ? 8 : 4;
     MXL_TRY(mx::dev_malloc(&D.partial, ((size_t)C.totalChunks * 64 + 64) * accBytes));
     MXL_TRY(hipMemsetAsync(D.partial, 0, ((size_t)C.totalChunks * 64 + 64) * accBytes, s));
-    if (fusedTaken) {
+    if (fusedTaken || D.fused) {
         // what the one-launch kernel needs beyond the two-launch arrays (which stay valid: the plan falls back on them)
-        std::vector<int> hSegIdx(nv1, 0), target;
-        MXL_TRY(hipMemcpyAsync(hSegIdx.data(), D.segIdx, nv1 * 4, hipMemcpyDeviceToHost, s));
-        MXL_TRY(hipStreamSynchronize(s));
-        fused_targets(rows, SP.nGroups, fusedPlaces, C.totalChunks, hSegPtr.data(), hSegIdx.data(), target);
-        D.nGroups = SP.nGroups;
-        D.maxWgGroups = SP.maxWgGroups;
-        D.placesPerRow = fusedPlaces;
-        if ((rc = up((void **)&D.wgGroups, SP.wgGroups.data(), SP.wgGroups.size() * 4))) return rc;
-        if ((rc = up((void **)&D.groupNeed, SP.groupNeed.data(), SP.groupNeed.size() * 4))) return rc;
-        const size_t nTarget = target.size() + 64;  // (64 spare entries, zero)
-        MXL_TRY(mx::dev_malloc((void **)&D.fusedTarget, nTarget * 4));
-        MXL_TRY(hipMemsetAsync(D.fusedTarget, 0, nTarget * 4, s));
-        MXL_TRY(hipMemcpyAsync(D.fusedTarget, target.data(), target.size() * 4, hipMemcpyHostToDevice, s));
-        const size_t nCount = (size_t)SP.nGroups + 1, nClaim = (size_t)SP.nWG + 1;
-        const size_t sumBytes = ((size_t)SP.nGroups * fusedPlaces * kFusedGroupRows + 64) * accBytes;
+        const size_t nTarget = (size_t)C.totalChunks * 64 + 64;  // (64 spare entries, zero)
+        if (D.fused) {
+            D.nGroups = F.nGroups;
+            D.maxWgGroups = F.maxWgGroups;
+            D.placesPerRow = F.places;
+            D.wgGroups = (int *)F.wgGroups.take();
+            D.groupNeed = (int *)F.groupNeed.take();
+            MXL_TRY(mx::dev_malloc((void **)&D.fusedTarget, nTarget * 4));
+            if ((rc = fused_targets_device(F.nGroups, F.places, C.totalChunks, (const int *)segPtr.p, D.segIdx, (const int *)vRow.p, nV, D.fusedTarget, s)))
+                return rc;
+        } else {
+            std::vector<int> hSegIdx(nv1, 0), target;
+            MXL_TRY(hipMemcpyAsync(hSegIdx.data(), D.segIdx, nv1 * 4, hipMemcpyDeviceToHost, s));
+            MXL_TRY(hipStreamSynchronize(s));
+            fused_targets(rows, SP.nGroups, fusedPlaces, SP.totalChunks, hSegPtr.data(), hSegIdx.data(), target);
+            D.nGroups = SP.nGroups;
+            D.maxWgGroups = SP.maxWgGroups;
+            D.placesPerRow = fusedPlaces;
+            if ((rc = up((void **)&D.wgGroups, SP.wgGroups.data(), SP.wgGroups.size() * 4))) return rc;
+            if ((rc = up((void **)&D.groupNeed, SP.groupNeed.data(), SP.groupNeed.size() * 4))) return rc;
+            MXL_TRY(mx::dev_malloc((void **)&D.fusedTarget, nTarget * 4));
+            MXL_TRY(hipMemsetAsync(D.fusedTarget, 0, nTarget * 4, s));
+            MXL_TRY(hipMemcpyAsync(D.fusedTarget, target.data(), target.size() * 4, hipMemcpyHostToDevice, s));
+            MXL_TRY(hipStreamSynchronize(s));  // `target` leaves scope
+        }
+        const size_t nCount = (size_t)D.nGroups + 1, nClaim = (size_t)C.nWG + 1;
+        const size_t sumBytes = ((size_t)D.nGroups * D.placesPerRow * kFusedGroupRows + 64) * accBytes;
         MXL_TRY(mx::dev_malloc((void **)&D.groupCount, nCount * 4));
         MXL_TRY(hipMemsetAsync(D.groupCount, 0, nCount * 4, s));
         MXL_TRY(mx::dev_malloc((void **)&D.claim, nClaim * 4));
         MXL_TRY(hipMemsetAsync(D.claim, 0, nClaim * 4, s));
         MXL_TRY(mx::dev_malloc(&D.fusedSums, sumBytes));
         MXL_TRY(hipMemsetAsync(D.fusedSums, 0, sumBytes, s));
-        MXL_TRY(hipStreamSynchronize(s));  // `target` leaves scope
         D.fused = true;
     }
     if (segPtrOut) {

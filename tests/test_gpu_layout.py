@@ -35,3 +35,70 @@ def test_chunks_are_dealt_as_on_the_host(mx, dtype, rows, cols, lengths, ncu):
     A = mx.Csr(rows, cols, ptr, rng.integers(0, cols, ptr[-1]).astype(np.int32), rng.uniform(-1, 1, ptr[-1]).astype(dtype))
     H = _same_layout(mx, A, ncu)
     assert H["chunks"] >= rows // 64
+
+
+def _fused_case(name, rng):
+    """(matrix, whether the one-launch form takes it when it is asked for)"""
+    def m(lens, col, cols, dtype=np.float64):
+        ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        row = np.repeat(np.arange(len(lens)), lens)
+        return len(lens), cols, ptr, np.asarray(col(row), np.int32), rng.uniform(-1, 1, ptr[-1]).astype(dtype)
+    anywhere = lambda cols: (lambda row: rng.integers(0, cols, row.size))
+    few = lambda rows: rng.integers(0, 9, rows)
+    if name == "fewer groups than XCDs":
+        return m(np.full(7 * 256, 16), anywhere(16384), 16384), False
+    if name == "a group each":
+        return m(np.full(8 * 256, 16), anywhere(16384), 16384), True
+    if name == "a row more":
+        return m(4 * few(8 * 256 + 1), anywhere(16384), 16384), True
+    if name == "all entries in the last rows":
+        lens = np.zeros(20000, int)
+        lens[-300:] = 200
+        return m(lens, anywhere(40000), 40000), None
+    if name == "eight places":
+        lens = few(20000)
+        lens[7000] = 4000
+        return m(lens, lambda row: np.where(row == 7000, rng.integers(0, 8, row.size) * 16384, rng.integers(0, 130000, row.size)), 131072), False
+    if name == "eight places, no more":
+        lens = few(20000)
+        lens[7000] = 8
+        return m(lens, lambda row: np.where(row == 7000, np.arange(row.size) % 8 * 16384, rng.integers(0, 130000, row.size)), 131072), True
+    if name == "nine places":
+        lens = few(20000)
+        lens[7000] = 9
+        return m(lens, lambda row: np.where(row == 7000, np.arange(row.size) % 9 * 16384, rng.integers(0, 140000, row.size)), 9 * 16384), False
+    if name == "more slices than workgroups of an XCD":
+        return m(np.full(100000, 6), anywhere(33 * 65536), 33 * 65536, np.float16), False
+    if name == "as many":
+        return m(np.full(100000, 6), anywhere(32 * 65536), 32 * 65536, np.float16), True
+    if name == "a small part":
+        return m(few(60000), lambda row: np.where(rng.random(row.size) < 1e-4, 70000, 0) + rng.integers(0, 60000, row.size), 140000, np.float16), True
+    if name == "too many chunks for a workgroup":
+        return m(np.full(1700000, 1), anywhere(60000), 60000, np.float16), False
+    if name == "as many as it may have":
+        return m(np.full(1500000, 1), anywhere(60000), 60000, np.float16), True
+    assert name == "repeats"
+    return m(few(30000), lambda row: row // 300 * 100, 30000), True
+
+
+@pytest.mark.parametrize("name", ["fewer groups than XCDs", "a group each", "a row more", "all entries in the last rows", "eight places", "eight places, no more",
+                                  "nine places", "more slices than workgroups of an XCD", "as many", "a small part", "too many chunks for a workgroup",
+                                  "as many as it may have", "repeats"])
+def test_one_launch_plan_is_the_hosts(mx, monkeypatch, name):
+    """The one-launch form planned on the device and on the host: taken or refused alike, and every array the same."""
+    import torch
+    rng = np.random.default_rng(len(name))
+    (rows, cols, ptr, col, val), takes = _fused_case(name, rng)
+    A = mx.Csr(rows, cols, ptr, col, val)
+    flags = mx.MX_PLAN_CSR_SLICES | mx.MX_PLAN_FUSE
+    D = mx.Plan.from_device_csr(*(torch.from_numpy(a).cuda() for a in (ptr, col, val)), cols, flags)
+    P = mx.Partition(A, 0.0, 0.0)
+    monkeypatch.setenv("MX_LAYOUT", "host")
+    H = mx.Plan(P, flags)
+    monkeypatch.delenv("MX_LAYOUT")
+    assert H.info["csr_variant"] == D.info["csr_variant"] == 1
+    assert H.info["csr_fused"] == D.info["csr_fused"], H.info
+    assert takes is None or bool(D.info["csr_fused"]) == takes
+    assert H.arrays() == D.arrays()
+    x = torch.from_numpy(rng.integers(-2, 3, cols).astype(val.dtype)).cuda()
+    assert bool((H.spmv(x) == D.spmv(x)).all())
