@@ -203,68 +203,76 @@ __global__ __launch_bounds__(kBlock) void csr_offsets_kernel(const int4 *__restr
 
 // ---- laying a matrix out ----------------------------------------------------------------------------------
 
-// The distinct offsets of every chunk (one wave each), ascending, into offs[chunk][kMaxOffsets] and their
-// number into count[chunk].  totals[0] = 1 as soon as a chunk has more than kMaxOffsets; the waves that
-// start after that leave at once.  (A matrix of another kind costs the walk to the 65th offset in every chunk that is
-// under way by then: 0.19 ms for 16 million entries in a million rows.)
-__global__ __launch_bounds__(64) void offset_lists_kernel(const int *__restrict__ rowPtr, const int *__restrict__ col, int rows,
-                                                          int chunkRows, int *__restrict__ offs, int *__restrict__ count,
-                                                          int *totals)
+// The distinct offsets of every chunk (one workgroup each), ascending, into offs[chunk][kMaxOffsets] and their
+// number into count[chunk].  totals[0] = 1 as soon as a chunk has more than kMaxOffsets; the workgroups that
+// start after that leave at once.  A workgroup takes the chunk's entries as they lie, so a matrix of another kind is left after its first
+// few of them.  (A wave to a chunk with a row to a lane walked the rows one entry at a time: 190 us for 700 thousand rows of a power law, so 19; a stencil of 290 thousand rows 33 and 31.)
+__global__ __launch_bounds__(kBlock) void offset_lists_kernel(const int *__restrict__ rowPtr, const int *__restrict__ col, int rows,
+                                                              int chunkRows, int *__restrict__ offs, int *__restrict__ count,
+                                                              int *totals)
 {
+    __shared__ int start[mx::offsets_chunk_rows(false) + 1];
     __shared__ int table[kTable];
     __shared__ int list[kMaxOffsets];
-    __shared__ int found, n;
-    const int c = blockIdx.x, lane = threadIdx.x;
-    if (*(volatile int *)totals) return;
-    for (int i = lane; i < kTable; i += 64) table[i] = kFree;
-    if (lane == 0) found = n = 0;
+    __shared__ int found, n, stop;
+    const int c = blockIdx.x, tid = threadIdx.x;
+    const int r0 = c * chunkRows, inside = min(chunkRows, rows - r0);
+    if (tid == 0) {
+        stop = *(volatile int *)totals;  // (looked at once: all threads go or all stay)
+        found = n = 0;
+    }
+    for (int i = tid; i <= inside; i += kBlock) start[i] = rowPtr[r0 + i];
+    for (int i = tid; i < kTable; i += kBlock) table[i] = kFree;
     __syncthreads();
-    const int r0 = c * chunkRows, r1 = min(r0 + chunkRows, rows);
+    if (stop) return;
     bool tooMany = false;
-    for (int r = r0 + lane; r < r1 && !tooMany; r += 64) {
-        for (int p = rowPtr[r], e = rowPtr[r + 1]; p < e; ++p) {
-            const int off = col[p] - r;
-            unsigned h = ((unsigned)off * 2654435761u) >> 25;  // the upper seven bits
-            static_assert(kTable == 128, "seven bits of the product number the slots");
-            bool placed = false;
-            for (int step = 0; step < kTable && !placed && !tooMany; ++step) {
-                int t = *(volatile int *)&table[h];
-                if (t == kFree) {
-                    if (*(volatile int *)&found >= kMaxOffsets) {
-                        tooMany = true;
-                    } else {
-                        t = atomicCAS(&table[h], kFree, off);
-                        if (t == kFree) {
-                            atomicAdd(&found, 1);
-                            placed = true;
-                        }
+    for (int p = start[0] + tid; p < start[inside] && !tooMany; p += kBlock) {
+        int r = 0;  // the last row that begins at or before p
+#pragma unroll
+        for (int half = mx::offsets_chunk_rows(false) / 2; half; half >>= 1)
+            if (r + half < inside && start[r + half] <= p) r += half;
+        const int off = col[p] - (r0 + r);
+        unsigned h = ((unsigned)off * 2654435761u) >> 25;  // the upper seven bits
+        static_assert(kTable == 128, "seven bits of the product number the slots");
+        bool placed = false;
+        for (int step = 0; step < kTable && !placed && !tooMany; ++step) {
+            int t = *(volatile int *)&table[h];
+            if (t == kFree) {
+                if (*(volatile int *)&found > kMaxOffsets) {
+                    tooMany = true;
+                } else {
+                    t = atomicCAS(&table[h], kFree, off);
+                    if (t == kFree) {
+                        atomicAdd(&found, 1);
+                        placed = true;
                     }
                 }
-                if (t == off) placed = true;
-                h = (h + 1) & (kTable - 1);
             }
-            tooMany = tooMany || !placed;
-            if (tooMany) break;
+            if (t == off) placed = true;
+            h = (h + 1) & (kTable - 1);
+            if (!placed && *(volatile int *)&found > kMaxOffsets) tooMany = true;
         }
+        tooMany = tooMany || !placed || *(volatile int *)&found > kMaxOffsets;
     }
     __syncthreads();
-    // (up to 63 lanes may have passed the test above together: the count decides)
-    if (tooMany || found > kMaxOffsets) {
-        *(volatile int *)totals = 1;
+    // (others may have passed the test above together: the count decides.  A table that is full before it has been counted past
+    // kMaxOffsets holds more than that, too)
+    if (__syncthreads_or(tooMany) || found > kMaxOffsets) {
+        if (tid == 0 && *(volatile int *)totals == 0) *(volatile int *)totals = 1;  // (stores to one word take turns)
         return;
     }
-    for (int i = lane; i < kTable; i += 64) {
+    for (int i = tid; i < kTable; i += kBlock) {
         const int t = table[i];
         if (t != kFree) list[atomicAdd(&n, 1)] = t;
     }
     __syncthreads();
-    for (int i = lane; i < n; i += 64) {
-        const int v = list[i];
+    if (tid < n) {
+        const int v = list[tid];
         int rank = 0;
         for (int k = 0; k < n; ++k) rank += list[k] < v;
         offs[(size_t)c * kMaxOffsets + rank] = v;
     }
-    if (lane == 0) count[c] = n;
+    if (tid == 0) count[c] = n;
 }
 
 // units[c] = units of chunk c (one more element, zero); totals[1] += units, totals[2] = most offsets of a chunk
@@ -404,7 +412,7 @@ int build_offsets_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     MXO_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
     MXO_TRY(hipMemsetAsync(totals.p, 0, 256, s));
     int *tot = (int *)totals.p;
-    hipLaunchKernelGGL(offset_lists_kernel, dim3(nChunks), dim3(64), 0, s, rowPtr_dev, col_dev, rows, chunkRows, (int *)lists.p, (int *)count.p, tot);
+    hipLaunchKernelGGL(offset_lists_kernel, dim3(nChunks), dim3(kBlock), 0, s, rowPtr_dev, col_dev, rows, chunkRows, (int *)lists.p, (int *)count.p, tot);
     // (with whole 16-byte units of values; a dictionary counts again below)
     int U = 16 / (R * elem_size(dtype));
     hipLaunchKernelGGL(chunk_units_kernel, grid((long long)nChunks + 1), dim3(kBlock), 0, s, (const int *)count.p, nChunks, U, (int *)units.p, tot);
