@@ -186,14 +186,17 @@ __global__ __launch_bounds__(kBlock) void pad_columns_kernel(const int *__restri
     }
 }
 
-// rowInfo and the marks of the two lists (rows with 2..lightSegs virtual rows, rows with more)
+// rowInfo and the marks of the two lists (rows with 2..lightSegs virtual rows, rows with more).  facts[workgroup] = the most virtual
+// rows of any of its rows, and of its listed rows with at most lightSegs: a word of its own, because atomics on one word take turns
+// (one from every wave that had more than there was: 182 us for 700 thousand rows; so 7, and 6 in row_totals_kernel).
 __global__ __launch_bounds__(kBlock) void row_info_kernel(const int *__restrict__ segPtr, const int *__restrict__ segIdx,
                                                           const char *__restrict__ elsewhere, int rows, int lightSegs,
                                                           int *__restrict__ rowInfo, int *__restrict__ isLight, int *__restrict__ isHeavy,
-                                                          int *__restrict__ over4, int *__restrict__ most)
+                                                          int2 *__restrict__ facts)
 {
+    __shared__ int2 part[kBlock / 64];
     const int r = blockIdx.x * kBlock + threadIdx.x;
-    int n = 0;
+    int n = 0, light = 0;
     if (r < rows) {
         const int a = segPtr[r];
         n = segPtr[r + 1] - a;
@@ -203,25 +206,47 @@ __global__ __launch_bounds__(kBlock) void row_info_kernel(const int *__restrict_
         const bool listed = n > 1 && !fetched;
         isLight[r] = listed && n <= lightSegs;
         isHeavy[r] = listed && n > lightSegs;
-        if (listed && n <= lightSegs && n > 4 && *(volatile int *)over4 == 0) atomicOr(over4, 1);
+        if (listed && n <= lightSegs) light = n;
     } else if (r == rows) {  // the scans run over rows + 1 elements
         isLight[r] = isHeavy[r] = 0;
     }
-    // the most virtual rows of any row: one atomic per wave that brings more than there is already (a wave's every time
-    // is 16 thousand on one word for a million rows, 0.24 ms; so 0.13)
-    int m = n;
-    for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
-    if ((threadIdx.x & 63) == 0 && m > 1 && m > *(volatile int *)most) atomicMax(most, m);
+    for (int off = 32; off > 0; off >>= 1) {
+        n = max(n, __shfl_xor(n, off));
+        light = max(light, __shfl_xor(light, off));
+    }
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = int2{n, light};
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; ++w) {
+            n = max(n, part[w].x);
+            light = max(light, part[w].y);
+        }
+        facts[blockIdx.x] = int2{n, light};
+    }
 }
 
 // What the host asks for after the row marks and their running counts, in one place: one copy instead of four.
-__global__ void row_totals_kernel(const int *__restrict__ over4, const int *__restrict__ lightPos, const int *__restrict__ heavyPos, int rows,
-                                  int *__restrict__ out)
+__global__ __launch_bounds__(kBlock) void row_totals_kernel(const int2 *__restrict__ facts, int blocks, const int *__restrict__ lightPos,
+                                                            const int *__restrict__ heavyPos, int rows, int *__restrict__ out)
 {
-    out[0] = over4[0];
-    out[1] = over4[1];
-    out[2] = lightPos[rows];
-    out[3] = heavyPos[rows];
+    __shared__ int most, light;
+    if (threadIdx.x == 0) most = light = 0;
+    __syncthreads();
+    int2 m = {0, 0};
+#pragma unroll 4
+    for (int b = threadIdx.x; b < blocks; b += kBlock) {
+        m.x = max(m.x, facts[b].x);
+        m.y = max(m.y, facts[b].y);
+    }
+    atomicMax(&most, m.x);
+    atomicMax(&light, m.y);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        out[0] = light;
+        out[1] = most;
+        out[2] = lightPos[rows];
+        out[3] = heavyPos[rows];
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void row_lists_kernel(const int *__restrict__ segPtr, const int *__restrict__ segIdx,
@@ -544,7 +569,6 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     MXL_TRY(mx::dev_malloc(&ord.p, std::max<size_t>((size_t)nnz, 1) * 4));
     MXL_TRY(mx::dev_malloc(&flag.p, 256));
     MXL_TRY(hipMemsetAsync(flag.p, 0, 256, s));
-    int *over4 = flag.as<int>() + 1;
     Buf tmp;
     size_t scanBytes = 0, b2 = 0;
     const size_t nScan = (size_t)std::max(nnz, rows + 1) + 1;
@@ -768,28 +792,30 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
         MXL_TRY(hipMemcpyAsync(D.rowInfo + rows, fill.data(), fill.size() * 4, hipMemcpyHostToDevice, s));
         MXL_TRY(hipStreamSynchronize(s));  // `fill` leaves scope
     }
-    Buf isLight, isHeavy, lightPos, heavyPos;
+    Buf isLight, isHeavy, lightPos, heavyPos, facts;
     const size_t r1 = (size_t)rows + 1;
+    const int rowBlocks = (int)(((long long)rows + kBlock) / kBlock);
+    MXL_TRY(mx::dev_malloc(&facts.p, (size_t)rowBlocks * 8));
     MXL_TRY(mx::dev_malloc(&isLight.p, r1 * 4));
     MXL_TRY(mx::dev_malloc(&isHeavy.p, r1 * 4));
     MXL_TRY(mx::dev_malloc(&lightPos.p, r1 * 4));
     MXL_TRY(mx::dev_malloc(&heavyPos.p, r1 * 4));
-    hipLaunchKernelGGL(row_info_kernel, grid((long long)rows + 1), dim3(kBlock), 0, s, (const int *)segPtr.p, (const int *)D.segIdx, elsewhere,
-                       rows, kSliceLightSegs, D.rowInfo, isLight.as<int>(), isHeavy.as<int>(), over4, over4 + 1);
+    hipLaunchKernelGGL(row_info_kernel, dim3((unsigned)rowBlocks), dim3(kBlock), 0, s, (const int *)segPtr.p, (const int *)D.segIdx, elsewhere,
+                       rows, kSliceLightSegs, D.rowInfo, isLight.as<int>(), isHeavy.as<int>(), facts.as<int2>());
     MXL_TRY(hipGetLastError());
     MXL_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)isLight.p, lightPos.as<int>(), 0, r1, rocprim::plus<int>(), s));
     MXL_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)isHeavy.p, heavyPos.as<int>(), 0, r1, rocprim::plus<int>(), s));
     int got[4] = {0, 0, 0, 0};
-    hipLaunchKernelGGL(row_totals_kernel, dim3(1), dim3(1), 0, s, (const int *)over4, (const int *)lightPos.p, (const int *)heavyPos.p, rows,
+    hipLaunchKernelGGL(row_totals_kernel, dim3(1), dim3(kBlock), 0, s, (const int2 *)facts.p, rowBlocks, (const int *)lightPos.p, (const int *)heavyPos.p, rows,
                        flag.as<int>() + 16);
     MXL_TRY(hipGetLastError());
     MXL_TRY(hipMemcpyAsync(got, flag.as<int>() + 16, sizeof(got), hipMemcpyDeviceToHost, s));
     MXL_TRY(hipStreamSynchronize(s));
-    const int anyOver4 = got[0], mostVrows = got[1], nLight = got[2], nHeavy = got[3];
+    const int mostLight = got[0], mostVrows = got[1], nLight = got[2], nHeavy = got[3];
     D.nLight = nLight;
     D.nHeavy = nHeavy;
     D.mostVrows = std::max(mostVrows, nV > 0 ? 1 : 0);
-    const int places = anyOver4 ? kSliceLightSegs : 4;
+    const int places = mostLight > 4 ? kSliceLightSegs : 4;
     D.lightQuads = places / 4;
     MXL_TRY(mx::dev_malloc((void **)&D.lightRow, ((size_t)nLight + 1) * 4));
     MXL_TRY(hipMemsetAsync(D.lightRow, 0, ((size_t)nLight + 1) * 4, s));

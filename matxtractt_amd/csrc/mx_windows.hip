@@ -208,12 +208,16 @@ __global__ __launch_bounds__(64 * WAVES) void csr_window_kernel(const int2 *__re
 constexpr int kBuckets = mx::kWindowBuckets;
 
 // totals[0] = 1 where a row has more than kWindowLongest entries: a matrix with a tail of long rows is not looked at any
-// further (16 million entries in a million rows: 0.28 ms of counting columns)
+// further (16 million entries in a million rows: 0.28 ms of counting columns).  Few workgroups, one store each: stores to
+// one word take turns (a wave of every 64 rows storing for itself: 61 us for a million rows with four in a thousand too long; so 13).
+constexpr int kRowsBlocks = 256;
 __global__ __launch_bounds__(kBlock) void window_rows_kernel(const int *__restrict__ rowPtr, int rows, int *totals)
 {
-    const int r = blockIdx.x * kBlock + threadIdx.x;
-    const bool tooLong = r < rows && rowPtr[r + 1] - rowPtr[r] > mx::kWindowLongest;
-    if (__any(tooLong) && (threadIdx.x & 63) == 0) *(volatile int *)totals = 1;
+    bool tooLong = false;
+#pragma unroll 8
+    for (long long r = (long long)blockIdx.x * kBlock + threadIdx.x; r < rows; r += kRowsBlocks * kBlock)
+        tooLong |= rowPtr[r + 1] - rowPtr[r] > mx::kWindowLongest;
+    if (__syncthreads_or(tooLong) && threadIdx.x == 0) *(volatile int *)totals = 1;
 }
 
 // The window of a workgroup's rows: of its entries' columns, counted in buckets, the stretch of at most `widest` elements
@@ -442,7 +446,8 @@ int build_windows_device(mx_dtype dtype, int rows, int cols, int nnz, const int 
     auto body = [&]() -> int {
         MXW_TRY(mx::dev_malloc((void **)&D.window, (size_t)nWG * 8));
         MXW_TRY(hipMemsetAsync(counts.p, 0, 256 + 3 * countB, s));
-        hipLaunchKernelGGL(window_rows_kernel, dim3((unsigned)(((long long)rows + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, rowPtr_dev, rows, tot);
+        hipLaunchKernelGGL(window_rows_kernel, dim3((unsigned)std::min<long long>(kRowsBlocks, ((long long)rows + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
+                           rowPtr_dev, rows, tot);
         MXW_TRY(hipGetLastError());
         hipLaunchKernelGGL(window_find_kernel, dim3(nWG), dim3(kBlock), 0, s, rowPtr_dev, col_dev, rows, cols, nChunks, waves, epv, widest,
                            (int2 *)D.window, units, farSteps, alone, tot);
