@@ -279,7 +279,8 @@ __global__ __launch_bounds__(kBlock) void row_lists_kernel(const int *__restrict
 // table is written only when a workgroup meets a value for the first time -- so what bounds it is reading the
 // values: the plan of a constant 27-point stencil of 26.5 million binary64 entries is made in 10.7 ms, 16.7 with
 // the values sorted (5.8 million binary16 entries: 6.5 and 11.9 ms).  A workgroup that meets more than `most`
-// values raises the flag, and everybody stops.  Slot kDictSlots belongs to the pattern that marks free slots.
+// values raises the flag -- at once, also in the middle of its first entries (7.6 million distinct values: 47 us when the first thousand were gone through to the
+// end and the flag was stored by all, 8 so) -- and everybody stops.  Slot kDictSlots belongs to the pattern that marks free slots.
 constexpr int kDictSlots = 1024;
 constexpr unsigned long long kDictFree = ~0ull;
 template <typename V>
@@ -322,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void value_set_kernel(const V *__restrict__
 #pragma unroll
         for (int j = 0; j < E; ++j) {
             const long long k = k0 + j * kBlock + threadIdx.x;
-            if (k >= nnz) continue;
+            if (k >= nnz || *(volatile int *)&found > most) continue;
             int h = kDictSlots;
             if (b[j] != kDictFree) {
                 h = (int)dict_hash(b[j]);
@@ -350,7 +351,7 @@ __global__ __launch_bounds__(kBlock) void value_set_kernel(const V *__restrict__
         __syncthreads();
         if (threadIdx.x == 0 && (over || found > most || *(volatile int *)flag)) {
             stop = 1;
-            *(volatile int *)flag = 1;
+            if (*(volatile int *)flag == 0) *(volatile int *)flag = 1;  // (stores to one word take turns)
         }
         __syncthreads();
         if (stop) return;
@@ -420,21 +421,33 @@ __global__ __launch_bounds__(kBlock) void check_csr_kernel(const int *__restrict
     if (i < nnz && (unsigned)col[i] >= (unsigned)cols) atomicOr(bad, 2);
 }
 // sum += distinct 64-byte lines of x that the 64 entries of every stride-th window name: a lane per entry, which counts
-// when no lane below it has its line (a thread per window, comparing 64 columns with each other in turn, took 0.43 ms for
-// 65536 windows; a wave per window takes 0.06).  One atomic per workgroup.
+// when no lane below it has its line.  The lanes with a lane's line are found bit by bit, one ballot for each that differs in the wave (compared
+// with the other lanes' lines in turn instead: 84 us for the 118 thousand windows of 7.6 million entries; so 40).  One atomic per workgroup.
 constexpr int kLinesBlocks = 2048;
 __global__ __launch_bounds__(kBlock) void window_lines_kernel(const int *__restrict__ col, long long sampled, long long stride, int perLine,
                                                               unsigned long long *__restrict__ sum)
 {
     __shared__ int part[kBlock / 64];
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, waves = gridDim.x * (kBlock / 64);
     int d = 0;
-    for (long long i = (blockIdx.x * kBlock + threadIdx.x) >> 6; i < sampled; i += gridDim.x * (kBlock / 64)) {
-        const int l = col[i * stride * 64 + lane] / perLine;
-        bool seen = false;
-#pragma unroll 8
-        for (int b = 0; b < 63; ++b) seen |= lane > b && l == __builtin_amdgcn_readlane(l, b);
-        d += __popcll(__ballot(!seen));
+    long long i = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+    int c = i < sampled ? col[i * stride * 64 + lane] : 0;
+    for (; i < sampled; i += waves) {
+        const int line = c / perLine;
+        c = col[min(i + waves, sampled - 1) * stride * 64 + lane];  // (the next window's, on its way meanwhile)
+        const unsigned x = (unsigned)(line ^ __builtin_amdgcn_readfirstlane(line));
+        unsigned lo = ~0u, hi = ~0u, done = 0;
+        // (a bit that differs among the lanes, then the next)
+        for (unsigned long long any = __ballot(x != 0); any; any = __ballot((x & ~done) != 0)) {
+            const unsigned one = (unsigned)__builtin_amdgcn_readlane((int)(x & ~done), __builtin_ctzll(any)), bit = one & (0u - one);
+            const unsigned set = (x & bit) ? ~0u : 0u;
+            const unsigned long long b = __ballot(set != 0);
+            lo &= ~((unsigned)b ^ set);
+            hi &= ~((unsigned)(b >> 32) ^ set);
+            done |= bit;
+        }
+        const int below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+        d += __popcll(__ballot(below == 0));
     }
     if (lane == 0) part[threadIdx.x >> 6] = d;
     __syncthreads();
