@@ -10,7 +10,7 @@
 namespace mxl {
 
 constexpr int kBlock = 256;
-inline dim3 grid(long long n) { return dim3((unsigned)((n > 1 ? n : 1) + kBlock - 1) / kBlock); }
+inline dim3 grid(long long n) { return dim3((unsigned)(((n > 1 ? n : 1) + kBlock - 1) / kBlock)); }
 
 struct Buf {  // device memory released at scope exit unless taken
     void *p = nullptr;

@@ -29,29 +29,6 @@
 
 namespace mxl {
 
-// The row and, for now, the place in the order of every entry; flag |= 1 when some row's columns are not ascending.
-// (13 million entries in a million rows: 0.11 ms; row heads, a running maximum over them and a pass that compared, 0.35 ms)
-__global__ __launch_bounds__(kBlock) void entry_rows_kernel(const int *__restrict__ rowPtr, const int *__restrict__ col, int rows, int nnz,
-                                                            int *__restrict__ row, int *__restrict__ ord, int *__restrict__ flag)
-{
-    __shared__ mxr::TileRows T;
-    const int t0 = blockIdx.x * mxr::kTile;
-    mxr::tile_rows(rowPtr, rows, nnz, t0, T);
-    bool descends = false;
-#pragma unroll
-    for (int j = 0; j < mxr::kPer; ++j) {
-        const int i = j * kBlock + threadIdx.x, k = t0 + i;
-        if (i >= nnz - t0) break;
-        const int r = T.row[i];
-        row[k] = r;
-        ord[k] = k;
-        descends |= k > 0 && col[k] < col[k - 1] && (i > 0 ? T.row[i - 1] == r : rowPtr[r] < k);
-    }
-    // (one atomic per wave at most, and none once the flag is up: a matrix whose rows are all out of order would
-    // put one per entry on the same word, and half a million of them take four milliseconds)
-    if (__any(descends) && (threadIdx.x & 63) == 0 && *(volatile int *)flag == 0) atomicOr(flag, 1);
-}
-
 // The order of a row's entries by column, made inside their workgroups.
 struct RowColumns {
     const int *col;
@@ -60,59 +37,146 @@ struct RowColumns {
     __device__ __forceinline__ void put(int, int, unsigned, int e, int k) const { ord[k] = e; }
 };
 
-__global__ __launch_bounds__(kBlock) void sort_keys_kernel(const int *__restrict__ row, const int *__restrict__ col, int nnz,
+__global__ __launch_bounds__(kBlock) void sort_keys_kernel(const int *__restrict__ rowPtr, const int *__restrict__ col, int rows, int nnz,
                                                            int colBits, unsigned long long *__restrict__ key, int *__restrict__ pay)
 {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= nnz) return;
-    key[k] = ((unsigned long long)(unsigned)row[k] << colBits) | (unsigned)col[k];
-    pay[k] = k;
+    __shared__ mxr::TileRows T;
+    const int t0 = blockIdx.x * mxr::kTile;
+    mxr::tile_rows(rowPtr, rows, nnz, t0, T);
+#pragma unroll
+    for (int j = 0; j < mxr::kPer; ++j) {
+        const int i = j * kBlock + threadIdx.x, k = t0 + i;
+        if (i >= nnz - t0) break;
+        key[k] = ((unsigned long long)(unsigned)T.row[i] << colBits) | (unsigned)col[k];
+        pay[k] = k;
+    }
 }
 
-// runHead[k] = k where a run of one (row, slice) starts at position k of the ordered entries, 0 elsewhere
-__global__ __launch_bounds__(kBlock) void run_heads_kernel(const int *__restrict__ rowPtr, const int *__restrict__ row,
-                                                           const int *__restrict__ col, const int *__restrict__ ord, int nnz,
-                                                           int SW, int *__restrict__ runHead)
+// ---- virtual rows ----
+// Where the virtual rows start, a bit per entry (of a tile of kTile entries kWords words) and their number per tile.  A virtual
+// row starts at every cap-th entry of a run, the entries of a row in one slice; the run that a tile begins in is searched for, the rest is
+// found among the tile's own.  ord: the entries in ascending columns inside their rows, null where they are taken to lie so; then
+// *flag |= 1 where they do not, and nothing else is to be used.
+// (7.6 million entries in 700 thousand rows: rows and order of every entry, run heads, their running maximum, starts and their running sum,
+// 200 us with the records, in arrays of the length of the matrix; so 68.)
+constexpr int kWords = mxr::kTile / 64;
+template <int SW>
+__global__ __launch_bounds__(kBlock) void vrow_starts_kernel(const int *__restrict__ rowPtr, const int *__restrict__ col, const int *__restrict__ ord,
+                                                             int rows, int nnz, int cap, unsigned long long *__restrict__ startBits,
+                                                             int *__restrict__ tileStarts, int *__restrict__ flag)
 {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= nnz) return;
-    const bool head = k == rowPtr[row[k]] || col[ord[k]] / SW != col[ord[k - 1]] / SW;
-    runHead[k] = head ? k : 0;
+    __shared__ mxr::TileRows T;
+    __shared__ unsigned long long heads[kWords];
+    __shared__ int carry, starts;
+    const int t0 = blockIdx.x * mxr::kTile, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    mxr::tile_rows(rowPtr, rows, nnz, t0, T);
+    auto column = [&](int k) { return col[ord ? ord[k] : k]; };
+    if (w == 0) {
+        // the first entry of the run that entry t0 belongs to: the row's first in a slice that is not before t0's
+        const int q = column(t0) / SW;
+        int lo = min(rowPtr[T.row[0]], t0), hi = t0;
+        while (lo < hi) {
+            const int step = (hi - lo + 63) / 64;
+            const long long at = lo + (long long)lane * step;
+            const int before = __popcll(__ballot(at < hi && column((int)min(at, (long long)t0)) / SW < q));
+            if (before == 0) break;
+            hi = (int)min((long long)hi, lo + (long long)before * step);
+            lo += (before - 1) * step + 1;
+        }
+        if (lane == 0) {
+            carry = lo;
+            starts = 0;
+        }
+    }
+    bool descends = false;
+    int c[mxr::kPer];
+#pragma unroll
+    for (int j = 0; j < mxr::kPer; ++j) c[j] = column(t0 + min(j * kBlock + tid, nnz - 1 - t0));
+#pragma unroll
+    for (int j = 0; j < mxr::kPer; ++j) {
+        const int i = j * kBlock + tid, k = t0 + i;
+        int before = __shfl_up(c[j], 1);
+        bool head = false;
+        if (i < nnz - t0) {
+            const int r = T.row[i];
+            if (i > 0 ? T.row[i - 1] != r : rowPtr[r] == k) {
+                head = true;
+            } else {
+                if (lane == 0) before = column(k - 1);
+                head = before / SW != c[j] / SW;
+                descends |= c[j] < before;
+            }
+        }
+        const unsigned long long m = __ballot(head);
+        if (lane == 0) heads[j * (kBlock / 64) + w] = m;
+    }
+    if (!ord && __any(descends) && lane == 0 && *(volatile int *)flag == 0) atomicOr(flag, 1);
+    __syncthreads();
+    int mine = 0;
+#pragma unroll
+    for (int j = 0; j < mxr::kPer; ++j) {
+        const int i = j * kBlock + tid, k = t0 + i, word = j * (kBlock / 64) + w;
+        // the last head at or before the entry: in its word, in an earlier one, or the carry
+        const unsigned long long m = heads[word] & (~0ull >> (63 - lane));
+        const unsigned long long some = __ballot(lane < word && heads[min(lane, kWords - 1)] != 0);
+        int run = carry;
+        if (m) run = t0 + word * 64 + 63 - __builtin_clzll(m);
+        else if (some) {
+            const int v = 63 - __builtin_clzll(some);
+            run = t0 + v * 64 + 63 - __builtin_clzll(heads[v]);
+        }
+        const int d = k - run;  // (hardly any run is longer than cap: the division is for waves that have one)
+        const unsigned long long s = __ballot(i < nnz - t0 && (d == 0 || (d >= cap && d % cap == 0)));
+        if (lane == 0 && t0 + word * 64 < nnz) startBits[(size_t)blockIdx.x * kWords + word] = s;
+        mine += __popcll(s);
+    }
+    if (lane == 0) atomicAdd(&starts, mine);
+    __syncthreads();
+    if (tid == 0) tileStarts[blockIdx.x] = starts;
 }
+static_assert(kWords <= 64 && kBlock % 64 == 0, "a lane per word of a tile");
 
-struct MaxOp {
-    __device__ __host__ int operator()(int a, int b) const { return a > b ? a : b; }
-};
-
-// start[k] = 1 where a virtual row starts: every cap-th position of a run
-__global__ __launch_bounds__(kBlock) void vrow_starts_kernel(const int *__restrict__ runStart, int nnz, int cap, int *__restrict__ start)
+// per virtual row: where it starts, its slice; wordBase[i] = virtual rows before the i-th word.  A workgroup takes a tile.
+template <int SW>
+__global__ __launch_bounds__(kBlock) void vrow_records_kernel(const unsigned long long *__restrict__ startBits, const int *__restrict__ tileBase,
+                                                              const int *__restrict__ col, const int *__restrict__ ord, int nnz, int *__restrict__ wordBase,
+                                                              int *__restrict__ vStart, int *__restrict__ vSlice)
 {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k < nnz) start[k] = ((k - runStart[k]) % cap == 0) ? 1 : 0;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, t0 = blockIdx.x * mxr::kTile, words = min(kWords, (nnz - t0 + 63) >> 6);
+    const int word0 = blockIdx.x * kWords, base = tileBase[blockIdx.x];
+    const unsigned long long mine = lane < words ? startBits[word0 + lane] : 0;
+    int run = __popcll(mine), at = run;  // running sum over the tile's words, a lane each
+#pragma unroll
+    for (int off = 1; off < kWords; off <<= 1) {
+        const int o = __shfl_up(run, off);
+        if (lane >= off) run += o;
+    }
+    at = base + run - at;
+    if (w == 0 && lane < words) wordBase[word0 + lane] = at;
+#pragma unroll
+    for (int j = 0; j < mxr::kPer; ++j) {
+        const int word = j * (kBlock / 64) + w;
+        const unsigned long long m = __shfl(mine, word);
+        const int first = __shfl(at, word), k = t0 + word * 64 + lane;
+        if (!((m >> lane) & 1)) continue;
+        const int t = first + __popcll(m & ~(~0ull << lane));
+        vStart[t] = k;
+        vSlice[t] = col[ord ? ord[k] : k] / SW;
+    }
 }
 
-// per virtual row: where it starts, its row and slice
-__global__ __launch_bounds__(kBlock) void vrow_records_kernel(const int *__restrict__ start, const int *__restrict__ vid,
-                                                              const int *__restrict__ row, const int *__restrict__ col,
-                                                              const int *__restrict__ ord, int nnz, int SW, int *__restrict__ vStart,
-                                                              int *__restrict__ vRow, int *__restrict__ vSlice)
-{
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= nnz || !start[k]) return;
-    const int t = vid[k];
-    vStart[t] = k;
-    vRow[t] = row[k];
-    vSlice[t] = col[ord[k]] / SW;
-}
-
-// segPtr[r] = virtual rows before row r
-__global__ __launch_bounds__(kBlock) void seg_ptr_kernel(const int *__restrict__ rowPtr, const int *__restrict__ vid, int rows, int nnz,
-                                                         int nV, int *__restrict__ segPtr)
+// segPtr[r] = virtual rows before row r, and the row of every virtual row
+__global__ __launch_bounds__(kBlock) void seg_ptr_kernel(const int *__restrict__ rowPtr, const unsigned long long *__restrict__ startBits,
+                                                         const int *__restrict__ wordBase, int rows, int nnz, int nV, int *__restrict__ segPtr,
+                                                         int *__restrict__ vRow)
 {
     const int r = blockIdx.x * kBlock + threadIdx.x;
     if (r > rows) return;
-    const int p = r < rows ? rowPtr[r] : nnz;
-    segPtr[r] = p < nnz ? vid[p] : nV;
+    auto before = [&](int p) { return p < nnz ? wordBase[p >> 6] + __popcll(startBits[p >> 6] & ~(~0ull << (p & 63))) : nV; };
+    const int a = r < rows ? before(rowPtr[r]) : nV;
+    segPtr[r] = a;
+    if (r < rows)
+        for (int t = a, e = before(rowPtr[r + 1]); t < e; ++t) vRow[t] = r;
 }
 
 // the sort key of every virtual row: (slice, cap - length, kind of its row)
@@ -144,34 +208,37 @@ __global__ __launch_bounds__(kBlock) void vrow_places_kernel(const int *__restri
 
 // every entry to its place in the streams (see DeviceSlices: lanes' column offsets of a batch
 // contiguous, binary16 values likewise, binary64 values in sub-blocks of two per lane)
+// (The other way round, a wave per batch that collects its 512 entries: 114 instead of 105 us for 7.6 million entries of a power law, and 520
+// instead of 137 for 10.5 million binary16 entries out of order.  The entries of a chunk lie in as many rows as it has lanes, so every one
+// costs its own line or two then; here they are read as they lie, and the caches put the lines of the streams together.)
 template <typename V>
-__global__ __launch_bounds__(kBlock) void place_entries_kernel(const int *__restrict__ start, const int *__restrict__ vid,
-                                                               const int *__restrict__ vStart, const int *__restrict__ vSlice,
-                                                               const int *__restrict__ segIdx, const long long *__restrict__ chunkStep0,
-                                                               const int *__restrict__ ord, const int *__restrict__ col,
-                                                               const V *__restrict__ val, const unsigned char *__restrict__ code,
-                                                               int nnz, int SW, unsigned short *__restrict__ ecol, V *__restrict__ eval,
-                                                               unsigned char *__restrict__ ecode)
+__global__ __launch_bounds__(kBlock) void place_entries_kernel(const unsigned long long *__restrict__ startBits, const int *__restrict__ wordBase,
+                                                               const int *__restrict__ vStart, const int *__restrict__ segIdx,
+                                                               const long long *__restrict__ chunkStep0, const int *__restrict__ ord,
+                                                               const int *__restrict__ col, const V *__restrict__ val,
+                                                               const unsigned char *__restrict__ code, int nnz, unsigned short *__restrict__ ecol,
+                                                               V *__restrict__ eval, unsigned char *__restrict__ ecode)
 {
-    constexpr int BE = mx::kSliceBatchEntries;
+    constexpr int BE = mx::kSliceBatchEntries, SW = mx::kSliceBytes / (int)sizeof(V);
     const int k = blockIdx.x * kBlock + threadIdx.x;
     if (k >= nnz) return;
-    const int t = vid[k] + start[k] - 1;  // vid counts the starts before k
+    const int t = wordBase[k >> 6] + __popcll(startBits[k >> 6] & (~0ull >> (63 - (k & 63)))) - 1;  // the last that starts at or before k
     const int place = segIdx[t], l = place & 63;
     const size_t st = (size_t)chunkStep0[place >> 6] + (size_t)(k - vStart[t]), batch = st / BE, j = st % BE;
     const size_t atc = (batch * 64 + l) * BE + j;
     const size_t atv = sizeof(V) == 8 ? batch * 64 * BE + (j / 2) * 128 + (size_t)l * 2 + j % 2 : atc;
-    const int p = ord[k];
-    ecol[atc] = (unsigned short)(col[p] - vSlice[t] * SW);
+    const int p = ord ? ord[k] : k;
+    ecol[atc] = (unsigned short)(col[p] & (SW - 1));
     eval[atv] = val[p];
     if (ecode) ecode[atc] = code[p];
 }
 
 // the padding of every virtual row up to its chunk's longest member names the row's own last column
+template <int SW>
 __global__ __launch_bounds__(kBlock) void pad_columns_kernel(const int *__restrict__ vStart, const int *__restrict__ vLen,
-                                                             const int *__restrict__ vSlice, const int *__restrict__ segIdx,
+                                                             const int *__restrict__ segIdx,
                                                              const long long *__restrict__ chunkStep0, const int *__restrict__ chunkSteps,
-                                                             const int *__restrict__ ord, const int *__restrict__ col, int nV, int SW,
+                                                             const int *__restrict__ ord, const int *__restrict__ col, int nV,
                                                              unsigned short *__restrict__ ecol)
 {
     constexpr int BE = mx::kSliceBatchEntries;
@@ -179,7 +246,9 @@ __global__ __launch_bounds__(kBlock) void pad_columns_kernel(const int *__restri
     if (t >= nV) return;
     const int len = vLen[t], place = segIdx[t], l = place & 63, c = place >> 6;
     if (len <= 0) return;
-    const unsigned short last = (unsigned short)(col[ord[vStart[t] + len - 1]] - vSlice[t] * SW);
+    if (chunkSteps[c] <= len) return;
+    const int k = vStart[t] + len - 1;
+    const unsigned short last = (unsigned short)(col[ord ? ord[k] : k] & (SW - 1));
     for (int n = len; n < chunkSteps[c]; ++n) {
         const size_t st = (size_t)chunkStep0[c] + n, batch = st / BE, j = st % BE;
         ecol[(batch * 64 + l) * BE + j] = last;
@@ -576,39 +645,51 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     D.cols = cols;
     D.sliceCols = SW;
     D.nnz = nnz;
-    // ---- rows in ascending column order
-    Buf row, ord, flag;
-    MXL_TRY(mx::dev_malloc(&row.p, std::max<size_t>((size_t)nnz, 1) * 4));
-    MXL_TRY(mx::dev_malloc(&ord.p, std::max<size_t>((size_t)nnz, 1) * 4));
+    // ---- virtual rows, from the entries as they lie; where some row's columns are not ascending, from their order
+    Buf ordBuf, flag, startBits, tileStarts, tileBase, wordBase;
+    const size_t tiles = ((size_t)nnz + mxr::kTile - 1) / mxr::kTile, words = ((size_t)nnz + 63) / 64;
     MXL_TRY(mx::dev_malloc(&flag.p, 256));
+    MXL_TRY(mx::dev_malloc(&startBits.p, (words + 1) * 8));
+    MXL_TRY(mx::dev_malloc(&tileStarts.p, (tiles + 1) * 4));
+    MXL_TRY(mx::dev_malloc(&tileBase.p, (tiles + 1) * 4));
+    MXL_TRY(mx::dev_malloc(&wordBase.p, (words + 1) * 4));
     MXL_TRY(hipMemsetAsync(flag.p, 0, 256, s));
+    MXL_TRY(hipMemsetAsync(tileStarts.as<int>() + tiles, 0, 4, s));
     Buf tmp;
-    size_t scanBytes = 0, b2 = 0;
-    const size_t nScan = (size_t)std::max(nnz, rows + 1) + 1;
-    MXL_TRY(rocprim::inclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, nScan, MaxOp(), s));
-    MXL_TRY(rocprim::exclusive_scan(nullptr, b2, (const int *)nullptr, (int *)nullptr, 0, nScan, rocprim::plus<int>(), s));
-    scanBytes = std::max(scanBytes, b2);
+    size_t scanBytes = 0;
+    const size_t nScan = std::max(tiles, (size_t)rows + 1) + 1;
+    MXL_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, nScan, rocprim::plus<int>(), s));
     MXL_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
-    if (nnz > 0) {
-        hipLaunchKernelGGL(entry_rows_kernel, mxr::tile_grid(nnz), dim3(kBlock), 0, s, rowPtr, col, rows, nnz, row.as<int>(), ord.as<int>(),
-                           flag.as<int>());
+    constexpr int SliceCols = kSliceBytes / (int)sizeof(V);
+    const int *ord = nullptr;
+    int nV = 0;
+    auto find_vrows = [&](int *unsorted) -> int {
+        int got = 0;
+        hipLaunchKernelGGL(vrow_starts_kernel<SliceCols>, mxr::tile_grid(nnz), dim3(kBlock), 0, s, rowPtr, col, ord, rows, nnz, cap,
+                           startBits.as<unsigned long long>(), tileStarts.as<int>(), flag.as<int>());
         MXL_TRY(hipGetLastError());
-    }
-    int unsorted = 0;
-    MXL_TRY(hipMemcpyAsync(&unsorted, flag.p, 4, hipMemcpyDeviceToHost, s));
-    MXL_TRY(hipStreamSynchronize(s));
+        MXL_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)tileStarts.p, tileBase.as<int>(), 0, tiles + 1, rocprim::plus<int>(), s));
+        MXL_TRY(hipMemcpyAsync(&nV, tileBase.as<int>() + tiles, 4, hipMemcpyDeviceToHost, s));
+        MXL_TRY(hipMemcpyAsync(&got, flag.p, 4, hipMemcpyDeviceToHost, s));
+        MXL_TRY(hipStreamSynchronize(s));
+        *unsorted = got;
+        return MX_OK;
+    };
+    int unsorted = 0, rc;
+    if (nnz > 0 && (rc = find_vrows(&unsorted))) return rc;
     if (unsorted) {
         // inside a workgroup per row or group of rows, where there is no row too long for that
         // (15.8 million entries in a million rows: keys and radix sort 0.91 ms, so 0.39)
         Buf list;
         mxs::RowClasses classes{};
         int *count = flag.as<int>() + 8;
+        MXL_TRY(mx::dev_malloc(&ordBuf.p, (size_t)nnz * 4));
         MXL_TRY(mx::dev_malloc(&list.p, mxs::list_ints(nnz) * 4));
         MXL_TRY(mxs::classify_rows(rowPtr, rows, nnz, list.as<int>(), count, s));
         MXL_TRY(hipMemcpyAsync(classes.n, count, sizeof(classes.n), hipMemcpyDeviceToHost, s));
         MXL_TRY(hipStreamSynchronize(s));
         if (classes.n[mxs::kClasses] == 0) {
-            MXL_TRY(mxs::sort_rows(rowPtr, rows, nnz, list.as<int>(), classes, RowColumns{col, ord.as<int>()}, s));
+            MXL_TRY(mxs::sort_rows(rowPtr, rows, nnz, list.as<int>(), classes, RowColumns{col, ordBuf.as<int>()}, s));
         } else {
             int colBits = 1, rowBits = 1;
             while (colBits < 31 && (1ll << colBits) < (long long)cols) ++colBits;
@@ -621,35 +702,15 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
             MXL_TRY(mx::dev_malloc(&keyOut.p, (size_t)nnz * 8));
             MXL_TRY(mx::dev_malloc(&payIn.p, (size_t)nnz * 4));
             MXL_TRY(mx::dev_malloc(&tmp.p, sortBytes + 256));
-            hipLaunchKernelGGL(sort_keys_kernel, grid(nnz), dim3(kBlock), 0, s, (const int *)row.p, col, nnz, colBits,
+            hipLaunchKernelGGL(sort_keys_kernel, mxr::tile_grid(nnz), dim3(kBlock), 0, s, rowPtr, col, rows, nnz, colBits,
                                keyIn.as<unsigned long long>(), payIn.as<int>());
             MXL_TRY(hipGetLastError());
             MXL_TRY(rocprim::radix_sort_pairs(tmp.p, sortBytes, (const unsigned long long *)keyIn.p, keyOut.as<unsigned long long>(),
-                                              (const int *)payIn.p, ord.as<int>(), (size_t)nnz, 0u, (unsigned)(colBits + rowBits), s));
+                                              (const int *)payIn.p, ordBuf.as<int>(), (size_t)nnz, 0u, (unsigned)(colBits + rowBits), s));
         }
+        ord = ordBuf.as<int>();
+        if ((rc = find_vrows(&unsorted))) return rc;
     }
-    // ---- virtual rows
-    Buf runHead, runStart, start, vid;
-    MXL_TRY(mx::dev_malloc(&runHead.p, ((size_t)nnz + 1) * 4));
-    MXL_TRY(mx::dev_malloc(&runStart.p, ((size_t)nnz + 1) * 4));
-    MXL_TRY(mx::dev_malloc(&start.p, ((size_t)nnz + 1) * 4));
-    MXL_TRY(mx::dev_malloc(&vid.p, ((size_t)nnz + 1) * 4));
-    int nV = 0;
-    if (nnz > 0) {
-        hipLaunchKernelGGL(run_heads_kernel, grid(nnz), dim3(kBlock), 0, s, rowPtr, (const int *)row.p, col, (const int *)ord.p, nnz, SW,
-                           runHead.as<int>());
-        MXL_TRY(hipGetLastError());
-        MXL_TRY(rocprim::inclusive_scan(tmp.p, scanBytes, (const int *)runHead.p, runStart.as<int>(), (size_t)nnz, MaxOp(), s));
-        hipLaunchKernelGGL(vrow_starts_kernel, grid(nnz), dim3(kBlock), 0, s, (const int *)runStart.p, nnz, cap, start.as<int>());
-        MXL_TRY(hipGetLastError());
-        MXL_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)start.p, vid.as<int>(), 0, (size_t)nnz, rocprim::plus<int>(), s));
-        int lastVid = 0, lastStart = 0;
-        MXL_TRY(hipMemcpyAsync(&lastVid, vid.as<int>() + (nnz - 1), 4, hipMemcpyDeviceToHost, s));
-        MXL_TRY(hipMemcpyAsync(&lastStart, start.as<int>() + (nnz - 1), 4, hipMemcpyDeviceToHost, s));
-        MXL_TRY(hipStreamSynchronize(s));
-        nV = lastVid + lastStart;
-    }
-    runHead.release();
     D.vrows = nV;
     Buf vStart, vRow, vSlice, vLen, segPtr, key, keyOut, pay, sorted;
     const size_t nv1 = (size_t)nV + 1;
@@ -662,13 +723,14 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
     MXL_TRY(mx::dev_malloc(&keyOut.p, nv1 * 4));
     MXL_TRY(mx::dev_malloc(&pay.p, nv1 * 4));
     MXL_TRY(mx::dev_malloc(&sorted.p, nv1 * 4));
+    const unsigned long long *bits = startBits.as<unsigned long long>();
     if (nnz > 0) {
-        hipLaunchKernelGGL(vrow_records_kernel, grid(nnz), dim3(kBlock), 0, s, (const int *)start.p, (const int *)vid.p, (const int *)row.p,
-                           col, (const int *)ord.p, nnz, SW, vStart.as<int>(), vRow.as<int>(), vSlice.as<int>());
+        hipLaunchKernelGGL(vrow_records_kernel<SliceCols>, mxr::tile_grid(nnz), dim3(kBlock), 0, s, bits, (const int *)tileBase.p, col, ord, nnz,
+                           wordBase.as<int>(), vStart.as<int>(), vSlice.as<int>());
         MXL_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL(seg_ptr_kernel, grid((long long)rows + 1), dim3(kBlock), 0, s, rowPtr, (const int *)vid.p, rows, nnz, nV,
-                       segPtr.as<int>());
+    hipLaunchKernelGGL(seg_ptr_kernel, grid((long long)rows + 1), dim3(kBlock), 0, s, rowPtr, bits, (const int *)wordBase.p, rows, nnz, nV,
+                       segPtr.as<int>(), vRow.as<int>());
     MXL_TRY(hipGetLastError());
     if (nV > 0) {
         hipLaunchKernelGGL(vrow_keys_kernel, grid(nV), dim3(kBlock), 0, s, (const int *)vStart.p, (const int *)vRow.p, (const int *)vSlice.p,
@@ -729,7 +791,6 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
         if (bytes) MXL_TRY(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, s));
         return MX_OK;
     };
-    int rc;
     Buf chunkFirst, chunkN, chunkSteps, chunkStep0;
     if (fusedTaken) {
         C.nWG = SP.nWG;
@@ -786,14 +847,12 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
         MXL_TRY(hipGetLastError());
     }
     if (nnz > 0) {
-        hipLaunchKernelGGL(place_entries_kernel<V>, grid(nnz), dim3(kBlock), 0, s, (const int *)start.p, (const int *)vid.p,
-                           (const int *)vStart.p, (const int *)vSlice.p, (const int *)D.segIdx, C.chunkStep0,
-                           (const int *)ord.p, col, val, (const unsigned char *)codes.p, nnz, SW, D.ecol, (V *)D.eval,
+        hipLaunchKernelGGL(place_entries_kernel<V>, grid(nnz), dim3(kBlock), 0, s, bits, (const int *)wordBase.p, (const int *)vStart.p,
+                           (const int *)D.segIdx, C.chunkStep0, ord, col, val, (const unsigned char *)codes.p, nnz, D.ecol, (V *)D.eval,
                            nDict > 0 ? D.ecode : nullptr);
         MXL_TRY(hipGetLastError());
-        hipLaunchKernelGGL(pad_columns_kernel, grid(nV), dim3(kBlock), 0, s, (const int *)vStart.p, (const int *)vLen.p, (const int *)vSlice.p,
-                           (const int *)D.segIdx, C.chunkStep0, C.chunkSteps, (const int *)ord.p, col, nV, SW,
-                           D.ecol);
+        hipLaunchKernelGGL(pad_columns_kernel<SliceCols>, grid(nV), dim3(kBlock), 0, s, (const int *)vStart.p, (const int *)vLen.p, (const int *)D.segIdx,
+                           C.chunkStep0, C.chunkSteps, ord, col, nV, D.ecol);
         MXL_TRY(hipGetLastError());
     }
     // ---- how the sums become y

@@ -37,6 +37,26 @@ def test_chunks_are_dealt_as_on_the_host(mx, dtype, rows, cols, lengths, ncu):
     assert H["chunks"] >= rows // 64
 
 
+@pytest.mark.parametrize("dtype,lens,cols", [
+    (np.float64, [5000] * 9, 40000),                            # rows of several tiles, runs that tiles begin in, cut at the cap
+    (np.float64, [1024, 1023, 1, 1024, 0, 0, 2048, 512, 512], 60000),    # rows that end with a tile, and one entry off
+    (np.float64, [64, 0, 64, 1, 63, 128, 960, 0] * 6, 16384),   # ... with a word; one slice
+    (np.float16, [9000] + [3] * 4000, 140000),
+    (np.float64, [0] * 500 + [4159] + [0] * 9000 + [1], 20000), # mostly rows without entries; a last tile of one word
+    (np.float16, [1] * 70000, 300000),                          # a virtual row to an entry
+])
+@pytest.mark.parametrize("order", ["ascending", "any"])
+def test_virtual_rows_are_cut_as_on_the_host(mx, dtype, lens, cols, order):
+    rng = np.random.default_rng(len(lens) + cols)
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    col = rng.integers(0, cols, ptr[-1]).astype(np.int32)
+    if order == "ascending":
+        for r in np.nonzero(lens)[0] if len(lens) < 5000 else []:
+            col[ptr[r]:ptr[r + 1]].sort()
+    A = mx.Csr(len(lens), cols, ptr, col, rng.integers(-9, 10, ptr[-1]).astype(dtype))
+    _same_layout(mx, A, 7)
+
+
 def _fused_case(name, rng):
     """(matrix, whether the one-launch form takes it when it is asked for)"""
     def m(lens, col, cols, dtype=np.float64):
