@@ -10,7 +10,7 @@
 // last line), --tune (pick the two fractions from the 5x5 grid by timing each on the device,
 // then run with them), --estimate-tau (pick them from counts over the same grid, nothing timed), --partition-cache FILE (read the partition from FILE when it was made for a
 // matrix of this shape with these fractions, otherwise compute it and write FILE), --device-prep / --host-prep (the extraction runs on the GPU /
-// on the host cores; same partition; without either the GPU takes matrices of two million entries or more), --device-plan (the matrix is uploaded as it is and everything after
+// on the host cores; same partition; without either the GPU takes matrices of 131072 entries or more), --device-plan (the matrix is uploaded as it is and everything after
 // that -- extraction, the plan's decisions, its layouts -- happens on the GPU: mx_plan_create_device;
 // same plan, no partition on the host, so no --partition-cache and no checksum in the JSON record).
 // Precision is the build's: -Dfp64 -> FP64 binary, otherwise FP16.
@@ -98,7 +98,7 @@ int main(int argc, char **argv)
     double scale = 1.0;
     unsigned long long seed = 0;
     bool keepValues = false, json = false, tune = false, estimate = false, devicePlan = false;
-    int devicePrep = -1;  // -1: the GPU for a matrix of two million entries or more, the host otherwise
+    int devicePrep = -1;  // -1: the GPU for a matrix of 131072 entries or more, the host otherwise
     std::string cachePath;
     for (int i = 1; i < argc; ++i) {
         std::string a = argv[i];
@@ -227,7 +227,7 @@ int main(int argc, char **argv)
         std::cout << "---------------------------------------------------------" << std::endl;
         std::cout << "---------------------Compression Info--------------------" << std::endl;
     }
-    if (devicePrep < 0) devicePrep = nnzA >= (1 << 21) && extracting && mx_device_count() > 0;
+    if (devicePrep < 0) devicePrep = nnzA >= (1 << 17) && extracting && mx_device_count() > 0;
     if (devicePrep || devicePlan) (void)hipFree(nullptr);  // the first use of the device is not part of the preprocessing time
     auto t0 = std::chrono::steady_clock::now();
     mx_partition *part = nullptr;

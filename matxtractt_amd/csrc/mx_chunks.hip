@@ -853,7 +853,8 @@ __global__ __launch_bounds__(kBlock) void spare_targets_kernel(int n, int spare,
     if (i < n + 64) target[i] = i < n ? spare + (i & 63) : 0;
 }
 
-bool fused_plan_on_device(int S, int cap) { return X * S <= mxd::kDigits && cap < mxd::kDigits; }
+constexpr int kVrowsLeast = 16384;
+bool fused_plan_on_device(int S, int cap, int nV) { return X * S <= mxd::kDigits && cap < mxd::kDigits && nV >= kVrowsLeast; }
 
 int plan_fused_device(mx_dtype dtype, int budget, int S, int rows, int nnz, int cap, int nV, int mode, const int *rowPtr, const int *segPtr,
                       const int *vRow, const int *vSlice, const int *vLen, int *sorted, ChunkPlan &P, FusedPlan &F, bool *taken, hipStream_t s)

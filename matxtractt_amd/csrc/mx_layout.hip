@@ -737,11 +737,11 @@ static int build_slices_device_t(mx_dtype dtype, int rows, int cols, int nnz, co
                            (const int *)segPtr.p, nV, nnz, cap, kSliceLightSegs, key.as<unsigned>(), pay.as<int>(), vLen.as<int>());
         MXL_TRY(hipGetLastError());
     }
-    // ---- the one-launch form, where it is wanted and the matrix suits it (on the host where its digits are too many for the device:
-    // the records of the virtual rows come down, the plan goes up)
+    // ---- the one-launch form, where it is wanted and the matrix suits it (on the host where there are few virtual rows, or its digits
+    // are too many for the device: their records come down, the plan goes up)
     ChunkPlan C;
     FusedPlan F;
-    if (fused && nV > 0 && !elsewhere && fused_plan_on_device(S, cap)) {
+    if (fused && nV > 0 && !elsewhere && fused_plan_on_device(S, cap, nV)) {
         bool taken = false;
         const int rc = plan_fused_device(dtype, budget, S, rows, nnz, cap, nV, fused, rowPtr, (const int *)segPtr.p, (const int *)vRow.p, (const int *)vSlice.p,
                                          (const int *)vLen.p, sorted.as<int>(), C, F, &taken, s);

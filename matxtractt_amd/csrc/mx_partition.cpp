@@ -334,16 +334,35 @@ int mx::check_partition_args(const mx_csr *A, float tau_c, float tau_r, mx_parti
         set_error("mx_partition_create: rowPtr does not span [0, nnz]");
         return MX_ERR_ARG;
     }
-    for (int r = 0; r < A->rows; ++r)
-        if (A->rowPtr[r + 1] < A->rowPtr[r]) {
-            set_error("mx_partition_create: rowPtr not monotone");
-            return MX_ERR_ARG;
-        }
-    for (int p = 0; p < A->nnz; ++p)
-        if ((unsigned)A->colInd[p] >= (unsigned)A->cols) {
-            set_error("mx_partition_create: column index out of range");
-            return MX_ERR_ARG;
-        }
+    // (what is wrong is collected, with no way out at every line and entry: 4 million columns take 1.4 ms with one; and by all cores where there is much to look at)
+    const int rows = A->rows, nnz = A->nnz, *ptr = A->rowPtr, *ind = A->colInd;
+    const unsigned cols = (unsigned)A->cols;
+    auto look = [=](int r0, int r1, int p0, int p1) {  // 1 = rowPtr falls, 2 = a column outside
+        unsigned f = 0, o = 0;
+#pragma omp simd reduction(| : f)
+        for (int r = r0; r < r1; ++r) f |= (unsigned)(ptr[r + 1] < ptr[r]);
+#pragma omp simd reduction(| : o)
+        for (int p = p0; p < p1; ++p) o |= (unsigned)((unsigned)ind[p] >= cols);
+        return f | o << 1;
+    };
+    unsigned wrong = 0;
+    if (rows + (long long)nnz < 400000) {
+        wrong = look(0, rows, 0, nnz);
+    } else {
+        constexpr int parts = 64;
+#pragma omp parallel for schedule(static) reduction(| : wrong)
+        for (int k = 0; k < parts; ++k)
+            wrong |= look((int)((long long)rows * k / parts), (int)((long long)rows * (k + 1) / parts), (int)((long long)nnz * k / parts),
+                          (int)((long long)nnz * (k + 1) / parts));
+    }
+    if (wrong & 1) {
+        set_error("mx_partition_create: rowPtr not monotone");
+        return MX_ERR_ARG;
+    }
+    if (wrong & 2) {
+        set_error("mx_partition_create: column index out of range");
+        return MX_ERR_ARG;
+    }
     return MX_OK;
 }
 

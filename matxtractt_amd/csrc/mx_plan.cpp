@@ -398,6 +398,7 @@ int mxp::try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *col
     return MX_OK;
 }
 
+constexpr int kHostArraysUp = 1 << 20;  // entries of a part in host memory from which on it is laid out where it goes
 // Puts the CSR part on the device.  A matrix whose rows repeat a pattern of offsets, or reach into one window of x, takes
 // the form made for that (try_forms) where no tiles are kept beside it and nothing asks for another.  Three executable
 // forms exist for any matrix: row tiles with direct x gathers; column slices with x resident in LDS; and a split in which the long rows (most of
@@ -420,6 +421,28 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
     const int nnz = rowPtr[rows];
     const size_t es = (size_t)mx::elem_size(plan->dtype);
     plan->csr_nnz = nnz;
+    // A large part goes up once, as it is, and takes the device's route: the same plan, without the counts over all entries
+    // that the host would decide from (a million entries and more: binary64 power law 1.4 ms either way, blocks 1.3 and 1.1, a band 2.3 and 1.4; 2 million, 2.4 and
+    // 2.0, 2.4 and 1.3, 4.0 and 1.8; half a million 0.9 and 0.9 to 1.1).  Where there is no memory for that beside the plan, the host's route
+    // needs less at a time.
+    if (nnz >= kHostArraysUp && !mx::opt().layout_host && mx::opt().csr_kernel != 3 && !plan_autotune()) {
+        int *rp = nullptr, *ci = nullptr;
+        void *va = nullptr, *marks = nullptr;
+        int rc = upload(&rp, rowPtr, (size_t)rows + 1);
+        if (!rc) rc = upload(&ci, col, (size_t)nnz);
+        if (!rc) rc = upload_bytes(&va, val, (size_t)nnz * es);
+        if (!rc && stripRows) rc = upload_bytes(&marks, stripRows, (size_t)rows);
+        if (!rc) rc = setup_csr_part_device(plan, nnz, rp, ci, va, flags, (const char *)marks, segOut, alone);
+        (void)mx::dev_free(rp);
+        (void)mx::dev_free(ci);
+        (void)mx::dev_free(va);
+        (void)mx::dev_free(marks);
+        if (rc != MX_ERR_ALLOC) return rc;
+        free_csr(plan->csr);
+        free_slices(plan->slices);
+        plan->csr_variant = 0;
+        plan->fused = false;
+    }
     if (alone && may_look_for_form(flags) && forms_may_suit(plan->dtype, rows, cols, rowPtr, col)) {
         // (the offset and window forms are found and laid out on the device, whatever MX_LAYOUT says)
         int *rp = nullptr, *ci = nullptr;

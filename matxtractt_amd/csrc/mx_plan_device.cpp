@@ -23,8 +23,8 @@ using namespace mxp;
 // matrix crosses to the host but its row pointers (for the row-tile form) or the lengths of its
 // chunks (for the slice form).  `elsewhere_dev` (optional): marks of rows that another kernel writes; `alone`: no tile
 // form has a part in the product.
-static int setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags,
-                                 const char *elsewhere_dev, std::pair<std::vector<int>, std::vector<int>> *segOut = nullptr, bool alone = true)
+int mxp::setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags,
+                               const char *elsewhere_dev, std::pair<std::vector<int>, std::vector<int>> *segOut, bool alone)
 {
     const mx_dtype dtype = plan->dtype;
     const int rows = plan->rows, cols = plan->cols;

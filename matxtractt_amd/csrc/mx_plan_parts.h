@@ -40,7 +40,7 @@ inline int upload(T **dst, const T *src, size_t n, size_t pad = 0)
     const size_t total = std::max<size_t>(n + pad, 1);
     MX_HIP(mx::dev_malloc((void **)dst, total * sizeof(T)));
     if (pad || n == 0) MX_HIP(hipMemset(*dst, 0, total * sizeof(T)));
-    if (n) MX_HIP(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
+    if (n) MX_HIP(mx::copy_up ? mx::copy_up(*dst, src, n * sizeof(T)) : hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
     return MX_OK;
 }
 int upload_bytes(void **dst, const void *src, size_t n, size_t pad = 0);
@@ -265,6 +265,8 @@ bool may_look_for_form(int flags);
 bool forms_may_suit(mx_dtype dtype, int rows, int cols, const int *rowPtr, const int *col);
 // Tries the offset form, then the window form, on a CSR part in device memory; *took says whether the plan has its CSR part now.
 int try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took);
+int setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags,
+                          const char *elsewhere_dev, std::pair<std::vector<int>, std::vector<int>> *segOut = nullptr, bool alone = true);
 int setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const void *val, int flags, const char *stripRows = nullptr,
                    std::pair<std::vector<int>, std::vector<int>> *segOut = nullptr, bool alone = true);
 int tiles_worth(mx_dtype dtype, int fragM, int fragK, bool blocks64, double generalEntries, double generalFrags, double stripEntries,

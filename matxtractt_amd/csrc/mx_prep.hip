@@ -944,10 +944,10 @@ extern "C" int mx_partition_create_device(const mx_csr *A, float tau_c, float ta
     W->dc = (int *)W->order;
     W->dr = (int *)((unsigned char *)W->order + dcB);
     int *dc = W->dc, *dr = W->dr;
-    MXP_TRY(hipMemcpy(rp, A->rowPtr, ((size_t)rows + 1) * 4, hipMemcpyHostToDevice));
+    MXP_TRY(mx::copy_up(rp, A->rowPtr, ((size_t)rows + 1) * 4));
     if (nnz > 0) {
-        MXP_TRY(hipMemcpy(ci, A->colInd, (size_t)nnz * 4, hipMemcpyHostToDevice));
-        MXP_TRY(hipMemcpy(va, A->val, (size_t)nnz * es, hipMemcpyHostToDevice));
+        MXP_TRY(mx::copy_up(ci, A->colInd, (size_t)nnz * 4));
+        MXP_TRY(mx::copy_up(va, A->val, (size_t)nnz * es));
     }
     mx_selection sel{};
     int rc = mx_select_device(rows, cols, nnz, rp, ci, tau_c, tau_r, dc, dr, &sel, nullptr);

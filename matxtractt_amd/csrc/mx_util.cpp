@@ -379,4 +379,8 @@ IdleFrees::~IdleFrees()
 
 }  // namespace mx
 
-extern "C" void mx_release_memory(void) { mx::release_idle_memory(); }
+extern "C" void mx_release_memory(void)
+{
+    if (mx::release_staging) mx::release_staging();
+    mx::release_idle_memory();
+}

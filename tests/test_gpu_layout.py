@@ -68,9 +68,9 @@ def _fused_case(name, rng):
     if name == "fewer groups than XCDs":
         return m(np.full(7 * 256, 16), anywhere(16384), 16384), False
     if name == "a group each":
-        return m(np.full(8 * 256, 16), anywhere(16384), 16384), True
+        return m(np.full(8 * 256, 32), lambda row: np.arange(row.size) % 8 * 16384 + rng.integers(0, 16384, row.size), 131072), True
     if name == "a row more":
-        return m(4 * few(8 * 256 + 1), anywhere(16384), 16384), True
+        return m(np.full(8 * 256 + 1, 32), lambda row: np.arange(row.size) % 8 * 16384 + rng.integers(0, 16384, row.size), 131072), True
     if name == "all entries in the last rows":
         lens = np.zeros(20000, int)
         lens[-300:] = 200
@@ -97,15 +97,17 @@ def _fused_case(name, rng):
         return m(np.full(1700000, 1), anywhere(60000), 60000, np.float16), False
     if name == "as many as it may have":
         return m(np.full(1500000, 1), anywhere(60000), 60000, np.float16), True
+    if name.startswith("virtual rows"):
+        return m(np.full(int(name.split()[-1]), 9), anywhere(16384), 16384), True
     assert name == "repeats"
     return m(few(30000), lambda row: row // 300 * 100, 30000), True
 
 
 @pytest.mark.parametrize("name", ["fewer groups than XCDs", "a group each", "a row more", "all entries in the last rows", "eight places", "eight places, no more",
                                   "nine places", "more slices than workgroups of an XCD", "as many", "a small part", "too many chunks for a workgroup",
-                                  "as many as it may have", "repeats"])
+                                  "as many as it may have", "repeats", "virtual rows 16383", "virtual rows 16384"])
 def test_one_launch_plan_is_the_hosts(mx, monkeypatch, name):
-    """The one-launch form planned on the device and on the host: taken or refused alike, and every array the same."""
+    """The one-launch form planned on the device (from 16384 virtual rows on) and on the host: taken or refused alike, and every array the same."""
     import torch
     rng = np.random.default_rng(len(name))
     (rows, cols, ptr, col, val), takes = _fused_case(name, rng)
