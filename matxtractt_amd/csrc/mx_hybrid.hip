@@ -1098,8 +1098,22 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         MXH_TRY(hipGetLastError());
         hipLaunchKernelGGL(iota_kernel, grid(I.nDD), dim3(kBlock), 0, s, payIn.as<int>(), I.nDD);
         MXH_TRY(hipGetLastError());
-        MXH_TRY(rocprim::radix_sort_pairs(sortTmp.p, sortBytes, (const unsigned long long *)keyIn.p, I.blkKey.as<unsigned long long>(),
-                                          (const int *)payIn.p, I.blkPay.as<int>(), n, 0u, 64u, s));
+        // (a large sort takes eight bits at a time: only those that the numbers have, and one more that the mark of a twin alone has; a
+        // small one compares whole keys)
+        unsigned bcBits = 1, brBits = 1;
+        while (bcBits < 31 && (1ll << bcBits) < (long long)cols / 8 + 1) ++bcBits;
+        while (brBits < 31 && (1ll << brBits) < (long long)rows / 8 + 1) ++brBits;
+        if (n >= 1000000 && (bcBits + 7) / 8 + (brBits + 8) / 8 < 8) {
+            MXH_TRY(rocprim::radix_sort_pairs(sortTmp.p, sortBytes, (const unsigned long long *)keyIn.p, I.blkKey.as<unsigned long long>(),
+                                              (const int *)payIn.p, I.blkPay.as<int>(), n, 0u, bcBits, s));
+            MXH_TRY(rocprim::radix_sort_pairs(sortTmp.p, sortBytes, (const unsigned long long *)I.blkKey.p, keyIn.as<unsigned long long>(),
+                                              (const int *)I.blkPay.p, payIn.as<int>(), n, 32u, 32u + brBits + 1, s));
+            std::swap(I.blkKey.p, keyIn.p);
+            std::swap(I.blkPay.p, payIn.p);
+        } else {
+            MXH_TRY(rocprim::radix_sort_pairs(sortTmp.p, sortBytes, (const unsigned long long *)keyIn.p, I.blkKey.as<unsigned long long>(),
+                                              (const int *)payIn.p, I.blkPay.as<int>(), n, 0u, 64u, s));
+        }
         hipLaunchKernelGGL(block_runs_kernel, count_grid(I.nDD), dim3(kBlock), 0, s, (const unsigned long long *)I.blkKey.p, I.nDD, 48, cols, tot + 2);
         MXH_TRY(hipGetLastError());
     }
