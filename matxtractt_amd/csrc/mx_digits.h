@@ -5,6 +5,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 namespace mxd {
 
 constexpr int kThreads = 1024, kPer = 8, kTile = kThreads * kPer;  // entries that a workgroup puts in order at a time
@@ -156,6 +158,66 @@ static __global__ __launch_bounds__(kThreads) void bucket_starts_kernel(const in
     out = __syncthreads_or(out);
     const bool crowded = __syncthreads_or(max(n0, n1) > most);
     if (b == 0) *flag = (int)out + 2 * (int)crowded;
+}
+
+// ---- buckets of consecutive lines (columns): entries by line in two steps, bucket and line inside it ----
+constexpr int kBucketMean = 6800;     // entries of a bucket on average: nearly all then have at most kTile
+constexpr int kBucketsLeast = 64;     // but not so few buckets that most of the device has none
+// Buckets of `lines` output lines.  c / lines as a product: exact for c < kDigits * lines with lines <= kDigits, since the
+// error of `inverse`, below one, times c stays below 2^42 / lines.
+struct Buckets {
+    int n, bits, lines, lineBits;
+    unsigned long long inverse;  // 2^42 / lines, rounded up
+    __device__ __forceinline__ int of(int c) const { return (int)(((unsigned long long)(unsigned)c * inverse) >> 42); }
+};
+
+// count[tile][bucket] entries; bad[tile]: an index lies outside [0, inner)
+static __global__ __launch_bounds__(kThreads) void bucket_counts_kernel(const int *__restrict__ ind, int inner, int nnz, Buckets B, int tiles,
+                                                                 int *__restrict__ count, int *__restrict__ bad)
+{
+    __shared__ int here[kDigits];
+    const int t = tile_of_block(tiles);
+    if (t >= tiles) return;
+    const int t0 = t * kTile, tid = threadIdx.x, lane = tid & 63;
+    here[tid] = here[tid + kThreads] = 0;
+    __syncthreads();
+    int b[kPer];
+    bool out = false;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int i = j * kThreads + tid;
+        b[j] = -1;
+        if (i >= nnz - t0) continue;
+        const int c = ind[t0 + i];
+        if ((unsigned)c < (unsigned)inner) b[j] = B.of(c);
+        else out = true;
+    }
+    // (neighbours often share a bucket, and an atomic takes as long as lanes want the same word: the first lane's bucket is counted at once)
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int first = __builtin_amdgcn_readfirstlane(b[j]);
+        const unsigned long long same = __ballot(b[j] == first);
+        if (first >= 0 && lane == __builtin_ctzll(same)) atomicAdd(&here[first], __popcll(same));
+        if (b[j] >= 0 && b[j] != first) atomicAdd(&here[b[j]], 1);
+    }
+    out = __syncthreads_or(out);
+    if (tid == 0) bad[t] = out;
+    for (int k = tid; k < B.n; k += kThreads) count[(size_t)t * B.n + k] = here[k];
+}
+
+inline bool buckets_hold(int lines) { return lines >= 1 && lines <= kDigits * kDigits; }
+inline Buckets make_buckets(int inner, int nnz)
+{
+    Buckets B;
+    const long long mean = ((long long)nnz + kBucketMean - 1) / kBucketMean, wide = ((long long)inner + kDigits - 1) / kDigits;
+    B.n = (int)std::min<long long>(kDigits, std::max<long long>(kBucketsLeast, std::max(mean, wide)));
+    B.lines = (inner + B.n - 1) / B.n;
+    B.n = (inner + B.lines - 1) / B.lines;
+    B.bits = B.lineBits = 0;
+    while ((1 << B.bits) < B.n) ++B.bits;
+    while ((1 << B.lineBits) < B.lines) ++B.lineBits;
+    B.inverse = ((1ull << 42) + B.lines - 1) / B.lines;
+    return B;
 }
 
 }  // namespace mxd

@@ -12,6 +12,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include "mx_device.h"
+#include "mx_digits.h"
 #include "mx_entry_rows.h"
 #include "mx_internal.h"
 #include "mx_row_sort.h"
@@ -34,6 +35,47 @@ __global__ __launch_bounds__(kBlock) void index_histogram_kernel(const int *__re
     else atomicAdd(&cnt[c], 1);
 }
 
+constexpr int kBucketCounts = 1 << 21;  // entries from which on the two steps are the faster way (atomics 28 us a million; so 58 us for 2.2 million with
+                                        // what five launches take, 68 for 4.3)
+// The same through buckets of columns: the entries' places in their buckets, in any order, then the columns of a bucket counted in LDS.
+// (Atomics on memory: 330 us for 15.8 million entries in a million columns; so 120.)
+__global__ __launch_bounds__(mxd::kThreads) void bucket_columns_kernel(const int *__restrict__ ind, int nnz, int inner, mxd::Buckets B, int tiles,
+                                                                       const int *__restrict__ before, const int *__restrict__ first,
+                                                                       unsigned short *__restrict__ column)
+{
+    __shared__ int next[mxd::kDigits];
+    const int t = mxd::tile_of_block(tiles), tid = threadIdx.x;
+    if (t >= tiles) return;
+    const int t0 = t * mxd::kTile;
+    for (int k = tid; k < B.n; k += mxd::kThreads) next[k] = first[k] + before[(size_t)t * B.n + k];
+    __syncthreads();
+    int c[mxd::kPer];
+#pragma unroll
+    for (int j = 0; j < mxd::kPer; ++j) c[j] = ind[min(t0 + j * mxd::kThreads + tid, nnz - 1)];
+#pragma unroll
+    for (int j = 0; j < mxd::kPer; ++j) {
+        if (j * mxd::kThreads + tid >= nnz - t0 || (unsigned)c[j] >= (unsigned)inner) continue;
+        const int b = B.of(c[j]);
+        column[atomicAdd(&next[b], 1)] = (unsigned short)(c[j] - b * B.lines);
+    }
+}
+__global__ __launch_bounds__(mxd::kThreads) void count_columns_kernel(const unsigned short *__restrict__ column, const int *__restrict__ first, int inner,
+                                                                      mxd::Buckets B, int *__restrict__ cnt)
+{
+    __shared__ int here[mxd::kDigits];
+    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, p0 = first[b], p1 = first[b + 1], c0 = b * B.lines, lines = min(B.lines, inner - c0);
+    for (int k = tid; k < lines; k += mxd::kThreads) here[k] = 0;
+    __syncthreads();
+    for (int p = p0 + tid; p < p1; p = mx::next_of(p, p1, mxd::kThreads)) {
+        const int c = column[p], one = __builtin_amdgcn_readfirstlane(c);
+        const unsigned long long same = __ballot(c == one);  // (a crowded column)
+        if (lane == __builtin_ctzll(same)) atomicAdd(&here[one], __popcll(same));
+        if (c != one) atomicAdd(&here[c], 1);
+    }
+    __syncthreads();
+    for (int k = tid; k < lines; k += mxd::kThreads) cnt[c0 + k] = here[k];
+}
+
 // bad |= bit where v[i] lies outside [0, lim): the index arrays of a caller are looked at before a
 // kernel uses them as addresses.
 __global__ __launch_bounds__(kBlock) void range_check_kernel(const int *__restrict__ v, int n, int lim, int bit,
@@ -52,10 +94,75 @@ __global__ __launch_bounds__(kBlock) void pointer_check_kernel(const int *__rest
     if ((i == 0 && p != 0) || (i == n && p != total) || (i < n && ptr[i + 1] < p) || p < 0 || p > total) atomicOr(bad, bit);
 }
 
-__global__ __launch_bounds__(kBlock) void iota_kernel(int *__restrict__ v, int n)
+// most[0] = the highest of cnt [0, n), most[1] = the longest of the rows (both zeroed before)
+__global__ __launch_bounds__(kBlock) void highest_kernel(const int *__restrict__ cnt, int n, const int *__restrict__ rowPtr, int rows, int *__restrict__ most)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) v[i] = i;
+    __shared__ int a, b;
+    if (threadIdx.x == 0) a = b = 0;
+    __syncthreads();
+    int c = 0, l = 0;
+    const long long step = (long long)gridDim.x * kBlock;
+#pragma unroll 4
+    for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += step) c = max(c, cnt[i]);
+#pragma unroll 4
+    for (long long r = (long long)blockIdx.x * kBlock + threadIdx.x; r < rows; r += step) l = max(l, rowPtr[r + 1] - rowPtr[r]);
+    atomicMax(&a, c);
+    atomicMax(&b, l);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        atomicMax(&most[0], a);
+        atomicMax(&most[1], b);
+    }
+}
+
+// ---- lines by count, the highest first, those of one count ascending: a counting sort, eleven bits of `most - count` at a time.
+// (Two orders of a million lines, counts up to some thousands: a stable radix sort of 32-bit counts, which rocPRIM makes a merge sort of twenty launches of at this size,
+// 390 us; so 100.)
+struct CountDigit {
+    const int *cnt, *before;  // `before`: the order so far, null for the lines as they are numbered
+    int most, shift;
+    __device__ __forceinline__ int line(int i) const { return before ? before[i] : i; }
+    __device__ __forceinline__ int operator()(int i) const { return (max(most - cnt[line(i)], 0) >> shift) & (mxd::kDigits - 1); }
+};
+__global__ __launch_bounds__(mxd::kThreads) void count_digits_kernel(CountDigit digit, int n, int values, int tiles, int *__restrict__ count)
+{
+    __shared__ int here[mxd::kDigits];
+    const int t = mxd::tile_of_block(tiles), tid = threadIdx.x;
+    if (t >= tiles) return;
+    for (int k = tid; k < values; k += mxd::kThreads) here[k] = 0;
+    __syncthreads();
+    for (int i = tid; i < mxd::kTile && t * mxd::kTile + i < n; i += mxd::kThreads) {
+        const int d = digit(t * mxd::kTile + i), one = __builtin_amdgcn_readfirstlane(d);
+        const unsigned long long same = __ballot(d == one);  // (most lines have a count like their neighbours')
+        if ((tid & 63) == __builtin_ctzll(same)) atomicAdd(&here[one], __popcll(same));
+        if (d != one) atomicAdd(&here[d], 1);
+    }
+    __syncthreads();
+    for (int k = tid; k < values; k += mxd::kThreads) count[(size_t)t * values + k] = here[k];
+}
+__global__ __launch_bounds__(mxd::kThreads, 8) void order_digits_kernel(CountDigit digit, int n, int values, int bits, int tiles,
+                                                                        const int *__restrict__ before, const int *__restrict__ first,
+                                                                        int *__restrict__ order, int *__restrict__ sortedCnt)
+{
+    using namespace mxd;
+    __shared__ Digits digits;
+    __shared__ int start[kDigits];
+    const int t = tile_of_block(tiles), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if (t >= tiles) return;
+    const int t0 = t * kTile, size = min(kTile, n - t0);
+    for (int k = tid; k < values; k += kThreads) start[k] = first[k] + before[(size_t)t * values + k];
+    int d[kPer], at[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) d[j] = digit(t0 + min(w * kWave + j * 64 + lane, size - 1));
+    place_by_digit<false>([&](int j) { return d[j]; }, size, bits, digits, start, (int *)nullptr, at);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int i = w * kWave + j * 64 + lane;
+        if (i >= size) continue;
+        const int line = digit.line(t0 + i);
+        order[at[j]] = line;
+        sortedCnt[at[j]] = digit.cnt[line];
+    }
 }
 
 // The shortest prefix of the sorted counts whose sum reaches `target`, from their running sums:
@@ -235,13 +342,17 @@ __global__ __launch_bounds__(kBlock) void chunk_starts_kernel(const int *__restr
     if (w <= chunkNum) first[w] = ddRowPtr[min(w * mx::kFragM, dRows)];
 }
 
-// reach[0] = where the last chunk ends that is too long for a workgroup
-__global__ __launch_bounds__(kBlock) void long_chunks_kernel(const int *__restrict__ first, int chunkNum, int *__restrict__ reach)
+// reach[0] = where the last chunk ends that is too long for a workgroup, *chunks = the chunks up to that one
+__global__ __launch_bounds__(kBlock) void long_chunks_kernel(const int *__restrict__ first, int chunkNum, int *__restrict__ reach,
+                                                            int *__restrict__ chunks)
 {
     const int w = blockIdx.x * kBlock + threadIdx.x;
     const bool big = w < chunkNum && first[w + 1] - first[w] > mxs::kLongest;
     const unsigned long long m = __ballot(big);
-    if (m && (threadIdx.x & 63) == 63 - __builtin_clzll(m)) atomicMax(reach, first[w + 1]);
+    if (m && (threadIdx.x & 63) == 63 - __builtin_clzll(m)) {
+        atomicMax(reach, first[w + 1]);
+        atomicMax(chunks, w + 1);
+    }
 }
 
 // key = [chunk of the entry's row][column], payload = the entry, for the first n entries of A_dd: those of the chunks up to
@@ -399,21 +510,40 @@ struct Scratch {
 
 namespace mxp {
 
-// order[0..n) = the lines by count descending, ties by ascending line (a stable descending sort
-// of the counts with the line numbers as payload); then the prefix that reaches `target`.
-// cnt, order: device arrays of n; work: 3 n ints + 4; returns the prefix length and its sum.
-static int order_and_reach(const int *cnt, int n, int target, int *order, int *work, void *sortTmp, size_t sortBytes,
+// order[0..n) = the lines by count descending, ties by ascending line; then the prefix that reaches `target`.
+// cnt, order: device arrays of n, no count above `most`; work: 3 n ints + 4, digitTmp: digit_bytes(n); returns the
+// prefix length and its sum.
+static size_t digit_bytes(size_t n)
+{
+    return ((n + mxd::kTile - 1) / mxd::kTile * mxd::kDigits + 2 * mxd::kDigits + 64) * sizeof(int);
+}
+static int order_and_reach(const int *cnt, int n, int most, int target, int *order, int *work, int *digitTmp,
                            void *scanTmp, size_t scanBytes, hipStream_t s, int *len, int *sum)
 {
     static const char who[] = "mx_select_device";
     *len = 0;
     *sum = 0;
     if (n == 0) return MX_OK;
-    int *ids = work, *sortedCnt = work + n, *run = work + 2 * (size_t)n, *res = work + 3 * (size_t)n;
-    const int blocks = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(iota_kernel, dim3(blocks), dim3(kBlock), 0, s, ids, n);
+    int *other = work, *sortedCnt = work + n, *run = work + 2 * (size_t)n, *res = work + 3 * (size_t)n;
+    const int blocks = (n + kBlock - 1) / kBlock, tiles = (int)(((long long)n + mxd::kTile - 1) / mxd::kTile);
+    int *total = digitTmp, *first = total + mxd::kDigits, *flag = first + mxd::kDigits + 1, *count = total + 2 * mxd::kDigits + 64;
+    int passes = 1;
+    while (passes < 3 && (most >> (mxd::kDigitBits * passes)) > 0) ++passes;
+    const int *before = nullptr;
+    for (int p = 0; p < passes; ++p) {
+        int *out = (passes - 1 - p) % 2 == 0 ? order : other;  // (the last one writes `order`)
+        const int shift = p * mxd::kDigitBits, values = std::min(mxd::kDigits, (most >> shift) + 1);
+        int bits = 0;
+        while ((1 << bits) < values) ++bits;
+        const CountDigit digit{cnt, before, most, shift};
+        hipLaunchKernelGGL(count_digits_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, digit, n, values, tiles, count);
+        hipLaunchKernelGGL(mxd::bucket_offsets_kernel, dim3((unsigned)((values + 15) / 16)), dim3(1024), 0, s, count, values, tiles, total);
+        hipLaunchKernelGGL(mxd::bucket_starts_kernel, dim3(1), dim3(mxd::kThreads), 0, s, (const int *)total, values, n, (const int *)nullptr, 0, first, flag);
+        hipLaunchKernelGGL(order_digits_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, digit, n, values, bits, tiles, (const int *)count,
+                           (const int *)first, out, sortedCnt);
+        before = out;
+    }
     MXP_TRY(hipGetLastError());
-    MXP_TRY(rocprim::radix_sort_pairs_desc(sortTmp, sortBytes, cnt, sortedCnt, (const int *)ids, order, (size_t)n, 0u, 32u, s));
     MXP_TRY(rocprim::inclusive_scan(scanTmp, scanBytes, (const int *)sortedCnt, run, (size_t)n, rocprim::plus<int>(), s));
     const int init[4] = {-1, 0, 0, 0};
     MXP_TRY(hipMemcpyAsync(res, init, sizeof(init), hipMemcpyHostToDevice, s));
@@ -449,38 +579,55 @@ extern "C" int mx_select_device(int rows, int cols, int nnz, const int *rowPtr_d
     mx::MemScope scope(s);
     *out = mx_selection{0, 0, 0, 0};
     const size_t n = (size_t)std::max(rows, cols);
-    size_t sortBytes = 0, scanBytes = 0;
-    if (n > 0) {
-        MXP_TRY(rocprim::radix_sort_pairs_desc(nullptr, sortBytes, (const int *)nullptr, (int *)nullptr, (const int *)nullptr,
-                                               (int *)nullptr, n, 0u, 32u, s));
-        MXP_TRY(rocprim::inclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, n, rocprim::plus<int>(), s));
-    }
-    sortBytes = (sortBytes + 255) & ~(size_t)255;
+    size_t scanBytes = 0;
+    if (n > 0) MXP_TRY(rocprim::inclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, n, rocprim::plus<int>(), s));
+    const size_t digitB = (digit_bytes(n) + 255) & ~(size_t)255;
     // counts [n], work [3 n + 4], flag, dense flags [cols], the library's storage
     const size_t cntB = (n * sizeof(int) + 255) & ~(size_t)255, workB = ((3 * n + 4) * sizeof(int) + 255) & ~(size_t)255;
     const size_t denseB = ((size_t)cols + 255) & ~(size_t)255;
     Scratch scratch;
-    MXP_TRY(mx::dev_malloc(&scratch.p, cntB + workB + 256 + denseB + sortBytes + scanBytes + 256));
+    MXP_TRY(mx::dev_malloc(&scratch.p, cntB + workB + 256 + denseB + digitB + scanBytes + 256));
     unsigned char *base = (unsigned char *)scratch.p;
     int *cnt = (int *)base, *work = (int *)(base + cntB), *bad = (int *)(base + cntB + workB);
     unsigned char *dense = base + cntB + workB + 256;
-    void *sortTmp = dense + denseB, *scanTmp = dense + denseB + sortBytes;
+    int *digitTmp = (int *)(dense + denseB);
+    void *scanTmp = dense + denseB + digitB;
     const int eblocks = (nnz + kBlock - 1) / kBlock;
 
     // ---- column pass (test/test_autotc_spmv.cpp:1122-1141)
     MXP_TRY(hipMemsetAsync(base, 0, cntB + workB + 256 + denseB, s));
-    if (nnz > 0) {
+    if (nnz >= kBucketCounts && mxd::buckets_hold(cols)) {
+        const mxd::Buckets B = mxd::make_buckets(cols, nnz);
+        const int tiles = (int)(((long long)nnz + mxd::kTile - 1) / mxd::kTile);
+        const size_t countB = ((size_t)tiles * (B.n + 1) * 4 + 255) & ~(size_t)255, firstB = (2 * mxd::kDigits + 64) * sizeof(int);
+        Scratch held;
+        MXP_TRY(mx::dev_malloc(&held.p, countB + firstB + (size_t)nnz * 2));
+        int *count = (int *)held.p, *badTile = count + (size_t)tiles * B.n, *first = (int *)((unsigned char *)held.p + countB), *total = first + mxd::kDigits + 1;
+        unsigned short *column = (unsigned short *)((unsigned char *)held.p + countB + firstB);
+        hipLaunchKernelGGL(mxd::bucket_counts_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, colInd_dev, cols, nnz, B, tiles, count, badTile);
+        hipLaunchKernelGGL(mxd::bucket_offsets_kernel, dim3((unsigned)((B.n + 15) / 16)), dim3(1024), 0, s, count, B.n, tiles, total);
+        hipLaunchKernelGGL(mxd::bucket_starts_kernel, dim3(1), dim3(mxd::kThreads), 0, s, (const int *)total, B.n, nnz, (const int *)badTile, tiles, first, bad);
+        hipLaunchKernelGGL(bucket_columns_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, colInd_dev, nnz, cols, B, tiles, (const int *)count,
+                           (const int *)first, column);
+        hipLaunchKernelGGL(count_columns_kernel, dim3((unsigned)B.n), dim3(mxd::kThreads), 0, s, (const unsigned short *)column, (const int *)first, cols, B, cnt);
+        MXP_TRY(hipGetLastError());
+    } else if (nnz > 0) {
         hipLaunchKernelGGL(index_histogram_kernel, dim3(eblocks), dim3(kBlock), 0, s, colInd_dev, nnz, cols, cnt, bad);
         MXP_TRY(hipGetLastError());
     }
-    int badHost = 0;
-    MXP_TRY(hipMemcpyAsync(&badHost, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+    // (what the orders need to know of their counts comes down with the flag; a row has no more entries in selected columns than it has)
+    if (n > 0)
+        hipLaunchKernelGGL(highest_kernel, dim3((unsigned)std::min<size_t>(256, (n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, (const int *)cnt, cols, rowPtr_dev,
+                           rows, bad + 1);
+    MXP_TRY(hipGetLastError());
+    int got[3] = {0, 0, 0};
+    MXP_TRY(hipMemcpyAsync(got, bad, sizeof(got), hipMemcpyDeviceToHost, s));
     MXP_TRY(hipStreamSynchronize(s));
-    if (badHost) {
+    if (got[0]) {
         mx::set_error("mx_select_device: column index out of range");
         return MX_ERR_ARG;
     }
-    int rc = order_and_reach(cnt, cols, mx::threshold(nnz, tau_c), descColId_dev, work, sortTmp, sortBytes, scanTmp, scanBytes,
+    int rc = order_and_reach(cnt, cols, got[1], mx::threshold(nnz, tau_c), descColId_dev, work, digitTmp, scanTmp, scanBytes,
                              s, &out->dCols, &out->nnzColD);
     if (rc != MX_OK) return rc;
 
@@ -496,7 +643,7 @@ extern "C" int mx_select_device(int rows, int cols, int nnz, const int *rowPtr_d
                            (const unsigned char *)dense, rows, nnz, cnt);
         MXP_TRY(hipGetLastError());
     }
-    rc = order_and_reach(cnt, rows, mx::threshold(nnz, tau_r), descRowId_dev, work, sortTmp, sortBytes, scanTmp, scanBytes, s,
+    rc = order_and_reach(cnt, rows, got[2], mx::threshold(nnz, tau_r), descRowId_dev, work, digitTmp, scanTmp, scanBytes, s,
                          &out->dRows, &out->nnzRowD);
     return rc;
 }
@@ -674,8 +821,7 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
     const size_t es = (size_t)mx::elem_size(dtype);
     int colBits = 1, chunkBits = 1;
     while (colBits < 31 && (1ll << colBits) < (long long)dCols) ++colBits;
-    while (chunkBits < 31 && (1ll << chunkBits) < (long long)chunkNum) ++chunkBits;
-    const unsigned keyBits = (unsigned)(colBits + chunkBits);
+    // (chunkBits: of the numbers of the chunks that the radix sort is for; all keys are shifted by colBits alone)
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     auto grid = [](long long m) { return dim3((unsigned)((m + kBlock - 1) / kBlock)); };
     size_t scanBytes = 0;
@@ -708,18 +854,20 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
     {
         // the caller's A_dd is about to be used for addressing: pointers and column ids are looked at first
         int *bad = (int *)((unsigned char *)scanTmp + scanBytes);  // in the 256 spare bytes at the end
-        MXP_TRY(hipMemsetAsync(bad, 0, (3 + mxs::kClasses) * sizeof(int), s));
+        MXP_TRY(hipMemsetAsync(bad, 0, (4 + mxs::kClasses) * sizeof(int), s));
         hipLaunchKernelGGL(pointer_check_kernel, grid((long long)dRows + 1), dim3(kBlock), 0, s, ddRowPtr_dev, dRows, n, 1, bad);
         if (n > 0) hipLaunchKernelGGL(range_check_kernel, grid(n), dim3(kBlock), 0, s, ddColInd_dev, n, dCols, 2, bad);
         hipLaunchKernelGGL(chunk_starts_kernel, grid((long long)chunkNum + 1), dim3(kBlock), 0, s, ddRowPtr_dev, dRows, chunkNum, chunkFirst);
-        hipLaunchKernelGGL(long_chunks_kernel, grid((long long)chunkNum + 1), dim3(kBlock), 0, s, (const int *)chunkFirst, chunkNum, bad + 1);
+        hipLaunchKernelGGL(long_chunks_kernel, grid((long long)chunkNum + 1), dim3(kBlock), 0, s, (const int *)chunkFirst, chunkNum, bad + 1,
+                           bad + 3 + mxs::kClasses);
         MXP_TRY(hipGetLastError());
         MXP_TRY(mxs::classify_rows(chunkFirst, chunkNum, n, list, bad + 2, s));
-        int got[3 + mxs::kClasses] = {};
+        int got[4 + mxs::kClasses] = {};
         MXP_TRY(hipMemcpyAsync(got, bad, sizeof(got), hipMemcpyDeviceToHost, s));
         MXP_TRY(hipStreamSynchronize(s));
         const int badHost = got[0];
         nLong = got[1];
+        while (chunkBits < 31 && (1ll << chunkBits) < (long long)got[3 + mxs::kClasses]) ++chunkBits;
         std::copy(got + 2, got + 3 + mxs::kClasses, classes.n);
         if (badHost) {
             mx::set_error((badHost & 1) ? "mx_tiles_device: ddRowPtr does not rise from 0 to nnzRowD"
@@ -734,7 +882,7 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
         if (nLong > 0) {
             size_t sortBytes = 0;
             MXP_TRY(rocprim::radix_sort_pairs(nullptr, sortBytes, (const unsigned long long *)nullptr, (unsigned long long *)nullptr,
-                                              (const int *)nullptr, (int *)nullptr, (size_t)nLong, 0u, keyBits, s));
+                                              (const int *)nullptr, (int *)nullptr, (size_t)nLong, 0u, (unsigned)(colBits + chunkBits), s));
             Scratch sort;
             const size_t inB = al((size_t)nLong * 8), payB = al((size_t)nLong * 4);
             MXP_TRY(mx::dev_malloc(&sort.p, inB + payB + sortBytes + 256));
@@ -744,7 +892,7 @@ extern "C" int mx_tiles_device(mx_dtype dtype, int dRows, int dCols, int nnzRowD
                                colBits, keyIn, payIn);
             MXP_TRY(hipGetLastError());
             MXP_TRY(rocprim::radix_sort_pairs((unsigned char *)sort.p + inB + payB, sortBytes, (const unsigned long long *)keyIn, keyOut,
-                                              (const int *)payIn, payOut, (size_t)nLong, 0u, keyBits, s));
+                                              (const int *)payIn, payOut, (size_t)nLong, 0u, (unsigned)(colBits + chunkBits), s));
         }
         hipLaunchKernelGGL(tile_heads_kernel, grid(n), dim3(kBlock), 0, s, (const unsigned long long *)keyOut, n, head);
         MXP_TRY(hipGetLastError());

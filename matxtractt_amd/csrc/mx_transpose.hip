@@ -42,53 +42,9 @@ constexpr int kBlock = 256;
 constexpr int kMaxCount = 2147483647 - 2 * kBlock;
 
 // ---- the two steps ------------------------------------------------------------------------
-constexpr int kBucketMean = 6800;     // entries of a bucket on average: nearly all then have at most kTile
-constexpr int kBucketsLeast = 64;     // but not so few buckets that most of the device has none
 // Entries of one bucket at most: its workgroup takes 11 us for every 8192 of them while the others are done, and the radix sort has
 // to be the slower way still (a million entries, 16 thousand of them in one line: 113 us, radix sort 231; 8 million, 60 thousand: 349, 620).
 inline int most_of_bucket(int nnz) { return 65536 + nnz / 64; }
-
-// Buckets of `lines` output lines.  c / lines as a product: exact for c < kDigits * lines with lines <= kDigits, since the
-// error of `inverse`, below one, times c stays below 2^42 / lines.
-struct Buckets {
-    int n, bits, lines, lineBits;
-    unsigned long long inverse;  // 2^42 / lines, rounded up
-    __device__ __forceinline__ int of(int c) const { return (int)(((unsigned long long)(unsigned)c * inverse) >> 42); }
-};
-
-// count[tile][bucket] entries; bad[tile]: an index lies outside [0, inner)
-__global__ __launch_bounds__(kThreads) void bucket_counts_kernel(const int *__restrict__ ind, int inner, int nnz, Buckets B, int tiles,
-                                                                 int *__restrict__ count, int *__restrict__ bad)
-{
-    __shared__ int here[kDigits];
-    const int t = tile_of_block(tiles);
-    if (t >= tiles) return;
-    const int t0 = t * kTile, tid = threadIdx.x, lane = tid & 63;
-    here[tid] = here[tid + kThreads] = 0;
-    __syncthreads();
-    int b[kPer];
-    bool out = false;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int i = j * kThreads + tid;
-        b[j] = -1;
-        if (i >= nnz - t0) continue;
-        const int c = ind[t0 + i];
-        if ((unsigned)c < (unsigned)inner) b[j] = B.of(c);
-        else out = true;
-    }
-    // (neighbours often share a bucket, and an atomic takes as long as lanes want the same word: the first lane's bucket is counted at once)
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int first = __builtin_amdgcn_readfirstlane(b[j]);
-        const unsigned long long same = __ballot(b[j] == first);
-        if (first >= 0 && lane == __builtin_ctzll(same)) atomicAdd(&here[first], __popcll(same));
-        if (b[j] >= 0 && b[j] != first) atomicAdd(&here[b[j]], 1);
-    }
-    out = __syncthreads_or(out);
-    if (tid == 0) bad[t] = out;
-    for (int k = tid; k < B.n; k += kThreads) count[(size_t)t * B.n + k] = here[k];
-}
 
 // An entry between the two steps, in one piece: a store of a wave goes to as many places as it has lanes, whatever a lane
 // stores (line, source line and value in arrays of their own, put in order in LDS to be written side by side: 89 + 89 us
@@ -323,16 +279,8 @@ static int transpose_by_buckets(int outer, int inner, int nnz, const int *ptr, c
                                 bool *done, bool *checked, hipStream_t s)
 {
     *done = *checked = false;
-    if (inner < 1 || inner > kDigits * kDigits) return MX_OK;
-    Buckets B;
-    const long long mean = ((long long)nnz + kBucketMean - 1) / kBucketMean, wide = ((long long)inner + kDigits - 1) / kDigits;
-    B.n = (int)std::min<long long>(kDigits, std::max<long long>(kBucketsLeast, std::max(mean, wide)));
-    B.lines = (inner + B.n - 1) / B.n;
-    B.n = (inner + B.lines - 1) / B.lines;
-    B.bits = B.lineBits = 0;
-    while ((1 << B.bits) < B.n) ++B.bits;
-    while ((1 << B.lineBits) < B.lines) ++B.lineBits;
-    B.inverse = ((1ull << 42) + B.lines - 1) / B.lines;
+    if (!buckets_hold(inner)) return MX_OK;
+    const Buckets B = make_buckets(inner, nnz);
     const int buckets = B.n, tiles = (int)(((long long)nnz + kTile - 1) / kTile);
     typedef typename Moved<V>::Word Word;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };

@@ -124,3 +124,22 @@ def test_one_launch_plan_is_the_hosts(mx, monkeypatch, name):
     assert H.arrays() == D.arrays()
     x = torch.from_numpy(rng.integers(-2, 3, cols).astype(val.dtype)).cuda()
     assert bool((H.spmv(x) == D.spmv(x)).all())
+
+
+@pytest.mark.parametrize("rows,cols", [(8191, 8192), (8193, 8191), (20000, 3), (3, 20000), (5000, 40000), (1, 1)])
+@pytest.mark.parametrize("tau", [(1.0, 1.0), (0.6, 0.2)])
+def test_lines_by_count_are_the_hosts(mx, rows, cols, tau):
+    """Columns and rows ordered by count on the device: counts of one digit and of two (columns that every row names, a row of 4100
+    entries), ties, lines without entries, and as many lines as a tile has, one fewer and one more."""
+    rng = np.random.default_rng(rows + cols)
+    lens = rng.integers(0, 7, rows)
+    lens[rng.integers(0, rows, 2)] = min(cols, 4100)
+    row = np.repeat(np.arange(rows), lens)
+    col = np.where(rng.random(row.size) < 0.5, rng.integers(0, min(cols, 5), row.size), rng.integers(0, cols, row.size))
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    A = mx.Csr(rows, cols, ptr, col.astype(np.int32), rng.integers(-9, 10, row.size).astype(np.float64))
+    D, H = mx.Partition(A, *tau, device=True), mx.Partition(A, *tau, device=False)
+    for k in ("dCols", "dRows", "nnzColD", "nnzRowD"):
+        assert getattr(D, k) == getattr(H, k), k
+    for k in ("descColId", "rId", "ddRowPtr", "ddColInd", "cdRowPtr", "cdColInd", "chunkPtr", "fragPtr", "sparse_AToX_index"):
+        assert np.array_equal(getattr(D, k), getattr(H, k)), k
