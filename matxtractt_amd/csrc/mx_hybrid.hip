@@ -173,29 +173,32 @@ __device__ bool row_blocks(const int *__restrict__ ddRowPtr, const int *__restri
 __global__ __launch_bounds__(kBlock) void strip_candidates_kernel(const int *__restrict__ ddRowPtr, const int *__restrict__ ddCol,
                                                                   const int *__restrict__ descColId, const int *__restrict__ rId,
                                                                   const int *__restrict__ cdRowPtr, int dRows, int cols,
-                                                                  int *__restrict__ isCand)
+                                                                  int *__restrict__ isCand, int4 *__restrict__ rowKey)
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= dRows) return;
     RowBlocks R;
-    isCand[i] = row_blocks(ddRowPtr, ddCol, descColId, rId, cdRowPtr, i, cols, R) ? 1 : 0;
+    const bool is = row_blocks(ddRowPtr, ddCol, descColId, rId, cdRowPtr, i, cols, R);
+    isCand[i] = is ? 1 : 0;
+    if (!is) return;
+    auto block = [&](int k) { return k < R.nb ? R.b[k] : -1; };
+    rowKey[2 * (size_t)i] = make_int4(block(0), block(1), block(2), block(3));
+    rowKey[2 * (size_t)i + 1] = make_int4(block(4), block(5), block(6), block(7));
 }
-// candidates in row order: their row of A_dd, the first columns of their blocks (-1 = none) and how many
-__global__ __launch_bounds__(kBlock) void candidate_keys_kernel(const int *__restrict__ ddRowPtr, const int *__restrict__ ddCol,
-                                                                const int *__restrict__ descColId, const int *__restrict__ rId,
-                                                                const int *__restrict__ cdRowPtr, const int *__restrict__ isCand,
-                                                                const int *__restrict__ candPos, int dRows, int cols,
-                                                                int *__restrict__ candRow, int *__restrict__ candKey,
-                                                                int *__restrict__ candNb)
+// candidates in row order: their row of A_dd, the first columns of their blocks (-1 = none, behind the others) and how many.
+// (A row's blocks are kept from when it was looked at: finding them again took 118 us for 1.05 million rows, reading them 6.)
+__global__ __launch_bounds__(kBlock) void candidate_keys_kernel(const int *__restrict__ isCand, const int *__restrict__ candPos,
+                                                                const int4 *__restrict__ rowKey, int dRows, int *__restrict__ candRow,
+                                                                int4 *__restrict__ candKey, int *__restrict__ candNb)
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= dRows || !isCand[i]) return;
-    RowBlocks R;
-    (void)row_blocks(ddRowPtr, ddCol, descColId, rId, cdRowPtr, i, cols, R);
     const int j = candPos[i];
+    const int4 a = rowKey[2 * (size_t)i], b = rowKey[2 * (size_t)i + 1];
     candRow[j] = i;
-    candNb[j] = R.nb;
-    for (int k = 0; k < 8; ++k) candKey[(size_t)j * 8 + k] = k < R.nb ? R.b[k] : -1;
+    candNb[j] = (a.x >= 0) + (a.y >= 0) + (a.z >= 0) + (a.w >= 0) + (b.x >= 0) + (b.y >= 0) + (b.z >= 0) + (b.w >= 0);
+    candKey[2 * (size_t)j] = a;
+    candKey[2 * (size_t)j + 1] = b;
 }
 // candidates by (block 0, .., block 7, row); they are numbered in row order, and -1 (no block) comes first
 struct CandidateOrder {
@@ -987,7 +990,7 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
 
     // ---- binary16: rows of dense strips, grouped by their set of blocks
     if (wantStrips && dtype == MX_F16 && I.dRows > 0 && I.nDD > 0) {
-        Buf isCand, candPos, tmp;
+        Buf isCand, candPos, rowKey, tmp;
         size_t scanBytes = 0, b2 = 0;
         MXH_TRY(rocprim::exclusive_scan(nullptr, scanBytes, (const int *)nullptr, (int *)nullptr, 0, (size_t)I.dRows + 1, rocprim::plus<int>(), s));
         MXH_TRY(rocprim::inclusive_scan(nullptr, b2, (const int *)nullptr, (int *)nullptr, (size_t)I.dRows + 1, rocprim::plus<int>(), s));
@@ -995,9 +998,10 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
         MXH_TRY(mx::dev_malloc(&isCand.p, ((size_t)I.dRows + 1) * 4));
         MXH_TRY(mx::dev_malloc(&candPos.p, ((size_t)I.dRows + 1) * 4));
         MXH_TRY(mx::dev_malloc(&tmp.p, scanBytes + 256));
+        MXH_TRY(mx::dev_malloc(&rowKey.p, (size_t)I.dRows * 2 * sizeof(int4)));
         MXH_TRY(hipMemsetAsync(isCand.p, 0, ((size_t)I.dRows + 1) * 4, s));
         hipLaunchKernelGGL(strip_candidates_kernel, grid(I.dRows), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc, (const int *)I.dc,
-                           (const int *)I.dr, (const int *)I.cdp, I.dRows, cols, isCand.as<int>());
+                           (const int *)I.dr, (const int *)I.cdp, I.dRows, cols, isCand.as<int>(), rowKey.as<int4>());
         MXH_TRY(hipGetLastError());
         MXH_TRY(rocprim::exclusive_scan(tmp.p, scanBytes, (const int *)isCand.p, candPos.as<int>(), 0, (size_t)I.dRows + 1, rocprim::plus<int>(), s));
         int nCand = 0;
@@ -1009,9 +1013,8 @@ static int analyse_tail(HybridDevice::Impl &I, bool wantGeneral, bool wantStrips
             MXH_TRY(mx::dev_malloc(&I.candRow.p, nc * 4));
             MXH_TRY(mx::dev_malloc(&I.candKey.p, nc * 8 * 4));
             MXH_TRY(mx::dev_malloc(&I.candNb.p, nc * 4));
-            hipLaunchKernelGGL(candidate_keys_kernel, grid(I.dRows), dim3(kBlock), 0, s, (const int *)I.ddp, (const int *)I.ddc,
-                               (const int *)I.dc, (const int *)I.dr, (const int *)I.cdp, (const int *)isCand.p, (const int *)candPos.p, I.dRows,
-                               cols, I.candRow.as<int>(), I.candKey.as<int>(), I.candNb.as<int>());
+            hipLaunchKernelGGL(candidate_keys_kernel, grid(I.dRows), dim3(kBlock), 0, s, (const int *)isCand.p, (const int *)candPos.p, (const int4 *)rowKey.p,
+                               I.dRows, I.candRow.as<int>(), I.candKey.as<int4>(), I.candNb.as<int>());
             MXH_TRY(hipGetLastError());
             // one sort of the candidates by their whole keys (a stable pass per block, eight of them with a gather
             // of keys before each, took 0.94 ms for 210000 candidates; this one takes 0.38)
