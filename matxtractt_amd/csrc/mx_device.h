@@ -426,8 +426,7 @@ constexpr int kSlicePadSteps = 16;  // spare zero steps after the last of the st
 // arrays of `D` equal those of the host route byte for byte.  `elsewhere_dev`: optional marks per
 // row (device memory) as in the host route.  segPtrOut / segIdxOut (optional): host copies of the
 // virtual rows of every row.  `fused` (1 or 2, as in plan_fused_records): the one-launch form where the matrix
-// suits it (D.fused says whether it did) -- the records of the virtual rows come down, the plan goes up, the
-// entries never leave the device.
+// suits it (D.fused says whether it did); who plans it, the device or the host, fused_plan_on_device says.
 int build_slices_device(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *col_dev, const void *val_dev,
                         int nCU, int S, const char *elsewhere_dev, DeviceSlices &D, hipStream_t s, std::vector<int> *segPtrOut = nullptr,
                         std::vector<int> *segIdxOut = nullptr, int fused = 0);

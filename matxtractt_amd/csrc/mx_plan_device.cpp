@@ -20,8 +20,8 @@ using namespace mxp;
 
 // The CSR part of a plan from arrays in device memory: the form is chosen as setup_csr_part chooses
 // it -- the same counts, taken on the device -- and only that form is built, there.  Nothing of the
-// matrix crosses to the host but its row pointers (for the row-tile form) or the lengths of its
-// chunks (for the slice form).  `elsewhere_dev` (optional): marks of rows that another kernel writes; `alone`: no tile
+// matrix crosses to the host but its row pointers (for the row-tile form).
+// `elsewhere_dev` (optional): marks of rows that another kernel writes; `alone`: no tile
 // form has a part in the product.
 int mxp::setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags,
                                const char *elsewhere_dev, std::pair<std::vector<int>, std::vector<int>> *segOut, bool alone)
@@ -62,8 +62,7 @@ int mxp::setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, co
     if (env == 2 && S > 0) want[1] = true, want[0] = false;
     if (want[1]) {
         // (the one-launch form where the matrix suits it and the device deals its workgroups as the form assumes:
-        // the layout is made for it in the same pass -- the records of the virtual rows go to the host, its plan
-        // comes back, the entries stay)
+        // the layout is made for it in the same pass)
         int wantFused = !elsewhere_dev ? fused_wanted(flags, dtype, rows, S, -1, nCU) : 0;
         if (wantFused) {
             int ok = 0;
@@ -116,8 +115,8 @@ int mxp::setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, co
 }
 
 // A plan for y = A x from a CSR matrix that lives in device memory: nothing of the matrix crosses
-// to the host but its row pointers (for the row-tile form) or the lengths of its chunks (for the
-// slice form).  The form is chosen as in mx_plan_create -- the same counts, taken on the device --
+// to the host but its row pointers (for the row-tile form).
+// The form is chosen as in mx_plan_create -- the same counts, taken on the device --
 // so the plan equals the one mx_plan_create makes from a partition of the same matrix with
 // tau = (0, 0).
 extern "C" int mx_plan_create_device_csr(mx_dtype dtype, int rows, int cols, int nnz, const int *rowPtr_dev, const int *colInd_dev,
