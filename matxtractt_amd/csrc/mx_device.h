@@ -41,7 +41,8 @@ struct IdleFrees {
     IdleFrees &operator=(const IdleFrees &) = delete;
 };
 
-// The next of the places p, p + stride, .. below n; n where there is none (p + stride may be more than an int holds).
+// The next of the places p, p + stride, .. below n; n where there is none (p + stride may be more than an int holds).  A thread's own first of
+// the places [p, n) is next_of(p, n, thread): its number on top of a p near n may be more than an int holds, too.
 __host__ __device__ inline int next_of(int p, int n, int stride) { return n - p > stride ? p + stride : n; }
 // Rows, columns and entries that the kernels of the offset and window forms can number: a chunk reaches past the last row by fewer
 // rows than this leaves.  (The other routes on the device refuse more than that; from host arrays row tiles take it.)

@@ -5,6 +5,8 @@
 
 #include <algorithm>
 
+#include "mx_device.h"
+
 namespace mxr {
 
 constexpr int kBlock = 256;
@@ -57,7 +59,7 @@ __device__ __forceinline__ void tile_rows(const int *__restrict__ ptr, int rows,
         __syncthreads();
         return;
     }
-    for (int r = lo + 1 + tid; r < rows; r += kBlock) {
+    for (int r = mx::next_of(lo, rows, 1 + tid); r < rows; r = mx::next_of(r, rows, kBlock)) {
         const long long at = (long long)ptr[r] - t0;
         if (at >= size) break;
         if (at >= 0 && ptr[r + 1] > ptr[r]) T.row[at] = r - lo;

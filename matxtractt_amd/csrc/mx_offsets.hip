@@ -328,19 +328,19 @@ __global__ __launch_bounds__(kBlock) void chunk_values_kernel(const int *__restr
     int wrong = 0;
     const int p0 = start[0], size = start[r1 - r0] - p0;
     constexpr int AHEAD = 4;  // entries of a thread on their way at a time
-    for (int i0 = tid; i0 < size; i0 += AHEAD * kBlock) {
+    for (int i0 = tid; i0 < size; i0 = mx::next_of(i0, size, AHEAD * kBlock)) {
         int ci[AHEAD];
         S vi[AHEAD];
 #pragma unroll
         for (int k = 0; k < AHEAD; ++k) {
-            const int p = p0 + min(i0 + k * kBlock, size - 1);
+            const int p = p0 + min(mx::next_of(i0, size, k * kBlock), size - 1);
             ci[k] = col[p];
             if constexpr (DICT) vi[k] = code[p];
             else vi[k] = __builtin_bit_cast(S, val[p]);
         }
 #pragma unroll
         for (int k = 0; k < AHEAD; ++k) {
-            const int i = i0 + k * kBlock;
+            const int i = mx::next_of(i0, size, k * kBlock);
             if (i >= size) break;
             int r = 0;  // the last row that begins at or before the entry
 #pragma unroll

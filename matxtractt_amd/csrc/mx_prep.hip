@@ -66,7 +66,7 @@ __global__ __launch_bounds__(mxd::kThreads) void count_columns_kernel(const unsi
     const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, p0 = first[b], p1 = first[b + 1], c0 = b * B.lines, lines = min(B.lines, inner - c0);
     for (int k = tid; k < lines; k += mxd::kThreads) here[k] = 0;
     __syncthreads();
-    for (int p = p0 + tid; p < p1; p = mx::next_of(p, p1, mxd::kThreads)) {
+    for (int p = mx::next_of(p0, p1, tid); p < p1; p = mx::next_of(p, p1, mxd::kThreads)) {
         const int c = column[p], one = __builtin_amdgcn_readfirstlane(c);
         const unsigned long long same = __ballot(c == one);  // (a crowded column)
         if (lane == __builtin_ctzll(same)) atomicAdd(&here[one], __popcll(same));

@@ -168,19 +168,24 @@ static void csr_blocks()
     CHECK(mx_plan_get_info(&plan, &info) == MX_OK && info.csr_blocks == 500);
 }
 
-// The entries that one thread of a counting kernel looks at: all below n and n at the end, also where n is close to what an int
-// holds (2^31 - 513 entries are accepted).
+// The entries that one thread of a kernel looks at: all below n and n at the end, also where n is close to what an int
+// holds (2^31 - 513 entries are accepted): by the threads of a grid of 1024 workgroups, of a workgroup, of four entries on their way for each of its
+// threads, by tiles of 8192.
 static void strides()
 {
-    const int n = 2147483647 - 512, stride = 1024 * 256;
-    for (const int first : {0, stride - 1, n - 1, n - stride - 1, n - stride}) {
-        int p = first, steps = 0;
-        for (; p < n; p = mx::next_of(p, n, stride)) {
-            CHECK(p >= 0);
-            CHECK(++steps <= n / stride + 2);
+    const int n = 2147483647 - 512;
+    for (const int stride : {1024 * 256, 1024, 4 * 256, 8192})
+        for (const int first : {n - 3000000, n - 3000000 + stride - 1, n - 1, n - stride - 1, n - stride, n - stride + 1}) {
+            int p = first, steps = 0;
+            for (; p < n; p = mx::next_of(p, n, stride)) {
+                CHECK(p >= 0);
+                CHECK(++steps <= 3000000 / stride + 2);
+            }
+            CHECK(p == n && steps == (n - 1 - first) / stride + 1);
         }
-        CHECK(p == n && steps == (n - 1 - first) / stride + 1);
-    }
+    // the first of a thread, in a stretch that begins among the last places
+    for (const int p0 : {n - 5000, n - 1024, n - 1023, n - 1, n})
+        for (const int thread : {0, 1, 255, 1023, 1024}) CHECK(mx::next_of(p0, n, thread) == (thread < n - p0 ? p0 + thread : n));
     CHECK(mx::next_of(5, 3, 2) == 3 && mx::next_of(0, 1, 262144) == 1);
     // ... and matrices whose last chunk would not be numbered in an int do not take the forms
     CHECK(mx::forms_can_number(n, n, n) && !mx::forms_can_number(n + 1, 5, 5) && !mx::forms_can_number(5, n + 1, 5) && !mx::forms_can_number(5, 5, n + 1));
