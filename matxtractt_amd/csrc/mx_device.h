@@ -44,8 +44,8 @@ struct IdleFrees {
 // The next of the places p, p + stride, .. below n; n where there is none (p + stride may be more than an int holds).  A thread's own first of
 // the places [p, n) is next_of(p, n, thread): its number on top of a p near n may be more than an int holds, too.
 __host__ __device__ inline int next_of(int p, int n, int stride) { return n - p > stride ? p + stride : n; }
-// Rows, columns and entries that the kernels of the offset and window forms can number: a chunk reaches past the last row by fewer
-// rows than this leaves.  (The other routes on the device refuse more than that; from host arrays row tiles take it.)
+// Rows, columns and entries that the kernels which lay a matrix out can number: they reach past the last row or entry by fewer
+// than this leaves.  (From device arrays a plan refuses more than that; from host arrays the host's layouts take it.)
 inline bool forms_can_number(int rows, int cols, int nnz)
 {
     constexpr int most = 2147483647 - 512;

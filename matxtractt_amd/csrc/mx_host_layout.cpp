@@ -719,10 +719,10 @@ int upload_slices(mx_dtype dtype, int rows, int cols, const int *rowPtr, const i
                   std::pair<std::vector<int>, std::vector<int>> *segOut, int fused)
 {
     // The whole matrix: the layout is made on the device (the same arrays, in a fraction of the
-    // time for a large matrix); MX_LAYOUT=host keeps the host route, which also serves row subsets.
-    if (!sel && !mx::opt().layout_host) {
+    // time for a large matrix); MX_LAYOUT=host keeps the host route, which also serves row subsets and what the device cannot number.
+    const int nnz = rowPtr[rows];
+    if (!sel && !mx::opt().layout_host && mx::forms_can_number(rows, cols, nnz)) {
         const size_t es = (size_t)mx::elem_size(dtype);
-        const int nnz = rowPtr[rows];
         int *dRowPtr = nullptr, *dCol = nullptr;
         void *dVal = nullptr, *dElse = nullptr;
         int rc = upload(&dRowPtr, rowPtr, (size_t)rows + 1);

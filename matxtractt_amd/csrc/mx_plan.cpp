@@ -399,6 +399,12 @@ int mxp::try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *col
 }
 
 constexpr int kHostArraysUp = 1 << 20;  // entries of a part in host memory from which on it is laid out where it goes
+bool mxp::part_goes_up(int rows, int cols, int nnz)
+{
+    const mx::Options &o = mx::opt();
+    // (what the device's kernels cannot number, and what only the host makes, stays with the host's layouts)
+    return nnz >= kHostArraysUp && mx::forms_can_number(rows, cols, nnz) && !o.layout_host && o.csr_kernel != 3 && !o.autotune;
+}
 // Puts the CSR part on the device.  A matrix whose rows repeat a pattern of offsets, or reach into one window of x, takes
 // the form made for that (try_forms) where no tiles are kept beside it and nothing asks for another.  Three executable
 // forms exist for any matrix: row tiles with direct x gathers; column slices with x resident in LDS; and a split in which the long rows (most of
@@ -424,8 +430,9 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
     // A large part goes up once, as it is, and takes the device's route: the same plan, without the counts over all entries
     // that the host would decide from (a million entries and more: binary64 power law 1.4 ms either way, blocks 1.3 and 1.1, a band 2.3 and 1.4; 2 million, 2.4 and
     // 2.0, 2.4 and 1.3, 4.0 and 1.8; half a million 0.9 and 0.9 to 1.1).  Where there is no memory for that beside the plan, the host's route
-    // needs less at a time.
-    if (nnz >= kHostArraysUp && !mx::opt().layout_host && mx::opt().csr_kernel != 3 && !plan_autotune()) {
+    // needs less at a time; and where the slices would have more places than an int numbers, which the device finds out when it lays them
+    // out (its one reason to refuse a matrix that was looked at), the host's route may not want slices at all.
+    if (part_goes_up(rows, cols, nnz)) {
         int *rp = nullptr, *ci = nullptr;
         void *va = nullptr, *marks = nullptr;
         int rc = upload(&rp, rowPtr, (size_t)rows + 1);
@@ -437,7 +444,7 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
         (void)mx::dev_free(ci);
         (void)mx::dev_free(va);
         (void)mx::dev_free(marks);
-        if (rc != MX_ERR_ALLOC) return rc;
+        if (rc != MX_ERR_ALLOC && rc != MX_ERR_ARG) return rc;
         free_csr(plan->csr);
         free_slices(plan->slices);
         plan->csr_variant = 0;

@@ -265,6 +265,8 @@ bool may_look_for_form(int flags);
 bool forms_may_suit(mx_dtype dtype, int rows, int cols, const int *rowPtr, const int *col);
 // Tries the offset form, then the window form, on a CSR part in device memory; *took says whether the plan has its CSR part now.
 int try_forms(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags, bool *took);
+// Whether a CSR part in host memory goes up as it is and takes the device's route.
+bool part_goes_up(int rows, int cols, int nnz);
 int setup_csr_part_device(mx_plan *plan, int nnz, const int *rowPtr_dev, const int *colInd_dev, const void *val_dev, int flags,
                           const char *elsewhere_dev, std::pair<std::vector<int>, std::vector<int>> *segOut = nullptr, bool alone = true);
 int setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const void *val, int flags, const char *stripRows = nullptr,

@@ -2,18 +2,19 @@
 // their names.  The sanitizer driver never reaches them.
 #include "mx_device.h"
 namespace mx {
+// (weak: a check may answer itself)
 hipError_t launch_tiles(mx_dtype, const DeviceTiles &, const void *, void *, int, hipStream_t, const void *) { return hipErrorUnknown; }
 hipError_t launch_csr(mx_dtype, const DeviceCsr &, const void *, void *, int, hipStream_t, void *) { return hipErrorUnknown; }
 hipError_t launch_slices(mx_dtype, const DeviceSlices &, const void *, void *, int, hipStream_t, int, const DeviceTiles *, void *) { return hipErrorUnknown; }
 hipError_t launch_fused(mx_dtype, const DeviceSlices &, const void *, void *, int, hipStream_t, void *, unsigned *, unsigned) { return hipErrorUnknown; }
-hipError_t fused_placement_ok(int, int *ok) { *ok = 0; return hipErrorUnknown; }
+__attribute__((weak)) hipError_t fused_placement_ok(int, int *ok) { *ok = 0; return hipErrorUnknown; }
 hipError_t prepare_slice_kernels(mx_dtype) { return hipErrorUnknown; }
 hipError_t static_scratch(void **p) { *p = nullptr; return hipErrorUnknown; }
-int build_slices_device(mx_dtype, int, int, int, const int *, const int *, const void *, int, int, const char *, DeviceSlices &, hipStream_t,
+__attribute__((weak)) int build_slices_device(mx_dtype, int, int, int, const int *, const int *, const void *, int, int, const char *, DeviceSlices &, hipStream_t,
                         std::vector<int> *, std::vector<int> *, int) { return MX_ERR_DEVICE; }
 int check_csr_device(int, int, int, const int *, const int *, hipStream_t, const char *) { return MX_ERR_DEVICE; }
-int lines_per_gather_device(mx_dtype, int, const int *, hipStream_t, double *) { return MX_ERR_DEVICE; }
-int upload_csr_device(mx_dtype, int, int, int, const int *, const int *, const void *, const std::vector<int> &, bool, DeviceCsr &, hipStream_t) { return MX_ERR_DEVICE; }
+__attribute__((weak)) int lines_per_gather_device(mx_dtype, int, const int *, hipStream_t, double *) { return MX_ERR_DEVICE; }
+__attribute__((weak)) int upload_csr_device(mx_dtype, int, int, int, const int *, const int *, const void *, const std::vector<int> &, bool, DeviceCsr &, hipStream_t) { return MX_ERR_DEVICE; }
 bool strips_can_ride(mx_dtype, const DeviceTiles &, const void *) { return false; }
 struct HybridDevice::Impl {};
 HybridDevice::~HybridDevice() { delete impl; }
