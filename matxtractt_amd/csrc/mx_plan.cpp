@@ -430,20 +430,25 @@ int mxp::setup_csr_part(mx_plan *plan, const int *rowPtr, const int *col, const 
     // A large part goes up once, as it is, and takes the device's route: the same plan, without the counts over all entries
     // that the host would decide from (a million entries and more: binary64 power law 1.4 ms either way, blocks 1.3 and 1.1, a band 2.3 and 1.4; 2 million, 2.4 and
     // 2.0, 2.4 and 1.3, 4.0 and 1.8; half a million 0.9 and 0.9 to 1.1).  Where there is no memory for that beside the plan, the host's route
-    // needs less at a time; and where the slices would have more places than an int numbers, which the device finds out when it lays them
-    // out (its one reason to refuse a matrix that was looked at), the host's route may not want slices at all.
+    // estimates first and lays out one form: row tiles go up as they are read, without the matrix beside them (slices are made from
+    // the matrix in device memory on either route).  And where the slices would have more places than an int numbers, which the device finds out when
+    // it lays them out (its one reason to refuse a matrix that was looked at), the host's route may not want slices at all.
     if (part_goes_up(rows, cols, nnz)) {
-        int *rp = nullptr, *ci = nullptr;
-        void *va = nullptr, *marks = nullptr;
-        int rc = upload(&rp, rowPtr, (size_t)rows + 1);
-        if (!rc) rc = upload(&ci, col, (size_t)nnz);
-        if (!rc) rc = upload_bytes(&va, val, (size_t)nnz * es);
-        if (!rc && stripRows) rc = upload_bytes(&marks, stripRows, (size_t)rows);
-        if (!rc) rc = setup_csr_part_device(plan, nnz, rp, ci, va, flags, (const char *)marks, segOut, alone);
-        (void)mx::dev_free(rp);
-        (void)mx::dev_free(ci);
-        (void)mx::dev_free(va);
-        (void)mx::dev_free(marks);
+        struct Matrix {
+            int *rp = nullptr, *ci = nullptr;
+            void *va = nullptr, *marks = nullptr;
+            ~Matrix()
+            {
+                for (void *p : {(void *)rp, (void *)ci, va, marks}) (void)mx::dev_free(p);
+            }
+        };
+        int rc = MX_ERR_ALLOC;  // (a matrix that does not get there is no failure: the host's route takes it)
+        {
+            Matrix M;
+            if (!upload(&M.rp, rowPtr, (size_t)rows + 1) && !upload(&M.ci, col, (size_t)nnz) && !upload_bytes(&M.va, val, (size_t)nnz * es) &&
+                (!stripRows || !upload_bytes(&M.marks, stripRows, (size_t)rows)))
+                rc = setup_csr_part_device(plan, nnz, M.rp, M.ci, M.va, flags, (const char *)M.marks, segOut, alone);
+        }
         if (rc != MX_ERR_ALLOC && rc != MX_ERR_ARG) return rc;
         free_csr(plan->csr);
         free_slices(plan->slices);

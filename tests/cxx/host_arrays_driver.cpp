@@ -5,6 +5,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -25,6 +26,7 @@ struct Device {
     hipError_t last = hipSuccess;
 } device;
 int slices_rc = MX_OK, rows_rc = MX_OK, slices_asked = 0, rows_asked = 0;
+bool slices_throw = false;
 }  // namespace
 
 extern "C" {
@@ -75,6 +77,7 @@ int build_slices_device(mx_dtype, int rows, int, int, const int *, const int *, 
                         std::vector<int> *, std::vector<int> *, int)
 {
     ++slices_asked;
+    if (slices_throw) throw std::bad_alloc();
     D = DeviceSlices();
     D.vrows = 4 * rows;
     if (dev_malloc((void **)&D.ecol, 1000) != hipSuccess) return MX_ERR_ALLOC;
@@ -153,6 +156,47 @@ static void refused()
     dropped(plan);
 }
 
+// A device without room for the matrix beside the plan, or that runs out while it lays the plan out: the part has its row tiles all the same.
+static void memory()
+{
+    const Band &b = band();
+    slices_rc = rows_rc = MX_OK;
+    for (const int flags : {MX_PLAN_DEFAULT, MX_PLAN_CSR_ROWS}) {
+        const size_t tiles = b.ptr.size() * 4 + (b.col.size() + mx::kCsrPad) * (sizeof(double) + 2) + 1000000;  // (16-bit columns)
+        CHECK(tiles < b.raw());
+        device.total = tiles;
+        {
+            mx_plan plan;
+            CHECK(made(plan, flags) == MX_OK && slices_asked + rows_asked == 0 && plan.csr_variant == 0 && plan.csr.nBlocks > 0);
+            dropped(plan);
+        }
+        device.total = b.raw() / 2;  // (nor for the tiles)
+        {
+            mx_plan plan;
+            CHECK(made(plan, flags) != MX_OK);
+            dropped(plan);
+        }
+        device.total = (size_t)4 << 30;
+        rows_rc = MX_ERR_ALLOC;
+        mx_plan plan;
+        CHECK(made(plan, flags) == MX_OK && rows_asked == 1 && plan.csr_variant == 0 && plan.csr.nBlocks > 0);
+        dropped(plan);
+        rows_rc = MX_OK;
+    }
+    // host memory that runs out meanwhile leaves nothing behind on the device
+    slices_throw = true;
+    mx_plan plan;
+    bool thrown = false;
+    try {
+        (void)made(plan, MX_PLAN_DEFAULT);
+    } catch (const std::bad_alloc &) {
+        thrown = true;
+    }
+    slices_throw = false;
+    CHECK(thrown);
+    dropped(plan);
+}
+
 // What the device's kernels cannot number does not go up.
 static void sizes()
 {
@@ -163,7 +207,7 @@ static void sizes()
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"refused", refused}, {"sizes", sizes}};
+    const std::map<std::string, void (*)()> checks = {{"refused", refused}, {"memory", memory}, {"sizes", sizes}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();

@@ -66,7 +66,7 @@ def host_arrays(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["refused", "sizes"])
+@pytest.mark.parametrize("check", ["refused", "memory", "sizes"])
 def test_parts_from_host_arrays(host_arrays, check):
     """tests/cxx/host_arrays_driver.cpp, one check at a time."""
     r = subprocess.run([host_arrays, check], capture_output=True, text=True, timeout=60)
