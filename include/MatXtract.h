@@ -106,6 +106,11 @@ inline void check(int rc, const char *what)
 }
 inline int warm() { return env_int("MATXTRACT_WARM", 200); }
 inline int iters() { return env_int("MATXTRACT_ITERS", 4000); }
+// Where matxtract_preprocess makes the extraction when the caller leaves the choice.
+inline bool extract_on_device(indT nnz, float colProp, float rowProp)
+{
+    return nnz >= (1 << 17) && (colProp != 0.0f || rowProp != 0.0f) && mx_device_count() > 0;
+}
 }  // namespace matxtract_detail
 
 /* include/MatXtract.h:3-5.  Y is IN/OUT: Y += A*X.  cdTime, cdPre in ms. */
@@ -214,11 +219,13 @@ inline void exclusive_scan(indT *input, int length)
  * (colProp < rowProp, as at :1064-1069).  Inspect with mx_partition_get(); release with
  * mx_partition_destroy().  onDevice: 1 = the extraction runs on the GPU (mx_partition_create_device: the
  * same partition, whose arrays come to the host when they are asked for), 0 = on the host, -1 (default) = on the
- * GPU for a matrix of 131072 entries or more when there is one, on the host otherwise. */
+ * GPU for a matrix of 131072 entries or more when there is one, on the host otherwise, and where the GPU has
+ * no room for it. */
 inline mx_partition *matxtract_preprocess(valT *csrVal, indT *csrRowPtr, indT *csrColInd, int rowA, int colA, indT nnzA,
                                           float colProp, float rowProp, int onDevice = -1)
 {
-    if (onDevice < 0) onDevice = nnzA >= (1 << 17) && (colProp != 0.0f || rowProp != 0.0f) && mx_device_count() > 0;
+    const bool choose = onDevice < 0;
+    if (choose) onDevice = matxtract_detail::extract_on_device(nnzA, colProp, rowProp);
     mx_csr A;
     A.rows = rowA;
     A.cols = colA;
@@ -228,7 +235,10 @@ inline mx_partition *matxtract_preprocess(valT *csrVal, indT *csrRowPtr, indT *c
     A.colInd = csrColInd;
     A.val = csrVal;
     mx_partition *p = nullptr;
-    if ((onDevice ? mx_partition_create_device(&A, colProp, rowProp, &p) : mx_partition_create(&A, colProp, rowProp, &p)) != MX_OK) {
+    int rc = onDevice ? mx_partition_create_device(&A, colProp, rowProp, &p) : MX_ERR_DEVICE;
+    // (what the GPU has no room for, or cannot take now, the host can)
+    if (!onDevice || (choose && (rc == MX_ERR_ALLOC || rc == MX_ERR_DEVICE))) rc = mx_partition_create(&A, colProp, rowProp, &p);
+    if (rc != MX_OK) {
         std::fprintf(stderr, "matxtract_preprocess: %s\n", mx_last_error());
         return nullptr;
     }

@@ -230,15 +230,19 @@ class Partition:
     def __init__(self, A, tau_c, tau_r, device=False):
         """device=True: the extraction runs on the GPU (mx_partition_create_device); same result.  device=None:
         what the reference's surface does (matxtract_preprocess, the CLI): the GPU for a matrix of 131072
-        entries or more when there is one, the host otherwise (plan and product included, from host arrays: 130 thousand
+        entries or more when there is one, the host otherwise and where the GPU has no room (plan and product included, from host arrays: 130 thousand
         entries 1.4 to 1.9 ms there, 1.5 to 3.6 with the extraction on the host; 65 thousand 1.2 to 1.8 and 1.2 to 1.9; 2 million 2.0 to 3.1 and 10 to 63)."""
         self._h = C.c_void_p()
         self._A = A  # keep the input arrays alive during the call
         st = A.struct()
-        if device is None:
-            device = A.nnz >= (1 << 17) and (tau_c != 0 or tau_r != 0) and _lib.load().mx_device_count() > 0
-        create = _lib.load().mx_partition_create_device if device else _lib.load().mx_partition_create
-        check(create(C.byref(st), float(tau_c), float(tau_r), C.byref(self._h)))
+        lib, choose = _lib.load(), device is None
+        if choose:
+            device = A.nnz >= (1 << 17) and (tau_c != 0 or tau_r != 0) and lib.mx_device_count() > 0
+        args = C.byref(st), float(tau_c), float(tau_r), C.byref(self._h)
+        rc = (lib.mx_partition_create_device if device else lib.mx_partition_create)(*args)
+        if device and choose and rc in (_lib.MX_ERR_ALLOC, _lib.MX_ERR_DEVICE):
+            rc = lib.mx_partition_create(*args)
+        check(rc)
         self._bind()
 
     @classmethod

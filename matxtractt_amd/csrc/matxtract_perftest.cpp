@@ -227,8 +227,8 @@ int main(int argc, char **argv)
         std::cout << "---------------------------------------------------------" << std::endl;
         std::cout << "---------------------Compression Info--------------------" << std::endl;
     }
-    if (devicePrep < 0) devicePrep = nnzA >= (1 << 17) && extracting && mx_device_count() > 0;
-    if (devicePrep || devicePlan) (void)hipFree(nullptr);  // the first use of the device is not part of the preprocessing time
+    const bool onDevice = devicePrep < 0 ? matxtract_detail::extract_on_device(nnzA, colProp, rowProp) : devicePrep != 0;
+    if (onDevice || devicePlan) (void)hipFree(nullptr);  // the first use of the device is not part of the preprocessing time
     auto t0 = std::chrono::steady_clock::now();
     mx_partition *part = nullptr;
     mx_plan *plan = nullptr;

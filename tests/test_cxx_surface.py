@@ -58,6 +58,21 @@ def test_surface_driver_builds_in_both_precisions(mx):
     assert all(os.path.exists(e) for e in exes.values())
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp16"])
+def test_extraction_on_the_host_where_the_device_has_no_room(mx, tmp_path, precision):
+    """tests/cxx/choice_driver.cpp: matxtract_preprocess on a device that refuses."""
+    _gxx()
+    exe = str(tmp_path / "choice")
+    lib = os.path.join(ROOT, "matxtractt_amd")
+    cmd = ["g++", "-std=c++17", "-O1", "-fopenmp", "-Wall", "-Wextra"] + (["-Dfp64"] if precision == "fp64" else []) + \
+          ["-I" + os.path.join(ROOT, "include"), os.path.join(CXX_DIR, "choice_driver.cpp"), "-o", exe, "-L" + lib, "-lmatxtract_hip",
+           "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath," + lib, "-Wl,-rpath,/opt/rocm/lib"]
+    b = subprocess.run(cmd, capture_output=True, text=True)
+    assert b.returncode == 0, b.stderr[-2000:]
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
 def _read_arrays(path, dtypes):
     buf = open(path, "rb").read()
     out, at = [], 0

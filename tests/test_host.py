@@ -89,6 +89,26 @@ def test_partition_bit_exact_on_hostile_inputs(mx, ora, seed, dtype):
         P.close()
 
 
+@pytest.mark.parametrize("code", ["MX_ERR_ALLOC", "MX_ERR_DEVICE", "MX_ERR_ARG"])
+def test_partition_on_the_host_where_the_device_has_no_room(mx, monkeypatch, code):
+    """device=None on a device that refuses: the host's partition, unless the arguments were at fault."""
+    from matxtractt_amd import _lib
+    lib = _lib.load()
+    A, _ = mx.gen_config(2, scale=1 / 8)
+    assert A.nnz > 262144
+    asked = []
+    monkeypatch.setattr(lib, "mx_device_count", lambda: 1)
+    monkeypatch.setattr(lib, "mx_partition_create_device", lambda *a: asked.append(1) or getattr(_lib, code))
+    if code == "MX_ERR_ARG":
+        with pytest.raises(_lib.MxError):
+            mx.Partition(A, 0.5, 0.25, device=None)
+    else:
+        assert mx.Partition(A, 0.5, 0.25, device=None).hash == mx.Partition(A, 0.5, 0.25).hash
+    assert len(asked) == 1
+    with pytest.raises(_lib.MxError):
+        mx.Partition(A, 0.5, 0.25, device=True)
+
+
 def test_partition_rejects_bad_arguments(mx):
     A, _ = mx.gen_config(1, scale=0.05)
     with pytest.raises(mx.MxError) as e:
