@@ -230,8 +230,9 @@ class Partition:
     def __init__(self, A, tau_c, tau_r, device=False):
         """device=True: the extraction runs on the GPU (mx_partition_create_device); same result.  device=None:
         what the reference's surface does (matxtract_preprocess, the CLI): the GPU for a matrix of 131072
-        entries or more when there is one, the host otherwise and where the GPU has no room (plan and product included, from host arrays: 130 thousand
-        entries 1.4 to 1.9 ms there, 1.5 to 3.6 with the extraction on the host; 65 thousand 1.2 to 1.8 and 1.2 to 1.9; 2 million 2.0 to 3.1 and 10 to 63)."""
+        entries or more when there is one, the host otherwise and where the GPU has no room (plan and product included, from host arrays,
+        ms, extraction on the host and on the GPU: 120 to 165 thousand entries in even rows 0.8 to 1.8 and 0.9 to 1.8, up to 22 % slower there; in blocks
+        2.0 to 2.3 and 1.5 to 1.6; in a power law up to 9.8 and 2.0.  From 196 thousand on nothing is slower: 0.9 to 15 and 0.9 to 2.1)."""
         self._h = C.c_void_p()
         self._A = A  # keep the input arrays alive during the call
         st = A.struct()
