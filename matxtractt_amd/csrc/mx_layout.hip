@@ -165,18 +165,24 @@ __global__ __launch_bounds__(kBlock) void vrow_records_kernel(const unsigned lon
     }
 }
 
-// segPtr[r] = virtual rows before row r, and the row of every virtual row
+// segPtr[r] = virtual rows before row r, and the row of every virtual row: a row's own thread names up to kOwnVrows of them, longer
+// lists are written by the wave, one after the other.  (One row of 3 million binary64 entries, 125 thousand virtual rows: 3.4 ms by its thread alone, so 0.05.)
+constexpr int kOwnVrows = 16;
 __global__ __launch_bounds__(kBlock) void seg_ptr_kernel(const int *__restrict__ rowPtr, const unsigned long long *__restrict__ startBits,
                                                          const int *__restrict__ wordBase, int rows, int nnz, int nV, int *__restrict__ segPtr,
                                                          int *__restrict__ vRow)
 {
-    const int r = blockIdx.x * kBlock + threadIdx.x;
-    if (r > rows) return;
+    const int r = blockIdx.x * kBlock + threadIdx.x, lane = threadIdx.x & 63;
     auto before = [&](int p) { return p < nnz ? wordBase[p >> 6] + __popcll(startBits[p >> 6] & ~(~0ull << (p & 63))) : nV; };
-    const int a = r < rows ? before(rowPtr[r]) : nV;
-    segPtr[r] = a;
-    if (r < rows)
-        for (int t = a, e = before(rowPtr[r + 1]); t < e; ++t) vRow[t] = r;
+    const int a = r < rows ? before(rowPtr[r]) : nV, e = r < rows ? before(rowPtr[r + 1]) : nV;
+    if (r <= rows) segPtr[r] = a;
+    const bool many = e - a > kOwnVrows;
+    if (!many)
+        for (int t = a; t < e; ++t) vRow[t] = r;
+    for (unsigned long long m = __ballot(many); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m), a_ = __builtin_amdgcn_readlane(a, l), e_ = __builtin_amdgcn_readlane(e, l), r_ = __builtin_amdgcn_readlane(r, l);
+        for (int t = a_ + lane; t < e_; t += 64) vRow[t] = r_;
+    }
 }
 
 // the sort key of every virtual row: (slice, cap - length, kind of its row)

@@ -57,6 +57,20 @@ def test_virtual_rows_are_cut_as_on_the_host(mx, dtype, lens, cols, order):
     _same_layout(mx, A, 7)
 
 
+@pytest.mark.parametrize("dtype,most", [(np.float64, 15), (np.float64, 16), (np.float64, 17), (np.float16, 17), (np.float64, 64), (np.float64, 65), (np.float16, 3000)])
+def test_rows_of_many_virtual_rows(mx, dtype, most):
+    """The list of a row's virtual rows by the row's own thread (up to 16 of them) or by its wave: a virtual row to an entry, rows without, short and long
+    lists side by side, long ones at both ends of a wave and in the last row."""
+    per = 16384 if dtype == np.float64 else 65536
+    lens = np.array(([0, 1, most, 2, most - 1] + [3] * 57 + [most, most] + [0] * 63 + [most]) * 3)
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    slices = min(most, 60)
+    col = np.concatenate([np.sort(np.arange(n) % slices * per + np.arange(n) // slices) for n in lens]).astype(np.int32)
+    A = mx.Csr(lens.size, slices * per, ptr, col, np.random.default_rng(most).uniform(-1, 1, ptr[-1]).astype(dtype))
+    H = _same_layout(mx, A, 30)
+    assert np.diff(H["segPtr"]).max() >= min(most, 60)
+
+
 def _fused_case(name, rng):
     """(matrix, whether the one-launch form takes it when it is asked for)"""
     def m(lens, col, cols, dtype=np.float64):
