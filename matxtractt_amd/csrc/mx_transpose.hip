@@ -171,11 +171,13 @@ __global__ __launch_bounds__(kThreads, 8) void bucket_lines_kernel(const typenam
     }
     next[2 * tid] = next[2 * tid + 1] = 0;
     __syncthreads();
-    for (int p = mx::next_of(p0, p1, tid); p < p1; p = mx::next_of(p, p1, kThreads)) {
-        const int c = M::line(moved[p]), one = __builtin_amdgcn_readfirstlane(c);
+    // (places are unsigned here: the step past the last entry is more than an int holds where the bucket ends near 2^31)
+    const unsigned end = (unsigned)p1;
+    for (unsigned p = (unsigned)p0; p < end; p += kThreads) {
+        const int c = p + tid < end ? M::line(moved[p + tid]) : -1, one = __builtin_amdgcn_readfirstlane(c);
         const unsigned long long same = __ballot(c == one);  // (a crowded line)
-        if (lane == __builtin_ctzll(same)) atomicAdd(&next[one], __popcll(same));
-        if (c != one) atomicAdd(&next[c], 1);
+        if (one >= 0 && lane == __builtin_ctzll(same)) atomicAdd(&next[one], __popcll(same));
+        if (c >= 0 && c != one) atomicAdd(&next[c], 1);
     }
     __syncthreads();
     {
@@ -185,9 +187,9 @@ __global__ __launch_bounds__(kThreads, 8) void bucket_lines_kernel(const typenam
         if (2 * tid < lines) tPtr[c0 + 2 * tid] = s;
         if (2 * tid + 1 < lines) tPtr[c0 + 2 * tid + 1] = s + n0;
     }
-    for (int q = p0; q < p1; q = mx::next_of(q, p1, kTile)) {
-        const int size = min(kTile, p1 - q);
-        load(q, size);
+    for (unsigned q = (unsigned)p0; q < end; q += kTile) {
+        const int size = min(kTile, (int)(end - q));
+        load((int)q, size);
         place_by_digit<true>([&](int j) { return d[j]; }, size, B.lineBits, U.digits, start, part, at);
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
