@@ -42,9 +42,14 @@ constexpr int kBlock = 256;
 constexpr int kMaxCount = 2147483647 - 2 * kBlock;
 
 // ---- the two steps ------------------------------------------------------------------------
-// Entries of one bucket at most: its workgroup takes 11 us for every 8192 of them while the others are done, and the radix sort has
-// to be the slower way still (a million entries, 16 thousand of them in one line: 113 us, radix sort 231; 8 million, 60 thousand: 349, 620).
-inline int most_of_bucket(int nnz) { return 65536 + nnz / 64; }
+// Entries of one bucket at most: its workgroup takes 10.5 us for every 8192 of them while the others are done.  So many, in binary64, take as long as
+// the radix sort and the counting that then was in vain, 25 to 35 us: 39 thousand of 60 thousand entries, 46 of 120, 86 of 300, 119 of a
+// million, 137 of 3 million, 237 of 8 million (in binary16 somewhat more).  Us by buckets, by the radix sort alone and after the counting: 32 of 60 thousand
+// 106, 91, 120; 64 of 300 thousand 172, 175, 200; 96 of a million 241, 243, 270; 200 thousand of 8 million 599, 626, 661.
+inline int most_of_bucket(int nnz) { return std::min(30000 + nnz / 6, 75000 + nnz / 50); }
+constexpr int kBucketsWorth = 1024;  // entries from which on the buckets are faster than a sort by one workgroup (800: 57 us, radix sort 50; 1250: 57, 59)
+// Whether it is worth counting: not where some bucket has too many entries whatever the indices are.
+inline bool buckets_worth(int nnz, const Buckets &B) { return nnz >= kBucketsWorth && nnz / B.n <= most_of_bucket(nnz); }
 
 // An entry between the two steps, in one piece: a store of a wave goes to as many places as it has lanes, whatever a lane
 // stores (line, source line and value in arrays of their own, put in order in LDS to be written side by side: 89 + 89 us
@@ -283,6 +288,7 @@ static int transpose_by_buckets(int outer, int inner, int nnz, const int *ptr, c
     *done = *checked = false;
     if (!buckets_hold(inner)) return MX_OK;
     const Buckets B = make_buckets(inner, nnz);
+    if (!buckets_worth(nnz, B)) return MX_OK;
     const int buckets = B.n, tiles = (int)(((long long)nnz + kTile - 1) / kTile);
     typedef typename Moved<V>::Word Word;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };

@@ -45,6 +45,21 @@ def test_transpose_of_crowded_lines(mx, share):
     _check(mx, ptr, ind, val, inner)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float16])
+@pytest.mark.parametrize("inner,nnz,crowd", [
+    (40, 1023, 0), (40, 1024, 0),                              # from 1024 entries on by buckets
+    (1, 36000, 0), (1, 36001, 0), (3, 216003, 0), (3, 216006, 0),  # some bucket has 36000 (66000) of them, one more
+    (5000, 60000, 39990), (5000, 60000, 40050),                # one line with about as many as a bucket may have
+    (100003, 3000000, 134000), (100003, 3000000, 136500),
+])
+def test_transpose_by_the_rule_for_buckets(mx, dtype, inner, nnz, crowd):
+    rng = np.random.default_rng(inner + nnz + crowd)
+    ptr, val = _matrix(rng, 700, nnz, dtype)
+    ind = rng.integers(0, inner, nnz)
+    ind[rng.permutation(nnz)[:crowd]] = inner // 3
+    _check(mx, ptr, ind, val, inner)
+
+
 def test_transpose_refuses_an_index_before_it_writes(mx):
     import ctypes
 
