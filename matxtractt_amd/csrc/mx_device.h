@@ -25,9 +25,8 @@ void release_idle_memory();
 // fill while the device reads them (a partition of 4.2 million binary64 entries, 50 MB, made on the device: 3.4 ms with hipMemcpy, of them 0.5 in
 // the look at the columns by one core, 2.2 so).  The buffers (16 MB) are kept until mx_release_memory; a thread that finds them
 // in use copies by hipMemcpy.
-// (weak: a link of some of the library's C++ files against a stub of the runtime has hipMemcpy only)
-__attribute__((weak)) hipError_t copy_up(void *dst, const void *src, size_t bytes);
-__attribute__((weak)) void release_staging();
+hipError_t copy_up(void *dst, const void *src, size_t bytes);
+void release_staging();
 struct MemScope {
     explicit MemScope(hipStream_t s);
     ~MemScope();

@@ -40,7 +40,7 @@ inline int upload(T **dst, const T *src, size_t n, size_t pad = 0)
     const size_t total = std::max<size_t>(n + pad, 1);
     MX_HIP(mx::dev_malloc((void **)dst, total * sizeof(T)));
     if (pad || n == 0) MX_HIP(hipMemset(*dst, 0, total * sizeof(T)));
-    if (n) MX_HIP(mx::copy_up ? mx::copy_up(*dst, src, n * sizeof(T)) : hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
+    if (n) MX_HIP(mx::copy_up(*dst, src, n * sizeof(T)));
     return MX_OK;
 }
 int upload_bytes(void **dst, const void *src, size_t n, size_t pad = 0);

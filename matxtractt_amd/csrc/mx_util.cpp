@@ -381,6 +381,6 @@ IdleFrees::~IdleFrees()
 
 extern "C" void mx_release_memory(void)
 {
-    if (mx::release_staging) mx::release_staging();
+    mx::release_staging();
     mx::release_idle_memory();
 }

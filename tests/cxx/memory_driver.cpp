@@ -5,6 +5,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <deque>
 #include <map>
 #include <mutex>
 #include <new>
@@ -27,6 +28,26 @@ struct Device {
     std::atomic<int> streams{0};
     bool refuse = false;  // waits for the device
     hipError_t last = hipSuccess;
+    // copies that run when they are waited for, in order; an event stands for those asked for before it
+    struct Copy {
+        void *to;
+        const void *from;
+        size_t n;
+    };
+    std::deque<Copy> copies;
+    size_t done = 0;  // copies that have run
+    std::map<hipEvent_t, size_t> events;
+    size_t made = 0, plain = 0, pinned = 0;  // events; copies by hipMemcpy; bytes of pinned memory
+    bool no_pinned = false;
+    int copies_left = -1;  // so many are taken, the next is refused
+    void run(size_t until)
+    {
+        for (; done < until; ++done) {
+            std::memcpy(copies.front().to, copies.front().from, copies.front().n);
+            copies.pop_front();
+        }
+    }
+    size_t asked() const { return done + copies.size(); }
 } device;
 
 #define CHECK(x)                                                     \
@@ -90,7 +111,71 @@ hipError_t hipFree(void *p)
 hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) { return *f = device.total - device.used, *t = device.total, hipSuccess; }
 hipError_t hipDeviceSynchronize() { return device.refuse ? hipErrorStreamCaptureUnsupported : hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    device.run(device.asked());
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    if (device.copies_left >= 0 && device.copies_left-- == 0) return hipErrorInvalidValue;
+    device.copies.push_back({to, from, n});
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void *to, const void *from, size_t n, hipMemcpyKind)
+{
+    {
+        std::lock_guard<std::mutex> hold(device.mu);
+        ++device.plain;
+    }
+    std::memcpy(to, from, n);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    if (device.no_pinned) return device.last = hipErrorOutOfMemory;
+    device.pinned += n;
+    size_t *at = (size_t *)std::malloc(n + 64);
+    *at = n;
+    return *p = (char *)at + 64, hipSuccess;
+}
+hipError_t hipHostFree(void *p)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    CHECK(device.copies.empty());  // (nothing reads it any more)
+    size_t *at = (size_t *)((char *)p - 64);
+    device.pinned -= *at;
+    std::free(at);
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    *e = (hipEvent_t)(uintptr_t)(1000 + ++device.made);
+    device.events[*e] = 0;
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    device.events.at(e) = device.asked();
+    return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    device.run(device.events.at(e));
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e)
+{
+    std::lock_guard<std::mutex> hold(device.mu);
+    CHECK(device.events.erase(e) == 1);
+    return hipSuccess;
+}
 hipError_t hipStreamCreate(hipStream_t *s)
 {
     std::this_thread::sleep_for(std::chrono::milliseconds(2));
@@ -229,9 +314,73 @@ static void host_memory()
     }
 }
 
+// Large copies go through pinned buffers, of which none is filled again before the device has read it (the copies here run as late as
+// the waits allow); small ones, and all where there is no pinned memory, by hipMemcpy.
+struct Bytes {
+    std::vector<unsigned char> from, to;
+    explicit Bytes(size_t n, unsigned seed) : from(n), to(n, 0)
+    {
+        for (auto &b : from) b = (unsigned char)((seed = seed * 1664525u + 1013904223u) >> 24);
+    }
+    hipError_t up() { return mx::copy_up(to.data(), from.data(), from.size()); }
+    bool same() const { return from == to; }
+};
+static void copies()
+{
+    constexpr size_t MB = (size_t)1 << 20;
+    for (const size_t n : {(size_t)0, (size_t)1, 8 * MB - 1}) {
+        Bytes b(n, 3);
+        const size_t plain = device.plain;
+        CHECK(b.up() == hipSuccess && b.same() && device.plain == plain + 1 && device.pinned == 0);
+    }
+    for (const size_t n : {8 * MB, 8 * MB + 1, 12 * MB - 1, 16 * MB, 16 * MB + 1, 20 * MB, 33 * MB + 12345}) {
+        Bytes b(n, (unsigned)n);
+        const size_t plain = device.plain;
+        CHECK(b.up() == hipSuccess && b.same() && device.plain == plain && device.events.empty());
+        CHECK(device.pinned == 16 * MB && device.copies.empty());
+    }
+    mx_release_memory();
+    CHECK(device.pinned == 0);
+    Bytes b(9 * MB, 7);
+    CHECK(b.up() == hipSuccess && b.same() && device.pinned == 16 * MB);
+    mx_release_memory();
+    device.no_pinned = true;
+    Bytes c(9 * MB, 8);
+    const size_t plain = device.plain;
+    CHECK(c.up() == hipSuccess && c.same() && device.plain == plain + 1 && hipGetLastError() == hipSuccess);
+}
+static void copies_of_threads()
+{
+    std::vector<std::thread> threads;
+    std::atomic<int> wrong{0};
+    for (int t = 0; t < 4; ++t)
+        threads.emplace_back([&, t]() {
+            for (int k = 0; k < 6; ++k) {
+                Bytes b(((size_t)10 << 20) + 4096 * t + k, 100 * t + k);
+                if (b.up() != hipSuccess || !b.same()) ++wrong;
+                if (t == 0) mx_release_memory();
+            }
+        });
+    for (auto &t : threads) t.join();
+    CHECK(wrong == 0 && device.events.empty() && device.copies.empty());
+    mx_release_memory();
+    CHECK(device.pinned == 0);
+}
+// A copy that the device refuses is an error; what was on its way is waited for.
+static void copies_refused()
+{
+    for (int after = 0; after < 6; ++after) {
+        Bytes b((size_t)40 << 20, 5);
+        device.copies_left = after;
+        CHECK(b.up() == hipErrorInvalidValue && device.copies.empty() && device.events.empty());
+        device.copies_left = -1;
+        CHECK(b.up() == hipSuccess && b.same());
+    }
+}
+
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"wait_refused", wait_refused}, {"bound", bound}, {"age", age}, {"scope_full", scope_full}, {"scope_share", scope_share}, {"one_stream", one_stream}, {"host_memory", host_memory}};
+    const std::map<std::string, void (*)()> checks = {{"copies", copies}, {"copies_of_threads", copies_of_threads}, {"copies_refused", copies_refused}, {"wait_refused", wait_refused}, {"bound", bound}, {"age", age}, {"scope_full", scope_full}, {"scope_share", scope_share}, {"one_stream", one_stream}, {"host_memory", host_memory}};
     const auto it = checks.find(argc > 1 ? argv[1] : "");
     if (it == checks.end()) return 2;
     it->second();
