@@ -891,7 +891,7 @@ int plan_fused_device(mx_dtype dtype, int budget, int S, int rows, int nnz, int 
     hipLaunchKernelGGL(xcd_groups_kernel, dim3(1), dim3(64), 0, s, rowPtr, (long long)nnz, parts, D.totals);
     hipLaunchKernelGGL(part_counts_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, parts, tiles, count);
     hipLaunchKernelGGL(mxd::bucket_offsets_kernel, dim3((unsigned)((n + 15) / 16)), dim3(1024), 0, s, count, n, tiles, total);
-    hipLaunchKernelGGL(mxd::bucket_starts_kernel, dim3(1), dim3(mxd::kThreads), 0, s, (const int *)total, n, nV, (const int *)nullptr, 0, first, flag);
+    hipLaunchKernelGGL(mxd::bucket_starts_kernel<false>, dim3(1), dim3(mxd::kThreads), 0, s, (const int *)total, n, mxd::BucketBound{}, (const int *)nullptr, 0, first, flag);
     hipLaunchKernelGGL(part_order_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, parts, bits_of(n), tiles, (const int *)count, (const int *)first, order,
                        length, partOf);
     MXL_TRY(hipGetLastError());

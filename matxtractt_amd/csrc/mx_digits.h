@@ -144,9 +144,16 @@ static __global__ __launch_bounds__(1024) void bucket_offsets_kernel(int *__rest
         }
     }
 }
-// first[b] = entries of the buckets before b, first[buckets] = all; *flag = 1 when a tile is bad, + 2 when a bucket has more than `most`
-static __global__ __launch_bounds__(kThreads) void bucket_starts_kernel(const int *__restrict__ total, int buckets, int most, const int *__restrict__ bad,
-                                                                 int tiles, int *__restrict__ first, int *__restrict__ flag)
+// How many entries a bucket may have for one workgroup to work on it.
+struct BucketBound {
+    int few, low, high;  // `low`, or `high` where more than `few` buckets have more than that
+};
+enum { kBucketsBad = 1, kBucketsCrowded = 2, kBucketsRefused = 4 };
+// first[b] = entries of the buckets before b, first[buckets] = all.  flag[0]: kBucketsBad when a tile is bad; with a bound, flag[1] = the one that
+// holds, kBucketsCrowded when some bucket has more than that, kBucketsRefused as well when more than `few` have.
+template <bool BOUND>
+static __global__ __launch_bounds__(kThreads) void bucket_starts_kernel(const int *__restrict__ total, int buckets, BucketBound bound,
+                                                                        const int *__restrict__ bad, int tiles, int *__restrict__ first, int *__restrict__ flag)
 {
     __shared__ int part[kWaves];
     const int b = 2 * threadIdx.x, n0 = b < buckets ? total[b] : 0, n1 = b + 1 < buckets ? total[b + 1] : 0, at = sum_before(n0 + n1, part);
@@ -156,8 +163,15 @@ static __global__ __launch_bounds__(kThreads) void bucket_starts_kernel(const in
     bool out = false;
     for (int t = threadIdx.x; t < tiles; t += kThreads) out |= bad[t] != 0;
     out = __syncthreads_or(out);
-    const bool crowded = __syncthreads_or(max(n0, n1) > most);
-    if (b == 0) *flag = (int)out + 2 * (int)crowded;
+    int crowded = 0;
+    if (BOUND) {
+        auto above = [&](int m) { return __syncthreads_count(n0 > m) + __syncthreads_count(n1 > m); };
+        if (__syncthreads_or(max(n0, n1) > bound.low)) crowded = above(bound.low);
+        const bool many = crowded > bound.few;
+        if (many) crowded = above(bound.high);
+        if (b == 0) flag[1] = many ? bound.high : bound.low;
+    }
+    if (b == 0) flag[0] = (out ? kBucketsBad : 0) + (crowded > 0 ? kBucketsCrowded : 0) + (crowded > bound.few ? kBucketsRefused : 0);
 }
 
 // ---- buckets of consecutive lines (columns): entries by line in two steps, bucket and line inside it ----

@@ -547,7 +547,7 @@ static int order_and_reach(const int *cnt, int n, int most, int target, int *ord
         }
         hipLaunchKernelGGL(count_digits_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, digit, n, values, tiles, count);
         hipLaunchKernelGGL(mxd::bucket_offsets_kernel, dim3((unsigned)((values + 15) / 16)), dim3(1024), 0, s, count, values, tiles, total);
-        hipLaunchKernelGGL(mxd::bucket_starts_kernel, dim3(1), dim3(mxd::kThreads), 0, s, (const int *)total, values, n, (const int *)nullptr, 0, first, flag);
+        hipLaunchKernelGGL(mxd::bucket_starts_kernel<false>, dim3(1), dim3(mxd::kThreads), 0, s, (const int *)total, values, mxd::BucketBound{}, (const int *)nullptr, 0, first, flag);
         hipLaunchKernelGGL(order_digits_kernel<false>, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, digit, n, values, bits, tiles, (const int *)count,
                            (const int *)first, out, sortedCnt);
         before = out;
@@ -615,7 +615,7 @@ extern "C" int mx_select_device(int rows, int cols, int nnz, const int *rowPtr_d
         unsigned short *column = (unsigned short *)((unsigned char *)held.p + countB + firstB);
         hipLaunchKernelGGL(mxd::bucket_counts_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, colInd_dev, cols, nnz, B, tiles, count, badTile);
         hipLaunchKernelGGL(mxd::bucket_offsets_kernel, dim3((unsigned)((B.n + 15) / 16)), dim3(1024), 0, s, count, B.n, tiles, total);
-        hipLaunchKernelGGL(mxd::bucket_starts_kernel, dim3(1), dim3(mxd::kThreads), 0, s, (const int *)total, B.n, nnz, (const int *)badTile, tiles, first, bad);
+        hipLaunchKernelGGL(mxd::bucket_starts_kernel<false>, dim3(1), dim3(mxd::kThreads), 0, s, (const int *)total, B.n, mxd::BucketBound{}, (const int *)badTile, tiles, first, bad);
         hipLaunchKernelGGL(bucket_columns_kernel, mxd::tile_blocks(tiles), dim3(mxd::kThreads), 0, s, colInd_dev, nnz, cols, B, tiles, (const int *)count,
                            (const int *)first, column);
         hipLaunchKernelGGL(count_columns_kernel, dim3((unsigned)B.n), dim3(mxd::kThreads), 0, s, (const unsigned short *)column, (const int *)first, cols, B, cnt);

@@ -17,8 +17,9 @@
 // steps, and 4 to count them first.  (7.6 million entries of a power law, 700001 x 412345, binary64: 217 us;
 // three passes of a radix sort over index and entry number, with the lines and values gathered at the end, 448; 2 million lines, 4.1 million output lines, binary16: 287, 1046; 12000 x 9000 with nine a line: 63, 103.)
 //
-// One workgroup works on a bucket: a matrix with so many of its entries in one place that the others would wait for
-// that workgroup, or with more output lines than the buckets hold (kDigits each), takes the radix sort.
+// One workgroup works on a bucket; a few crowded ones are counted and put in order by as many workgroups as they have tiles (line_counts_kernel,
+// line_entries_kernel), after a look by the host at which those are.  A matrix with many of them, or with more output lines than the
+// buckets hold (kDigits each), takes the radix sort.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -42,14 +43,19 @@ constexpr int kBlock = 256;
 constexpr int kMaxCount = 2147483647 - 2 * kBlock;
 
 // ---- the two steps ------------------------------------------------------------------------
-// Entries of one bucket at most: its workgroup takes 10.5 us for every 8192 of them while the others are done.  So many, in binary64, take as long as
-// the radix sort and the counting that then was in vain, 25 to 35 us: 39 thousand of 60 thousand entries, 46 of 120, 86 of 300, 119 of a
-// million, 137 of 3 million, 237 of 8 million (in binary16 somewhat more).  Us by buckets, by the radix sort alone and after the counting: 32 of 60 thousand
-// 106, 91, 120; 64 of 300 thousand 172, 175, 200; 96 of a million 241, 243, 270; 200 thousand of 8 million 599, 626, 661.
-inline int most_of_bucket(int nnz) { return std::min(30000 + nnz / 6, 75000 + nnz / 50); }
+// A bucket's workgroup takes 10.5 us for every 8192 of its entries while the others are done.  A bucket with too many is crowded: its tiles are put in order by
+// workgroups of their own (line_entries_kernel), which takes a look by the host at which buckets those are and four launches for each.
+// That is 30 us, as long as three rounds of its own workgroup; for 8 million binary16 entries, where the others take longer, as four.  Us, binary64, n entries of which m
+// name one line of many, by the bucket's own workgroup / by workgroups for its tiles / by the radix sort alone: n = 60 thousand, m = 32 thousand
+// 106 / 94 / 89; 300 and 96 thousand 221 / 99 / 176; a million and 32 thousand 142 / 113 / 247; a million and 300 thousand 584 / 112 / 239; 8 million and
+// 300 thousand 769 / 285 / 626.
+constexpr int kCrowdedMost = 8;  // crowded buckets at most; where more have so many, they may have as many as take as long as the radix sort and the counting
+inline BucketBound bucket_bound(int nnz)
+{
+    constexpr int low = 24576;
+    return BucketBound{kCrowdedMost, low, std::max(low, std::min(30000 + nnz / 6, 75000 + nnz / 50))};
+}
 constexpr int kBucketsWorth = 1024;  // entries from which on the buckets are faster than a sort by one workgroup (800: 57 us, radix sort 50; 1250: 57, 59)
-// Whether it is worth counting: not where some bucket has too many entries whatever the indices are.
-inline bool buckets_worth(int nnz, const Buckets &B) { return nnz >= kBucketsWorth && nnz / B.n <= most_of_bucket(nnz); }
 
 // An entry between the two steps, in one piece: a store of a wave goes to as many places as it has lanes, whatever a lane
 // stores (line, source line and value in arrays of their own, put in order in LDS to be written side by side: 89 + 89 us
@@ -80,6 +86,8 @@ struct Moved<uint16_t> {
     static __device__ __forceinline__ uint16_t value(const Word &w) { return (uint16_t)((unsigned)w.y >> 16); }
 };
 
+__device__ __forceinline__ bool refused(int flag) { return flag & (kBucketsBad | kBucketsRefused); }
+
 // The entries of a tile to their buckets, in source order.
 template <typename V>
 __global__ __launch_bounds__(kThreads, 8) void bucket_entries_kernel(const int *__restrict__ ptr, const int *__restrict__ ind, const V *__restrict__ val,
@@ -93,7 +101,7 @@ __global__ __launch_bounds__(kThreads, 8) void bucket_entries_kernel(const int *
     } U;
     __shared__ int start[kDigits];
     const int t = tile_of_block(tiles);
-    if (t >= tiles || *flag) return;
+    if (t >= tiles || refused(flag[0])) return;
     const int t0 = t * kTile, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, size = min(kTile, nnz - t0);
     mxr::tile_rows(ptr, outer, nnz, t0, U.rows);
     int row[kPer], c[kPer], at[kPer];  // (c: bucket and line)
@@ -136,10 +144,11 @@ __global__ __launch_bounds__(kThreads, 8) void bucket_lines_kernel(const typenam
     } U;
     __shared__ int next[kDigits], part[kWaves];
     __shared__ unsigned short start[kDigits];
-    if (*flag) return;
+    if (refused(flag[0])) return;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, b = blockIdx.x;
     const int c0 = b * B.lines, lines = min(B.lines, inner - c0), p0 = first[b], p1 = first[b + 1];
     if (b == B.n - 1 && tid == 0) tPtr[inner] = p1;
+    if (p1 - p0 > flag[1]) return;  // (crowded)
     int d[kPer], at[kPer], row[kPer];
     V v[kPer];
     auto load = [&](int q, int size) {
@@ -207,6 +216,60 @@ __global__ __launch_bounds__(kThreads, 8) void bucket_lines_kernel(const typenam
         const int s0 = start[2 * tid], s1 = start[2 * tid + 1], s2 = tid + 1 < kThreads ? start[2 * tid + 2] : size;
         next[2 * tid] += s1 - s0;
         next[2 * tid + 1] += s2 - s1;
+    }
+}
+
+// ---- a crowded bucket, by as many workgroups as it has tiles ----
+// count[tile][line] entries
+template <typename V>
+__global__ __launch_bounds__(kThreads) void line_counts_kernel(const typename Moved<V>::Word *__restrict__ moved, int n, int lines, int tiles,
+                                                               int *__restrict__ count)
+{
+    __shared__ int here[kDigits];
+    const int t = tile_of_block(tiles), tid = threadIdx.x, lane = tid & 63;
+    if (t >= tiles) return;
+    const int t0 = t * kTile, size = min(kTile, n - t0);
+    here[tid] = here[tid + kThreads] = 0;
+    __syncthreads();
+    for (int i = tid; i < size; i += kThreads) {
+        const int c = Moved<V>::line(moved[t0 + i]), one = __builtin_amdgcn_readfirstlane(c);
+        const unsigned long long same = __ballot(c == one);  // (a crowded line)
+        if (lane == __builtin_ctzll(same)) atomicAdd(&here[one], __popcll(same));
+        if (c != one) atomicAdd(&here[c], 1);
+    }
+    __syncthreads();
+    for (int k = tid; k < lines; k += kThreads) count[(size_t)t * lines + k] = here[k];
+}
+// Every entry to its place, from the entries of its line in the tiles before (`before`) and of the lines before (`first`); the pointers of the lines.
+template <typename V>
+__global__ __launch_bounds__(kThreads, 8) void line_entries_kernel(const typename Moved<V>::Word *__restrict__ moved, int n, int lines, int lineBits, int tiles,
+                                                                   const int *__restrict__ before, const int *__restrict__ first, int p0,
+                                                                   int *__restrict__ tPtr, int *__restrict__ tInd, V *__restrict__ tVal)
+{
+    __shared__ Digits digits;
+    __shared__ int start[kDigits];
+    const int t = tile_of_block(tiles), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if (t >= tiles) return;
+    const int t0 = t * kTile, size = min(kTile, n - t0);
+    for (int k = tid; k < lines; k += kThreads) {
+        start[k] = first[k] + before[(size_t)t * lines + k];
+        if (t == 0) tPtr[k] = p0 + first[k];
+    }
+    int d[kPer], at[kPer], row[kPer];
+    V v[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const typename Moved<V>::Word e = moved[t0 + min(w * kWave + j * 64 + lane, size - 1)];
+        d[j] = Moved<V>::line(e);
+        row[j] = Moved<V>::source(e);
+        v[j] = Moved<V>::value(e);
+    }
+    place_by_digit<false>([&](int j) { return d[j]; }, size, lineBits, digits, start, (int *)nullptr, at);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        if (w * kWave + j * 64 + lane >= size) continue;
+        tInd[at[j]] = row[j];
+        tVal[at[j]] = v[j];
     }
 }
 
@@ -288,34 +351,55 @@ static int transpose_by_buckets(int outer, int inner, int nnz, const int *ptr, c
     *done = *checked = false;
     if (!buckets_hold(inner)) return MX_OK;
     const Buckets B = make_buckets(inner, nnz);
-    if (!buckets_worth(nnz, B)) return MX_OK;
+    const BucketBound bound = bucket_bound(nnz);
+    // (nor is it worth counting where the buckets have too many entries on the average: so few lines are one pass of the radix sort)
+    if (nnz < kBucketsWorth || nnz / B.n > bound.high) return MX_OK;
     const int buckets = B.n, tiles = (int)(((long long)nnz + kTile - 1) / kTile);
     typedef typename Moved<V>::Word Word;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t countB = al((size_t)tiles * buckets * 4 + (size_t)tiles * 4), firstB = al((size_t)(2 * kDigits + 1) * 4);
+    const size_t countB = al((size_t)tiles * buckets * 4 + (size_t)tiles * 4), firstB = al((size_t)(2 * kDigits + 3) * 4);
     Scratch scratch;
-    MXT_TRY(mx::dev_malloc(&scratch.p, countB + firstB + 256 + (size_t)nnz * sizeof(Word)));
+    MXT_TRY(mx::dev_malloc(&scratch.p, countB + firstB + (size_t)nnz * sizeof(Word)));
     unsigned char *b = (unsigned char *)scratch.p;
-    int *count = (int *)b, *bad = count + (size_t)tiles * buckets, *first = (int *)(b + countB), *total = first + kDigits + 1, *flag = (int *)(b + countB + firstB);
-    b += countB + firstB + 256;
-    Word *moved = (Word *)b;
+    int *count = (int *)b, *bad = count + (size_t)tiles * buckets, *flag = (int *)(b + countB), *first = flag + 2, *total = first + kDigits + 1;
+    Word *moved = (Word *)(b + countB + firstB);
     hipLaunchKernelGGL(bucket_counts_kernel, tile_blocks(tiles), dim3(kThreads), 0, s, ind, inner, nnz, B, tiles, count, bad);
     hipLaunchKernelGGL(bucket_offsets_kernel, dim3((unsigned)((buckets + 15) / 16)), dim3(1024), 0, s, count, buckets, tiles, total);
-    hipLaunchKernelGGL(bucket_starts_kernel, dim3(1), dim3(kThreads), 0, s, (const int *)total, buckets, most_of_bucket(nnz), (const int *)bad, tiles,
+    hipLaunchKernelGGL(bucket_starts_kernel<true>, dim3(1), dim3(kThreads), 0, s, (const int *)total, buckets, bound, (const int *)bad, tiles,
                        first, flag);
     hipLaunchKernelGGL(bucket_entries_kernel<V>, tile_blocks(tiles), dim3(kThreads), 0, s, ptr, ind, val, outer, nnz, B, tiles, (const int *)count,
                        (const int *)first, (const int *)flag, moved);
     hipLaunchKernelGGL(bucket_lines_kernel<V>, dim3((unsigned)buckets), dim3(kThreads), 0, s, (const Word *)moved, (const int *)first, inner, B, (const int *)flag, tPtr, tInd, tVal);
     MXT_TRY(hipGetLastError());
-    int got = 0;
-    MXT_TRY(hipMemcpyAsync(&got, flag, 4, hipMemcpyDeviceToHost, s));
+    int got[2 + kDigits + 1];  // (flag and first)
+    MXT_TRY(hipMemcpyAsync(got, flag, ((size_t)buckets + 3) * 4, hipMemcpyDeviceToHost, s));
     MXT_TRY(hipStreamSynchronize(s));
-    if (got & 1) {
+    if (got[0] & kBucketsBad) {
         mx::set_error("mx_transpose_device: index out of range");
         return MX_ERR_ARG;
     }
-    *done = got == 0;
     *checked = true;
+    *done = !(got[0] & kBucketsRefused);
+    if (!(got[0] & kBucketsCrowded) || !*done) return MX_OK;
+    const int *from = got + 2;
+    int most = 0;
+    for (int k = 0; k < buckets; ++k) most = std::max(most, from[k + 1] - from[k]);
+    const size_t lineCountB = al((size_t)((most - 1) / kTile + 1) * B.lines * 4);
+    Scratch crowd;
+    MXT_TRY(mx::dev_malloc(&crowd.p, lineCountB + al((size_t)(2 * kDigits + 2) * 4)));
+    int *lineCount = (int *)crowd.p, *lineFirst = (int *)((unsigned char *)crowd.p + lineCountB), *lineTotal = lineFirst + kDigits + 1, *unused = lineTotal + kDigits;
+    for (int k = 0; k < buckets; ++k) {
+        const int p0 = from[k], n = from[k + 1] - p0, c0 = k * B.lines, lines = std::min(B.lines, inner - c0), lineTiles = (n - 1) / kTile + 1;
+        if (n <= got[1]) continue;
+        const Word *here = moved + p0;
+        hipLaunchKernelGGL(line_counts_kernel<V>, tile_blocks(lineTiles), dim3(kThreads), 0, s, here, n, lines, lineTiles, lineCount);
+        hipLaunchKernelGGL(bucket_offsets_kernel, dim3((unsigned)((lines + 15) / 16)), dim3(1024), 0, s, lineCount, lines, lineTiles, lineTotal);
+        hipLaunchKernelGGL(bucket_starts_kernel<false>, dim3(1), dim3(kThreads), 0, s, (const int *)lineTotal, lines, BucketBound{}, (const int *)nullptr, 0, lineFirst, unused);
+        hipLaunchKernelGGL(line_entries_kernel<V>, tile_blocks(lineTiles), dim3(kThreads), 0, s, here, n, lines, B.lineBits, lineTiles, (const int *)lineCount,
+                           (const int *)lineFirst, p0, tPtr + c0, tInd + p0, tVal + p0);
+    }
+    MXT_TRY(hipGetLastError());
+    MXT_TRY(hipStreamSynchronize(s));
     return MX_OK;
 }
 

@@ -46,17 +46,25 @@ def test_transpose_of_crowded_lines(mx, share):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float16])
-@pytest.mark.parametrize("inner,nnz,crowd", [
-    (40, 1023, 0), (40, 1024, 0),                              # from 1024 entries on by buckets
-    (1, 36000, 0), (1, 36001, 0), (3, 216003, 0), (3, 216006, 0),  # some bucket has 36000 (66000) of them, one more
-    (5000, 60000, 39990), (5000, 60000, 40050),                # one line with about as many as a bucket may have
-    (100003, 3000000, 134000), (100003, 3000000, 136500),
+@pytest.mark.parametrize("inner,nnz,crowds", [
+    (40, 1023, []), (40, 1024, []),                               # from 1024 entries on by buckets
+    (1, 24576, []), (1, 24577, []), (1, 90000, []),               # one bucket of one line: as many as its workgroup takes, one more
+    (64, 700000, [(0, 24576)]), (64, 700000, [(0, 24577)]), (64, 700000, [(63, 40961)]),  # a line to a bucket; the first and the last of them
+    (40000, 1000000, [(0, 50000)]), (40000, 1000000, [(39999, 50000), (39998, 9), (0, 26000), (1, 40000)]),  # several lines of a bucket
+    (4000, 500000, [(500 * k, 25000) for k in range(8)]), (4000, 500000, [(440 * k, 25000) for k in range(9)]),  # eight crowded buckets, nine
+    (4000, 1200000, [(440 * k, 110000) for k in range(9)]),       # nine that are too many for one workgroup each: the radix sort
+    (10, 3000000, []),                                            # ... without counting
 ])
-def test_transpose_by_the_rule_for_buckets(mx, dtype, inner, nnz, crowd):
-    rng = np.random.default_rng(inner + nnz + crowd)
+def test_transpose_of_crowded_buckets(mx, dtype, inner, nnz, crowds):
+    """crowds: (line, entries)"""
+    rng = np.random.default_rng(inner + nnz + len(crowds))
     ptr, val = _matrix(rng, 700, nnz, dtype)
-    ind = rng.integers(0, inner, nnz)
-    ind[rng.permutation(nnz)[:crowd]] = inner // 3
+    ind, places, at = np.empty(nnz, int), rng.permutation(nnz), 0
+    for line, n in crowds:
+        ind[places[at:at + n]] = line
+        at += n
+    named = {line for line, _ in crowds} if inner < 100 else set()  # (a crowd of exactly so many)
+    ind[places[at:]] = rng.choice([c for c in range(inner) if c not in named], nnz - at)
     _check(mx, ptr, ind, val, inner)
 
 
