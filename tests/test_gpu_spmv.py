@@ -21,6 +21,13 @@ def oracle_y(ora, mx, A, x):
     return ora.spmv_f16_f32acc(A.val, A.rowPtr, A.colInd, x)[0]
 
 
+def host_plan(mx, monkeypatch, part, flags=0):
+    """The plan with its CSR part decided on and laid out by the host (a part of a million entries or more takes the device's route otherwise)."""
+    with monkeypatch.context() as m:
+        m.setenv("MX_LAYOUT", "host")
+        return mx.Plan(part, flags)
+
+
 def test_mfma_operand_layout_f64(mx):
     """v_mfma_f64_16x16x4_f64: A[i][k] in lane 16k+i, B[k][j] in lane 16k+j, D[i][j] in
     accumulator register i//4 of lane 16*(i%4)+j -- the mapping tile_kernel<double> relies on."""
@@ -250,7 +257,7 @@ def test_full_size_workloads_match_oracle(mx, ora, cfg, taus):
             part.close()
 
 
-def test_full_size_mixed_workload_with_its_strips(mx, ora):
+def test_full_size_mixed_workload_with_its_strips(mx, ora, monkeypatch):
     """Workload 5 at the point the benchmark picks, tau = (1, 1): the 20 % strip rows run through
     the strip form of the binary16 tile kernel (26.8 M entries), everything else through the CSR
     part; y against the oracle."""
@@ -277,6 +284,12 @@ def test_full_size_mixed_workload_with_its_strips(mx, ora):
     torch.cuda.synchronize()
     assert torch.equal(y, yd)
     dplan.close()
+    # ... and as the host makes all of it
+    hplan = host_plan(mx, monkeypatch, part)
+    for k in ("csr_variant", "csr_nnz", "csr_blocks", "tile_nnz", "tile_chunks", "tile_frags", "tile_variant", "tile_strip_nnz"):
+        assert hplan.info[k] == info[k], (k, hplan.info[k], info[k])
+    assert torch.equal(hplan.spmv(xd), y)
+    hplan.close()
     plan.close()
     part.close()
 
@@ -1159,8 +1172,9 @@ def test_entries_kept_in_the_caches_or_streamed(mx, ora, monkeypatch):
         # ... and the plan made from device arrays decides as the one made from the host's
         D = mx.Plan.from_device_csr(torch.from_numpy(A.rowPtr).cuda(), torch.from_numpy(A.colInd).cuda(), torch.from_numpy(A.val).cuda(),
                                     A.cols, flags)
-        assert D.info["csr_keep"] == kept and D.info["csr_fused"] == d.info["csr_fused"]
-        for pl in (d, k, t, e, D):
+        H = host_plan(mx, monkeypatch, P, flags)
+        assert D.info["csr_keep"] == H.info["csr_keep"] == kept and D.info["csr_fused"] == H.info["csr_fused"] == d.info["csr_fused"]
+        for pl in (d, k, t, e, D, H):
             pl.close()
         P.close()
 
@@ -1671,11 +1685,11 @@ def test_slice_layout_by_the_device_route_is_the_same_layout(mx, monkeypatch):
 
 
 @pytest.mark.gpu
-def test_plan_from_a_matrix_in_device_memory(mx, ora):
+def test_plan_from_a_matrix_in_device_memory(mx, ora, monkeypatch):
     """mx_plan_create_device_csr: the plan made from device arrays alone is the plan mx_plan_create
     makes from the host matrix -- same form, same estimates behind the choice, same value
     dictionary, and a y that is equal bit for bit -- in both forms and both precisions, on rows in
-    any order; a bad index is refused before it is used."""
+    any order, whether the host decides and lays it out or sends it up; a bad index is refused before it is used."""
     import torch
     rng = np.random.default_rng(5)
     cases = [mx.gen_config(c, scale=sc)[0] for c, sc in ((1, 1.0), (2, 1.0), (2, 1 / 8), (3, 0.1), (4, 0.25), (5, 0.1))]
@@ -1691,17 +1705,18 @@ def test_plan_from_a_matrix_in_device_memory(mx, ora):
         part = mx.Partition(A, 0.0, 0.0)
         for flags in (mx.MX_PLAN_DEFAULT, mx.MX_PLAN_CSR_ROWS, mx.MX_PLAN_CSR_SLICES):
             print("device csr plan: case %d rows=%d nnz=%d flags=%d" % (i, A.rows, A.nnz, flags), flush=True)
-            H = mx.Plan(part, flags)
             D = mx.Plan.from_device_csr(rp, ci, va, A.cols, flags)
-            for k in ("csr_variant", "csr_value_dict", "csr_nnz", "csr_blocks", "tile_nnz", "csr_fused"):
-                assert H.info[k] == D.info[k], (i, flags, k, H.info[k], D.info[k])
-            if flags == mx.MX_PLAN_DEFAULT and H.info["est_rows_us"] > 0:
-                assert abs(H.info["est_rows_us"] - D.info["est_rows_us"]) < 1e-9 and abs(H.info["est_slices_us"] - D.info["est_slices_us"]) < 1e-9
-            yh, yd = H.spmv(xd).cpu().numpy(), D.spmv(xd).cpu().numpy()
-            assert np.array_equal(yh.view(np.uint8), yd.view(np.uint8)), (i, flags)
+            yd = D.spmv(xd).cpu().numpy()
             assert rel_l2(yd, ref) <= (F64_TOL if A.dtype == mx.MX_F64 else F16_TOL)
+            for H in (host_plan(mx, monkeypatch, part, flags), mx.Plan(part, flags)):
+                for k in ("csr_variant", "csr_value_dict", "csr_nnz", "csr_blocks", "tile_nnz", "csr_fused"):
+                    assert H.info[k] == D.info[k], (i, flags, k, H.info[k], D.info[k])
+                if flags == mx.MX_PLAN_DEFAULT and H.info["est_rows_us"] > 0:
+                    assert abs(H.info["est_rows_us"] - D.info["est_rows_us"]) < 1e-9 and abs(H.info["est_slices_us"] - D.info["est_slices_us"]) < 1e-9
+                yh = H.spmv(xd).cpu().numpy()
+                assert np.array_equal(yh.view(np.uint8), yd.view(np.uint8)), (i, flags)
+                H.close()
             seen.add((D.info["csr_variant"], D.info["csr_value_dict"] > 0))
-            H.close()
             D.close()
         part.close()
     assert {(0, False), (1, False), (1, True), (0, True)} <= seen, seen
@@ -1756,11 +1771,12 @@ def _strip_matrix(mx, rng, rows, cols, dtype=np.float16):
 
 
 @pytest.mark.gpu
-def test_hybrid_plan_made_on_the_device(mx, ora):
+def test_hybrid_plan_made_on_the_device(mx, ora, monkeypatch):
     """mx_plan_create_device: extraction, decisions and layouts made on the device from a matrix
     in device memory give the plan mx_plan_create makes from mx_partition_create of the same
     matrix -- every counted fact, every array of the layouts byte for byte, y bit for bit --
-    whether the plan keeps strips, general tiles, binary64 blocks or nothing."""
+    whether the plan keeps strips, general tiles, binary64 blocks or nothing, and whether the host lays its CSR part out
+    or sends it up."""
     import torch
     rng = np.random.default_rng(12)
     cases = []
@@ -1780,31 +1796,35 @@ def test_hybrid_plan_made_on_the_device(mx, ora):
         for flags in (mx.MX_PLAN_DEFAULT, mx.MX_PLAN_KEEP_TILES, mx.MX_PLAN_NO_TILES, mx.MX_PLAN_CSR_ROWS, mx.MX_PLAN_ALL_TILES,
                       mx.MX_PLAN_ALL_TILES | mx.MX_PLAN_CSR_ROWS):
             print("device hybrid plan: %s tau=(%g, %g) flags=%d rows=%d nnz=%d" % (name, tc, tr, flags, A.rows, A.nnz), flush=True)
-            H = mx.Plan(part, flags)
             D = mx.Plan.from_device(rp, ci, va, A.cols, tc, tr, flags)
             routes.add(D.info["prep_route"])
-            for k in ("csr_variant", "csr_value_dict", "csr_nnz", "csr_blocks", "tile_nnz", "tile_chunks", "tile_frags", "tile_variant",
-                      "tile_strip_nnz"):
-                assert H.info[k] == D.info[k], (name, tc, tr, flags, k, H.info[k], D.info[k])
-            assert abs(H.info["est_rows_us"] - D.info["est_rows_us"]) < 1e-9 and abs(H.info["est_slices_us"] - D.info["est_slices_us"]) < 1e-9
-            ah, ad = H.arrays(), D.arrays()
-            assert sorted(ah) == sorted(ad), (name, flags, sorted(ah), sorted(ad))
-            for k in ah:
-                assert len(ah[k]) == len(ad[k]), (name, flags, k, len(ah[k]), len(ad[k]))
-                if ah[k] != ad[k]:
-                    a, b = np.frombuffer(ah[k], np.uint8), np.frombuffer(ad[k], np.uint8)
-                    at = int(np.flatnonzero(a != b)[0])
-                    raise AssertionError("%s tau=(%g, %g) flags=%d: %s differs from byte %d of %d" % (name, tc, tr, flags, k, at, a.size))
+            ad, yd = D.arrays(), D.spmv(xd).cpu().numpy()
+            assert rel_l2(yd, ref) <= (F64_TOL if A.dtype == mx.MX_F64 else F16_TOL)
+            plans = [host_plan(mx, monkeypatch, part, flags)]
+            if D.info["csr_nnz"] >= 1 << 20:
+                plans.append(mx.Plan(part, flags))  # (sends its CSR part up)
+            for H in plans:
+                for k in ("csr_variant", "csr_value_dict", "csr_nnz", "csr_blocks", "tile_nnz", "tile_chunks", "tile_frags", "tile_variant",
+                          "tile_strip_nnz"):
+                    assert H.info[k] == D.info[k], (name, tc, tr, flags, k, H.info[k], D.info[k])
+                assert abs(H.info["est_rows_us"] - D.info["est_rows_us"]) < 1e-9 and abs(H.info["est_slices_us"] - D.info["est_slices_us"]) < 1e-9
+                ah = H.arrays()
+                assert sorted(ah) == sorted(ad), (name, flags, sorted(ah), sorted(ad))
+                for k in ah:
+                    assert len(ah[k]) == len(ad[k]), (name, flags, k, len(ah[k]), len(ad[k]))
+                    if ah[k] != ad[k]:
+                        a, b = np.frombuffer(ah[k], np.uint8), np.frombuffer(ad[k], np.uint8)
+                        at = int(np.flatnonzero(a != b)[0])
+                        raise AssertionError("%s tau=(%g, %g) flags=%d: %s differs from byte %d of %d" % (name, tc, tr, flags, k, at, a.size))
+                yh = H.spmv(xd).cpu().numpy()
+                assert np.array_equal(yh.view(np.uint8), yd.view(np.uint8)), (name, flags)
+                H.close()
             if D.info["prep_route"] == 1 and D.info["tile_strip_nnz"] > 0:
                 strip_plans += 1
             if D.info["prep_route"] == 1 and D.info["tile_variant"] == 2:
                 block_plans += 1
             if D.info["prep_route"] == 1 and D.info["tile_nnz"] > D.info["tile_strip_nnz"]:
                 general_plans.add((A.dtype, D.info["tile_strip_nnz"] > 0))
-            yh, yd = H.spmv(xd).cpu().numpy(), D.spmv(xd).cpu().numpy()
-            assert np.array_equal(yh.view(np.uint8), yd.view(np.uint8)), (name, flags)
-            assert rel_l2(yd, ref) <= (F64_TOL if A.dtype == mx.MX_F64 else F16_TOL)
-            H.close()
             D.close()
         part.close()
     assert routes == {1}, routes
