@@ -464,7 +464,7 @@ int mx_estimate_tau(const mx_csr *A, int levels, float *tau_c, float *tau_r, mx_
 
 /* Making and destroying plans and partitions takes and gives back device memory by the hundred arrays; what was given
  * back is kept for the next call (at most 1/128 of a device's memory once a call has returned, and nothing for longer than 64 such
- * calls).  This gives all of it back to the device now.  No counterpart in the reference, which allocates and frees on every call
+ * calls); so are 16 MB of pinned host memory, through which large host arrays go up.  This gives all of it back now.  No counterpart in the reference, which allocates and frees on every call
  * (src/spmv_kernel/cdSpMV.cu:407-418). */
 void mx_release_memory(void);
 

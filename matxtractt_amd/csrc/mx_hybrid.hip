@@ -116,7 +116,8 @@ __global__ __launch_bounds__(kBlock) void iota_kernel(int *__restrict__ v, int n
 // named twice, a block that would reach past the end of x, more than eight blocks, or blocks less than
 // half full.
 // (The list is walked whole, by constant indexes: it stays in registers, where the search for a place in it put it in
-// private memory.  1.05 million rows, 15.8 million entries: 185 us, so 128.)
+// private memory.  1.05 million rows, 15.8 million entries: 185 us, so 128; 4.2 million rows, where neighbouring lanes' rows miss the caches: 1150 and 1194 with
+// the blocks stored, which spares candidate_keys_kernel 920.)
 constexpr int kNoBlock = 0x7fffffff;
 struct RowBlocks {
     int nb;
@@ -202,7 +203,7 @@ __global__ __launch_bounds__(kBlock) void strip_candidates_kernel(const int *__r
     rowKey[2 * (size_t)i + 1] = make_int4(block(4), block(5), block(6), block(7));
 }
 // candidates in row order: their row of A_dd, the first columns of their blocks (-1 = none, behind the others) and how many.
-// (A row's blocks are kept from when it was looked at: finding them again took 118 us for 1.05 million rows, reading them 6.)
+// (A row's blocks are kept from when it was looked at: finding them again took 118 us for 1.05 million rows, reading them 6; 4.2 million rows 937, 15.)
 __global__ __launch_bounds__(kBlock) void candidate_keys_kernel(const int *__restrict__ isCand, const int *__restrict__ candPos,
                                                                 const int4 *__restrict__ rowKey, int dRows, int *__restrict__ candRow,
                                                                 int4 *__restrict__ candKey, int *__restrict__ candNb)
