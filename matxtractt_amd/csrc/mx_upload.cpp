@@ -51,7 +51,8 @@ hipError_t mx::copy_up(void *dst, const void *src, size_t bytes)
         const unsigned char *from = (const unsigned char *)src + at;
         constexpr size_t piece = (size_t)256 << 10;
         const int pieces = (int)((n + piece - 1) / piece);
-#pragma omp parallel for schedule(static) num_threads(8)
+// (by as many threads as the host's other loops: a team of another size ends threads and starts them again, 0.15 ms of a plan that both are in)
+#pragma omp parallel for schedule(static)
         for (int k = 0; k < pieces; ++k) std::memcpy(to + k * piece, from + k * piece, std::min(piece, n - k * piece));
         e = hipMemcpyAsync((unsigned char *)dst + at, to, n, hipMemcpyHostToDevice, nullptr);
         if (e == hipSuccess) e = hipEventRecord(read[b], nullptr);
