@@ -1,4 +1,4 @@
-"""GPU tests of mx_transpose_device's two routes (buckets of output lines, radix sort) at the edges of their tiles."""
+"""GPU tests of mx_transpose_device's routes (buckets of output lines, crowded buckets, radix sort) at the edges of their tiles."""
 import numpy as np
 import pytest
 
@@ -35,9 +35,9 @@ def test_transpose_at_the_edges(mx, dtype, outer, inner, nnz):
     _check(mx, ptr, rng.integers(0, inner, nnz), val, inner)
 
 
-@pytest.mark.parametrize("share", [0.02, 0.07, 0.5, 1.0])
+@pytest.mark.parametrize("share", [0.005, 0.015, 0.02, 0.07, 0.5, 1.0])
 def test_transpose_of_crowded_lines(mx, share):
-    """Many entries in one line: a bucket of several rounds (2 and 7 %), one that would keep a workgroup too long (the radix sort)."""
+    """Many entries in one line: a bucket of two and of three rounds (0.5 and 1.5 %), one that its tiles' own workgroups put in order."""
     rng = np.random.default_rng(5)
     outer, inner, nnz = 30000, 40000, 1000000
     ptr, val = _matrix(rng, outer, nnz, np.float64)
@@ -56,7 +56,7 @@ def test_transpose_of_crowded_lines(mx, share):
     (10, 3000000, []),                                            # ... without counting
 ])
 def test_transpose_of_crowded_buckets(mx, dtype, inner, nnz, crowds):
-    """crowds: (line, entries)"""
+    """Buckets by their own workgroup, by workgroups for their tiles, and the radix sort, on both sides of the lines between them.  crowds: (line, entries)"""
     rng = np.random.default_rng(inner + nnz + len(crowds))
     ptr, val = _matrix(rng, 700, nnz, dtype)
     ind, places, at = np.empty(nnz, int), rng.permutation(nnz), 0
